@@ -1,4 +1,6 @@
-"""Shared host side of the two attention entry points: buffer allocation and the C-ABI call."""
+"""What the two attention entry points keep for the backward, and their forward and backward as plain functions: buffers
+allocated here, the C ABI called through ctypes, thresholds and tile mask returned.  (``adasplash`` and its kin run the same
+calls natively, ``csrc/torch_binding.cpp``.)"""
 
 import torch
 
@@ -43,6 +45,11 @@ def get_keep_supports():
         env = os.environ.get("ADSP_KEEP_SUPPORTS", "auto").lower()
         _keep_mode = {"0": "never", "1": "always"}.get(env, env if env in _KEEP_MODES else "auto")
     return _keep_mode
+
+
+def keep_code():
+    """The mode as the native host path takes it: an index into ("never", "always", "auto")."""
+    return {"never": 0, "always": 1, "auto": 2}[_keep_mode or get_keep_supports()]
 
 
 def _keeps(sup_bytes, q):

@@ -1,4 +1,5 @@
-"""ctypes binding of ``libadasplash_hip.so`` (the C ABI in ``include/adasplash_hip.h``).
+"""ctypes binding of ``libadasplash_hip.so`` (the C ABI in ``include/adasplash_hip.h``), and the loader of the native host
+path (``csrc/torch_binding.cpp``) that the public entry points go through.
 
 There is no CPU or eager fallback: if the library has not been built, or a tensor is not on a
 ROCm device, the call fails.
@@ -11,6 +12,7 @@ from pathlib import Path
 import torch
 
 _LIB_PATH = Path(__file__).resolve().parent / "lib" / "libadasplash_hip.so"
+BINDING_PATH = _LIB_PATH.with_name("_adsp_torch.so")
 _lib = None
 
 ADSP_F32, ADSP_BF16, ADSP_F16 = 0, 1, 2
@@ -67,6 +69,31 @@ def load():
         _check_build_id(lib)
         _lib = lib
     return _lib
+
+
+_module = None
+
+
+def native():
+    """The native host path of the public entry points (``lib/_adsp_torch.so``), loaded once."""
+    global _module
+    if _module is None:
+        import importlib.machinery
+        import importlib.util
+
+        from . import build as _build
+
+        load()  # (the C library first: the module is linked to it, and its build id is checked here)
+        if not BINDING_PATH.exists():
+            raise RuntimeError(f"{BINDING_PATH} not found: build it with `python -m adasplash_amd.build`.")
+        loader = importlib.machinery.ExtensionFileLoader("_adsp_torch", str(BINDING_PATH))
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_adsp_torch", BINDING_PATH, loader=loader))
+        loader.exec_module(mod)
+        if _build.BINDING_SRC.exists() and mod.build_id != _build.binding_id():
+            raise RuntimeError(f"{BINDING_PATH} is stale: it was built from other sources or for another torch. "
+                               "Rebuild with `python -m adasplash_amd.build`.")
+        _module = mod
+    return _module
 
 
 def build_id() -> str:

@@ -2,51 +2,13 @@
 
 Same call surface as the reference module of this name:
 ``sparse_attn(q, k, v, alpha=1.5, is_causal=False, varlen=None, niter=10)``
-(``adasplash/adasplash_block_mask.py:1213-1232``), same argument checks as its autograd wrapper
+(``adasplash/adasplash_block_mask.py:1213-1232``), same argument checks as the autograd wrapper there
 (``adasplash/adasplash_block_mask.py:922-960``).
 """
 
 import torch
 
-from . import _attention
-
-
-class _SparseAttentionV1(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, q, k, v, alpha=1.5, is_causal=False, varlen=None, niter=10):
-        B, N_H, N_CTX, H_DIM = q.shape
-        assert H_DIM in {16, 32, 64, 128, 256}
-        if varlen is None:
-            assert N_CTX.bit_count() == 1, "If varlen is not used, the context length must be a power of two."
-        else:
-            assert varlen.dim() == 1, "varlen must be a one-dimensional tensor."
-            assert varlen.shape[0] == B, f"varlen must have one entry per batch item (B={B})."
-        assert k.shape == q.shape and v.shape == q.shape, "q, k and v must share one shape (no GQA in v1)."
-        _attention.assert_contiguous(q, k, v, msg="Q, K and/or V are not contiguous.")
-        if varlen is not None and not varlen.is_contiguous():
-            varlen = varlen.contiguous()
-
-        # (when a gradient will be asked for, the forward keeps the supports it found: the backward then finds none again)
-        keep = any(ctx.needs_input_grad[:3])
-        res = _attention.launch_forward(
-            q, k, v, version=1, alpha=alpha, is_causal=is_causal, niter=niter, varlen=varlen,
-            keep_supports=keep,
-        )
-        out, taus, bmask = res[:3]
-        supports = res[3] if keep else None
-        ctx.save_for_backward(q, k, v, taus, bmask, supports)
-        ctx.alpha = alpha
-        ctx.is_causal = is_causal
-        ctx.varlen = varlen
-        return out
-
-    @staticmethod
-    def backward(ctx, do):
-        q, k, v, taus, bmask, supports = ctx.saved_tensors
-        dq, dk, dv = _attention.launch_backward(
-            q, k, v, do, taus, bmask, alpha=ctx.alpha, is_causal=ctx.is_causal, varlen=ctx.varlen, supports=supports
-        )
-        return dq, dk, dv, None, None, None, None
+from . import _attention, _lib
 
 
 def sparse_attn(q, k, v, alpha=1.5, is_causal=False, varlen=None, niter=10):
@@ -56,7 +18,8 @@ def sparse_attn(q, k, v, alpha=1.5, is_causal=False, varlen=None, niter=10):
     ``(batch,)`` valid lengths (right padding), padded output rows are zero; ``niter``: Halley /
     bisection passes of the threshold solver.
     """
-    return _SparseAttentionV1.apply(q, k, v, alpha, is_causal, varlen, niter)
+    # (checks, buffers, launches and autograd: csrc/torch_binding.cpp)
+    return _lib.native().attention(q, k, v, 1, alpha, is_causal, niter, varlen, _attention.keep_code())
 
 
 def tile_sparsity(q, k, v, alpha=1.5, is_causal=False, varlen=None, niter=10):

@@ -10,6 +10,8 @@ linked into ``adasplash_amd/lib/libadasplash_hip.so`` (the C ABI declared in ``i
   profiling builds).  ``source_id(extra)`` recomputes the id from the tree for the library's own extra flags, and the
   loader and the tests compare the two, so a library that is older than the sources next to it is an error instead
   of a silent stale binary, whatever the environment of the process that loads it.
+* ``lib/_adsp_torch.so``, the native host path of the Python entry points, is compiled with g++ against the installed torch
+  and linked to the library; it carries an id of its own (``binding_id()``).
 * The link step always runs, and the library is replaced atomically after a successful link only.
 """
 
@@ -27,6 +29,8 @@ INCLUDE = PKG.parent / "include"
 LIB_DIR = PKG / "lib"
 LIB_PATH = LIB_DIR / "libadasplash_hip.so"
 OBJ_DIR = PKG / "build"
+BINDING_SRC = CSRC / "torch_binding.cpp"
+BINDING_PATH = LIB_DIR / "_adsp_torch.so"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -123,6 +127,43 @@ def _compile(unit, build_id: str, force: bool):
     return obj, True
 
 
+def _binding_cmd():
+    """The command that builds the native host path (a Python module against torch's C++ API), without id and output."""
+    import sysconfig
+
+    import torch
+
+    inc = Path(torch.__file__).resolve().parent / "include"
+    libs = Path(torch.__file__).resolve().parent / "lib"
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-I{inc}", f"-I{inc}/torch/csrc/api/include", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}",
+            str(BINDING_SRC), f"-L{libs}", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python", f"-L{LIB_DIR}",
+            "-ladasplash_hip", "-Wl,-rpath,$ORIGIN"]
+
+
+def binding_id() -> str:
+    """Hash of what the native host path is built from: its source, the C ABI's header and torch's version."""
+    import torch
+
+    return _digest([BINDING_SRC.read_bytes(), (INCLUDE / "adasplash_hip.h").read_bytes(), torch.__version__])[:16]
+
+
+def _build_binding(force: bool):
+    cmd, ident = _binding_cmd(), binding_id()
+    sig_file = OBJ_DIR / "torch_binding.sig"
+    sig = _digest([" ".join(cmd), ident])
+    if not force and BINDING_PATH.exists() and sig_file.exists() and sig_file.read_text() == sig:
+        return False
+    sig_file.unlink(missing_ok=True)
+    tmp = BINDING_PATH.with_suffix(".so.tmp")
+    res = subprocess.run(cmd + [f'-DADSP_BINDING_ID="{ident}"', "-o", str(tmp)], capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"the native host path did not compile:\n{res.stderr}")
+    os.replace(tmp, BINDING_PATH)
+    sig_file.write_text(sig)
+    return True
+
+
 def build(jobs: int = 8, verbose: bool = True, force: bool = False) -> Path:
     """Compile what changed (everything with ``force``), link, and return the path of the shared library."""
     OBJ_DIR.mkdir(exist_ok=True)
@@ -145,6 +186,7 @@ def build(jobs: int = 8, verbose: bool = True, force: bool = False) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    _build_binding(force)
     if verbose:
         n = sum(1 for _, done in results if done)
         print(f"[adasplash_amd.build] compiled {n} of {len(objs)} objects, wrote {LIB_PATH}", flush=True)

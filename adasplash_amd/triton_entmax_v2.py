@@ -6,47 +6,16 @@ Same call surface as the reference module of this name (``adasplash/triton_entma
 Triton is involved.
 """
 
-import torch
-
 from . import _lib
 
 
-class _EntmaxRows(torch.autograd.Function):
-    """Counterpart of ``_entmax_triton`` (``adasplash/triton_entmax_v2.py:620-687``)."""
+class _EntmaxRows:
+    """Counterpart of ``_entmax_triton`` (``adasplash/triton_entmax_v2.py:620-687``): ``apply(x, alpha, n_iter, use_histogram,
+    fast_math)`` runs in the native host path (``csrc/torch_binding.cpp``), gradient included."""
 
     @staticmethod
-    def forward(ctx, x, alpha=1.5, n_iter=10, use_histogram=True, fast_math=False):
-        size_n = x.shape[-1]
-        assert x.is_contiguous(), "x must be contiguous"
-        _lib.require_device(x)
-        lib = _lib.load()
-        y = torch.empty_like(x)  # the kernel writes every element, zeros included
-        rows = x.numel() // size_n if size_n > 0 else 0
-        with _lib.device_guard(x.device):
-            st = lib.adsp_entmax_rows_fwd(x.data_ptr(), y.data_ptr(), rows, size_n, _lib.dtype_code(x), float(alpha),
-                                          int(n_iter), int(bool(use_histogram)), int(bool(fast_math)),
-                                          _lib.current_stream(x.device))
-        _lib.check(st, "adsp_entmax_rows_fwd")
-        ctx.save_for_backward(y)
-        ctx.alpha = alpha
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        (y,) = ctx.saved_tensors
-        size_n = y.shape[-1]
-        if not dy.is_contiguous():
-            dy = dy.contiguous()
-        if dy.dtype != y.dtype:
-            dy = dy.to(y.dtype)
-        dx = torch.empty_like(dy)
-        rows = y.numel() // size_n if size_n > 0 else 0
-        lib = _lib.load()
-        with _lib.device_guard(y.device):
-            st = lib.adsp_entmax_rows_bwd(y.data_ptr(), dy.data_ptr(), dx.data_ptr(), rows, size_n, _lib.dtype_code(y),
-                                          float(ctx.alpha), _lib.current_stream(y.device))
-        _lib.check(st, "adsp_entmax_rows_bwd")
-        return dx, None, None, None, None
+    def apply(x, alpha=1.5, n_iter=10, use_histogram=True, fast_math=False):
+        return _lib.native().entmax_rows(x, alpha, n_iter, use_histogram, fast_math)
 
 
 def triton_entmax(x, alpha=1.5, n_iter=2, use_histogram=True, fast_math=False):
