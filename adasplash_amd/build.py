@@ -57,6 +57,7 @@ def units(extra=None):
     attn_flags = ATTN_FLAGS + (EXTRA_ATTN_FLAGS if extra is None else list(extra))
     out = [("attn_api", "attn_api.hip", []), ("entmax_rows", "entmax_rows.hip", [])]
     for tag, ty in TYPES.items():
+        out.append((f"entmax_rows_{tag}", "entmax_rows_unit.hip", [f"-DADSP_T={ty}", f"-DADSP_TAG={tag}"]))
         for d in HEAD_DIMS:
             base = [f"-DADSP_T={ty}", f"-DADSP_TAG={tag}", f"-DADSP_D={d}"]
             for multi in (0, 1):

@@ -82,8 +82,7 @@ const char* adsp_status_string(int status);
 /*
  * Row-wise alpha-entmax over the last dimension: y[r, :] = [(alpha-1) x[r, :] - tau_r]_+^(1/(alpha-1)).
  *   x, y      : contiguous [rows, cols] arrays of `dtype`; y is fully overwritten (zeros included).
- *   alpha     : > 1.  n_iter : refinement steps after initialisation (>= 0).
- *   use_histogram : non-zero = histogram initialisation of tau (honoured for alpha in {1.5, 2}).
+ *   alpha     : > 1.  n_iter (>= 0), use_histogram, fast_math: accepted; the solver runs to convergence whatever they say.
  *   fast_math : accepted for signature parity; the generic-alpha power always uses exp2/log2.
  * Replaces the launch at adasplash/triton_entmax_v2.py:650-658.
  */

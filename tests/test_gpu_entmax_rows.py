@@ -215,3 +215,31 @@ def test_forward_across_the_dispatch_boundaries(cols, alpha, dtype):
     flat = torch.zeros(5, cols).to(dtype)
     y = A.triton_entmax(flat.to(DEV), alpha=alpha)
     assert (y.float().cpu() - 1.0 / cols).abs().max().item() < (1e-6 if dtype == torch.float32 else 2e-3 / cols + 1e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("alpha", ALPHAS)
+@pytest.mark.parametrize("cols", [7, 14, 15, 16, 31, 129, 511, 2049, 4097, 8195, 16389, 32769, 65537])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_rows_that_start_and_end_off_a_16_byte_boundary(cols, alpha, dtype, offset):
+    """Odd row lengths around the borders of the dispatch (and the shortest the edge slots take), on buffers that start on a
+    16-byte boundary or one element behind one, forward and backward; the element behind the last row stays untouched.
+    Tolerances as in the tests above."""
+    from adasplash_amd import _lib
+    g = torch.Generator().manual_seed(cols + offset)
+    rows = 7
+    x0 = (3 * torch.randn(rows, cols, generator=g)).to(dtype)
+    dy0 = torch.randn(rows, cols, generator=g).to(dtype)
+    bufs = [torch.full((rows * cols + offset + 1,), 7.0, device=DEV, dtype=dtype) for _ in range(4)]
+    x, y, dy, dx = (b[offset:offset + rows * cols].view(rows, cols) for b in bufs)
+    x.copy_(x0)
+    dy.copy_(dy0)
+    lib, stream = _lib.load(), _lib.current_stream(x.device)
+    assert lib.adsp_entmax_rows_fwd(x.data_ptr(), y.data_ptr(), rows, cols, _lib.dtype_code(x), alpha, 2, 1, 0, stream) == 0
+    assert lib.adsp_entmax_rows_bwd(y.data_ptr(), dy.data_ptr(), dx.data_ptr(), rows, cols, _lib.dtype_code(x), alpha, stream) == 0
+    assert max_err(y, exact.entmax_rows(x0, alpha)) < tol_for(dtype, alpha)
+    want = _rows_backward_reference(y, dy0, alpha)
+    tol = (1e-5 if alpha in (1.5, 2.0) else 1e-4) if dtype == torch.float32 else 1e-2
+    assert (dx.double().cpu() - want).abs().max().item() < tol * max(1.0, want.abs().max().item())
+    for b in bufs:
+        assert float(b[-1]) == 7.0 and (offset == 0 or float(b[0]) == 7.0)
