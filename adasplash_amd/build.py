@@ -55,7 +55,8 @@ def units(extra=None):
     """(object stem, source file, extra flags) of every translation unit; ``extra``: flags added to the attention units
     (default: ``ADSP_ATTN_FLAGS`` of this process)."""
     attn_flags = ATTN_FLAGS + (EXTRA_ATTN_FLAGS if extra is None else list(extra))
-    out = [("attn_api", "attn_api.hip", []), ("entmax_rows", "entmax_rows.hip", [])]
+    out = [("attn_api", "attn_api.hip", []), ("entmax_rows", "entmax_rows.hip", []),
+           ("attn_decode", "attn_decode.hip", [])]
     for tag, ty in TYPES.items():
         out.append((f"entmax_rows_{tag}", "entmax_rows_unit.hip", [f"-DADSP_T={ty}", f"-DADSP_TAG={tag}"]))
         for d in HEAD_DIMS:

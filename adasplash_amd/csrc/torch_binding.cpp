@@ -246,6 +246,40 @@ void check_attention(const Tensor& q, const Tensor& k, const Tensor& v, AttnCall
           "varlen must be int32/int64; got ", c.varlen.defined() ? c.varlen.scalar_type() : at::kInt, ".");
 }
 
+// ---- a few queries against a cache of keys --------------------------------------------------------------------------
+// Undefined where adsp_attn_decode_fwd does not take the call: a gradient is asked for, many queries, other head dims or types, an
+// inner stride.
+Tensor decode_forward(const Tensor& q, const Tensor& k, const Tensor& v, double alpha, const Tensor& varlen, bool causal, bool left,
+                      const Tensor& slopes) {
+  const int64_t B = q.size(0), H = q.size(1), q_len = q.size(2), D = q.size(3), k_len = k.size(2);
+  const auto t = q.scalar_type();
+  if (!q.is_cuda() || !k.is_cuda() || !v.is_cuda() || k.device() != q.device() || v.device() != q.device()) return Tensor();
+  if ((t != at::kFloat && t != at::kBFloat16 && t != at::kHalf) || k.scalar_type() != t || v.scalar_type() != t) return Tensor();
+  if (q_len < 1 || q_len > 16 || (D != 32 && D != 64 && D != 128 && D != 256) || k_len < 1 || k_len > (1 << 24)) return Tensor();
+  if (B < 1 || H < 1 || B * H > 65535 || !(alpha > 1.0)) return Tensor();
+  if (varlen.defined() && (q_len == k_len || (varlen.scalar_type() != at::kInt && varlen.scalar_type() != at::kLong))) return Tensor();
+  const int64_t per16 = 16 / q.element_size();
+  for (const Tensor* x : {&k, &v}) {
+    if (x->stride(3) != 1 || x->stride(0) % per16 || x->stride(1) % per16 || x->stride(2) % per16 || (uintptr_t)x->data_ptr() % 16)
+      return Tensor();
+  }
+  const c10::DeviceGuard guard(q.device());
+  Tensor qc = q.contiguous();
+  if ((uintptr_t)qc.data_ptr() % 16) qc = qc.clone();
+  Tensor vl = varlen, sl = slopes;
+  if (vl.defined()) vl = vl.to(q.device()).contiguous();
+  if (sl.defined()) sl = sl.to(q.device(), at::kFloat).contiguous();
+  Tensor out = at::empty(q.sizes(), v.options());
+  const size_t ws_bytes = adsp_attn_decode_workspace_bytes((int)B, (int)H, (int)q_len, (int)k_len);
+  Tensor ws = bytes(ws_bytes, q);
+  check(adsp_attn_decode_fwd(qc.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), data(vl),
+                             !vl.defined() ? 0 : (vl.scalar_type() == at::kLong ? 64 : 32), left, (const float*)data(sl), (int)B, (int)H,
+                             (int)q_len, (int)k_len, (int)D, k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2),
+                             dtype_code(q), alpha, causal, ws.data_ptr(), ws_bytes, stream_of(q)),
+        "adsp_attn_decode_fwd");
+  return out;
+}
+
 bool wants_grad(const Tensor& t) { return t.requires_grad(); }
 
 // ---- Python side ----------------------------------------------------------------------------------------------------
@@ -317,9 +351,32 @@ PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// decode_attention(q, k, v, alpha, varlen, is_causal, left_padding, slopes) -> tensor, or None where the kernels do not take the call
+PyObject* py_decode_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  expect_args(n, 8);
+  const Tensor &q = tensor_arg(a[0], "q"), &k = tensor_arg(a[1], "k"), &v = tensor_arg(a[2], "v");
+  const double alpha = double_arg(a[3]);
+  Tensor varlen, slopes;
+  if (a[4] != Py_None) varlen = tensor_arg(a[4], "varlen");
+  const bool causal = bool_arg(a[5]), left = bool_arg(a[6]);
+  if (a[7] != Py_None) slopes = tensor_arg(a[7], "alibi_slopes");
+  if (at::GradMode::is_enabled() && (wants_grad(q) || wants_grad(k) || wants_grad(v) || (slopes.defined() && wants_grad(slopes))))
+    Py_RETURN_NONE;
+  Tensor out;
+  {
+    pybind11::gil_scoped_release no_gil;
+    out = decode_forward(q, k, v, alpha, varlen, causal, left, slopes);
+  }
+  if (!out.defined()) Py_RETURN_NONE;
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
     {"entmax_rows", (PyCFunction)(void (*)(void))py_entmax_rows, METH_FASTCALL, "alpha-entmax of the last dimension, with autograd"},
     {"attention", (PyCFunction)(void (*)(void))py_attention, METH_FASTCALL, "sparse entmax attention, with autograd"},
+    {"decode_attention", (PyCFunction)(void (*)(void))py_decode_attention, METH_FASTCALL, "a few queries against a cache of keys"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_adsp_torch", nullptr, -1, methods};
 }  // namespace

@@ -83,7 +83,6 @@ const char* adsp_status_string(int status);
  * Row-wise alpha-entmax over the last dimension: y[r, :] = [(alpha-1) x[r, :] - tau_r]_+^(1/(alpha-1)).
  *   x, y      : contiguous [rows, cols] arrays of `dtype`; y is fully overwritten (zeros included).
  *   alpha     : > 1.  n_iter (>= 0), use_histogram, fast_math: accepted; the solver runs to convergence whatever they say.
- *   fast_math : accepted for signature parity; the generic-alpha power always uses exp2/log2.
  * Replaces the launch at adasplash/triton_entmax_v2.py:650-658.
  */
 int adsp_entmax_rows_fwd(const void* x, void* y, int64_t rows, int64_t cols, int dtype, double alpha,
@@ -219,6 +218,23 @@ int adsp_attn_bwd(const void* q, const void* k, const void* v, const void* dout,
                   const int32_t* bmask, const void* varlen, int varlen_bits, void* dq, void* dk, void* dv,
                   float* delta, float* zinv, int B, int Hq, int Hkv, int N, int D, int dtype, double alpha,
                   int is_causal, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * Entmax attention of a few queries against a cache of keys (a decoding step): entmax_alpha(q k^T / sqrt(D) + bias) v.
+ *   q, out    : contiguous [B, H, q_len, D], q_len <= 16; k, v: [B, H, k_len, D] with unit stride along D and the strides given
+ *               (in elements; multiples of 16 bytes), D in {32, 64, 128, 256}; base pointers 16-byte aligned.
+ *   varlen    : NULL, or [B] valid key counts (varlen_bits 32 or 64): the first ones of a sequence, or with left_padding the last.
+ *   alibi_slopes : NULL, or [H] fp32: adds slope * (key position - query position) to the scores.
+ *   is_causal : the queries are the last q_len positions of k_len.
+ *   workspace : adsp_attn_decode_workspace_bytes() bytes (the scores in fp32).
+ * A query that sees no key gets a row of zeros.  Replaces the dense path of examples/attention.py:34-91 for such calls.
+ */
+size_t adsp_attn_decode_workspace_bytes(int B, int H, int q_len, int k_len);
+int adsp_attn_decode_fwd(const void* q, const void* k, const void* v, void* out, const void* varlen, int varlen_bits,
+                         int left_padding, const float* alibi_slopes, int B, int H, int q_len, int k_len, int D,
+                         int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_b, int64_t v_stride_h,
+                         int64_t v_stride_n, int dtype, double alpha, int is_causal, void* workspace, size_t workspace_bytes,
+                         void* stream);
 
 #ifdef __cplusplus
 }

@@ -121,3 +121,34 @@ def test_flash_name_routes_to_the_fused_kernels():
     a = dense.flash_entmax_attention(q, k, v, niter=10)  # the default single step is good to ~1e-3 only
     b = dense.slow_entmax_attention(q, k, v, is_causal=True, niter=10)
     assert (a - b).abs().max().item() < 3e-4  # each side is within 1e-4 of the exact result
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 2e-2), (torch.float16, 2e-2)])
+@pytest.mark.parametrize("q_len,k_len,D,alpha,padding", [
+    (1, 1, 64, 1.5, "right"), (1, 63, 32, 1.5, "left"), (16, 257, 64, 1.5, "left"), (3, 300, 128, 1.333, "right"),
+    (2, 1500, 256, 2.0, "left"), (1, 1300, 64, 1.5, "right")])
+def test_decoding_kernels(q_len, k_len, D, alpha, padding, dtype, tol):
+    """Calls that csrc/attn_decode.hip serves: edges of its 64- and 256-key granules, every type and head dim, caches that are
+    views of larger buffers, lengths that leave whole granules out, a sequence without keys (zeros), flat scores whose
+    candidates overflow the list of 1024 (the last shape, with q scaled down).  Same oracle and tolerances as above."""
+    g = torch.Generator().manual_seed(k_len)
+    B, H = 3, 2
+    q = torch.randn(B, H, q_len, D, generator=g).to(dtype) * (0.01 if k_len == 1300 else 1.0)
+    big = [torch.randn(B, H, k_len + 8, D, generator=g).to(dtype) for _ in range(2)]
+    k, v = (t[:, :, :k_len] for t in big)
+    kd, vd = (t.to(DEV)[:, :, :k_len] for t in big)
+    slopes = torch.tensor([0.02, 0.001])
+    for varlen in (None, torch.tensor([k_len, max(1, k_len // 3), 1]) if q_len == 1 else torch.tensor([k_len, k_len // 2, q_len])):
+        kw = dict(alpha=alpha, is_causal=True, padding=padding, alibi_slopes=slopes)
+        if varlen is not None and q_len == k_len:
+            continue
+        if varlen is not None and padding == "right" and q_len > 1:
+            kw["is_causal"] = False  # (right padding leaves the last queries of a causal call without keys)
+        got = dense.slow_entmax_attention(q.to(DEV), kd, vd, niter=10, varlen=None if varlen is None else varlen.to(DEV),
+                                          **{n: x.to(DEV) if torch.is_tensor(x) else x for n, x in kw.items()})
+        want = exact.dense_entmax_attention_general(q, k, v, varlen=varlen, **kw)
+        assert got.shape == q.shape and got.dtype == dtype
+        assert (got.double().cpu() - want).abs().max().item() < tol
+    zero = dense.slow_entmax_attention(q.to(DEV), kd, vd, alpha=alpha, padding=padding,
+                                       varlen=torch.zeros(B, dtype=torch.int64, device=DEV)) if q_len != k_len else None
+    assert zero is None or (zero == 0).all()
