@@ -9,7 +9,7 @@
 //    support (z >= max - 1) go to a list in LDS, the threshold is solved on the list as in the rows kernels, and only the V rows
 //    of the support are read.
 // A step of 16 x 16 heads against caches of up to 4096 keys (D = 64, bf16, 84 MB of K in use): 265 us as fp32 copies of q and
-// K, a library product, ten elementwise launches, the rows kernel and a second product; measured now: see the host function.
+// K, a library product, ten elementwise launches, the rows kernel and a second product; 27 us now (20 us = 4.2 TB/s and 6.7 us).
 #include "entmax_rows_kernel.h"
 #include "../../include/adasplash_hip.h"
 #include <math.h>
@@ -125,10 +125,22 @@ template <typename T, int D, int AM> __global__ __launch_bounds__(256) void deco
   const int c0 = first >> 2, c1 = first < last ? (last + 3) >> 2 : c0;
   const f32x4* const z4 = reinterpret_cast<const f32x4*>(zrow);
   if (tid == 0) list_n = 0;
+  // eight loads of a thread under way together; a row of up to 8192 keys is then in registers for the second look as well
+  constexpr int kHold = 8;
+  f32x4 held[kHold];
+  const f32x4 none = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  auto load_held = [&](int from) {
+#pragma unroll
+    for (int i = 0; i < kHold; ++i) {
+      const int c = from + i * 256 + tid;
+      held[i] = c < c1 ? z4[c] : none;
+    }
+  };
   float m = -INFINITY;
-  for (int c = c0 + tid; c < c1; c += 256) {
-    const f32x4 z = z4[c];
-    m = fmaxf(m, fmaxf(fmaxf(z[0], z[1]), fmaxf(z[2], z[3])));
+  for (int from = c0; from < c1; from += kHold * 256) {
+    load_held(from);
+#pragma unroll
+    for (int i = 0; i < kHold; ++i) m = fmaxf(m, fmaxf(fmaxf(held[i][0], held[i][1]), fmaxf(held[i][2], held[i][3])));
   }
   m = row_max<256>(m, sm);
   float acc[kVec];
@@ -136,15 +148,19 @@ template <typename T, int D, int AM> __global__ __launch_bounds__(256) void deco
   for (int e = 0; e < kVec; ++e) acc[e] = 0.f;
   if (m > -INFINITY) {  // (a query that sees no key at all is a row of zeros)
     const float thr = m - 1.f;
-    for (int c = c0 + tid; c < c1; c += 256) {
-      const f32x4 z = z4[c];
+    for (int from = c0; from < c1; from += kHold * 256) {
+      if (c1 - c0 > kHold * 256) load_held(from);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (z[e] >= thr) {
-          const int at = atomicAdd(&list_n, 1);
-          if (at < kDecodeCap) {
-            list_z[at] = z[e];
-            list_key[at] = c * 4 + e;
+      for (int i = 0; i < kHold; ++i) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float z = held[i][e];
+          if (z >= thr) {
+            const int at = atomicAdd(&list_n, 1);
+            if (at < kDecodeCap) {
+              list_z[at] = z;
+              list_key[at] = (from + i * 256 + tid) * 4 + e;
+            }
           }
         }
       }
@@ -153,8 +169,8 @@ template <typename T, int D, int AM> __global__ __launch_bounds__(256) void deco
     const int n = list_n;
     const int grp = tid / kLanes, col = tid % kLanes;
     const char* const vbase = (const char*)p.v + ((size_t)(b * p.v_sb + h * p.v_sh) + col * kVec) * elem_traits<T>::kBytes;
-    auto add_row = [&](float w, int key) {
-      const u32x4 raw = *reinterpret_cast<const u32x4*>(vbase + key * p.v_sn * elem_traits<T>::kBytes);
+    auto row_of = [&](int key) { return *reinterpret_cast<const u32x4*>(vbase + key * p.v_sn * elem_traits<T>::kBytes); };
+    auto add_row = [&](float w, u32x4 raw) {
 #pragma unroll
       for (int e = 0; e < kVec; ++e) acc[e] = fmaf(w, chunk_elem<T>(raw, e), acc[e]);
     };
@@ -169,10 +185,40 @@ template <typename T, int D, int AM> __global__ __launch_bounds__(256) void deco
         lr.load(list_z, n, lane);
         tau = solve_row<AM, 64>(lr, m, p.rows, sm);
       }
-#pragma unroll 4
-      for (int i = grp; i < n; i += kGroups) {
-        const float w = prob<AM>(list_z[i] - tau, p.rows.c0);
-        if (w > 0.f) add_row(w, list_key[i]);
+      // the support, in the list's place: every entry is in a register before the first is written back
+      float w[kDecodeCap / 256];
+      int key[kDecodeCap / 256];
+#pragma unroll
+      for (int c = 0; c < kDecodeCap / 256; ++c) {
+        const int i = c * 256 + tid;
+        w[c] = i < n ? prob<AM>(list_z[i] - tau, p.rows.c0) : 0.f;
+        key[c] = i < n ? list_key[i] : 0;
+      }
+      __syncthreads();
+      if (tid == 0) list_n = 0;
+      __syncthreads();
+#pragma unroll
+      for (int c = 0; c < kDecodeCap / 256; ++c) {
+        if (w[c] > 0.f) {
+          const int at = atomicAdd(&list_n, 1);
+          list_z[at] = w[c];
+          list_key[at] = key[c];
+        }
+      }
+      __syncthreads();
+      const int members = list_n;
+      // four rows of a group under way together; a slot past the end takes the first member's row with weight zero
+      for (int i = grp; i < members; i += 4 * kGroups) {
+        u32x4 raw[4];
+        float wt[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int at = i + u * kGroups;
+          wt[u] = at < members ? list_z[at] : 0.f;
+          raw[u] = row_of(list_key[at < members ? at : 0]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) add_row(wt[u], raw[u]);
       }
     } else {
       // a flat row: more candidates than the list holds; solved on the scores in memory, and every key is looked at
@@ -181,7 +227,7 @@ template <typename T, int D, int AM> __global__ __launch_bounds__(256) void deco
 #pragma unroll 4
       for (int key = first + grp; key < last; key += kGroups) {
         const float w = prob<AM>(zrow[key] - tau, p.rows.c0);
-        if (w > 0.f) add_row(w, key);
+        if (w > 0.f) add_row(w, row_of(key));
       }
     }
   }
