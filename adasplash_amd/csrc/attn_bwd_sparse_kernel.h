@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
   static_assert(AM == ATT_15 || AM == ATT_2 || AM == ATT_GEN, "alpha = 1.5, 2 or any other in (1, 2)");
   constexpr int NW = SG::kNW, BM = SG::kBM;
   __shared__ __align__(1024) unsigned char lds_all[SG::kLds];
-  __shared__ int s_item, s_skip;
+  __shared__ int s_item, s_skip, s_draw;
   // a lane ran out of event slots, or a wave out of list room.  Two words: the walks write the one of the tile's
   // parity and read the other one behind the next barrier, so no wave can read a word another one is still setting
   __shared__ uint32_t s_giveup[2];
@@ -116,8 +116,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
   const int N = p.N;
   const int n_mblk = (N + BM - 1) / BM;
   const int group = p.Hq / p.Hkv;
-  const long long total = (long long)p.B * p.Hkv * n_mblk * group;
-  const long long per_xcd = (total + 7) / 8;
+  const int total = p.B * p.Hkv * n_mblk * group;  // (below 2^31, see the dispatch)
+  const int per_xcd = (total + 7) / 8;
   const float qs = p.qscale, inv_qs = 1.f / p.qscale;
   constexpr int kKPer = (G::kKLoads + NW - 1) / NW;
   constexpr bool kKStep = (NW * 64 / KS::kC) % 16 == 0 && (NW * 64) % KS::kC == 0;
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
     if (blockIdx.x == 0 && threadIdx.x == 0) p.queue[kCtrlAllDense] = 1u;
     return;
   }
-  int queues_tried = 0;  // thread 0: how many of the eight counters were found empty
+  if (threadIdx.x == 0) s_draw = 0;
   for (;;) {
     // The lane's constants are formed anew for every row block (the empty asm hides that they repeat): hoisted out
     // of this loop they would stay live through both walks, and the walks have no registers to spare.
@@ -141,17 +141,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
 
     __syncthreads();  // the previous row block is done with LDS and with s_item
     if (tid == 0) {
-      int got = -1;
-      while (queues_tried < 8) {
-        const int x = ((int)(blockIdx.x & 7) + queues_tried) & 7;
-        const long long i = (long long)atomicAdd(&p.queue[x], 1u);
-        const long long logical = (long long)x * per_xcd + i;
-        if (i < per_xcd && logical < total) {
-          got = (int)logical;
-          break;
-        }
-        ++queues_tried;
-      }
+      const int got = draw_item(p.queue, per_xcd, total, &s_draw);
       s_item = got;
       s_skip = 0;
       if (got >= 0) {  // the K/V head of the row block, as decoded below
@@ -736,7 +726,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
   static_assert(AM == ATT_15 || AM == ATT_2 || AM == ATT_GEN, "alpha = 1.5, 2 or any other in (1, 2)");
   constexpr int NW = SG::kNW, BM = SG::kBM;
   __shared__ __align__(1024) unsigned char lds_all[SG::kLds];
-  __shared__ int s_item, s_skip;
+  __shared__ int s_item, s_skip, s_draw;
   // a lane ran out of event slots, or a wave out of list room.  Two words: the walks write the one of the tile's
   // parity and read the other one behind the next barrier, so no wave can read a word another one is still setting
   __shared__ uint32_t s_giveup[2];
@@ -746,8 +736,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
   const int N = p.N;
   const int n_mblk = (N + BM - 1) / BM;
   const int group = p.Hq / p.Hkv;
-  const long long total = (long long)p.B * p.Hkv * n_mblk * group;
-  const long long per_xcd = (total + 7) / 8;
+  const int total = p.B * p.Hkv * n_mblk * group;  // (below 2^31, see the dispatch)
+  const int per_xcd = (total + 7) / 8;
   const float qs = p.qscale, inv_qs = 1.f / p.qscale;
   constexpr int kKPer = (G::kKLoads + NW - 1) / NW;
   constexpr bool kKStep = (NW * 64 / KS::kC) % 16 == 0 && (NW * 64) % KS::kC == 0;
@@ -758,7 +748,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
     if (blockIdx.x == 0 && threadIdx.x == 0) p.queue2[kCtrlAllDense] = 1u;
     return;
   }
-  int queues_tried = 0;  // thread 0: how many of the eight counters were found empty
+  if (threadIdx.x == 0) s_draw = 0;
   for (;;) {
     // The lane's constants are formed anew for every row block (the empty asm hides that they repeat): hoisted out
     // of this loop they would stay live through both walks, and the walks have no registers to spare.
@@ -771,17 +761,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
 
     __syncthreads();  // the previous row block is done with LDS and with s_item
     if (tid == 0) {
-      int got = -1;
-      while (queues_tried < 8) {
-        const int x = ((int)(blockIdx.x & 7) + queues_tried) & 7;
-        const long long i = (long long)atomicAdd(&p.queue2[x], 1u);
-        const long long logical = (long long)x * per_xcd + i;
-        if (i < per_xcd && logical < total) {
-          got = (int)logical;
-          break;
-        }
-        ++queues_tried;
-      }
+      const int got = draw_item(p.queue2, per_xcd, total, &s_draw);
       s_item = got;
       s_skip = 0;
       if (got >= 0) {  // the K/V head of the row block, as decoded below
@@ -1264,15 +1244,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_DKDV_W
   static_assert(AM == ATT_15 || AM == ATT_2 || AM == ATT_GEN, "alpha = 1.5, 2 or any other in (1, 2)");
   constexpr int NW = SG::kNW, BM = SG::kBM;
   __shared__ __align__(16) unsigned char lds_all[NW * SG::kWaveLds];
-  __shared__ int s_item, s_skip;
+  __shared__ int s_item, s_skip, s_draw;
 
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int tid = threadIdx.x, lane = tid & 63;
   const int N = p.N;
   const int n_mblk = (N + BM - 1) / BM;
   const int group = p.Hq / p.Hkv;
-  const long long total = (long long)p.B * p.Hkv * n_mblk * group;
-  const long long per_xcd = (total + 7) / 8;
+  const int total = p.B * p.Hkv * n_mblk * group;  // (below 2^31, see the dispatch)
+  const int per_xcd = (total + 7) / 8;
   const float qs = p.qscale;
 
   // (the probe left too little to this kernel: the dense kernel serves everything)
@@ -1280,21 +1260,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_DKDV_W
     if (blockIdx.x == 0 && threadIdx.x == 0) p.queue2[kCtrlAllDense] = 1u;
     return;
   }
-  int queues_tried = 0;  // thread 0: how many of the eight counters were found empty
+  if (threadIdx.x == 0) s_draw = 0;
   for (;;) {
     __syncthreads();  // the previous item is done with s_item
     if (tid == 0) {
-      int got = -1;
-      while (queues_tried < 8) {
-        const int x = ((int)(blockIdx.x & 7) + queues_tried) & 7;
-        const long long i = (long long)atomicAdd(&p.queue2[x], 1u);
-        const long long logical = (long long)x * per_xcd + i;
-        if (i < per_xcd && logical < total) {
-          got = (int)logical;
-          break;
-        }
-        ++queues_tried;
-      }
+      const int got = draw_item(p.queue2, per_xcd, total, &s_draw);
       s_item = got;
       s_skip = 0;
       if (got >= 0) {  // the K/V head of the key block, as decoded below: marked dense by the probe?

@@ -130,6 +130,41 @@ __device__ __forceinline__ bool sparse_steps_aside(const uint32_t* hints, const 
   return 2ull * s_work[1] < s_work[0] || s_work[1] == 0ull;
 }
 
+// The next item of a persistent kernel's work list, called by one thread of a workgroup; -1: there is none left.  The list
+// is dealt in eight parts of `per_xcd` items, one per XCD with a counter each; a workgroup draws from its own XCD's part and,
+// when that has run dry, from the others.  An access to a counter costs 0.1-0.3 us and those of the eight, which lie in one
+// line, follow one another: a launch of few items per workgroup spent most of its time in the increments by which every
+// workgroup found all eight counters exhausted (encoder batch of 16 x 12 heads, N = 500, D = 64: 768 items, 114 us, of
+// which about 85).  So with up to two items per workgroup each takes the items of its own number -- the second ones in
+// reverse, the longest items coming first -- and no counter is touched.  (First items by number in a long launch too, or a
+// look at a counter before it is incremented: 1-2 % slower at 16384 items.)
+// `drawn` is in LDS (0 in front of the first call) and everything else is formed anew on every call -- the empty asm hides
+// that it repeats --: the kernels have no registers to spare for it between two draws.
+__device__ __forceinline__ int draw_item(uint32_t* queue, int per_xcd, int total, int* drawn) {
+  uint32_t bid = blockIdx.x, per_part = gridDim.x >> 3;
+  asm volatile("" : "+s"(bid), "+s"(per_part));
+  const int own = (int)(bid & 7u), n = (int)per_part;
+  int k = *drawn, got = -1;
+  if (2 * n >= per_xcd) {  // k: items taken
+    for (; k < 2 && got < 0; ++k) {
+      const int i = k == 0 ? (int)(bid >> 3) : 2 * n - 1 - (int)(bid >> 3);
+      const int logical = own * per_xcd + i;
+      if (i < per_xcd && logical < total) got = logical;
+    }
+  } else {  // k: parts found dry
+    for (; k < 8; ++k) {
+      const int x = (own + k) & 7;
+      const int at = x * per_xcd + (int)atomicAdd(&queue[x], 1u);
+      if (at < (x + 1) * per_xcd && at < total) {
+        got = at;
+        break;
+      }
+    }
+  }
+  *drawn = k;
+  return got;
+}
+
 template <typename T, int D> struct SparseGeo {
   using G = TileGeo<T, D>;
   static constexpr int kNW = 4;
@@ -167,7 +202,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
   static_assert(AM == ATT_15 || AM == ATT_2 || AM == ATT_GEN, "alpha = 1.5, 2 or any other in (1, 2)");
   constexpr int NW = SG::kNW, BM = SG::kBM;
   __shared__ __align__(1024) unsigned char lds_all[SG::kLds];
-  __shared__ int s_item;
+  __shared__ int s_item, s_draw;
   // a lane ran out of event slots, or a wave out of list room.  Two words: the walks write the one of the tile's
   // parity and read the other one behind the next barrier, so no wave can read a word another one is still setting
   __shared__ uint32_t s_giveup[2];
@@ -177,8 +212,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
   const int N = p.N;
   const int n_mblk = (N + BM - 1) / BM;
   const int group = p.Hq / p.Hkv;
-  const long long total = (long long)p.B * p.Hkv * n_mblk * group;
-  const long long per_xcd = (total + 7) / 8;
+  const int total = p.B * p.Hkv * n_mblk * group;  // (below 2^31, see the dispatch)
+  const int per_xcd = (total + 7) / 8;
   const float qs = p.qscale, inv_qs = 1.f / p.qscale;
   constexpr int kKPer = (G::kKLoads + NW - 1) / NW;
   constexpr int kK8Per = SG::kK8Loads / NW;
@@ -191,7 +226,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
     if (blockIdx.x == 0 && threadIdx.x == 0) p.queue[kCtrlAllDense] = 1u;
     return;
   }
-  int queues_tried = 0;  // thread 0: how many of the eight counters were found empty
+  if (threadIdx.x == 0) s_draw = 0;
   for (;;) {
     // The lane's constants are formed anew for every row block (the empty asm hides that they repeat): hoisted out
     // of this loop they would stay live through both walks, and the walks have no registers to spare.
@@ -207,17 +242,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
 
     __syncthreads();  // the previous row block is done with LDS and with s_item
     if (tid == 0) {
-      int got = -1;
-      while (queues_tried < 8) {
-        const int x = ((int)(blockIdx.x & 7) + queues_tried) & 7;
-        const long long i = (long long)atomicAdd(&p.queue[x], 1u);
-        const long long logical = (long long)x * per_xcd + i;
-        if (i < per_xcd && logical < total) {
-          got = (int)logical;
-          break;
-        }
-        ++queues_tried;
-      }
+      const int got = draw_item(p.queue, per_xcd, total, &s_draw);
       s_item = got;
       s_giveup[0] = 0u;
       s_giveup[1] = 0u;
