@@ -67,6 +67,8 @@ def units(extra=None):
             if tag != "f32" and d in (64, 128):
                 out.append((f"attn_sparse_{tag}_d{d}", "attn_sparse_unit.hip", base + attn_flags))
                 out.append((f"attn_bwd_sparse_{tag}_d{d}", "attn_bwd_sparse_unit.hip", base + attn_flags))
+    for d in (64, 128):
+        out.append((f"attn_f32_d{d}", "attn_f32_unit.hip", [f"-DADSP_D={d}"]))
     return out
 
 

@@ -29,6 +29,12 @@ int launch_attn_bwd_sparse_bf16_d128(const AttnBwdParams&, int, int, int, hipStr
 int launch_attn_bwd_sparse_f16_d64(const AttnBwdParams&, int, int, int, hipStream_t);
 int launch_attn_bwd_sparse_f16_d128(const AttnBwdParams&, int, int, int, hipStream_t);
 
+// the single-precision kernels on 32 rows a workgroup (attn_f32_unit.hip): head dims 64 and 128
+int launch_attn_f32_fwd_d64(const AttnParams&, int, hipStream_t);
+int launch_attn_f32_fwd_d128(const AttnParams&, int, hipStream_t);
+int launch_attn_f32_bwd_d64(const AttnBwdParams&, int, hipStream_t);
+int launch_attn_f32_bwd_d128(const AttnBwdParams&, int, hipStream_t);
+
 typedef int (*attn_fwd_fn)(const AttnParams&, int, hipStream_t);
 typedef int (*attn_bwd_fn)(const AttnBwdParams&, int, int, hipStream_t);
 #define ADSP_FWD_ROW(tag, d) {launch_attn_fwd_##tag##_d##d##_m0, launch_attn_fwd_##tag##_d##d##_m1}
@@ -289,6 +295,13 @@ static int dkdv_merge256() {
   return v < 0 ? 0 : (v > 256 ? 256 : v);
 }
 
+// Whether a single-precision call takes the kernels of attn_f32_kernel.h: the head dims they are made for, key indices that
+// fit their 16-bit list entries, and an alpha whose powers u^(1 / (alpha - 1)) stay inside fp32 (the limit of the other
+// list-keeping kernels).
+static bool f32_split(int N, int D, int dtype, double alpha) {
+  return dtype == ADSP_F32 && (D == 64 || D == 128) && N <= 65536 && alpha >= 1.125 && alpha <= 2.0;
+}
+
 static int attn_common(const void* q, const void* k, const void* v, void* out, float* taus, int32_t* bmask,
                        const void* varlen, int varlen_bits, int B, int Hq, int Hkv, int N, int D, int dtype,
                        double alpha, int is_causal, int niter, int use_hist, void* workspace, size_t workspace_bytes,
@@ -353,6 +366,14 @@ static int attn_common(const void* q, const void* k, const void* v, void* out, f
   p.save_streams = nullptr;
 
   (void)hipGetLastError();
+  if (!tile_counts && f32_split(N, D, dtype, alpha)) {
+    if (bmask) {  // several workgroups share a row block's words
+      const long long words = (long long)B * Hq * p.n_mblk * p.mask_words;
+      hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((words + 255) / 256 > 1024 ? 1024 : (words + 255) / 256)), dim3(256), 0, s, bmask, words);
+    }
+    if ((D == 64 ? launch_attn_f32_fwd_d64(p, am, s) : launch_attn_f32_fwd_d128(p, am, s)) != 0) return ADSP_ERR_LAUNCH;
+    return hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
+  }
   if (dtype != ADSP_F32) {
     const SupportsLayout sl = supports ? supports_layout(B, Hq, Hkv, N, D, dtype) : SupportsLayout{};
     if (sl.total && (supports_bytes < sl.total || ((uintptr_t)supports & 15) != 0)) return ADSP_ERR_WORKSPACE;
@@ -409,6 +430,10 @@ extern "C" size_t adsp_attn_workspace_bytes(int B, int Hq, int Hkv, int N, int D
 extern "C" size_t adsp_attn_supports_bytes(int B, int Hq, int Hkv, int N, int D, int dtype) {
   if (dtype == ADSP_F32 || B <= 0 || Hq <= 0 || Hkv <= 0 || N <= 0 || D <= 0) return 0;
   return adsp::supports_layout(B, Hq, Hkv, N, D, dtype).total;
+}
+
+extern "C" int adsp_attn_bwd_reads_bmask(int N, int D, int dtype, double alpha) {
+  return adsp::f32_split(N, D, dtype, alpha) ? 0 : 1;
 }
 
 extern "C" size_t adsp_attn_bmask_words(int N) {
@@ -737,6 +762,10 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
       }
       if (rc != 0) return ADSP_ERR_LAUNCH;
     }
+  }
+  if (f32_split(N, D, dtype, alpha)) {
+    if ((D == 64 ? launch_attn_f32_bwd_d64(p, am, s) : launch_attn_f32_bwd_d128(p, am, s)) != 0) return ADSP_ERR_LAUNCH;
+    return hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
   }
   if (!sparse) {
     if (kBwdTable[dtype][head_dim_slot(D)](p, am, 3, s) != 0) return ADSP_ERR_LAUNCH;

@@ -1,0 +1,761 @@
+// Sparse entmax attention in single precision for gfx950, head dims 64 and 128: forward, dQ and dK/dV kernels.
+//
+// What bounds them: the fp32 matrix pipe (v_mfma_f32_32x32x2_f32, 64 cycles for 32 x 32 x 2) on large problems, and on
+// ordinary ones the length of a workgroup's walk over the keys, because a K/V head of N keys has only N / rows workgroups.
+//
+// Split: a workgroup is four waves and owns 32 rows (queries; keys in the dK/dV kernel); the waves share the rows and
+// take the 32-row blocks of the other side in turn, and meet in LDS at the end of a walk.  Against 128 rows per workgroup,
+// 32 per wave, a walk is a quarter as long and there are four times as many workgroups.  A wave's operands come through a
+// ring of three 4 KB chunks ([32 rows][32 columns]) of LDS of its own, loaded two chunks ahead with direct 16-byte loads:
+// a chunk lasts 1024 cycles of matrix work, so the waves need no barrier inside a walk and no tile shared by them.  Each
+// operand block is read by one workgroup of 32 rows instead of 128, about 16 bytes per cycle and CU out of L2.
+//
+// Forward, one product per (row, key) where supports are short: tau over a subset of the keys is a lower bound of tau over
+// all of them, so a wave lists the scores above its row's bound while it walks, and after 1, 2, 4, 8, ... steps the
+// workgroup solves the rows on what is listed so far and drops what fell below.  Between two such points about as
+// many scores join as a support holds.  Behind the last step the solution is the threshold itself, to fp32 rounding,
+// and the output gathers the V rows of the support.  A row whose part of a wave's list overflows (flat scores) sends the
+// workgroup to walks: Newton steps on (sum u^c0)^(1/c0) - 1 from the bound the lists gave, until a step is below 2e-5, and
+// an output walk.
+//
+// Measured, B = 2, 8 heads, N = 1500 and 375, D = 64, causal (us, 128-row workgroups -> here): see the launch rule in
+// attn_api.hip.
+#pragma once
+#include "attn_bwd_kernel.h"
+
+namespace adsp {
+namespace f32path {
+
+constexpr int kRows = 32;        // rows per workgroup, and per block of the other side
+constexpr int kWaves = 4;
+constexpr int kChunk = 4096;     // bytes of a chunk: 32 rows of 128 bytes, 16-byte pieces swizzled
+constexpr int kStages = 3;
+constexpr int kRing = kWaves * kStages * kChunk;
+constexpr int kCap = 32;         // list entries per row and wave
+constexpr int kListBytes = kWaves * kCap * kRows * 6;  // a score (fp32) and a key index (16 bits) per entry
+
+// position of 16-byte piece c of chunk row r
+__device__ __forceinline__ int piece_sw(int row) { return (row >> 1) & 7; }
+
+// A wave's ring of chunks and its place in it.
+struct Ring {
+  unsigned char* base;  // the wave's three chunks
+  int lane;
+  int st;  // stage of the next chunk to be consumed
+  // chunk c (32 columns) of rows [row0, row0 + 32) of a row-major tensor with `stride` bytes per row into stage `s`; rows
+  // from `limit` on are replaced by the last one in front of it
+  __device__ __forceinline__ void issue(const unsigned char* g, int row0, int limit, int stride, int c, int s) const {
+    const unsigned char* gb = uniform_ptr(g + c * 128);
+    unsigned char* l = base + s * kChunk;
+    const int p0 = (lane & 7) ^ (lane >> 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      int r = row0 + 8 * j + (lane >> 3);
+      r = r < limit ? r : limit - 1;
+      dma16s(gb, (uint32_t)r * (uint32_t)stride + (uint32_t)((p0 ^ (4 * (j & 1))) * 16), l + j * 1024);
+    }
+  }
+  // Waits for the oldest of the two chunks under way and for the wave's own LDS reads (the stage the caller fills next is
+  // the one it has just read); returns the LDS address of the chunk.
+  __device__ __forceinline__ uint32_t arrive() const {
+    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+    return (uint32_t)(uintptr_t)(base + st * kChunk);
+  }
+  __device__ __forceinline__ int ahead() const { return st == 0 ? 2 : st - 1; }  // stage of the chunk after next
+  __device__ __forceinline__ void advance() { st = st == 2 ? 0 : st + 1; }
+  __device__ __forceinline__ void drain() const { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
+};
+
+// Walks the blocks wave, wave + 4, ... below n_blk.  Each block is SEQ chunks, src(blk, s, ring, stage) issues number s of
+// them; body(blk, next) consumes them by SEQ calls of next(s) in order, which return the chunk's LDS address.
+template <int SEQ, typename Src, typename Body>
+__device__ __forceinline__ void walk(Ring& ring, int first, int n_blk, int step, Src&& src, Body&& body) {
+  if (first >= n_blk) return;
+  ring.st = 0;
+  src(first, 0, 0);
+  src(first, 1, 1);
+  for (int blk = first; blk < n_blk; blk += step) {
+    const int blk_next = blk + step < n_blk ? blk + step : blk;  // (past the end: loads that nothing reads keep the count)
+    body(blk, [&](int s) -> uint32_t {
+      const uint32_t a = ring.arrive();
+      if (s + 2 < SEQ) src(blk, s + 2, ring.ahead());
+      else src(blk_next, s + 2 - SEQ, ring.ahead());
+      ring.advance();
+      return a;
+    });
+  }
+  ring.drain();
+}
+
+// acc += (chunk rows) . (the lane's own row), columns 32 c .. 32 c + 31: f holds the lane's row, 8 g + 4 lh .. + 3 of every 8
+__device__ __forceinline__ void dot_chunk(f32x16& acc, uint32_t chunk, uint32_t row_lane, const uint32_t* f) {
+  f32x4 a[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) a[g] = __builtin_bit_cast(f32x4, lds_read16((chunk + row_lane) ^ (g << 5)));
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g][e], __builtin_bit_cast(float, f[g * 4 + e]), acc, 0, 0, 0);
+}
+// o[column of the chunk][lane's row] += sum over the chunk's rows of chunk[row][column] * w[row]; w in accumulator order
+__device__ __forceinline__ void acc_chunk(f32x16& o, uint32_t chunk, uint32_t col_lane, const float (&w)[16]) {
+  float a[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    // row 8 (i / 4) + 4 lh + i % 4: its swizzle differs from the lane's constant part by an immediate
+    const int x = (4 * ((i >> 2) & 1)) ^ ((i >> 1) & 1);
+    a[i] = *(const __attribute__((address_space(3))) float*)(((chunk + col_lane) ^ (x << 4)) + (8 * (i >> 2) + (i & 3)) * 128);
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) o = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], w[i], o, 0, 0, 0);
+}
+__device__ __forceinline__ uint32_t row_lane_of(int lq, int lh) { return (uint32_t)(lq * 128 + ((lh ^ piece_sw(lq)) << 4)); }
+__device__ __forceinline__ uint32_t col_lane_of(int lq, int lh) {
+  return (uint32_t)(4 * lh * 128 + (((lq >> 2) ^ (2 * lh)) << 4) + (lq & 3) * 4);
+}
+
+// Adds up the four waves' o (32 columns per block, accumulator layout) in LDS and writes scale[row] * sum to the rows
+// [row0, row0 + 32) below n of a row-major tensor.  `smem` holds 4 x 32 x D floats; every wave is done with what it held.
+template <int D, typename Scale>
+__device__ __forceinline__ void combine_store(const f32x16 (&o)[D / 32], unsigned char* smem, float* out, int row0, int n, int wave,
+                                              int lane, Scale&& scale) {
+  using KS = Swz<D * 4>;
+  const int lq = lane & 31, lh = lane >> 5, tid = wave * 64 + lane;
+  unsigned char* mine = smem + wave * (kRows * D * 4);
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(mine + KS::off(lq, db * 8 + 2 * g + lh)) =
+          f32x4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]};
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kRows * D / 4 / 256; ++j) {
+    const int id = j * 256 + tid, row = id / (D / 4), c = id % (D / 4);
+    const int at = KS::off(row, c);
+    f32x4 s = *reinterpret_cast<const f32x4*>(smem + at);
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(smem + w * (kRows * D * 4) + at);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] += x[e];
+    }
+    const float k = scale(row);
+    if (row0 + row < n) *reinterpret_cast<f32x4*>(out + (size_t)(row0 + row) * D + c * 4) = f32x4{s[0] * k, s[1] * k, s[2] * k, s[3] * k};
+  }
+}
+
+template <int D> __device__ __forceinline__ void load_row(const float* row, int lh, uint32_t (&f)[D / 2]) {
+#pragma unroll
+  for (int g = 0; g < D / 8; ++g) {
+    const u32x4 raw = *reinterpret_cast<const u32x4*>(row + 8 * g + 4 * lh);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[g * 4 + e] = raw[e];
+  }
+}
+
+__device__ __forceinline__ float sum8(float x) {
+  x += __shfl_xor(x, 1, 64);
+  x += __shfl_xor(x, 2, 64);
+  return x + __shfl_xor(x, 4, 64);
+}
+
+// u^c0 and u^(c0 - 1) of u >= 0
+template <int AM> __device__ __forceinline__ void powers(float u, float c0, float& e0, float& e1) {
+  if constexpr (AM == ATT_15) {
+    e0 = u * u;
+    e1 = u;
+  } else if constexpr (AM == ATT_2) {
+    e0 = u;
+    e1 = u > 0.f ? 1.f : 0.f;
+  } else {
+    const bool pos = u > 0.f;
+    const float x = pos ? u : 1.f;
+    const float e = fast_exp2(fast_log2(x) * c0);
+    e0 = pos ? e : 0.f;
+    e1 = pos ? e * fast_rcp(x) : 0.f;
+  }
+}
+// Newton step on (sum u^c0)^(1/c0) - 1: convex and decreasing in the threshold, nearly linear where the support is settled
+template <int AM> __device__ __forceinline__ float norm_step(float s0, float s1, float c0) {
+  const float g = AM == ATT_15 ? sqrtf(s0) : (AM == ATT_2 ? s0 : fast_exp2(fast_log2(s0) / c0));
+  return (g - 1.f) * s0 / (g * s1);
+}
+
+// ---------------------------------------------------------------------------------------------------------
+// forward
+// ---------------------------------------------------------------------------------------------------------
+template <int D> constexpr int fwd_smem() {
+  const int a = kRing + kListBytes, b = kWaves * kRows * D * 4;
+  return a > b ? a : b;
+}
+
+template <int D, int AM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_f32_fwd_kernel(AttnParams p) {
+  constexpr int NC = D / 32;
+  constexpr int kStride = D * 4;
+  __shared__ __align__(4096) unsigned char smem[fwd_smem<D>()];
+  __shared__ float t_lds[kRows];
+  __shared__ uint8_t n_lds[kWaves][2][kRows];
+  __shared__ float red[2][kWaves][3][kRows];
+  __shared__ uint32_t over_flag;
+  float* const list_s = reinterpret_cast<float*>(smem + kRing);                                   // [wave][slot][row]
+  uint16_t* const list_k = reinterpret_cast<uint16_t*>(smem + kRing + kWaves * kCap * kRows * 4);  // likewise
+
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
+  const int N = p.N, group = p.Hq / p.Hkv, n_rblk = (N + kRows - 1) / kRows;
+  int bkv, mi, hg;
+  if (!xcd_block_map(p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
+  const int b = bkv / p.Hkv, kvh = bkv % p.Hkv, h = kvh * group + hg;
+  const int m0 = (n_rblk - 1 - mi) * kRows;
+  int L = N;
+  if (p.varlen) {
+    const long long l = p.varlen_bits == 64 ? ((const long long*)p.varlen)[b] : (long long)((const int*)p.varlen)[b];
+    L = (int)(l < 0 ? 0 : (l > N ? N : l));
+  }
+  const size_t q_row0 = (size_t)(b * p.Hq + h) * N;
+  float* const out = reinterpret_cast<float*>(p.out) + q_row0 * D;
+  if (m0 >= L) {
+    const int rows = N - m0 < kRows ? N - m0 : kRows;
+    for (int i = tid; i < rows * (D / 4); i += 256) reinterpret_cast<f32x4*>(out + (size_t)m0 * D)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    return;
+  }
+  const unsigned char* kg = reinterpret_cast<const unsigned char*>(p.k) + (size_t)bkv * N * kStride;
+  const unsigned char* vg = reinterpret_cast<const unsigned char*>(p.v) + (size_t)bkv * N * kStride;
+  const int qi = m0 + lq;
+  const bool live = qi < L;
+  const int lim = p.causal ? (qi < L - 1 ? qi : L - 1) : L - 1;  // last key of the lane's row
+  const int key_hi = p.causal ? (m0 + kRows < L ? m0 + kRows : L) : L;
+  const int n_kblk = (key_hi + kRows - 1) / kRows;
+  const float qs = p.qscale, inv_qs = 1.f / p.qscale, c0 = p.c0;
+  uint32_t qf[D / 2];
+  load_row<D>(reinterpret_cast<const float*>(p.q) + (q_row0 + (live ? qi : L - 1)) * D, lh, qf);
+
+  Ring ring{smem + wave * (kStages * kChunk), lane, 0};
+  const uint32_t rl = row_lane_of(lq, lh), cl = col_lane_of(lq, lh);
+  auto src_k = [&](int blk, int s, int st) { ring.issue(kg, blk * kRows, L, kStride, s, st); };
+  // scores of a block less `sub`, -inf on the keys the row may not see
+  auto scores = [&](int blk, float init, auto&& next) -> f32x16 {
+    f32x16 acc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = init;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) dot_chunk(acc, next(c), rl, qf + c * 16);
+    const int k0 = blk * kRows;
+    if (k0 + kRows > L || (p.causal && k0 + kRows - 1 > m0)) {
+      const int jb = k0 + 4 * lh;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[i] = jb + 8 * (i >> 2) + (i & 3) <= lim ? acc[i] : -INFINITY;
+    }
+    return acc;
+  };
+
+  // ---- the walk that lists: rows are solved on the lists after 1, 2, 4, ... steps of four blocks and behind the last ----
+  if (tid == 0) over_flag = 0u;
+  float t_raw = -INFINITY;  // bound of the lane's row, raw score units
+  int n_mine = 0;           // entries of this lane: lh = 0 fills the wave's slots of the row from the front, lh = 1 from the back
+  bool over = false;
+  const int n_steps = (n_kblk + kWaves - 1) / kWaves;
+  float* const my_s = list_s + wave * (kCap * kRows) + lq;
+  uint16_t* const my_k = list_k + wave * (kCap * kRows) + lq;
+  auto slot_of = [&](int e) -> int { return (lh ? kCap - 1 - e : e) * kRows; };
+  // solver's view: eight lanes per row, wave w has rows 8 w .. 8 w + 7
+  const int srow = wave * 8 + (lane >> 3), sj = lane & 7;
+  float sv[16];  // the lane's share of the row's listed scores, relative to their maximum, in z units
+  float s_max = 0.f, s_tau = 0.f;
+  auto solve = [&]() {
+    float x[16];
+    s_max = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const int n0 = n_lds[w][0][srow], n1 = n_lds[w][1][srow];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int slot = sj + 8 * k;
+        const bool ok = slot < n0 || slot >= kCap - n1;
+        const float v = list_s[w * (kCap * kRows) + slot * kRows + srow];
+        x[w * 4 + k] = ok ? v : -INFINITY;
+        s_max = fmaxf(s_max, x[w * 4 + k]);
+      }
+    }
+    s_max = fmaxf(s_max, __shfl_xor(s_max, 1, 64));
+    s_max = fmaxf(s_max, __shfl_xor(s_max, 2, 64));
+    s_max = fmaxf(s_max, __shfl_xor(s_max, 4, 64));
+    const float m = s_max > -INFINITY ? s_max : 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sv[i] = (x[i] - m) * qs;
+    s_tau = -1.f;
+    bool go = s_max > -INFINITY;
+    for (int it = 0; it < 40 && __builtin_amdgcn_ballot_w64(go) != 0ull; ++it) {
+      float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        float e0, e1;
+        powers<AM>(fmaxf(sv[i] - s_tau, 0.f), c0, e0, e1);
+        s0 += e0;
+        s1 += e1;
+      }
+      s0 = sum8(s0);
+      s1 = sum8(s1);
+      const float step = norm_step<AM>(s0, s1, c0);
+      if (go) s_tau = fminf(s_tau + step, 0.f);
+      go = go && step > 2e-7f;
+    }
+  };
+  bool fallback = false;
+  {
+    int step_no = 0, next_sync = 1;
+    // solves the rows on the lists and keeps what is above the new bound; true when the workgroup gives its lists up
+    auto sync = [&]() -> bool {
+      n_lds[wave][lh][lq] = (uint8_t)n_mine;
+      if (over) over_flag = 1u;
+      __syncthreads();
+      solve();
+      if (sj == 0) {
+        // (the margin covers the rounding of the difference and of the product back to raw units)
+        t_lds[srow] = s_max > -INFINITY ? (s_max + (s_tau - 1e-6f) * inv_qs) - 4e-7f * fabsf(s_max) : -INFINITY;
+      }
+      const bool given_up = over_flag != 0u;  // (read in front of the barrier: behind it a faster wave may set it again)
+      __syncthreads();
+      t_raw = fmaxf(t_raw, t_lds[lq]);
+      return given_up;
+    };
+    auto compact = [&]() {
+      int kept = 0;
+      for (int e = 0; __builtin_amdgcn_ballot_w64(e < n_mine) != 0ull; ++e) {
+        if (e < n_mine) {
+          const float s = my_s[slot_of(e)];
+          const uint16_t k = my_k[slot_of(e)];
+          if (s > t_raw) {
+            my_s[slot_of(kept)] = s;
+            my_k[slot_of(kept)] = k;
+            ++kept;
+          }
+        }
+      }
+      n_mine = kept;
+    };
+    __syncthreads();  // over_flag is clear
+    // one segment of the walk per solve: the blocks of the steps [step_no, next_sync)
+    while (true) {
+      const int seg_end = next_sync < n_steps ? next_sync : n_steps;
+      walk<NC>(ring, step_no * kWaves + wave, seg_end * kWaves < n_kblk ? seg_end * kWaves : n_kblk, kWaves, src_k, [&](int blk, auto&& next) {
+        const f32x16 s = scores(blk, 0.f, next);
+        float bm = s[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) bm = fmaxf(bm, s[i]);
+        if (over || __builtin_amdgcn_ballot_w64(live && bm > t_raw) == 0ull) return;
+        int c = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) c += s[i] > t_raw ? 1 : 0;
+        c = live ? c : 0;
+        const int need = n_mine + c;
+        if (__builtin_amdgcn_ballot_w64(need + __shfl_xor(need, 32, 64) > kCap) != 0ull) {
+          over = true;  // uniform over the wave
+          return;
+        }
+        const int jb = blk * kRows + 4 * lh;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          if (live && s[i] > t_raw) {
+            my_s[slot_of(n_mine)] = s[i];
+            my_k[slot_of(n_mine)] = (uint16_t)(jb + 8 * (i >> 2) + (i & 3));
+            ++n_mine;
+          }
+        }
+      });
+      step_no = seg_end;
+      if (sync()) {
+        fallback = true;
+        break;
+      }
+      if (step_no == n_steps) break;
+      compact();
+      next_sync = step_no * 2;
+    }
+  }
+
+  if (!fallback) {
+    // ---- output from the lists: the solver's lanes hold the row's scores; members to a dense list in the idle ring ----
+    float pr[16];
+    float psum = 0.f;
+    int members = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float e1;
+      powers<AM>(fmaxf(sv[i] - s_tau, 0.f), c0, pr[i], e1);
+      psum += pr[i];
+      members += pr[i] > 0.f ? 1 : 0;
+    }
+    psum = sum8(psum);
+    const float inv = psum > 0.f ? 1.f / psum : 0.f;
+    int before = 0, total = members;
+#pragma unroll
+    for (int d = 1; d < 8; d <<= 1) {
+      const int o = __shfl_xor(total, d, 64);
+      if (sj & d) before += o;
+      total += o;
+    }
+    float* const mem_p = reinterpret_cast<float*>(smem) + srow * 128;
+    uint32_t* const mem_k = reinterpret_cast<uint32_t*>(smem) + kRows * 128 + srow * 128;
+    uint32_t bits_done = 0xffffffffu;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      if (pr[i] > 0.f) {
+        const uint32_t key = list_k[(i >> 2) * (kCap * kRows) + (sj + 8 * (i & 3)) * kRows + srow];
+        mem_p[before] = pr[i];
+        mem_k[before] = key;
+        ++before;
+        if (p.bmask && (key >> 6) != bits_done) {
+          bits_done = key >> 6;
+          atomicOr(reinterpret_cast<uint32_t*>(p.bmask) + ((size_t)(b * p.Hq + h) * p.n_mblk + m0 / kMaskRows) * p.mask_words + (bits_done >> 5),
+                   1u << (bits_done & 31));
+        }
+      }
+    }
+    // (a row's eight lanes belong to one wave, whose LDS accesses stay in order)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+    const int row = m0 + srow;
+    if (p.taus && sj == 0 && row < L) p.taus[q_row0 + row] = fmaf(s_max, qs, s_tau);
+    f32x4 acc[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const f32x4* v4 = reinterpret_cast<const f32x4*>(vg);
+    for (int e = 0; __builtin_amdgcn_ballot_w64(e < total) != 0ull; e += 4) {
+      f32x4 r[4][NC];
+      float w[4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const bool ok = e + x < total;
+        w[x] = ok ? mem_p[e + x] : 0.f;
+        const uint32_t key = ok ? mem_k[e + x] : mem_k[0];
+        const f32x4* vr = v4 + (size_t)(total > 0 ? key : 0u) * (D / 4) + sj;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) r[x][c] = vr[8 * c];
+      }
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        if (e + x < total)
+#pragma unroll
+          for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[c][k] = fmaf(w[x], r[x][c][k], acc[c][k]);
+    }
+    if (row < N) {
+      f32x4* o4 = reinterpret_cast<f32x4*>(out + (size_t)row * D) + sj;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) o4[8 * c] = f32x4{acc[c][0] * inv, acc[c][1] * inv, acc[c][2] * inv, acc[c][3] * inv};
+    }
+    return;
+  }
+
+  // ---- walks: t_raw is finite for live rows (every row sees key 0, which the first solve has), a lower bound of tau ----
+  float t = live && t_raw > -INFINITY ? t_raw : 0.f;
+  for (int it = 0; it < 24; ++it) {
+    float a0 = 0.f, a1 = 0.f, mx = -INFINITY;
+    walk<NC>(ring, wave, n_kblk, kWaves, src_k, [&](int blk, auto&& next) {
+      const f32x16 s = scores(blk, -t, next);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        mx = fmaxf(mx, s[i]);
+        float e0, e1;
+        powers<AM>(fmaxf(s[i], 0.f) * qs, c0, e0, e1);
+        a0 += e0;
+        a1 += e1;
+      }
+    });
+    a0 += __shfl_xor(a0, 32, 64);
+    a1 += __shfl_xor(a1, 32, 64);
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    float(*rd)[3][kRows] = red[it & 1];
+    if (lh == 0) {
+      rd[wave][0][lq] = a0;
+      rd[wave][1][lq] = a1;
+      rd[wave][2][lq] = mx;
+    }
+    __syncthreads();
+    a0 = (rd[0][0][lq] + rd[1][0][lq]) + (rd[2][0][lq] + rd[3][0][lq]);
+    a1 = (rd[0][1][lq] + rd[1][1][lq]) + (rd[2][1][lq] + rd[3][1][lq]);
+    mx = fmaxf(fmaxf(rd[0][2][lq], rd[1][2][lq]), fmaxf(rd[2][2][lq], rd[3][2][lq]));
+    // never below the row maximum less 1, where the sums of a score far above the bound would also leave fp32
+    float step = mx * qs - 1.f;
+    if (a0 > 0.f && a0 < 1e30f && a1 > 0.f && a1 < 1e30f) step = fmaxf(step, norm_step<AM>(a0, a1, c0));
+    if (live) t += step * inv_qs;
+    if (__builtin_amdgcn_ballot_w64(live && fabsf(step) > 2e-5f) == 0ull) break;  // (the same sums in every wave)
+  }
+  if (live && lh == 0 && wave == 0 && p.taus) p.taus[q_row0 + qi] = t * qs;
+
+  f32x16 o[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[c][i] = 0.f;
+  float psum = 0.f;
+  auto src_kv = [&](int blk, int s, int st) { ring.issue(s < NC ? kg : vg, blk * kRows, L, kStride, s < NC ? s : s - NC, st); };
+  walk<2 * NC>(ring, wave, n_kblk, kWaves, src_kv, [&](int blk, auto&& next) {
+    const f32x16 s = scores(blk, -t, next);
+    float w[16];
+    float bs = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float e1;
+      powers<AM>(live ? fmaxf(s[i], 0.f) * qs : 0.f, c0, w[i], e1);
+      bs += w[i];
+    }
+    psum += bs;
+    const bool any = __builtin_amdgcn_ballot_w64(bs > 0.f) != 0ull;
+    if (any && p.bmask && lane == 0)
+      atomicOr(reinterpret_cast<uint32_t*>(p.bmask) + ((size_t)(b * p.Hq + h) * p.n_mblk + m0 / kMaskRows) * p.mask_words + (blk >> 6),
+               1u << ((blk >> 1) & 31));
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const uint32_t a = next(NC + c);
+      if (any) acc_chunk(o[c], a, cl, w);
+    }
+  });
+  psum += __shfl_xor(psum, 32, 64);
+  __syncthreads();  // the sums of the last step have been read, every wave is done with its ring
+  if (lh == 0) red[0][wave][0][lq] = psum;
+  combine_store<D>(o, smem, out, m0, N, wave, lane, [&](int row) {
+    const float z = (red[0][0][0][row] + red[0][1][0][row]) + (red[0][2][0][row] + red[0][3][0][row]);
+    return z > 0.f ? 1.f / z : 0.f;
+  });
+}
+
+// ---------------------------------------------------------------------------------------------------------
+// dQ: one walk for sum p, sum u, sum u dP, one for dX and dQ^T += K^T dX^T
+// ---------------------------------------------------------------------------------------------------------
+template <int D> constexpr int bwd_smem() { return kRing > kWaves * kRows * D * 4 ? kRing : kWaves * kRows * D * 4; }
+
+template <int D, int AM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_f32_dq_kernel(AttnBwdParams p) {
+  constexpr int NC = D / 32;
+  constexpr int kStride = D * 4;
+  __shared__ __align__(4096) unsigned char smem[bwd_smem<D>()];
+  __shared__ float red[kWaves][3][kRows];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
+  const int N = p.N, group = p.Hq / p.Hkv, n_rblk = (N + kRows - 1) / kRows;
+  int bkv, mi, hg;
+  if (!xcd_block_map(p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
+  const int b = bkv / p.Hkv, kvh = bkv % p.Hkv, h = kvh * group + hg;
+  const int m0 = (n_rblk - 1 - mi) * kRows;
+  const int L = bwd_seq_len(p, b);
+  const size_t q_row0 = (size_t)(b * p.Hq + h) * N;
+  float* const dq = reinterpret_cast<float*>(p.dq) + q_row0 * D;
+  if (m0 >= L) {
+    const int rows = N - m0 < kRows ? N - m0 : kRows;
+    for (int i = tid; i < rows * (D / 4); i += 256) reinterpret_cast<f32x4*>(dq + (size_t)m0 * D)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    return;
+  }
+  const unsigned char* kg = reinterpret_cast<const unsigned char*>(p.k) + (size_t)bkv * N * kStride;
+  const unsigned char* vg = reinterpret_cast<const unsigned char*>(p.v) + (size_t)bkv * N * kStride;
+  const int qi = m0 + lq;
+  const bool live = qi < L;
+  const int lim = p.causal ? (qi < L - 1 ? qi : L - 1) : L - 1;
+  const int key_hi = p.causal ? (m0 + kRows < L ? m0 + kRows : L) : L;
+  const int n_kblk = (key_hi + kRows - 1) / kRows;
+  const float tau = live ? p.taus[q_row0 + qi] : INFINITY;
+  uint32_t qf[D / 2], dof[D / 2];
+  {
+    const size_t r = q_row0 + (live ? qi : L - 1);
+    load_row<D>(reinterpret_cast<const float*>(p.q) + r * D, lh, qf);
+    load_row<D>(reinterpret_cast<const float*>(p.dout) + r * D, lh, dof);
+  }
+  Ring ring{smem + wave * (kStages * kChunk), lane, 0};
+  const uint32_t rl = row_lane_of(lq, lh), cl = col_lane_of(lq, lh);
+  // chunks of a block: K, V and, for the second walk, K again
+  auto src = [&](int blk, int s, int st) {
+    ring.issue(s < NC || s >= 2 * NC ? kg : vg, blk * kRows, L, kStride, s < NC ? s : (s < 2 * NC ? s - NC : s - 2 * NC), st);
+  };
+  // r = z - tau (-inf where the row may not look); false when no row of the block has a member, whose dP is then not formed
+  auto block_terms = [&](int blk, auto&& next, float (&r)[16], f32x16& dp) -> bool {
+    f32x16 s;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) dot_chunk(s, next(c), rl, qf + c * 16);
+    const int jb = blk * kRows + 4 * lh;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      r[i] = jb + 8 * (i >> 2) + (i & 3) <= lim ? fmaf(s[i], p.qscale, -tau) : -INFINITY;
+      mx = fmaxf(mx, r[i]);
+    }
+    const bool any = __builtin_amdgcn_ballot_w64(mx > 0.f) != 0ull;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const uint32_t a = next(NC + c);
+      if (any) dot_chunk(dp, a, rl, dof + c * 16);
+    }
+    return any;
+  };
+  float zsum = 0.f, usum = 0.f, udp = 0.f;
+  walk<2 * NC>(ring, wave, n_kblk, kWaves, src, [&](int blk, auto&& next) {
+    float r[16];
+    f32x16 dp;
+    if (!block_terms(blk, next, r, dp)) return;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float pr, u;
+      bwd_prob<AM>(r[i], p.c0, pr, u);
+      zsum += pr;
+      usum += u;
+      udp += u > 0.f ? u * dp[i] : 0.f;
+    }
+  });
+  zsum += __shfl_xor(zsum, 32, 64);
+  usum += __shfl_xor(usum, 32, 64);
+  udp += __shfl_xor(udp, 32, 64);
+  if (lh == 0) {
+    red[wave][0][lq] = zsum;
+    red[wave][1][lq] = usum;
+    red[wave][2][lq] = udp;
+  }
+  __syncthreads();
+  auto all = [&](int k) { return (red[0][k][lq] + red[1][k][lq]) + (red[2][k][lq] + red[3][k][lq]); };
+  zsum = all(0);
+  usum = all(1);
+  udp = all(2);
+  const float delta = usum > 0.f ? udp / usum : 0.f;
+  if (live && wave == 0 && lh == 0) {
+    p.delta[q_row0 + qi] = delta;
+    p.zinv[q_row0 + qi] = zsum > 0.f ? 1.f / zsum : 0.f;
+  }
+  f32x16 o[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[c][i] = 0.f;
+  walk<3 * NC>(ring, wave, n_kblk, kWaves, src, [&](int blk, auto&& next) {
+    float r[16], dx[16];
+    f32x16 dp;
+    const bool any = block_terms(blk, next, r, dp);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float pr, u;
+      bwd_prob<AM>(r[i], p.c0, pr, u);
+      dx[i] = u > 0.f ? u * (dp[i] - delta) : 0.f;
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const uint32_t a = next(2 * NC + c);
+      if (any) acc_chunk(o[c], a, cl, dx);
+    }
+  });
+  __syncthreads();  // every wave is done with its ring
+  const float sm = p.sm_scale;
+  combine_store<D>(o, smem, dq, m0, N, wave, lane, [&](int) { return sm; });
+}
+
+// ---------------------------------------------------------------------------------------------------------
+// dK, dV: one walk over the (query block, query head) pairs of a K/V head, dV^T += dO^T P and dK^T += Q^T dX
+// ---------------------------------------------------------------------------------------------------------
+template <int D, int AM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void attn_f32_dkdv_kernel(AttnBwdParams p) {
+  constexpr int NC = D / 32;
+  constexpr int kStride = D * 4;
+  __shared__ __align__(4096) unsigned char smem[bwd_smem<D>()];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
+  const int N = p.N, group = p.Hq / p.Hkv, n_rblk = (N + kRows - 1) / kRows;
+  int bkv, kblk, member_unused;
+  if (!xcd_block_map(p.B * p.Hkv, n_rblk, 1, p.causal != 0, 2ll * group * N * kStride, bkv, kblk, member_unused)) return;
+  const int b = bkv / p.Hkv, kvh = bkv % p.Hkv;
+  const int L = bwd_seq_len(p, b);
+  const int n0 = kblk * kRows;
+  const size_t kv_row0 = (size_t)bkv * N;
+  float* const dk = reinterpret_cast<float*>(p.dk) + kv_row0 * D;
+  float* const dv = reinterpret_cast<float*>(p.dv) + kv_row0 * D;
+  if (n0 >= L) {
+    const int rows = N - n0 < kRows ? N - n0 : kRows;
+    for (int i = tid; i < rows * (D / 4); i += 256) {
+      reinterpret_cast<f32x4*>(dk + (size_t)n0 * D)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      reinterpret_cast<f32x4*>(dv + (size_t)n0 * D)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    return;
+  }
+  const int kj = n0 + lq;
+  const bool live = kj < L;
+  uint32_t kf[D / 2], vf[D / 2];
+  {
+    const size_t r = kv_row0 + (live ? kj : L - 1);
+    load_row<D>(reinterpret_cast<const float*>(p.k) + r * D, lh, kf);
+    load_row<D>(reinterpret_cast<const float*>(p.v) + r * D, lh, vf);
+  }
+  const int q_first = p.causal ? kblk : 0;            // first query block that sees the keys
+  const int n_q = (L + kRows - 1) / kRows - q_first;  // query blocks per head
+  const size_t q_head0 = (size_t)(b * p.Hq + kvh * group) * N;
+  Ring ring{smem + wave * (kStages * kChunk), lane, 0};
+  const uint32_t rl = row_lane_of(lq, lh), cl = col_lane_of(lq, lh);
+  // item x = head * n_q + query block - q_first; its chunks: Q, dO, dO and Q again
+  auto src = [&](int x, int s, int st) {
+    const int g = x / n_q, qb = q_first + (x - g * n_q);
+    const unsigned char* base = reinterpret_cast<const unsigned char*>(s < NC || s >= 3 * NC ? p.q : p.dout) + (q_head0 + (size_t)g * N) * kStride;
+    ring.issue(base, qb * kRows, L, kStride, s % NC, st);
+  };
+  f32x16 ov[NC], ok[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) ov[c][i] = ok[c][i] = 0.f;
+  walk<4 * NC>(ring, wave, n_q * group, kWaves, src, [&](int x, auto&& next) {
+    const int g = x / n_q, q0 = (q_first + (x - g * n_q)) * kRows;
+    f32x16 s, dp;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) dot_chunk(s, next(c), rl, kf + c * 16);
+    const float* tau = p.taus + q_head0 + (size_t)g * N;
+    const float* zi = p.zinv + q_head0 + (size_t)g * N;
+    const float* de = p.delta + q_head0 + (size_t)g * N;
+    float r[16], w[16], dx[16];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int qrow = q0 + 8 * (i >> 2) + 4 * lh + (i & 3);
+      const int qc = qrow < L ? qrow : L - 1;
+      const bool see = live && qrow < L && (!p.causal || kj <= qrow);
+      r[i] = see ? fmaf(s[i], p.qscale, -tau[qc]) : -INFINITY;
+      mx = fmaxf(mx, r[i]);
+    }
+    const bool any = __builtin_amdgcn_ballot_w64(mx > 0.f) != 0ull;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const uint32_t a = next(NC + c);
+      if (any) dot_chunk(dp, a, rl, vf + c * 16);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int qrow = q0 + 8 * (i >> 2) + 4 * lh + (i & 3);
+      const int qc = qrow < L ? qrow : L - 1;
+      float pr, u;
+      bwd_prob<AM>(r[i], p.c0, pr, u);
+      w[i] = pr > 0.f ? pr * zi[qc] : 0.f;
+      dx[i] = u > 0.f ? u * (dp[i] - de[qc]) : 0.f;
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const uint32_t a = next(2 * NC + c);
+      if (any) acc_chunk(ov[c], a, cl, w);
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const uint32_t a = next(3 * NC + c);
+      if (any) acc_chunk(ok[c], a, cl, dx);
+    }
+  });
+  __syncthreads();  // every wave is done with its ring
+  combine_store<D>(ov, smem, dv, n0, N, wave, lane, [](int) { return 1.f; });
+  __syncthreads();
+  const float sm = p.sm_scale;
+  combine_store<D>(ok, smem, dk, n0, N, wave, lane, [&](int) { return sm; });
+}
+
+}  // namespace f32path
+}  // namespace adsp

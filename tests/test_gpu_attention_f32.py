@@ -1,0 +1,68 @@
+"""The single-precision kernels on 32 rows a workgroup (head dims 64 and 128) against the oracle, at the sizes where their split
+can go wrong: lengths around a block of 32 and a step of four of them, lists that overflow (flat scores, which send a
+workgroup from the lists to walks) and that do not, padding that holds NaN, grouped K/V heads, every alpha mode.
+
+Tolerance 1e-4 as in the other single-precision tests of forward and backward."""
+
+import pytest
+import torch
+
+import adasplash_amd as A
+from oracle import exact
+from tests.gpu_util import DEV, max_err
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-4
+
+
+def run(q, k, v, dout, varlen, alpha, causal, grouped):
+    qg, kg, vg = (t.to(DEV).requires_grad_(True) for t in (q, k, v))
+    vl = None if varlen is None else varlen.to(DEV)
+    if grouped:
+        out = A.adasplash_v2(qg, kg, vg, varlen=vl)
+    else:
+        out = A.adasplash_v1(qg, kg, vg, alpha=alpha, is_causal=causal, varlen=vl)
+    out.backward(dout.to(DEV))
+    return out.detach(), qg.grad, kg.grad, vg.grad
+
+
+@pytest.mark.parametrize("scale", [0.125, 1.0, 3.0])  # of q: flat scores (lists overflow), ordinary, peaked
+@pytest.mark.parametrize("alpha,causal,Hq,Hkv,D", [(1.5, True, 4, 2, 64), (1.5, True, 2, 2, 128), (1.333, False, 2, 2, 64),
+                                                   (2.0, False, 1, 1, 128), (1.5, False, 2, 2, 64), (1.125, True, 1, 1, 64)])
+def test_lengths_around_blocks_and_steps(alpha, causal, Hq, Hkv, D, scale):
+    g = torch.Generator().manual_seed(3)
+    N = 517
+    varlen = torch.tensor([517, 1, 32, 33, 127, 129, 384], dtype=torch.int32)
+    B = len(varlen)
+    q = scale * torch.randn(B, Hq, N, D, generator=g)
+    k, v = (torch.randn(B, Hkv, N, D, generator=g) for _ in range(2))
+    dout = torch.randn(B, Hq, N, D, generator=g)
+    want = [exact.dense_entmax_attention(q, k, v, alpha, causal, varlen)]
+    want += list(exact.dense_entmax_attention_grads(q, k, v, dout, alpha, causal, varlen))
+    for b, n in enumerate(varlen.tolist()):  # the padding may hold anything
+        for t in (q, k, v):
+            t[b, :, n:] = float("nan")
+    got = run(q, k, v, dout, varlen, alpha, causal, Hq != Hkv)
+    for name, a, w in zip(("out", "dq", "dk", "dv"), got, want):
+        assert torch.isfinite(a).all(), name
+        for b, n in enumerate(varlen.tolist()):
+            assert (a[b, :, n:] == 0).all(), name
+        assert max_err(a, w) < TOL, name
+
+
+@pytest.mark.parametrize("N,scale", [(64, 1.0), (2048, 1.0), (2048, 0.125), (4096, 3.0)])
+def test_same_bits_on_every_call_and_long_rows(N, scale):
+    g = torch.Generator().manual_seed(4)
+    q = scale * torch.randn(1, 4, N, 64, generator=g)
+    k, v = (torch.randn(1, 1, N, 64, generator=g) for _ in range(2))
+    dout = torch.randn(1, 4, N, 64, generator=g)
+    first = run(q, k, v, dout, None, 1.5, True, True)
+    again = run(q, k, v, dout, None, 1.5, True, True)
+    assert all(torch.equal(a, b) for a, b in zip(first, again))
+    want = [exact.dense_entmax_attention(q, k, v, 1.5, True)]
+    want += list(exact.dense_entmax_attention_grads(q, k, v, dout, 1.5, True))
+    # Beyond unit scale the bound grows with q: scores of that size round by as much more, a probability's root u moves by
+    # what its score is off, and dK sums u (dP - delta) q.
+    tol = TOL * max(1.0, scale)
+    for name, a, w in zip(("out", "dq", "dk", "dv"), first, want):
+        assert max_err(a, w) < tol, name
