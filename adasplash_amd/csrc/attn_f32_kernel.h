@@ -37,22 +37,34 @@ constexpr int kListBytes = kWaves * kCap * kRows * 6;  // a score (fp32) and a k
 // position of 16-byte piece c of chunk row r
 __device__ __forceinline__ int piece_sw(int row) { return (row >> 1) & 7; }
 
-// A wave's ring of chunks and its place in it.
-struct Ring {
+// A wave's ring of chunks and its place in it; kStride: bytes per row of the tensors its chunks come from.
+template <int kStride> struct Ring {
   unsigned char* base;  // the wave's three chunks
   int lane;
-  int st;  // stage of the next chunk to be consumed
-  // chunk c (32 columns) of rows [row0, row0 + 32) of a row-major tensor with `stride` bytes per row into stage `s`; rows
-  // from `limit` on are replaced by the last one in front of it
-  __device__ __forceinline__ void issue(const unsigned char* g, int row0, int limit, int stride, int c, int s) const {
-    const unsigned char* gb = uniform_ptr(g + c * 128);
+  uint32_t off[2];      // the lane's place in an even / odd group of eight rows, from the group's first row
+  int st;               // stage of the next chunk to be consumed
+  __device__ __forceinline__ Ring(unsigned char* b, int l) : base(b), lane(l), st(0) {
+    const int p0 = (l & 7) ^ (l >> 4);
+    off[0] = (uint32_t)((l >> 3) * kStride + p0 * 16);
+    off[1] = (uint32_t)((l >> 3) * kStride + (p0 ^ 4) * 16);
+  }
+  // chunk c (32 columns) of rows [row0, row0 + 32) of a row-major tensor into stage `s`; rows from `limit` on are replaced
+  // by the last one in front of it
+  __device__ __forceinline__ void issue(const unsigned char* g, int row0, int limit, int c, int s) const {
     unsigned char* l = base + s * kChunk;
-    const int p0 = (lane & 7) ^ (lane >> 4);
+    if (row0 + kRows <= limit) {
+      const unsigned char* gb = uniform_ptr(g + (size_t)row0 * kStride + c * 128);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      int r = row0 + 8 * j + (lane >> 3);
-      r = r < limit ? r : limit - 1;
-      dma16s(gb, (uint32_t)r * (uint32_t)stride + (uint32_t)((p0 ^ (4 * (j & 1))) * 16), l + j * 1024);
+      for (int j = 0; j < 4; ++j) dma16s(gb + j * (8 * kStride), off[j & 1], l + j * 1024);
+    } else {
+      const unsigned char* gb = uniform_ptr(g + c * 128);
+      const int p0 = (lane & 7) ^ (lane >> 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        int r = row0 + 8 * j + (lane >> 3);
+        r = r < limit ? r : limit - 1;
+        dma16s(gb, (uint32_t)r * (uint32_t)kStride + (uint32_t)((p0 ^ (4 * (j & 1))) * 16), l + j * 1024);
+      }
     }
   }
   // Waits for the oldest of the two chunks under way and for the wave's own LDS reads (the stage the caller fills next is
@@ -68,8 +80,8 @@ struct Ring {
 
 // Walks the blocks wave, wave + 4, ... below n_blk.  Each block is SEQ chunks, src(blk, s, ring, stage) issues number s of
 // them; body(blk, next) consumes them by SEQ calls of next(s) in order, which return the chunk's LDS address.
-template <int SEQ, typename Src, typename Body>
-__device__ __forceinline__ void walk(Ring& ring, int first, int n_blk, int step, Src&& src, Body&& body) {
+template <int SEQ, typename R, typename Src, typename Body>
+__device__ __forceinline__ void walk(R& ring, int first, int n_blk, int step, Src&& src, Body&& body) {
   if (first >= n_blk) return;
   ring.st = 0;
   src(first, 0, 0);
@@ -87,15 +99,22 @@ __device__ __forceinline__ void walk(Ring& ring, int first, int n_blk, int step,
   ring.drain();
 }
 
-// acc += (chunk rows) . (the lane's own row), columns 32 c .. 32 c + 31: f holds the lane's row, 8 g + 4 lh .. + 3 of every 8
-__device__ __forceinline__ void dot_chunk(f32x16& acc, uint32_t chunk, uint32_t row_lane, const uint32_t* f) {
+// acc += (chunk rows) . (the lane's own row), columns 32 c .. 32 c + 31: f holds the lane's row, 8 g + 4 lh .. + 3 of every
+// 8.  kParts: a chunk's 32 products are added up from zero and the chunks' sums then, shorter chains of smaller numbers (where
+// the registers allow it).
+template <bool kParts> __device__ __forceinline__ void dot_chunk(f32x16& acc, uint32_t chunk, uint32_t row_lane, const uint32_t* f) {
   f32x4 a[4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) a[g] = __builtin_bit_cast(f32x4, lds_read16((chunk + row_lane) ^ (g << 5)));
+  f32x16 part;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) part[i] = kParts ? 0.f : acc[i];
 #pragma unroll
   for (int g = 0; g < 4; ++g)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g][e], __builtin_bit_cast(float, f[g * 4 + e]), acc, 0, 0, 0);
+    for (int e = 0; e < 4; ++e) part = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g][e], __builtin_bit_cast(float, f[g * 4 + e]), part, 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = kParts ? acc[i] + part[i] : part[i];
 }
 // o[column of the chunk][lane's row] += sum over the chunk's rows of chunk[row][column] * w[row]; w in accumulator order
 __device__ __forceinline__ void acc_chunk(f32x16& o, uint32_t chunk, uint32_t col_lane, const float (&w)[16]) {
@@ -154,10 +173,19 @@ template <int D> __device__ __forceinline__ void load_row(const float* row, int 
   }
 }
 
+// over the eight lanes of a row: two quad permutations and a mirror of eight lanes, without a trip through LDS
+template <int kCtrl> __device__ __forceinline__ float dpp(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), kCtrl, 0xf, 0xf, true));
+}
 __device__ __forceinline__ float sum8(float x) {
-  x += __shfl_xor(x, 1, 64);
-  x += __shfl_xor(x, 2, 64);
-  return x + __shfl_xor(x, 4, 64);
+  x += dpp<0xb1>(x);   // quad_perm [1, 0, 3, 2]
+  x += dpp<0x4e>(x);   // quad_perm [2, 3, 0, 1]
+  return x + dpp<0x141>(x);  // row_half_mirror
+}
+__device__ __forceinline__ float max8(float x) {
+  x = fmaxf(x, dpp<0xb1>(x));
+  x = fmaxf(x, dpp<0x4e>(x));
+  return fmaxf(x, dpp<0x141>(x));
 }
 
 // u^c0 and u^(c0 - 1) of u >= 0
@@ -233,16 +261,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   uint32_t qf[D / 2];
   load_row<D>(reinterpret_cast<const float*>(p.q) + (q_row0 + (live ? qi : L - 1)) * D, lh, qf);
 
-  Ring ring{smem + wave * (kStages * kChunk), lane, 0};
+  Ring<kStride> ring(smem + wave * (kStages * kChunk), lane);
   const uint32_t rl = row_lane_of(lq, lh), cl = col_lane_of(lq, lh);
-  auto src_k = [&](int blk, int s, int st) { ring.issue(kg, blk * kRows, L, kStride, s, st); };
+  auto src_k = [&](int blk, int s, int st) { ring.issue(kg, blk * kRows, L, s, st); };
   // scores of a block less `sub`, -inf on the keys the row may not see
   auto scores = [&](int blk, float init, auto&& next) -> f32x16 {
     f32x16 acc;
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = init;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) dot_chunk(acc, next(c), rl, qf + c * 16);
+    for (int c = 0; c < NC; ++c) dot_chunk<true>(acc, next(c), rl, qf + c * 16);
     const int k0 = blk * kRows;
     if (k0 + kRows > L || (p.causal && k0 + kRows - 1 > m0)) {
       const int jb = k0 + 4 * lh;
@@ -254,6 +282,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   // ---- the walk that lists: rows are solved on the lists after 1, 2, 4, ... steps of four blocks and behind the last ----
   if (tid == 0) over_flag = 0u;
+  if (tid < kRows) t_lds[tid] = -INFINITY;
   float t_raw = -INFINITY;  // bound of the lane's row, raw score units
   int n_mine = 0;           // entries of this lane: lh = 0 fills the wave's slots of the row from the front, lh = 1 from the back
   bool over = false;
@@ -265,7 +294,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int srow = wave * 8 + (lane >> 3), sj = lane & 7;
   float sv[16];  // the lane's share of the row's listed scores, relative to their maximum, in z units
   float s_max = 0.f, s_tau = 0.f;
-  auto solve = [&]() {
+  auto solve = [&](bool last) {
     float x[16];
     s_max = -INFINITY;
 #pragma unroll
@@ -280,15 +309,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         s_max = fmaxf(s_max, x[w * 4 + k]);
       }
     }
-    s_max = fmaxf(s_max, __shfl_xor(s_max, 1, 64));
-    s_max = fmaxf(s_max, __shfl_xor(s_max, 2, 64));
-    s_max = fmaxf(s_max, __shfl_xor(s_max, 4, 64));
+    s_max = max8(s_max);
     const float m = s_max > -INFINITY ? s_max : 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) sv[i] = (x[i] - m) * qs;
-    s_tau = -1.f;
+    // from the bound the row has already; on the way a few steps do, each of which ends on a bound
+    s_tau = fmaxf(-1.f, (t_lds[srow] - m) * qs);
     bool go = s_max > -INFINITY;
-    for (int it = 0; it < 40 && __builtin_amdgcn_ballot_w64(go) != 0ull; ++it) {
+    const int most = last ? 40 : 4;
+    for (int it = 0; it < most && __builtin_amdgcn_ballot_w64(go) != 0ull; ++it) {
       float s0 = 0.f, s1 = 0.f;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
@@ -301,7 +330,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       s1 = sum8(s1);
       const float step = norm_step<AM>(s0, s1, c0);
       if (go) s_tau = fminf(s_tau + step, 0.f);
-      go = go && step > 2e-7f;
+      go = go && step > (last ? 1e-7f : 1e-3f);
     }
   };
   bool fallback = false;
@@ -312,7 +341,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       n_lds[wave][lh][lq] = (uint8_t)n_mine;
       if (over) over_flag = 1u;
       __syncthreads();
-      solve();
+      solve(step_no == n_steps);
       if (sj == 0) {
         // (the margin covers the rounding of the difference and of the product back to raw units)
         t_lds[srow] = s_max > -INFINITY ? (s_max + (s_tau - 1e-6f) * inv_qs) - 4e-7f * fabsf(s_max) : -INFINITY;
@@ -494,7 +523,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[c][i] = 0.f;
   float psum = 0.f;
-  auto src_kv = [&](int blk, int s, int st) { ring.issue(s < NC ? kg : vg, blk * kRows, L, kStride, s < NC ? s : s - NC, st); };
+  auto src_kv = [&](int blk, int s, int st) { ring.issue(s < NC ? kg : vg, blk * kRows, L, s < NC ? s : s - NC, st); };
   walk<2 * NC>(ring, wave, n_kblk, kWaves, src_kv, [&](int blk, auto&& next) {
     const f32x16 s = scores(blk, -t, next);
     float w[16];
@@ -566,11 +595,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     load_row<D>(reinterpret_cast<const float*>(p.q) + r * D, lh, qf);
     load_row<D>(reinterpret_cast<const float*>(p.dout) + r * D, lh, dof);
   }
-  Ring ring{smem + wave * (kStages * kChunk), lane, 0};
+  Ring<kStride> ring(smem + wave * (kStages * kChunk), lane);
   const uint32_t rl = row_lane_of(lq, lh), cl = col_lane_of(lq, lh);
   // chunks of a block: K, V and, for the second walk, K again
   auto src = [&](int blk, int s, int st) {
-    ring.issue(s < NC || s >= 2 * NC ? kg : vg, blk * kRows, L, kStride, s < NC ? s : (s < 2 * NC ? s - NC : s - 2 * NC), st);
+    ring.issue(s < NC || s >= 2 * NC ? kg : vg, blk * kRows, L, s < NC ? s : (s < 2 * NC ? s - NC : s - 2 * NC), st);
   };
   // r = z - tau (-inf where the row may not look); false when no row of the block has a member, whose dP is then not formed
   auto block_terms = [&](int blk, auto&& next, float (&r)[16], f32x16& dp) -> bool {
@@ -578,7 +607,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) dot_chunk(s, next(c), rl, qf + c * 16);
+    for (int c = 0; c < NC; ++c) dot_chunk<D == 64>(s, next(c), rl, qf + c * 16);
     const int jb = blk * kRows + 4 * lh;
     float mx = -INFINITY;
 #pragma unroll
@@ -590,7 +619,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(NC + c);
-      if (any) dot_chunk(dp, a, rl, dof + c * 16);
+      if (any) dot_chunk<D == 64>(dp, a, rl, dof + c * 16);
     }
     return any;
   };
@@ -691,13 +720,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   const int q_first = p.causal ? kblk : 0;            // first query block that sees the keys
   const int n_q = (L + kRows - 1) / kRows - q_first;  // query blocks per head
   const size_t q_head0 = (size_t)(b * p.Hq + kvh * group) * N;
-  Ring ring{smem + wave * (kStages * kChunk), lane, 0};
+  Ring<kStride> ring(smem + wave * (kStages * kChunk), lane);
   const uint32_t rl = row_lane_of(lq, lh), cl = col_lane_of(lq, lh);
   // item x = head * n_q + query block - q_first; its chunks: Q, dO, dO and Q again
   auto src = [&](int x, int s, int st) {
     const int g = x / n_q, qb = q_first + (x - g * n_q);
     const unsigned char* base = reinterpret_cast<const unsigned char*>(s < NC || s >= 3 * NC ? p.q : p.dout) + (q_head0 + (size_t)g * N) * kStride;
-    ring.issue(base, qb * kRows, L, kStride, s % NC, st);
+    ring.issue(base, qb * kRows, L, s % NC, st);
   };
   f32x16 ov[NC], ok[NC];
 #pragma unroll
@@ -709,35 +738,54 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     f32x16 s, dp;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
+    // tau, 1 / sum p and delta of the lane's sixteen queries
+    const size_t at = q_head0 + (size_t)g * N;
+    const bool whole = q0 + kRows <= L;
+    auto scalars = [&](const float* x, float (&y)[16]) {
+      typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+      if (whole) {
 #pragma unroll
-    for (int c = 0; c < NC; ++c) dot_chunk(s, next(c), rl, kf + c * 16);
-    const float* tau = p.taus + q_head0 + (size_t)g * N;
-    const float* zi = p.zinv + q_head0 + (size_t)g * N;
-    const float* de = p.delta + q_head0 + (size_t)g * N;
+        for (int i = 0; i < 4; ++i) {
+          const f32x4_u v4 = *reinterpret_cast<const f32x4_u*>(x + at + q0 + 8 * i + 4 * lh);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[4 * i + e] = v4[e];
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int qrow = q0 + 8 * (i >> 2) + 4 * lh + (i & 3);
+          y[i] = x[at + (qrow < L ? qrow : L - 1)];
+        }
+      }
+    };
+    float tau[16], zi[16], de[16];
+    scalars(p.taus, tau);
+    scalars(p.zinv, zi);
+    scalars(p.delta, de);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) dot_chunk<D == 64>(s, next(c), rl, kf + c * 16);
     float r[16], w[16], dx[16];
     float mx = -INFINITY;
+    const bool plain = whole && n0 + kRows <= L && (!p.causal || n0 + kRows - 1 <= q0);  // every query of the block sees every key
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int qrow = q0 + 8 * (i >> 2) + 4 * lh + (i & 3);
-      const int qc = qrow < L ? qrow : L - 1;
-      const bool see = live && qrow < L && (!p.causal || kj <= qrow);
-      r[i] = see ? fmaf(s[i], p.qscale, -tau[qc]) : -INFINITY;
+      const bool see = plain || (live && qrow < L && (!p.causal || kj <= qrow));
+      r[i] = see ? fmaf(s[i], p.qscale, -tau[i]) : -INFINITY;
       mx = fmaxf(mx, r[i]);
     }
     const bool any = __builtin_amdgcn_ballot_w64(mx > 0.f) != 0ull;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(NC + c);
-      if (any) dot_chunk(dp, a, rl, vf + c * 16);
+      if (any) dot_chunk<D == 64>(dp, a, rl, vf + c * 16);
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int qrow = q0 + 8 * (i >> 2) + 4 * lh + (i & 3);
-      const int qc = qrow < L ? qrow : L - 1;
       float pr, u;
       bwd_prob<AM>(r[i], p.c0, pr, u);
-      w[i] = pr > 0.f ? pr * zi[qc] : 0.f;
-      dx[i] = u > 0.f ? u * (dp[i] - de[qc]) : 0.f;
+      w[i] = pr > 0.f ? pr * zi[i] : 0.f;
+      dx[i] = u > 0.f ? u * (dp[i] - de[i]) : 0.f;
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
