@@ -92,49 +92,68 @@ static int mask_words_of(int N) { return ((N + kBN - 1) / kBN + 31) / 32; }
 // sparse-support kernels leave the row blocks that see more keys to the dense kernels without spending a walk on
 // them.  The prediction only decides which kernel does the work (a row block it gets wrong is caught by the kernel's
 // own checks), and it depends on the inputs alone: the same call takes the same way every time.
-template <typename T>
-__global__ __launch_bounds__(256) void attn_probe_kernel(AttnParams p, int D, int am) {
-  __shared__ float qrows[4][256];
+//
+// What bounds it is latency, one workgroup per K/V head in front of the real work: the sampled keys' rows are all under way
+// before the query rows are waited for, and the length whose predicted support just fits comes from the support point instead
+// of the other way round -- a lane takes an a, n(a) = 1 / (mass above a per key) and support n(a) Q(a) are closed forms that
+// grow with a, and a second look between the two neighbouring lanes refines it (bisecting a for 64 lengths
+// took 14 rounds, each an integral of 32 terms at a generic alpha).  192 heads, D = 64: 10.7 -> 6.7 us a launch.
+//
+// In front of a backward it clears the control words and flags of the dK/dV kernels as well (`ctrl2`, `kv_flags`).
+template <typename T, int D>
+__global__ __launch_bounds__(256) void attn_probe_kernel(AttnParams p, int am, uint32_t* ctrl2, int32_t* kv_flags) {
+  __shared__ __align__(16) float qrows[4][D];
   __shared__ float red[4][2][4];
   __shared__ float ksum[4];
   const int u = blockIdx.x, tid = threadIdx.x;
   const int units = p.B * p.Hkv;
   uint32_t* const ctrl = p.queue;
-  if (u == 0 && tid < 11) ctrl[tid] = 0u;
-  if (u == 0 && tid < 2) ctrl[64 + 2 * units + tid] = 0u;
-  if (tid < 2) ctrl[64 + 2 * u + tid] = 0u;
   const int b = u / p.Hkv, kvh = u % p.Hkv, group = p.Hq / p.Hkv;
-  if (p.save_flags)  // supports kept for the backward: no row block of this K/V head has a valid stream yet
-    for (int i = tid; i < group * p.n_mblk; i += 256) p.save_flags[(size_t)(b * p.Hq + kvh * group) * p.n_mblk + i] = 0;
   int L = p.N;
   if (p.varlen) {
     long long l = p.varlen_bits == 64 ? ((const long long*)p.varlen)[b] : (long long)((const int*)p.varlen)[b];
     L = (int)(l < 0 ? 0 : (l > p.N ? p.N : l));
   }
+  if (u == 0 && tid < 11) ctrl[tid] = 0u;
+  if (u == 0 && tid < 2) ctrl[64 + 2 * units + tid] = 0u;
+  if (tid < 2) ctrl[64 + 2 * u + tid] = 0u;
+  if (ctrl2 && u == 0 && tid < 11) ctrl2[tid] = 0u;
+  if (kv_flags) {
+    const int n_mblk = (p.N + kMaskRows - 1) / kMaskRows;
+    for (int i = tid; i < n_mblk; i += 256) kv_flags[(size_t)u * n_mblk + i] = 0;
+  }
+  if (p.save_flags)  // supports kept for the backward: no row block of this K/V head has a valid stream yet
+    for (int i = tid; i < group * p.n_mblk; i += 256) p.save_flags[(size_t)(b * p.Hq + kvh * group) * p.n_mblk + i] = 0;
   if (p.w1_scales && tid < 4) p.w1_scales[4 * u + tid] = tid < 2 ? 1.f : (tid == 2 ? INFINITY : 0.f);
   if (L < 256) return;  // short sequences: finding out in the kernel costs little
   int rows[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) rows[j] = L - 1 - j * (L / 16);
-  const uint16_t* qbase = reinterpret_cast<const uint16_t*>(p.q) + ((size_t)(b * p.Hq + kvh * group) * p.N) * D;
-  for (int i = tid; i < 4 * D; i += 256) {
-    const uint32_t w = qbase[(size_t)rows[i / D] * D + i % D];
-    qrows[i / D][i % D] = elem_traits<T>::kIsBf16 ? bf16_bits_to_float(w) : f16_bits_to_float(w);
-  }
-  __syncthreads();
   const int span = (p.causal ? rows[3] + 1 : L);
   const int key = (int)(((long long)tid * span) / 256);
-  const uint16_t* krow = reinterpret_cast<const uint16_t*>(p.k) + ((size_t)(b * p.Hkv + kvh) * p.N + key) * D;
+  const u32x4* krow = reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p.k) + ((size_t)(b * p.Hkv + kvh) * p.N + key) * D);
+  u32x4 kw[D / 8];
+#pragma unroll
+  for (int c = 0; c < D / 8; ++c) kw[c] = krow[c];
+  const uint16_t* qbase = reinterpret_cast<const uint16_t*>(p.q) + ((size_t)(b * p.Hq + kvh * group) * p.N) * D;
+#pragma unroll
+  for (int x = 0; x < 4 * D / 256; ++x) {
+    const int i = x * 256 + tid, j = i / D;
+    const uint32_t w = qbase[(size_t)(L - 1 - j * (L / 16)) * D + i % D];
+    qrows[j][i % D] = elem_traits<T>::kIsBf16 ? bf16_bits_to_float(w) : f16_bits_to_float(w);
+  }
+  __syncthreads();
   float dot[4] = {0.f, 0.f, 0.f, 0.f};
   float ksq = 0.f;
-  for (int d = 0; d < D; d += 8) {
-    const u32x4 w = *reinterpret_cast<const u32x4*>(krow + d);
+#pragma unroll
+  for (int c = 0; c < D / 8; ++c) {
+    __builtin_amdgcn_sched_barrier(0);  // (all of the query rows' LDS reads ahead of the first product would not fit the registers)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float lo = unpack_lo<T>(w[e]), hi = unpack_hi<T>(w[e]);
+      const float lo = unpack_lo<T>(kw[c][e]), hi = unpack_hi<T>(kw[c][e]);
       ksq = fmaf(lo, lo, fmaf(hi, hi, ksq));
 #pragma unroll
-      for (int j = 0; j < 4; ++j) dot[j] = fmaf(lo, qrows[j][d + 2 * e], fmaf(hi, qrows[j][d + 2 * e + 1], dot[j]));
+      for (int j = 0; j < 4; ++j) dot[j] = fmaf(lo, qrows[j][8 * c + 2 * e], fmaf(hi, qrows[j][8 * c + 2 * e + 1], dot[j]));
     }
   }
 #pragma unroll
@@ -168,10 +187,8 @@ __global__ __launch_bounds__(256) void attn_probe_kernel(AttnParams p, int D, in
     }
   }
   if (tid >= 64) return;
-  // The first wave: the score spread pooled over the four sampled rows, and for 64 row lengths n (a geometric grid from
-  // 64 to a million keys, one per lane) the support a Gaussian score distribution of that spread would have.  The
-  // prediction grows with n; the largest n whose support still fits is what the sparse-support kernels compare a row
-  // block's keys with.
+  // The first wave: the score spread pooled over the four sampled rows, and the largest n whose support, were the scores
+  // Gaussian with that spread, still fits: what the sparse-support kernels compare a row block's keys with.
   float var = 0.f;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -181,30 +198,47 @@ __global__ __launch_bounds__(256) void attn_probe_kernel(AttnParams p, int D, in
     var += 0.25f * fmaxf(s2 / 256.f - mean * mean, 0.f);
   }
   const float sd = sqrtf(var);
-  const float n = 64.f * exp2f((float)tid * (14.f / 63.f));
-  float lo = -2.f, hi = 7.f;
-  for (int it = 0; it < 14; ++it) {
-    const float a = 0.5f * (lo + hi);
+  // keys whose rows have their threshold `a` spreads above the mean, and the support of such a row
+  auto keys_at = [&](float a, float& support) -> float {
     const float Q = 0.5f * erfcf(a * 0.70710678f), phi = 0.39894228f * __expf(-0.5f * a * a);
-    float f;
-    if (am == ATT_2) f = n * sd * (phi - a * Q);
-    else if (am == ATT_15) f = n * var * ((1.f + a * a) * Q - a * phi);
-    else {  // any alpha: n E[(sd (Z - a))_+^c0] by the midpoint rule over [a, a + 8]
+    float f;  // mass of one key
+    if (am == ATT_2) f = sd * (phi - a * Q);
+    else if (am == ATT_15) f = var * ((1.f + a * a) * Q - a * phi);
+    else {  // any alpha: E[(sd (Z - a))_+^c0] by the midpoint rule over [a, a + 8]
       float acc = 0.f;
+#pragma unroll 4
       for (int i = 0; i < 32; ++i) {
         const float x = 0.25f * ((float)i + 0.5f);
         acc += __expf(p.c0 * __logf(sd * x)) * 0.39894228f * __expf(-0.5f * (a + x) * (a + x));
       }
-      f = n * acc * 0.25f;
+      f = acc * 0.25f;
     }
-    if (f > 1.f) lo = a;
-    else hi = a;
+    const float n = f > 0.f ? 1.f / f : INFINITY;
+    support = n * Q;
+    return n;
+  };
+  float lo = -2.f, width = 9.f, n_true = 0.f;
+  for (int round = 0; round < 2; ++round) {
+    const float step = width * (1.f / 63.f);
+    float support;
+    const float n = keys_at(lo + (float)tid * step, support);
+    const unsigned long long fits = __builtin_amdgcn_ballot_w64(support <= p.probe_max_support);
+    // (support grows with a: the lanes that fit are the first ones.  None: the threshold lies below every key of any length
+    // considered, the support is the whole row; a spread of zero or a NaN ends here too)
+    const int last = fits == ~0ull ? 63 : __builtin_ctzll(~fits) - 1;
+    if (last < 0) {
+      if (round == 0) n_true = p.probe_max_support * (1.f / 0.97725f);
+      break;
+    }
+    // (all of them: even the shortest lengths have their threshold above the range, and so few keys there that any fits)
+    n_true = round == 0 && last == 63 ? INFINITY : __shfl(n, last, 64);
+    lo += (float)last * step;
+    width = step;
+    if (last == 63) break;
   }
-  const float support = n * 0.5f * erfcf(0.5f * (lo + hi) * 0.70710678f);
-  const unsigned long long fits = __builtin_amdgcn_ballot_w64(support <= p.probe_max_support);
-  // (a spread of zero or a NaN predicts nothing: every length fits, and the kernels find out for themselves)
-  const int top = fits == 0ull ? -1 : 63 - __builtin_clzll(fits);
-  const float n_fit = top < 0 ? 0.f : (top == 63 ? INFINITY : 64.f * exp2f((float)top * (14.f / 63.f)));
+  // on a geometric grid of lengths from 64 to a million keys, rounded down
+  const float top = floorf(log2f(n_true * (1.f / 64.f)) * (63.f / 14.f) + 1e-4f);
+  const float n_fit = n_true < 64.f ? 0.f : (top >= 63.f ? INFINITY : 64.f * exp2f(top * (14.f / 63.f)));
   if (tid != 0) return;
   // A head goes one way as a whole: by its longest rows, which see all L keys and hold most of the work.  (Serving only
   // its shorter row blocks from their supports was measured and loses: for a row block of few tiles the fixed cost of the
@@ -264,6 +298,18 @@ static SupportsLayout supports_layout(int B, int Hq, int Hkv, int N, int D, int 
 }
 __global__ __launch_bounds__(256) void fill_zero_kernel(int32_t* x, long long n) {
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) x[i] = 0;
+}
+
+// the kernel for the head dims the sparse-support kernels serve
+static void launch_probe(const AttnParams& p, int D, int dtype, int am, uint32_t* ctrl2, int32_t* kv_flags, hipStream_t s) {
+  const dim3 grid((unsigned)(p.B * p.Hkv));
+  if (dtype == ADSP_BF16) {
+    if (D == 64) hipLaunchKernelGGL((attn_probe_kernel<bf16_t, 64>), grid, dim3(256), 0, s, p, am, ctrl2, kv_flags);
+    else hipLaunchKernelGGL((attn_probe_kernel<bf16_t, 128>), grid, dim3(256), 0, s, p, am, ctrl2, kv_flags);
+  } else {
+    if (D == 64) hipLaunchKernelGGL((attn_probe_kernel<f16_t, 64>), grid, dim3(256), 0, s, p, am, ctrl2, kv_flags);
+    else hipLaunchKernelGGL((attn_probe_kernel<f16_t, 128>), grid, dim3(256), 0, s, p, am, ctrl2, kv_flags);
+  }
 }
 
 // ADSP_SPARSE=0 in the environment keeps every row block on the dense kernel (for comparisons and tests).
@@ -395,11 +441,10 @@ static int attn_common(const void* q, const void* k, const void* v, void* out, f
         p.save_streams = sp + sl.streams_off;
       }
       const dim3 k8_grid((unsigned)(((long long)p.Npad * (D / 16) + 255) / 256), (unsigned)(B * Hkv));
+      launch_probe(p, D, dtype, am, nullptr, nullptr, s);
       if (dtype == ADSP_BF16) {
-        hipLaunchKernelGGL(attn_probe_kernel<bf16_t>, dim3((unsigned)(B * Hkv)), dim3(256), 0, s, p, D, am);
         hipLaunchKernelGGL(k8_layout_kernel<bf16_t>, k8_grid, dim3(256), 0, s, (const uint16_t*)k, ws + w.k8_off, N, p.Npad, D, (const uint32_t*)p.hints, (const float*)p.w1_scales);
       } else {
-        hipLaunchKernelGGL(attn_probe_kernel<f16_t>, dim3((unsigned)(B * Hkv)), dim3(256), 0, s, p, D, am);
         hipLaunchKernelGGL(k8_layout_kernel<f16_t>, k8_grid, dim3(256), 0, s, (const uint16_t*)k, ws + w.k8_off, N, p.Npad, D, (const uint32_t*)p.hints, (const float*)p.w1_scales);
       }
       int rc = dtype == ADSP_BF16 ? (D == 64 ? launch_attn_sparse_bf16_d64(p, am, w.slots, s) : launch_attn_sparse_bf16_d128(p, am, w.slots, s))
@@ -540,10 +585,10 @@ static BwdWorkspace bwd_workspace(int B, int Hq, int Hkv, int N, int D, int dtyp
     w.queue_off = align256(w.copies_bytes);
     w.flags_off = align256(w.queue_off + 256 + ((size_t)B * Hkv + 1) * 8);
     w.events_off = align256(w.flags_off + (size_t)items * 4);
-    // the dK/dV kernel: control words and the probe's verdict per K/V head once more, a flag per (K/V head, key
+    // the dK/dV kernel: control words, a flag per (K/V head, key
     // block), fp32 sums per workgroup and fp32 partial rows of dK and dV per query head
     w.queue2_off = align256(w.events_off + (size_t)slots * kSparseSlotBytes);
-    w.kvflags_off = align256(w.queue2_off + 256 + ((size_t)B * Hkv + 1) * 8);
+    w.kvflags_off = align256(w.queue2_off + 256);
     // (fp32 sums of an item worked off in parts: 32 rows of dK | dV per wave of every workgroup)
     w.scratch_off = align256(w.kvflags_off + (size_t)B * Hkv * mblocks_of(N) * 4);
     w.part_off = align256(w.scratch_off + (size_t)slots * 4 * 32 * 2 * D * 4);
@@ -564,20 +609,6 @@ static BwdWorkspace bwd_workspace(int B, int Hq, int Hkv, int N, int D, int dtyp
     w.total = w.dir_off + align256((size_t)items * 4 * w.dir_stride * 2);
   }
   return w;
-}
-
-// Clears the control words and key-block flags of the sparse-support dK/dV kernel and copies the probe's verdict per
-// K/V head (the dQ kernel's words) into the kernel's own.
-__global__ __launch_bounds__(256) void bwd_ctrl_clear_kernel(uint32_t* ctrl2, const uint32_t* hints1, int units, int32_t* kv_flags,
-                                                            long long n_flags) {
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (i < 10) ctrl2[i] = 0u;
-  if (i < units) {
-    ctrl2[64 + 2 * i] = hints1[2 * i] >= (1u << 20) ? (1u << 20) : 0u;
-    ctrl2[64 + 2 * i + 1] = 0u;
-  }
-  if (i < 2) ctrl2[64 + 2 * units + i] = 0u;
-  for (long long j = i; j < n_flags; j += (long long)gridDim.x * 256) kv_flags[j] = 0;
 }
 
 // dK, dV = sum over the query heads of a K/V head of the sparse-support kernel's fp32 partial rows; key blocks left to
@@ -688,7 +719,6 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   p.hints = nullptr;
   p.events = nullptr;
   p.queue2 = nullptr;
-  p.hints2 = nullptr;
   p.kv_flags = nullptr;
   p.dk_part = nullptr;
   p.dv_part = nullptr;
@@ -752,12 +782,11 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
       pp.queue = p.queue;
       pp.hints = p.hints;
       pp.probe_max_support = probe_max_support();
+      launch_probe(pp, D, dtype, am, (uint32_t*)(ws + w.queue2_off), (int32_t*)(ws + w.kvflags_off), s);
       int rc;
       if (dtype == ADSP_BF16) {
-        hipLaunchKernelGGL(attn_probe_kernel<bf16_t>, dim3((unsigned)(B * Hkv)), dim3(256), 0, s, pp, D, am);
         rc = D == 64 ? launch_attn_bwd_sparse_bf16_d64(p, am, 0, w.slots, s) : launch_attn_bwd_sparse_bf16_d128(p, am, 0, w.slots, s);
       } else {
-        hipLaunchKernelGGL(attn_probe_kernel<f16_t>, dim3((unsigned)(B * Hkv)), dim3(256), 0, s, pp, D, am);
         rc = D == 64 ? launch_attn_bwd_sparse_f16_d64(p, am, 0, w.slots, s) : launch_attn_bwd_sparse_f16_d128(p, am, 0, w.slots, s);
       }
       if (rc != 0) return ADSP_ERR_LAUNCH;
@@ -778,7 +807,6 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   {
     unsigned char* ws = (unsigned char*)workspace;
     p.queue2 = (uint32_t*)(ws + w.queue2_off);
-    p.hints2 = p.queue2 + 64;
     p.kv_flags = (int32_t*)(ws + w.kvflags_off);
     p.part_scratch = (float*)(ws + w.scratch_off);
     if (p.streams) p.merge256 = w.merge256;
@@ -787,13 +815,6 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
       p.dk_part = (float*)(ws + w.part_off);
       p.dv_part = (float*)(ws + w.part_off + w.part_bytes);
     }
-    const long long n_flags = (long long)B * Hkv * mblocks_of(N);
-    long long clear_items = n_flags > (long long)B * Hkv ? n_flags : (long long)B * Hkv;  // (at least one thread per K/V head and per control word)
-    if (clear_items < 10) clear_items = 10;
-    long long clear_blocks = (clear_items + 255) / 256;
-    if (clear_blocks > 1024) clear_blocks = 1024;
-    hipLaunchKernelGGL(bwd_ctrl_clear_kernel, dim3((unsigned)clear_blocks), dim3(256), 0, s, p.queue2, (const uint32_t*)p.hints, B * Hkv,
-                       p.kv_flags, n_flags);
     int rc;
     const int kind = p.streams ? 2 : 1;  // from the dQ kernel's streams, or with a walk of its own
     if (dtype == ADSP_BF16) rc = D == 64 ? launch_attn_bwd_sparse_bf16_d64(p, am, kind, w.slots, s) : launch_attn_bwd_sparse_bf16_d128(p, am, kind, w.slots, s);

@@ -28,7 +28,6 @@ struct AttnBwdParams {
   // [B, Hq, part_rows, D] when a K/V head serves several query heads (null otherwise), and per workgroup and wave 32 fp32
   // rows of dK | dV for the sums of an item that is worked off in parts; the streams are shared
   uint32_t* queue2;
-  uint32_t* hints2;
   int32_t* kv_flags;  // [B, Hkv, n_mblk] 1 = key block left to attn_bwd_dkdv_kernel
   float* dk_part;
   float* dv_part;

@@ -744,7 +744,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
   static_assert(kKStep && G::kKLoads % NW == 0, "head dims 32 .. 128");
 
   // (the probe left too little to this kernel: the dense kernel serves everything)
-  if (sparse_steps_aside(p.hints2, p.varlen, p.varlen_bits, p.B, p.Hkv, p.N)) {
+  if (sparse_steps_aside(p.hints, p.varlen, p.varlen_bits, p.B, p.Hkv, p.N)) {
     if (blockIdx.x == 0 && threadIdx.x == 0) p.queue2[kCtrlAllDense] = 1u;
     return;
   }
@@ -768,7 +768,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
         int unit = got / (group * n_mblk);
         const int units = p.B * p.Hkv;
         if (units % 8 == 0) unit = (unit % (units / 8)) * 8 + unit / (units / 8);
-        s_skip = __hip_atomic_load(p.hints2 + 2 * unit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= (1u << 20) ? 1 : 0;
+        s_skip = __hip_atomic_load(p.hints + 2 * unit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= (1u << 20) ? 1 : 0;
       }
       s_giveup[0] = 0u;
       s_giveup[1] = 0u;
@@ -1256,7 +1256,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_DKDV_W
   const float qs = p.qscale;
 
   // (the probe left too little to this kernel: the dense kernel serves everything)
-  if (sparse_steps_aside(p.hints2, p.varlen, p.varlen_bits, p.B, p.Hkv, p.N)) {
+  if (sparse_steps_aside(p.hints, p.varlen, p.varlen_bits, p.B, p.Hkv, p.N)) {
     if (blockIdx.x == 0 && threadIdx.x == 0) p.queue2[kCtrlAllDense] = 1u;
     return;
   }
@@ -1271,7 +1271,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_DKDV_W
         int unit = got / (group * n_mblk);
         const int units = p.B * p.Hkv;
         if (units % 8 == 0) unit = (unit % (units / 8)) * 8 + unit / (units / 8);
-        s_skip = __hip_atomic_load(p.hints2 + 2 * unit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= (1u << 20) ? 1 : 0;
+        s_skip = __hip_atomic_load(p.hints + 2 * unit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= (1u << 20) ? 1 : 0;
       }
     }
     __syncthreads();
