@@ -37,6 +37,14 @@ constexpr int kListBytes = kWaves * kCap * kRows * 6;  // a score (fp32) and a k
 // position of 16-byte piece c of chunk row r
 __device__ __forceinline__ int piece_sw(int row) { return (row >> 1) & 7; }
 
+// 4-byte global -> LDS copy per lane: lane i writes the i-th word behind the wave-uniform `lds`
+__device__ __forceinline__ void dma4(const float* g, float* lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
+               :
+               : "v"(g), "s"(__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds))
+               : "memory");
+}
+
 // A wave's ring of chunks and its place in it; kStride: bytes per row of the tensors its chunks come from.
 template <int kStride> struct Ring {
   unsigned char* base;  // the wave's three chunks
@@ -292,27 +300,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   auto slot_of = [&](int e) -> int { return (lh ? kCap - 1 - e : e) * kRows; };
   // solver's view: eight lanes per row, wave w has rows 8 w .. 8 w + 7
   const int srow = wave * 8 + (lane >> 3), sj = lane & 7;
-  float sv[16];  // the lane's share of the row's listed scores, relative to their maximum, in z units
+  float sv[16];  // the lane's share of the row's listed scores, relative to their maximum, in z units: kK per wave
+  uint32_t sslot[16];
   float s_max = 0.f, s_tau = 0.f;
-  auto solve = [&](bool last) {
-    float x[16];
+  // kK: the lane's entries per wave's list, enough for the longest of the eight rows' lists
+  auto solve_k = [&](auto kc, bool last) {
+    constexpr int kK = decltype(kc)::value;
+    float x[4 * kK];
     s_max = -INFINITY;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
       const int n0 = n_lds[w][0][srow], n1 = n_lds[w][1][srow];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int slot = sj + 8 * k;
-        const bool ok = slot < n0 || slot >= kCap - n1;
-        const float v = list_s[w * (kCap * kRows) + slot * kRows + srow];
-        x[w * 4 + k] = ok ? v : -INFINITY;
-        s_max = fmaxf(s_max, x[w * 4 + k]);
+      for (int k = 0; k < kK; ++k) {
+        const int e = sj + 8 * k;  // the wave's entries of the row, those from the front first
+        const bool ok = e < n0 + n1;
+        const uint32_t at = (uint32_t)(w * (kCap * kRows) + (e < n0 ? e : kCap - 1 - (e - n0)) * kRows + srow);
+        sslot[w * kK + k] = ok ? at : (uint32_t)srow;
+        const float v = list_s[sslot[w * kK + k]];
+        x[w * kK + k] = ok ? v : -INFINITY;
+        s_max = fmaxf(s_max, x[w * kK + k]);
       }
     }
     s_max = max8(s_max);
     const float m = s_max > -INFINITY ? s_max : 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) sv[i] = (x[i] - m) * qs;
+    for (int i = 0; i < 16; ++i) sv[i] = i < 4 * kK ? (x[i < 4 * kK ? i : 0] - m) * qs : -INFINITY;
     // from the bound the row has already; on the way a few steps do, each of which ends on a bound
     s_tau = fmaxf(-1.f, (t_lds[srow] - m) * qs);
     bool go = s_max > -INFINITY;
@@ -320,7 +333,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int it = 0; it < most && __builtin_amdgcn_ballot_w64(go) != 0ull; ++it) {
       float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
+      for (int i = 0; i < 4 * kK; ++i) {
         float e0, e1;
         powers<AM>(fmaxf(sv[i] - s_tau, 0.f), c0, e0, e1);
         s0 += e0;
@@ -332,6 +345,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (go) s_tau = fminf(s_tau + step, 0.f);
       go = go && step > (last ? 1e-7f : 1e-3f);
     }
+  };
+  auto solve = [&](bool last) {
+    int most = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const int n = n_lds[w][0][srow] + n_lds[w][1][srow];
+      most = n > most ? n : most;
+    }
+    if (__builtin_amdgcn_ballot_w64(most > 16) != 0ull) solve_k(std::integral_constant<int, 4>{}, last);
+    else if (__builtin_amdgcn_ballot_w64(most > 8) != 0ull) solve_k(std::integral_constant<int, 2>{}, last);
+    else solve_k(std::integral_constant<int, 1>{}, last);
   };
   bool fallback = false;
   {
@@ -433,7 +457,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       if (pr[i] > 0.f) {
-        const uint32_t key = list_k[(i >> 2) * (kCap * kRows) + (sj + 8 * (i & 3)) * kRows + srow];
+        const uint32_t key = list_k[sslot[i]];
         mem_p[before] = pr[i];
         mem_k[before] = key;
         ++before;
@@ -453,11 +477,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int c = 0; c < NC; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
     const f32x4* v4 = reinterpret_cast<const f32x4*>(vg);
-    for (int e = 0; __builtin_amdgcn_ballot_w64(e < total) != 0ull; e += 4) {
-      f32x4 r[4][NC];
-      float w[4];
+    constexpr int kRowsAhead = D == 64 ? 8 : 4;  // rows of V under way
+    for (int e = 0; __builtin_amdgcn_ballot_w64(e < total) != 0ull; e += kRowsAhead) {
+      f32x4 r[kRowsAhead][NC];
+      float w[kRowsAhead];
 #pragma unroll
-      for (int x = 0; x < 4; ++x) {
+      for (int x = 0; x < kRowsAhead; ++x) {
         const bool ok = e + x < total;
         w[x] = ok ? mem_p[e + x] : 0.f;
         const uint32_t key = ok ? mem_k[e + x] : mem_k[0];
@@ -466,7 +491,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int c = 0; c < NC; ++c) r[x][c] = vr[8 * c];
       }
 #pragma unroll
-      for (int x = 0; x < 4; ++x)
+      for (int x = 0; x < kRowsAhead; ++x)
         if (e + x < total)
 #pragma unroll
           for (int c = 0; c < NC; ++c)
@@ -689,6 +714,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   constexpr int NC = D / 32;
   constexpr int kStride = D * 4;
   __shared__ __align__(4096) unsigned char smem[bwd_smem<D>()];
+  __shared__ __align__(256) float scal[kWaves][4 * kRows];  // of the wave's block: tau, 1 / sum p, delta (and delta once more)
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
@@ -726,6 +752,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   auto src = [&](int x, int s, int st) {
     const int g = x / n_q, qb = q_first + (x - g * n_q);
     const unsigned char* base = reinterpret_cast<const unsigned char*>(s < NC || s >= 3 * NC ? p.q : p.dout) + (q_head0 + (size_t)g * N) * kStride;
+    if (s == 0) {  // tau and 1 / sum p (half a wave each) and delta of its queries, in front of the block's first chunk
+      int row = qb * kRows + (lane & 31);
+      row = row < L ? row : L - 1;
+      const size_t at = q_head0 + (size_t)g * N + row;
+      dma4((lane < 32 ? p.taus : p.zinv) + at, &scal[wave][0]);
+      dma4(p.delta + at, &scal[wave][64]);
+    }
     ring.issue(base, qb * kRows, L, s % NC, st);
   };
   f32x16 ov[NC], ok[NC];
@@ -738,32 +771,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     f32x16 s, dp;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
-    // tau, 1 / sum p and delta of the lane's sixteen queries
-    const size_t at = q_head0 + (size_t)g * N;
-    const bool whole = q0 + kRows <= L;
-    auto scalars = [&](const float* x, float (&y)[16]) {
-      typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
-      if (whole) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const f32x4_u v4 = *reinterpret_cast<const f32x4_u*>(x + at + q0 + 8 * i + 4 * lh);
+    for (int c = 0; c < NC; ++c) dot_chunk<D == 64>(s, next(c), rl, kf + c * 16);
+    // tau, 1 / sum p and delta of the lane's sixteen queries: they came in front of the block's first chunk
+    auto scalars = [&](int which, float (&y)[16]) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) y[4 * i + e] = v4[e];
-        }
-      } else {
+      for (int i = 0; i < 4; ++i) {
+        const f32x4 v4 = *reinterpret_cast<const f32x4*>(&scal[wave][which * kRows + 8 * i + 4 * lh]);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int qrow = q0 + 8 * (i >> 2) + 4 * lh + (i & 3);
-          y[i] = x[at + (qrow < L ? qrow : L - 1)];
-        }
+        for (int e = 0; e < 4; ++e) y[4 * i + e] = v4[e];
       }
     };
     float tau[16], zi[16], de[16];
-    scalars(p.taus, tau);
-    scalars(p.zinv, zi);
-    scalars(p.delta, de);
-#pragma unroll
-    for (int c = 0; c < NC; ++c) dot_chunk<D == 64>(s, next(c), rl, kf + c * 16);
+    scalars(0, tau);
+    scalars(1, zi);
+    scalars(2, de);
+    const bool whole = q0 + kRows <= L;
     float r[16], w[16], dx[16];
     float mx = -INFINITY;
     const bool plain = whole && n0 + kRows <= L && (!p.causal || n0 + kRows - 1 <= q0);  // every query of the block sees every key
