@@ -214,8 +214,13 @@ template <int AM> __device__ __forceinline__ void powers(float u, float c0, floa
 }
 // Newton step on (sum u^c0)^(1/c0) - 1: convex and decreasing in the threshold, nearly linear where the support is settled
 template <int AM> __device__ __forceinline__ float norm_step(float s0, float s1, float c0) {
-  const float g = AM == ATT_15 ? sqrtf(s0) : (AM == ATT_2 ? s0 : fast_exp2(fast_log2(s0) / c0));
-  return (g - 1.f) * s0 / (g * s1);
+  if constexpr (AM == ATT_2) return (s0 - 1.f) * fast_rcp(s1);
+  if constexpr (AM == ATT_15) {
+    const float g = __builtin_amdgcn_sqrtf(s0);  // g - 1 = (s0 - 1) / (g + 1): exact where it is small
+    return (s0 - 1.f) * s0 * fast_rcp((g + 1.f) * g * s1);
+  }
+  const float g = fast_exp2(fast_log2(s0) / c0);
+  return (g - 1.f) * s0 * fast_rcp(g * s1);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -375,15 +380,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       t_raw = fmaxf(t_raw, t_lds[lq]);
       return given_up;
     };
+    // only where a wave's list of a row is more than half full; entries below the bound do no harm otherwise
     auto compact = [&]() {
+      if (__builtin_amdgcn_ballot_w64(n_mine + __shfl_xor(n_mine, 32, 64) > kCap / 2) == 0ull) return;
       int kept = 0;
-      for (int e = 0; __builtin_amdgcn_ballot_w64(e < n_mine) != 0ull; ++e) {
-        if (e < n_mine) {
-          const float s = my_s[slot_of(e)];
-          const uint16_t k = my_k[slot_of(e)];
-          if (s > t_raw) {
-            my_s[slot_of(kept)] = s;
-            my_k[slot_of(kept)] = k;
+      for (int e0 = 0; __builtin_amdgcn_ballot_w64(e0 < n_mine) != 0ull; e0 += 8) {
+        float s[8];
+        uint16_t k[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+          s[x] = my_s[slot_of(e0 + x < kCap ? e0 + x : 0)];
+          k[x] = my_k[slot_of(e0 + x < kCap ? e0 + x : 0)];
+        }
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+          if (e0 + x < n_mine && s[x] > t_raw) {
+            my_s[slot_of(kept)] = s[x];
+            my_k[slot_of(kept)] = k[x];
             ++kept;
           }
         }
@@ -391,43 +404,61 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       n_mine = kept;
     };
     __syncthreads();  // over_flag is clear
-    // one segment of the walk per solve: the blocks of the steps [step_no, next_sync)
-    while (true) {
-      const int seg_end = next_sync < n_steps ? next_sync : n_steps;
-      walk<NC>(ring, step_no * kWaves + wave, seg_end * kWaves < n_kblk ? seg_end * kWaves : n_kblk, kWaves, src_k, [&](int blk, auto&& next) {
-        const f32x16 s = scores(blk, 0.f, next);
-        float bm = s[0];
+    // (as walk() does it, with the loads of the coming step under way across a solve)
+    auto list_block = [&](int blk, auto&& next) {
+      const f32x16 s = scores(blk, 0.f, next);
+      float bm = s[0];
 #pragma unroll
-        for (int i = 1; i < 16; ++i) bm = fmaxf(bm, s[i]);
-        if (over || __builtin_amdgcn_ballot_w64(live && bm > t_raw) == 0ull) return;
-        int c = 0;
+      for (int i = 1; i < 16; ++i) bm = fmaxf(bm, s[i]);
+      if (over || __builtin_amdgcn_ballot_w64(live && bm > t_raw) == 0ull) return;
+      int c = 0;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) c += s[i] > t_raw ? 1 : 0;
-        c = live ? c : 0;
-        const int need = n_mine + c;
-        if (__builtin_amdgcn_ballot_w64(need + __shfl_xor(need, 32, 64) > kCap) != 0ull) {
-          over = true;  // uniform over the wave
-          return;
-        }
-        const int jb = blk * kRows + 4 * lh;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          if (live && s[i] > t_raw) {
-            my_s[slot_of(n_mine)] = s[i];
-            my_k[slot_of(n_mine)] = (uint16_t)(jb + 8 * (i >> 2) + (i & 3));
-            ++n_mine;
-          }
-        }
-      });
-      step_no = seg_end;
-      if (sync()) {
-        fallback = true;
-        break;
+      for (int i = 0; i < 16; ++i) c += s[i] > t_raw ? 1 : 0;
+      c = live ? c : 0;
+      const int need = n_mine + c;
+      if (__builtin_amdgcn_ballot_w64(need + __shfl_xor(need, 32, 64) > kCap) != 0ull) {
+        over = true;  // uniform over the wave
+        return;
       }
-      if (step_no == n_steps) break;
-      compact();
-      next_sync = step_no * 2;
+      const int jb = blk * kRows + 4 * lh;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if (live && s[i] > t_raw) {
+          my_s[slot_of(n_mine)] = s[i];
+          my_k[slot_of(n_mine)] = (uint16_t)(jb + 8 * (i >> 2) + (i & 3));
+          ++n_mine;
+        }
+      }
+    };
+    if (wave < n_kblk) {
+      src_k(wave, 0, 0);
+      src_k(wave, 1, 1);
     }
+    while (true) {
+      const int blk = step_no * kWaves + wave;
+      if (blk < n_kblk) {
+        const int blk_next = blk + kWaves < n_kblk ? blk + kWaves : blk;
+        list_block(blk, [&](int s) -> uint32_t {
+          const uint32_t a = ring.arrive();
+          if (s + 2 < NC) src_k(blk, s + 2, ring.ahead());
+          else src_k(blk_next, s + 2 - NC, ring.ahead());
+          ring.advance();
+          return a;
+        });
+      }
+      ++step_no;
+      if (step_no == n_steps) ring.drain();  // (the output takes the ring's place behind the solve)
+      if (step_no == next_sync || step_no == n_steps) {
+        if (sync()) {
+          fallback = true;
+          break;
+        }
+        if (step_no == n_steps) break;
+        compact();
+        next_sync = step_no * 2;
+      }
+    }
+    ring.drain();
   }
 
   if (!fallback) {
