@@ -797,7 +797,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((BwdTiles<T
 // which: 1 = the dQ kernel, 2 = the dK/dV kernel, 3 = both, in that order
 template <typename T, int D> static int launch_attn_bwd_d(const AttnBwdParams& p, int am, int which, hipStream_t s) {
   const long long nq = (p.N + kBwdRows - 1) / kBwdRows;
-  const dim3 gq((unsigned)(((long long)p.B * p.Hq * nq + 7) / 8 * 8)), gk((unsigned)(((long long)p.B * p.Hkv * nq + 7) / 8 * 8));
+  const dim3 gq(xcd_grid((long long)p.B * p.Hkv, nq * (p.Hq / p.Hkv))), gk(xcd_grid((long long)p.B * p.Hkv, nq));
   if (am == ATT_15) {
     if (which & 1) hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, ATT_15>), gq, dim3(256), 0, s, p);
     if (which & 2) hipLaunchKernelGGL((attn_bwd_dkdv_kernel<T, D, ATT_15>), gk, dim3(256), 0, s, p);

@@ -10,14 +10,12 @@ template <typename T, int D, int AM, bool kMulti> static int launch_attn_one(con
   auto kern = attn_fwd_kernel<T, D, AM, kMulti>;
   const long long group = p.Hq / p.Hkv;
   const long long n_mblk = (p.N + G::kBM - 1) / G::kBM;
-  const long long total = (long long)p.B * p.Hkv * n_mblk * group;
-  const long long per_xcd = (total + 7) / 8;
   // dynamic LDS: the tile masks, and in the instance with the candidate lists, up to 128K keys, the
   // per-wave block bits as well (beyond that they would cost occupancy)
   AttnParams q = p;
   q.fine_masks = (kMulti && p.mask_words <= 64) ? 1 : 0;
   const size_t words = (size_t)(q.fine_masks ? 4 + 4 * G::kNW : 4) * p.mask_words + G::kPoolTail;  // + the candidate lists' bookkeeping
-  hipLaunchKernelGGL(kern, dim3((unsigned)(per_xcd * 8)), dim3(G::kThreads), words * sizeof(uint32_t), s, q);
+  hipLaunchKernelGGL(kern, dim3(xcd_grid((long long)p.B * p.Hkv, n_mblk * group)), dim3(G::kThreads), words * sizeof(uint32_t), s, q);
   return 0;
 }
 
