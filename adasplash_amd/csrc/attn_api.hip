@@ -35,6 +35,12 @@ int launch_attn_f32_fwd_d128(const AttnParams&, int, hipStream_t);
 int launch_attn_f32_bwd_d64(const AttnBwdParams&, int, hipStream_t);
 int launch_attn_f32_bwd_d128(const AttnBwdParams&, int, hipStream_t);
 
+// their forward for the 16-bit types (attn_rows32_unit.hip)
+int launch_attn_rows32_bf16_d64(const AttnParams&, int, hipStream_t);
+int launch_attn_rows32_bf16_d128(const AttnParams&, int, hipStream_t);
+int launch_attn_rows32_f16_d64(const AttnParams&, int, hipStream_t);
+int launch_attn_rows32_f16_d128(const AttnParams&, int, hipStream_t);
+
 typedef int (*attn_fwd_fn)(const AttnParams&, int, hipStream_t);
 typedef int (*attn_bwd_fn)(const AttnBwdParams&, int, int, hipStream_t);
 #define ADSP_FWD_ROW(tag, d) {launch_attn_fwd_##tag##_d##d##_m0, launch_attn_fwd_##tag##_d##d##_m1}
@@ -348,6 +354,25 @@ static bool f32_split(int N, int D, int dtype, double alpha) {
   return dtype == ADSP_F32 && (D == 64 || D == 128) && N <= 65536 && alpha >= 1.125 && alpha <= 2.0;
 }
 
+// Whether a 16-bit forward of which nobody wants the tile mask or the supports takes the single kernel on 32 rows a workgroup
+// (attn_f32_kernel.h): a short problem, for which the probe, the copy of K, the sparse-support kernel's items of 128 rows and
+// the dense kernel behind it take longer than the work.  Two workgroups fit a CU: up to 512 run at once.  With flat scores,
+// where the lists overflow and each workgroup walks several times, a second round of them is one too many on causal problems
+// of a few hundred keys (16 heads, N = 256: 8 sequences 30 -> 42 us, 5 of N = 512: 40 -> 60, against 57 -> 27 and 75 -> 43
+// with unit spread), and not on longer or full ones or where a workgroup has no more than one step.  The second
+// condition is the time the work itself takes, about 20 ns a workgroup and 1.35 ns a block of 32 x 32 scores with the chip full.
+// Measured at the line, four launches -> this kernel, us for q of spread 1, 3 and 1/8: 16/4 heads, D = 128, 4 sequences of
+// N = 256: 76 -> 18 and 38 -> 31 (1 and 1/8); 2 of 512: 99 -> 24, 52 -> 32; 32/8 heads, N = 1024: 131 -> 53, 80 -> 74; 16/4
+// heads, N = 2048: 132 -> 93, 89 -> 54, 135 -> 124; 4 x 16 heads, N = 512, not causal: 67 -> 46, 47 -> 34, 95 -> 54; 32 x 16
+// heads, N = 128: 59 -> 42, 44 -> 36, 70 -> 66; beyond it 32/8 heads, N = 2048: 147 -> 132, 96 -> 100, 139 -> 236.
+static bool rows32_16bit(int B, int Hq, int N, int D, int dtype, double alpha, bool causal) {
+  if (dtype == ADSP_F32 || (D != 64 && D != 128) || N > 65536 || !(alpha >= 1.125 && alpha <= 2.0) || !sparse_enabled()) return false;
+  const long long r = (N + 31) / 32, heads = (long long)B * Hq, groups = heads * r;
+  const double blocks = (double)heads * (causal ? 0.5 * (double)r * (double)(r + 1) : (double)r * (double)r);
+  const long long most = N <= 128 ? 2048 : ((N >= 1024 || !causal) ? 1024 : 512);
+  return groups <= most && 20.0 * (double)groups + 1.35 * blocks <= 66e3;
+}
+
 static int attn_common(const void* q, const void* k, const void* v, void* out, float* taus, int32_t* bmask,
                        const void* varlen, int varlen_bits, int B, int Hq, int Hkv, int N, int D, int dtype,
                        double alpha, int is_causal, int niter, int use_hist, void* workspace, size_t workspace_bytes,
@@ -419,6 +444,11 @@ static int attn_common(const void* q, const void* k, const void* v, void* out, f
     }
     if ((D == 64 ? launch_attn_f32_fwd_d64(p, am, s) : launch_attn_f32_fwd_d128(p, am, s)) != 0) return ADSP_ERR_LAUNCH;
     return hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
+  }
+  if (!tile_counts && !bmask && !supports && rows32_16bit(B, Hq, N, D, dtype, alpha, is_causal != 0)) {
+    const int rc = dtype == ADSP_BF16 ? (D == 64 ? launch_attn_rows32_bf16_d64(p, am, s) : launch_attn_rows32_bf16_d128(p, am, s))
+                                      : (D == 64 ? launch_attn_rows32_f16_d64(p, am, s) : launch_attn_rows32_f16_d128(p, am, s));
+    return rc == 0 && hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
   }
   if (dtype != ADSP_F32) {
     const SupportsLayout sl = supports ? supports_layout(B, Hq, Hkv, N, D, dtype) : SupportsLayout{};

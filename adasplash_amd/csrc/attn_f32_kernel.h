@@ -75,6 +75,18 @@ template <int kStride> struct Ring {
       }
     }
   }
+  // the same in the layout of the transposing reads (16-bit V; see BwdTiles::tsw): row r's pieces moved by 2 r
+  __device__ __forceinline__ void issue_t(const unsigned char* g, int row0, int limit, int c, int s) const {
+    const unsigned char* gb = uniform_ptr(g + c * 128);
+    unsigned char* l = base + s * kChunk;
+    const int piece = (lane & 7) ^ ((2 * (lane >> 3)) & 7);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      int r = row0 + 8 * j + (lane >> 3);
+      r = r < limit ? r : limit - 1;
+      dma16s(gb, (uint32_t)r * (uint32_t)kStride + (uint32_t)(piece * 16), l + j * 1024);
+    }
+  }
   // Waits for the oldest of the two chunks under way and for the wave's own LDS reads (the stage the caller fills next is
   // the one it has just read); returns the LDS address of the chunk.
   __device__ __forceinline__ uint32_t arrive() const {
@@ -86,31 +98,42 @@ template <int kStride> struct Ring {
   __device__ __forceinline__ void drain() const { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
 };
 
-// Walks the blocks wave, wave + 4, ... below n_blk.  Each block is SEQ chunks, src(blk, s, ring, stage) issues number s of
-// them; body(blk, next) consumes them by SEQ calls of next(s) in order, which return the chunk's LDS address.
+// A walk takes the blocks first, first + step, ... below n_blk, each SEQ chunks that src(blk, s, stage) issues.  `start` issues
+// the first two chunks; `take` waits for chunk s of blk, issues the chunk after next (past the end: one that nothing reads,
+// to keep the count) and returns the LDS address.
+template <int SEQ, typename Src> __device__ __forceinline__ void start(int first, int n_blk, int step, Src&& src) {
+  src(first, 0, 0);
+  if constexpr (SEQ == 1) src(first + step < n_blk ? first + step : first, 0, 1);
+  else src(first, 1, 1);
+}
+template <int SEQ, typename R, typename Src> __device__ __forceinline__ uint32_t take(R& ring, int blk, int s, int n_blk, int step, Src&& src) {
+  const uint32_t a = ring.arrive();
+  const int nb = blk + (s + 2) / SEQ * step;
+  src(nb < n_blk ? nb : blk, (s + 2) % SEQ, ring.ahead());
+  ring.advance();
+  return a;
+}
+// The whole walk: body(blk, next) consumes a block's chunks by calls of next(0), next(1), ... in order.
 template <int SEQ, typename R, typename Src, typename Body>
 __device__ __forceinline__ void walk(R& ring, int first, int n_blk, int step, Src&& src, Body&& body) {
   if (first >= n_blk) return;
   ring.st = 0;
-  src(first, 0, 0);
-  src(first, 1, 1);
-  for (int blk = first; blk < n_blk; blk += step) {
-    const int blk_next = blk + step < n_blk ? blk + step : blk;  // (past the end: loads that nothing reads keep the count)
-    body(blk, [&](int s) -> uint32_t {
-      const uint32_t a = ring.arrive();
-      if (s + 2 < SEQ) src(blk, s + 2, ring.ahead());
-      else src(blk_next, s + 2 - SEQ, ring.ahead());
-      ring.advance();
-      return a;
-    });
-  }
+  start<SEQ>(first, n_blk, step, src);
+  for (int blk = first; blk < n_blk; blk += step) body(blk, [&](int s) -> uint32_t { return take<SEQ>(ring, blk, s, n_blk, step, src); });
   ring.drain();
 }
 
-// acc += (chunk rows) . (the lane's own row), columns 32 c .. 32 c + 31: f holds the lane's row, 8 g + 4 lh .. + 3 of every
-// 8.  kParts: a chunk's 32 products are added up from zero and the chunks' sums then, shorter chains of smaller numbers (where
+// acc += (chunk rows) . (the lane's own row) over the chunk's columns: f holds of the lane's row piece 2 g + lh of every pair.  kParts: a chunk's 32 products are added up from zero and the chunks' sums then, shorter chains of smaller numbers (where
 // the registers allow it).
-template <bool kParts> __device__ __forceinline__ void dot_chunk(f32x16& acc, uint32_t chunk, uint32_t row_lane, const uint32_t* f) {
+template <bool kParts, typename T = float> __device__ __forceinline__ void dot_chunk(f32x16& acc, uint32_t chunk, uint32_t row_lane, const uint32_t* f) {
+  if constexpr (is16<T>::value) {
+    u32x4 a[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) a[g] = lds_read16((chunk + row_lane) ^ (g << 5));
+#pragma unroll
+    for (int g = 0; g < 4; ++g) acc = mfma_16bit<T>(a[g], u32x4{f[4 * g], f[4 * g + 1], f[4 * g + 2], f[4 * g + 3]}, acc);
+    return;
+  }
   f32x4 a[4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) a[g] = __builtin_bit_cast(f32x4, lds_read16((chunk + row_lane) ^ (g << 5)));
@@ -136,6 +159,27 @@ __device__ __forceinline__ void acc_chunk(f32x16& o, uint32_t chunk, uint32_t co
 #pragma unroll
   for (int i = 0; i < 16; ++i) o = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], w[i], o, 0, 0, 0);
 }
+// the same for a 16-bit chunk of 64 columns (issue_t): o[0] takes columns 0 .. 31, o[1] the others
+template <typename T> __device__ __forceinline__ void acc_chunk_16(f32x16 (&o)[2], uint32_t chunk, int lane, const float (&w)[16]) {
+  const int a4 = lane & 15, grp = lane >> 4, r = a4 >> 2, c = a4 & 3, dl = grp & 1;
+  uint32_t ta[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int x = 4 * (grp >> 1) + r + 8 * h;
+    ta[h] = chunk + (uint32_t)(x * 128 + (((2 * dl + (c >> 1)) ^ ((2 * x) & 7)) << 4) + (c & 1) * 8);
+  }
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const u32x4 b = {pack2<T>(w[8 * s], w[8 * s + 1]), pack2<T>(w[8 * s + 2], w[8 * s + 3]), pack2<T>(w[8 * s + 4], w[8 * s + 5]),
+                     pack2<T>(w[8 * s + 6], w[8 * s + 7])};
+#pragma unroll
+    for (int db = 0; db < 2; ++db) {
+      const u32x2_t a0 = lds_read8_tr(ta[0] ^ (db << 6), 16 * s * 128);
+      const u32x2_t a1 = lds_read8_tr(ta[1] ^ (db << 6), 16 * s * 128);
+      o[db] = mfma_16bit<T>(u32x4{a0[0], a0[1], a1[0], a1[1]}, b, o[db]);
+    }
+  }
+}
 __device__ __forceinline__ uint32_t row_lane_of(int lq, int lh) { return (uint32_t)(lq * 128 + ((lh ^ piece_sw(lq)) << 4)); }
 __device__ __forceinline__ uint32_t col_lane_of(int lq, int lh) {
   return (uint32_t)(4 * lh * 128 + (((lq >> 2) ^ (2 * lh)) << 4) + (lq & 3) * 4);
@@ -143,8 +187,8 @@ __device__ __forceinline__ uint32_t col_lane_of(int lq, int lh) {
 
 // Adds up the four waves' o (32 columns per block, accumulator layout) in LDS and writes scale[row] * sum to the rows
 // [row0, row0 + 32) below n of a row-major tensor.  `smem` holds 4 x 32 x D floats; every wave is done with what it held.
-template <int D, typename Scale>
-__device__ __forceinline__ void combine_store(const f32x16 (&o)[D / 32], unsigned char* smem, float* out, int row0, int n, int wave,
+template <int D, typename T, typename Scale>
+__device__ __forceinline__ void combine_store(const f32x16 (&o)[D / 32], unsigned char* smem, T* out, int row0, int n, int wave,
                                               int lane, Scale&& scale) {
   using KS = Swz<D * 4>;
   const int lq = lane & 31, lh = lane >> 5, tid = wave * 64 + lane;
@@ -168,14 +212,18 @@ __device__ __forceinline__ void combine_store(const f32x16 (&o)[D / 32], unsigne
       for (int e = 0; e < 4; ++e) s[e] += x[e];
     }
     const float k = scale(row);
-    if (row0 + row < n) *reinterpret_cast<f32x4*>(out + (size_t)(row0 + row) * D + c * 4) = f32x4{s[0] * k, s[1] * k, s[2] * k, s[3] * k};
+    if (row0 + row >= n) continue;
+    unsigned char* at_out = reinterpret_cast<unsigned char*>(out) + ((size_t)(row0 + row) * D + c * 4) * (is16<T>::value ? 2 : 4);
+    if constexpr (is16<T>::value) *reinterpret_cast<u32x2*>(at_out) = u32x2{pack2<T>(s[0] * k, s[1] * k), pack2<T>(s[2] * k, s[3] * k)};
+    else *reinterpret_cast<f32x4*>(at_out) = f32x4{s[0] * k, s[1] * k, s[2] * k, s[3] * k};
   }
 }
 
-template <int D> __device__ __forceinline__ void load_row(const float* row, int lh, uint32_t (&f)[D / 2]) {
+// kPairs pairs of 16-byte pieces of a row, the lane's half of each
+template <int kPairs> __device__ __forceinline__ void load_row(const unsigned char* row, int lh, uint32_t (&f)[4 * kPairs]) {
 #pragma unroll
-  for (int g = 0; g < D / 8; ++g) {
-    const u32x4 raw = *reinterpret_cast<const u32x4*>(row + 8 * g + 4 * lh);
+  for (int g = 0; g < kPairs; ++g) {
+    const u32x4 raw = *reinterpret_cast<const u32x4*>(row + 32 * g + 16 * lh);
 #pragma unroll
     for (int e = 0; e < 4; ++e) f[g * 4 + e] = raw[e];
   }
@@ -231,12 +279,13 @@ template <int D> constexpr int fwd_smem() {
   return a > b ? a : b;
 }
 
-template <int D, int AM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_f32_fwd_kernel(AttnParams p) {
-  constexpr int NC = D / 32;
-  constexpr int kStride = D * 4;
+template <typename T, int D, int AM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_rows32_fwd_kernel(AttnParams p) {
+  constexpr bool k16 = is16<T>::value;
+  constexpr int kStride = D * (k16 ? 2 : 4);
+  constexpr int NC = kStride / 128;  // chunks per block
   __shared__ __align__(4096) unsigned char smem[fwd_smem<D>()];
-  __shared__ float t_lds[kRows];
+  __shared__ float t_lds[kRows], est_lds[kRows];
   __shared__ uint8_t n_lds[kWaves][2][kRows];
   __shared__ float red[2][kWaves][3][kRows];
   __shared__ uint32_t over_flag;
@@ -257,10 +306,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     L = (int)(l < 0 ? 0 : (l > N ? N : l));
   }
   const size_t q_row0 = (size_t)(b * p.Hq + h) * N;
-  float* const out = reinterpret_cast<float*>(p.out) + q_row0 * D;
+  unsigned char* const out = reinterpret_cast<unsigned char*>(p.out) + q_row0 * kStride;
   if (m0 >= L) {
     const int rows = N - m0 < kRows ? N - m0 : kRows;
-    for (int i = tid; i < rows * (D / 4); i += 256) reinterpret_cast<f32x4*>(out + (size_t)m0 * D)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = tid; i < rows * (kStride / 16); i += 256) reinterpret_cast<f32x4*>(out + (size_t)m0 * kStride)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     return;
   }
   const unsigned char* kg = reinterpret_cast<const unsigned char*>(p.k) + (size_t)bkv * N * kStride;
@@ -271,8 +320,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int key_hi = p.causal ? (m0 + kRows < L ? m0 + kRows : L) : L;
   const int n_kblk = (key_hi + kRows - 1) / kRows;
   const float qs = p.qscale, inv_qs = 1.f / p.qscale, c0 = p.c0;
-  uint32_t qf[D / 2];
-  load_row<D>(reinterpret_cast<const float*>(p.q) + (q_row0 + (live ? qi : L - 1)) * D, lh, qf);
+  uint32_t qf[16 * NC];
+  load_row<4 * NC>(reinterpret_cast<const unsigned char*>(p.q) + (q_row0 + (live ? qi : L - 1)) * kStride, lh, qf);
 
   Ring<kStride> ring(smem + wave * (kStages * kChunk), lane);
   const uint32_t rl = row_lane_of(lq, lh), cl = col_lane_of(lq, lh);
@@ -283,7 +332,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = init;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) dot_chunk<true>(acc, next(c), rl, qf + c * 16);
+    for (int c = 0; c < NC; ++c) dot_chunk<true, T>(acc, next(c), rl, qf + c * 16);
     const int k0 = blk * kRows;
     if (k0 + kRows > L || (p.causal && k0 + kRows - 1 > m0)) {
       const int jb = k0 + 4 * lh;
@@ -295,7 +344,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   // ---- the walk that lists: rows are solved on the lists after 1, 2, 4, ... steps of four blocks and behind the last ----
   if (tid == 0) over_flag = 0u;
-  if (tid < kRows) t_lds[tid] = -INFINITY;
+  if (tid < kRows) t_lds[tid] = est_lds[tid] = -INFINITY;
   float t_raw = -INFINITY;  // bound of the lane's row, raw score units
   int n_mine = 0;           // entries of this lane: lh = 0 fills the wave's slots of the row from the front, lh = 1 from the back
   bool over = false;
@@ -371,6 +420,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (over) over_flag = 1u;
       __syncthreads();
       solve(step_no == n_steps);
+      if (step_no == 1 && n_steps > 1) {
+        // More than half of the first 128 keys in a row's support so far: its list is about to overflow.  The threshold of
+        // a row whose other keys are like these is where the walks then start (a Newton step from beyond tau ends below it).
+        float members = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) members += sv[i] > s_tau ? 1.f : 0.f;
+        if (__builtin_amdgcn_ballot_w64(sum8(members) > 64.f) != 0ull) {
+          const int row = m0 + srow, keys = p.causal ? (row < L - 1 ? row + 1 : L) : L;
+          const float ratio = (float)keys * (1.f / 128.f);
+          float e = s_tau;
+          for (int it = 0; it < 6; ++it) {
+            float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              float e0, e1;
+              powers<AM>(fmaxf(sv[i] - e, 0.f), c0, e0, e1);
+              s0 += e0;
+              s1 += e1;
+            }
+            s0 = sum8(s0) * ratio;
+            s1 = sum8(s1) * ratio;
+            const float step = norm_step<AM>(s0, s1, c0);
+            if (s0 > 0.f && s1 > 0.f) e += step;
+          }
+          if (sj == 0 && keys > 128 && e < 0.f && e > s_tau) est_lds[srow] = s_max + e * inv_qs;
+        }
+      }
       if (sj == 0) {
         // (the margin covers the rounding of the difference and of the product back to raw units)
         t_lds[srow] = s_max > -INFINITY ? (s_max + (s_tau - 1e-6f) * inv_qs) - 4e-7f * fabsf(s_max) : -INFINITY;
@@ -430,22 +506,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
       }
     };
-    if (wave < n_kblk) {
-      src_k(wave, 0, 0);
-      src_k(wave, 1, 1);
-    }
+    if (wave < n_kblk) start<NC>(wave, n_kblk, kWaves, src_k);
     while (true) {
       const int blk = step_no * kWaves + wave;
-      if (blk < n_kblk) {
-        const int blk_next = blk + kWaves < n_kblk ? blk + kWaves : blk;
-        list_block(blk, [&](int s) -> uint32_t {
-          const uint32_t a = ring.arrive();
-          if (s + 2 < NC) src_k(blk, s + 2, ring.ahead());
-          else src_k(blk_next, s + 2 - NC, ring.ahead());
-          ring.advance();
-          return a;
-        });
-      }
+      if (blk < n_kblk) list_block(blk, [&](int s) -> uint32_t { return take<NC>(ring, blk, s, n_kblk, kWaves, src_k); });
       ++step_no;
       if (step_no == n_steps) ring.drain();  // (the output takes the ring's place behind the solve)
       if (step_no == next_sync || step_no == n_steps) {
@@ -504,20 +568,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __builtin_amdgcn_wave_barrier();
     const int row = m0 + srow;
     if (p.taus && sj == 0 && row < L) p.taus[q_row0 + row] = fmaf(s_max, qs, s_tau);
-    f32x4 acc[NC];
+    constexpr int kPer = k16 ? 8 : 4;  // values per 16-byte piece; a lane has piece sj + 8 c of its row
+    float acc[NC][kPer];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const f32x4* v4 = reinterpret_cast<const f32x4*>(vg);
-    constexpr int kRowsAhead = D == 64 ? 8 : 4;  // rows of V under way
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) acc[c][k] = 0.f;
+    const u32x4* v4 = reinterpret_cast<const u32x4*>(vg);
+    constexpr int kRowsAhead = NC <= 2 ? 8 : 4;  // rows of V under way
     for (int e = 0; __builtin_amdgcn_ballot_w64(e < total) != 0ull; e += kRowsAhead) {
-      f32x4 r[kRowsAhead][NC];
+      u32x4 r[kRowsAhead][NC];
       float w[kRowsAhead];
 #pragma unroll
       for (int x = 0; x < kRowsAhead; ++x) {
         const bool ok = e + x < total;
         w[x] = ok ? mem_p[e + x] : 0.f;
         const uint32_t key = ok ? mem_k[e + x] : mem_k[0];
-        const f32x4* vr = v4 + (size_t)(total > 0 ? key : 0u) * (D / 4) + sj;
+        const u32x4* vr = v4 + (size_t)(total > 0 ? key : 0u) * (kStride / 16) + sj;
 #pragma unroll
         for (int c = 0; c < NC; ++c) r[x][c] = vr[8 * c];
       }
@@ -527,18 +594,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
           for (int c = 0; c < NC; ++c)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) acc[c][k] = fmaf(w[x], r[x][c][k], acc[c][k]);
+            for (int k = 0; k < 4; ++k) {
+              const uint32_t word = r[x][c][k];
+              if constexpr (k16) {
+                acc[c][2 * k] = fmaf(w[x], unpack_lo<T>(word), acc[c][2 * k]);
+                acc[c][2 * k + 1] = fmaf(w[x], unpack_hi<T>(word), acc[c][2 * k + 1]);
+              } else {
+                acc[c][k] = fmaf(w[x], __builtin_bit_cast(float, word), acc[c][k]);
+              }
+            }
     }
     if (row < N) {
-      f32x4* o4 = reinterpret_cast<f32x4*>(out + (size_t)row * D) + sj;
+      u32x4* o4 = reinterpret_cast<u32x4*>(out + (size_t)row * kStride) + sj;
 #pragma unroll
-      for (int c = 0; c < NC; ++c) o4[8 * c] = f32x4{acc[c][0] * inv, acc[c][1] * inv, acc[c][2] * inv, acc[c][3] * inv};
+      for (int c = 0; c < NC; ++c) {
+        u32x4 w;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if constexpr (k16) w[k] = pack2<T>(acc[c][2 * k] * inv, acc[c][2 * k + 1] * inv);
+          else w[k] = __builtin_bit_cast(uint32_t, acc[c][k] * inv);
+        }
+        o4[8 * c] = w;
+      }
     }
     return;
   }
 
-  // ---- walks: t_raw is finite for live rows (every row sees key 0, which the first solve has), a lower bound of tau ----
-  float t = live && t_raw > -INFINITY ? t_raw : 0.f;
+  // ---- walks: t_raw is finite for live rows (every row sees key 0, which the first solve has), a lower bound of tau; the
+  // estimate may lie beyond it ----
+  float t = live && t_raw > -INFINITY ? fmaxf(t_raw, est_lds[lq]) : 0.f;
   for (int it = 0; it < 24; ++it) {
     float a0 = 0.f, a1 = 0.f, mx = -INFINITY;
     walk<NC>(ring, wave, n_kblk, kWaves, src_k, [&](int blk, auto&& next) {
@@ -573,13 +657,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   if (live && lh == 0 && wave == 0 && p.taus) p.taus[q_row0 + qi] = t * qs;
 
-  f32x16 o[NC];
+  f32x16 o[NC][k16 ? 2 : 1];  // per chunk of V, 32 columns each
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) o[c][i] = 0.f;
+    for (int d = 0; d < (k16 ? 2 : 1); ++d)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[c][d][i] = 0.f;
   float psum = 0.f;
-  auto src_kv = [&](int blk, int s, int st) { ring.issue(s < NC ? kg : vg, blk * kRows, L, s < NC ? s : s - NC, st); };
+  auto src_kv = [&](int blk, int s, int st) {
+    if (s < NC) ring.issue(kg, blk * kRows, L, s, st);
+    else if constexpr (k16) ring.issue_t(vg, blk * kRows, L, s - NC, st);
+    else ring.issue(vg, blk * kRows, L, s - NC, st);
+  };
   walk<2 * NC>(ring, wave, n_kblk, kWaves, src_kv, [&](int blk, auto&& next) {
     const f32x16 s = scores(blk, -t, next);
     float w[16];
@@ -588,6 +678,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int i = 0; i < 16; ++i) {
       float e1;
       powers<AM>(live ? fmaxf(s[i], 0.f) * qs : 0.f, c0, w[i], e1);
+      if constexpr (k16) w[i] = unpack_lo<T>(pack2<T>(w[i], 0.f));  // what the product weighs V with
       bs += w[i];
     }
     psum += bs;
@@ -598,13 +689,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(NC + c);
-      if (any) acc_chunk(o[c], a, cl, w);
+      if constexpr (k16) {
+        if (any) acc_chunk_16<T>(o[c], a, lane, w);
+      } else {
+        if (any) acc_chunk(o[c][0], a, cl, w);
+      }
     }
   });
   psum += __shfl_xor(psum, 32, 64);
   __syncthreads();  // the sums of the last step have been read, every wave is done with its ring
   if (lh == 0) red[0][wave][0][lq] = psum;
-  combine_store<D>(o, smem, out, m0, N, wave, lane, [&](int row) {
+  combine_store<D>(reinterpret_cast<const f32x16(&)[D / 32]>(o), smem, reinterpret_cast<T*>(out), m0, N, wave, lane, [&](int row) {
     const float z = (red[0][0][0][row] + red[0][1][0][row]) + (red[0][2][0][row] + red[0][3][0][row]);
     return z > 0.f ? 1.f / z : 0.f;
   });
@@ -648,8 +743,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   uint32_t qf[D / 2], dof[D / 2];
   {
     const size_t r = q_row0 + (live ? qi : L - 1);
-    load_row<D>(reinterpret_cast<const float*>(p.q) + r * D, lh, qf);
-    load_row<D>(reinterpret_cast<const float*>(p.dout) + r * D, lh, dof);
+    load_row<D / 8>(reinterpret_cast<const unsigned char*>(p.q) + r * kStride, lh, qf);
+    load_row<D / 8>(reinterpret_cast<const unsigned char*>(p.dout) + r * kStride, lh, dof);
   }
   Ring<kStride> ring(smem + wave * (kStages * kChunk), lane);
   const uint32_t rl = row_lane_of(lq, lh), cl = col_lane_of(lq, lh);
@@ -771,8 +866,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   uint32_t kf[D / 2], vf[D / 2];
   {
     const size_t r = kv_row0 + (live ? kj : L - 1);
-    load_row<D>(reinterpret_cast<const float*>(p.k) + r * D, lh, kf);
-    load_row<D>(reinterpret_cast<const float*>(p.v) + r * D, lh, vf);
+    load_row<D / 8>(reinterpret_cast<const unsigned char*>(p.k) + r * kStride, lh, kf);
+    load_row<D / 8>(reinterpret_cast<const unsigned char*>(p.v) + r * kStride, lh, vf);
   }
   const int q_first = p.causal ? kblk : 0;            // first query block that sees the keys
   const int n_q = (L + kRows - 1) / kRows - q_first;  // query blocks per head

@@ -14,7 +14,7 @@ template <int AM> static void launch_bwd(const AttnBwdParams& p, hipStream_t s) 
   hipLaunchKernelGGL((attn_f32_dkdv_kernel<ADSP_D, AM>), grid_of(p.B, p.Hkv, 1, p.N), dim3(256), 0, s, p);
 }
 template <int AM> static void launch_fwd(const AttnParams& p, hipStream_t s) {
-  hipLaunchKernelGGL((attn_f32_fwd_kernel<ADSP_D, AM>), grid_of(p.B, p.Hkv, p.Hq / p.Hkv, p.N), dim3(256), 0, s, p);
+  hipLaunchKernelGGL((attn_rows32_fwd_kernel<float, ADSP_D, AM>), grid_of(p.B, p.Hkv, p.Hq / p.Hkv, p.N), dim3(256), 0, s, p);
 }
 int ADSP_CAT(launch_attn_f32_fwd_d, ADSP_D)(const AttnParams& p, int am, hipStream_t s) {
   if (am == ATT_15) launch_fwd<ATT_15>(p, s);

@@ -136,7 +136,7 @@ Tensor attn_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Att
     wp = ws_bytes ? kp + align256(l.total) : nullptr;
   }
   float* taus = (float*)kp;
-  int32_t* bmask = adsp_attn_bwd_reads_bmask(N, D, dt, c.alpha) ? (int32_t*)(kp + l.bmask_off) : nullptr;
+  int32_t* bmask = keep && adsp_attn_bwd_reads_bmask(N, D, dt, c.alpha) ? (int32_t*)(kp + l.bmask_off) : nullptr;
   void* supports = sup ? kp + l.supports_off : nullptr;
   void* stream = stream_of(q);
   if (c.version == 2) {

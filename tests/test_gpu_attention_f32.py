@@ -66,3 +66,29 @@ def test_same_bits_on_every_call_and_long_rows(N, scale):
     tol = TOL * max(1.0, scale)
     for name, a, w in zip(("out", "dq", "dk", "dv"), first, want):
         assert max_err(a, w) < tol, name
+
+
+@pytest.mark.parametrize("scale", [0.125, 1.0, 3.0])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("alpha,causal,Hq,Hkv,D", [(1.5, True, 4, 2, 64), (1.5, True, 2, 2, 128), (1.333, False, 2, 2, 64), (2.0, False, 1, 1, 128)])
+def test_16bit_inference_lengths_around_blocks_and_steps(dtype, alpha, causal, Hq, Hkv, D, scale):
+    """Without a gradient short 16-bit calls take the same forward; the bound is that of the other 16-bit forward tests."""
+    g = torch.Generator().manual_seed(5)
+    N = 517
+    varlen = torch.tensor([517, 1, 32, 33, 127, 129, 384], dtype=torch.int32)
+    B = len(varlen)
+    q = (scale * torch.randn(B, Hq, N, D, generator=g)).to(dtype)
+    k, v = (torch.randn(B, Hkv, N, D, generator=g).to(dtype) for _ in range(2))
+    want = exact.dense_entmax_attention(q, k, v, alpha, causal, varlen)
+    for b, n in enumerate(varlen.tolist()):
+        for t in (q, k, v):
+            t[b, :, n:] = float("nan")
+    args = [t.to(DEV) for t in (q, k, v)]
+    vl = varlen.to(DEV)
+    run16 = lambda: A.adasplash_v2(*args, varlen=vl) if Hq != Hkv else A.adasplash_v1(*args, alpha=alpha, is_causal=causal, varlen=vl)
+    got = run16()
+    assert torch.equal(got, run16())
+    assert torch.isfinite(got).all()
+    for b, n in enumerate(varlen.tolist()):
+        assert (got[b, :, n:] == 0).all()
+    assert max_err(got, want) < 2e-2
