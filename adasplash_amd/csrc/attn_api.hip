@@ -446,6 +446,7 @@ static int attn_common(const void* q, const void* k, const void* v, void* out, f
     return hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
   }
   if (!tile_counts && !bmask && !supports && rows32_16bit(B, Hq, N, D, dtype, alpha, is_causal != 0)) {
+    if (w.total && (!workspace || workspace_bytes < w.total || ((uintptr_t)workspace & 15) != 0)) return ADSP_ERR_WORKSPACE;  // (as below)
     const int rc = dtype == ADSP_BF16 ? (D == 64 ? launch_attn_rows32_bf16_d64(p, am, s) : launch_attn_rows32_bf16_d128(p, am, s))
                                       : (D == 64 ? launch_attn_rows32_f16_d64(p, am, s) : launch_attn_rows32_f16_d128(p, am, s));
     return rc == 0 && hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;

@@ -1,6 +1,7 @@
-// Sparse entmax attention in single precision for gfx950, head dims 64 and 128: forward, dQ and dK/dV kernels.
+// Sparse entmax attention on workgroups of 32 rows for gfx950, head dims 64 and 128: single-precision forward, dQ and dK/dV
+// kernels, and the same forward for short 16-bit problems.
 //
-// What bounds them: the fp32 matrix pipe (v_mfma_f32_32x32x2_f32, 64 cycles for 32 x 32 x 2) on large problems, and on
+// What bounds them: the fp32 matrix pipe (v_mfma_f32_32x32x2_f32, 64 cycles) on large problems, and on
 // ordinary ones the length of a workgroup's walk over the keys, because a K/V head of N keys has only N / rows workgroups.
 //
 // Split: a workgroup is four waves and owns 32 rows (queries; keys in the dK/dV kernel); the waves share the rows and
@@ -18,8 +19,10 @@
 // workgroup to walks: Newton steps on (sum u^c0)^(1/c0) - 1 from the bound the lists gave, until a step is below 2e-5, and
 // an output walk.
 //
-// Measured, B = 2, 8 heads, N = 1500 and 375, D = 64, causal (us, 128-row workgroups -> here): see the launch rule in
-// attn_api.hip.
+// Measured (fp32, causal, forward and backward; kernels on 128 rows a workgroup -> these): 2 x 8 heads, N = 1500 and 375,
+// D = 64: 1140 -> 287 us (forward 65, dQ 128, dK/dV 108, where one walk of the longest rows is 10 us of matrix work a
+// product); flat scores 1139 -> 380; 4 x 16/4 heads, N = 1024, D = 128: 2885 -> 927.  Eight waves to the 32 rows, one
+// workgroup per CU: 330 us for the first.  Where 16-bit calls come here: rows32_16bit in attn_api.hip.
 #pragma once
 #include "attn_bwd_kernel.h"
 

@@ -116,13 +116,14 @@ int adsp_attn_bwd_reads_bmask(int N, int D, int dtype, double alpha);
  * AdaSplash-2 forward: causal entmax-1.5 attention with GQA and right-padded variable lengths.
  *   q, out : [B, Hq, N, D]; k, v : [B, Hkv, N, D], contiguous, Hq % Hkv == 0, D in {16,32,64,128,256}.
  *   taus   : [B, Hq, N] fp32, receives the per-row threshold (rows past the valid length untouched).
- *   bmask  : [B, Hq, adsp_attn_bmask_words(N)] int32, receives the per-(128-row, 64-key) tile mask,
+ *   bmask  : NULL, or [B, Hq, adsp_attn_bmask_words(N)] int32, receives the per-(128-row, 64-key) tile mask,
  *            bit (c % 32) of word c / 32 of a row block = key tile c holds a non-zero probability.
  *   varlen : NULL, or [B] valid lengths as int32 (varlen_bits = 32) or int64 (varlen_bits = 64);
  *            keys >= length are masked, output rows >= length are written as zeros.
- *   niter  : Halley/bisection refinement passes after the histogram bracket (>= 0).  fp32 takes niter + 1 of them,
- *            as the reference does (adasplash/adasplash_v2.py:567-611 and :617-681); the 16-bit types take niter on
- *            the dense kernel, and the sparse-support kernel (head dims 64 / 128) iterates to convergence.
+ *   niter  : Halley/bisection refinement passes after the histogram bracket (>= 0).  where the dense kernel serves
+ *            a call alone it takes niter + 1 of them, as the reference does (adasplash/adasplash_v2.py:567-611 and
+ *            :617-681); behind the sparse-support kernel it takes niter.  That kernel, and those that serve fp32 at head
+ *            dims 64 / 128 and short 16-bit calls without bmask, iterate to convergence.
  * Replaces the four launches at adasplash/adasplash_v2.py:1288-1419.
  */
 int adsp_attn_v2_fwd(const void* q, const void* k, const void* v, void* out, float* taus, int32_t* bmask,
