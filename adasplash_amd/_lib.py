@@ -32,7 +32,7 @@ _SIGNATURES = {
                                   _dbl, _i, _vp, _sz, _vp]),
     "adsp_attn_workspace_bytes": (_sz, [_i, _i, _i, _i, _i, _i]),
     "adsp_attn_bmask_words": (_sz, [_i]),
-    "adsp_attn_bwd_reads_bmask": (_i, [_i, _i, _i, _dbl]),
+    "adsp_attn_bwd_reads_bmask": (_i, [_i, _i, _i, _i, _i, _i, _dbl, _i]),
     "adsp_attn_v2_fwd": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _sz, _vp]),
     "adsp_attn_v2_fwd_noalloc_max_bytes": (_sz, []),
     "adsp_attn_v2_fwd_noalloc": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp]),

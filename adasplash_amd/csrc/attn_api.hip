@@ -35,11 +35,14 @@ int launch_attn_f32_fwd_d128(const AttnParams&, int, hipStream_t);
 int launch_attn_f32_bwd_d64(const AttnBwdParams&, int, hipStream_t);
 int launch_attn_f32_bwd_d128(const AttnBwdParams&, int, hipStream_t);
 
-// their forward for the 16-bit types (attn_rows32_unit.hip)
-int launch_attn_rows32_bf16_d64(const AttnParams&, int, hipStream_t);
-int launch_attn_rows32_bf16_d128(const AttnParams&, int, hipStream_t);
-int launch_attn_rows32_f16_d64(const AttnParams&, int, hipStream_t);
-int launch_attn_rows32_f16_d128(const AttnParams&, int, hipStream_t);
+// the same for the 16-bit types (attn_rows32_unit.hip)
+#define ADSP_DECL_ROWS32(tag, d)                                            \
+  int launch_attn_rows32_fwd_##tag##_d##d(const AttnParams&, int, hipStream_t); \
+  int launch_attn_rows32_bwd_##tag##_d##d(const AttnBwdParams&, int, hipStream_t);
+ADSP_DECL_ROWS32(bf16, 64)
+ADSP_DECL_ROWS32(bf16, 128)
+ADSP_DECL_ROWS32(f16, 64)
+ADSP_DECL_ROWS32(f16, 128)
 
 typedef int (*attn_fwd_fn)(const AttnParams&, int, hipStream_t);
 typedef int (*attn_bwd_fn)(const AttnBwdParams&, int, int, hipStream_t);
@@ -365,12 +368,27 @@ static bool f32_split(int N, int D, int dtype, double alpha) {
 // N = 256: 76 -> 18 and 38 -> 31 (1 and 1/8); 2 of 512: 99 -> 24, 52 -> 32; 32/8 heads, N = 1024: 131 -> 53, 80 -> 74; 16/4
 // heads, N = 2048: 132 -> 93, 89 -> 54, 135 -> 124; 4 x 16 heads, N = 512, not causal: 67 -> 46, 47 -> 34, 95 -> 54; 32 x 16
 // heads, N = 128: 59 -> 42, 44 -> 36, 70 -> 66; beyond it 32/8 heads, N = 2048: 147 -> 132, 96 -> 100, 139 -> 236.
+static double rows32_cost_ns(int B, int Hq, int N, bool causal) {
+  const double heads = (double)B * Hq, r = (N + 31) / 32;
+  return heads * (20.0 * r + 1.35 * (causal ? 0.5 * r * (r + 1.0) : r * r));
+}
 static bool rows32_16bit(int B, int Hq, int N, int D, int dtype, double alpha, bool causal) {
   if (dtype == ADSP_F32 || (D != 64 && D != 128) || N > 65536 || !(alpha >= 1.125 && alpha <= 2.0) || !sparse_enabled()) return false;
-  const long long r = (N + 31) / 32, heads = (long long)B * Hq, groups = heads * r;
-  const double blocks = (double)heads * (causal ? 0.5 * (double)r * (double)(r + 1) : (double)r * (double)r);
+  const long long groups = (long long)B * Hq * ((N + 31) / 32);
   const long long most = N <= 128 ? 2048 : ((N >= 1024 || !causal) ? 1024 : 512);
-  return groups <= most && 20.0 * (double)groups + 1.35 * blocks <= 66e3;
+  return groups <= most && rows32_cost_ns(B, Hq, N, causal) <= 66e3;
+}
+// Of those, the calls whose backward goes the same way (and whose forward then keeps nothing for it): a dK/dV workgroup walks
+// the query blocks of all heads of its group, which only few-headed problems can afford at length.  Forward and backward, us,
+// q of spread 1, 3 and 1/8: 8 heads, 4 sequences of N = 256, D = 64: 136 -> 35, 93 -> 36, 74 -> 48; 2 x 16 heads, N = 512: 158 -> 50,
+// 103 -> 46, 103 -> 55; 8 heads, N = 2048: 238 -> 131, 134 -> 100, 273 -> 122; 16/4 heads, N = 1024: 202 -> 113, 118 -> 107,
+// 285 -> 118; 32 x 16 heads, N = 128: 144 -> 95, 109 -> 90, 136 -> 120; beyond the line 2 x 16/4 heads, N = 1024: 216 -> 143,
+// 121 -> 133, 288 -> 151; 32/8 heads, D = 128: 325 -> 201, 162 -> 190.
+static bool rows32_16bit_training(int B, int Hq, int Hkv, int N, int D, int dtype, double alpha, bool causal) {
+  if (!rows32_16bit(B, Hq, N, D, dtype, alpha, causal)) return false;
+  const double cost = rows32_cost_ns(B, Hq, N, causal);
+  const long long walk = (long long)(Hq / Hkv) * ((N + 31) / 32);
+  return walk <= 64 ? cost <= 50e3 : (walk <= 128 && cost <= 25e3);
 }
 
 static int attn_common(const void* q, const void* k, const void* v, void* out, float* taus, int32_t* bmask,
@@ -447,8 +465,8 @@ static int attn_common(const void* q, const void* k, const void* v, void* out, f
   }
   if (!tile_counts && !bmask && !supports && rows32_16bit(B, Hq, N, D, dtype, alpha, is_causal != 0)) {
     if (w.total && (!workspace || workspace_bytes < w.total || ((uintptr_t)workspace & 15) != 0)) return ADSP_ERR_WORKSPACE;  // (as below)
-    const int rc = dtype == ADSP_BF16 ? (D == 64 ? launch_attn_rows32_bf16_d64(p, am, s) : launch_attn_rows32_bf16_d128(p, am, s))
-                                      : (D == 64 ? launch_attn_rows32_f16_d64(p, am, s) : launch_attn_rows32_f16_d128(p, am, s));
+    const int rc = dtype == ADSP_BF16 ? (D == 64 ? launch_attn_rows32_fwd_bf16_d64(p, am, s) : launch_attn_rows32_fwd_bf16_d128(p, am, s))
+                                      : (D == 64 ? launch_attn_rows32_fwd_f16_d64(p, am, s) : launch_attn_rows32_fwd_f16_d128(p, am, s));
     return rc == 0 && hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
   }
   if (dtype != ADSP_F32) {
@@ -508,8 +526,9 @@ extern "C" size_t adsp_attn_supports_bytes(int B, int Hq, int Hkv, int N, int D,
   return adsp::supports_layout(B, Hq, Hkv, N, D, dtype).total;
 }
 
-extern "C" int adsp_attn_bwd_reads_bmask(int N, int D, int dtype, double alpha) {
-  return adsp::f32_split(N, D, dtype, alpha) ? 0 : 1;
+extern "C" int adsp_attn_bwd_reads_bmask(int B, int Hq, int Hkv, int N, int D, int dtype, double alpha, int is_causal) {
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || N <= 0) return 1;
+  return adsp::f32_split(N, D, dtype, alpha) || adsp::rows32_16bit_training(B, Hq, Hkv, N, D, dtype, alpha, is_causal != 0) ? 0 : 1;
 }
 
 extern "C" size_t adsp_attn_bmask_words(int N) {
@@ -768,13 +787,14 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   BwdWorkspace w = {};
 
   (void)hipGetLastError();
+  const bool short16 = !bmask && !supports && rows32_16bit_training(B, Hq, Hkv, N, D, dtype, alpha, is_causal != 0);
   if (dtype != ADSP_F32) {
     w = bwd_workspace(B, Hq, Hkv, N, D, dtype, is_causal ? 1 : 0);
     const size_t need = w.total;
     if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0)) return ADSP_ERR_WORKSPACE;
     // Sparse-support dQ kernel first (alpha 1.5 / 2): it serves the row blocks whose supports are short and flags the
     // others for attn_bwd_dq_kernel below; the dK/dV kernel reads delta and 1 / sum p from whichever of the two wrote them.
-    sparse = w.slots > 0 && (am == ATT_15 || am == ATT_2 || (alpha >= 1.125 && alpha < 2.0)) &&
+    sparse = !short16 && w.slots > 0 && (am == ATT_15 || am == ATT_2 || (alpha >= 1.125 && alpha < 2.0)) &&
              (long long)B * Hq * mblocks_of(N) < (1ll << 31) && sparse_enabled();
     if (sparse) {
       unsigned char* ws = (unsigned char*)workspace;
@@ -822,6 +842,11 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
       }
       if (rc != 0) return ADSP_ERR_LAUNCH;
     }
+  }
+  if (short16) {
+    const int rc = dtype == ADSP_BF16 ? (D == 64 ? launch_attn_rows32_bwd_bf16_d64(p, am, s) : launch_attn_rows32_bwd_bf16_d128(p, am, s))
+                                      : (D == 64 ? launch_attn_rows32_bwd_f16_d64(p, am, s) : launch_attn_rows32_bwd_f16_d128(p, am, s));
+    return rc == 0 && hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
   }
   if (f32_split(N, D, dtype, alpha)) {
     if ((D == 64 ? launch_attn_f32_bwd_d64(p, am, s) : launch_attn_f32_bwd_d128(p, am, s)) != 0) return ADSP_ERR_LAUNCH;

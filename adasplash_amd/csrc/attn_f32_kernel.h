@@ -1,5 +1,6 @@
 // Sparse entmax attention on workgroups of 32 rows for gfx950, head dims 64 and 128: single-precision forward, dQ and dK/dV
-// kernels, and the same forward for short 16-bit problems.
+// kernels, and the same for short 16-bit problems (there dQ's fp32 weights are split into two 16-bit operands; dK's and dV's are
+// rounded to one, as in the other 16-bit kernels).
 //
 // What bounds them: the fp32 matrix pipe (v_mfma_f32_32x32x2_f32, 64 cycles) on large problems, and on
 // ordinary ones the length of a workgroup's walk over the keys, because a K/V head of N keys has only N / rows workgroups.
@@ -713,10 +714,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // ---------------------------------------------------------------------------------------------------------
 template <int D> constexpr int bwd_smem() { return kRing > kWaves * kRows * D * 4 ? kRing : kWaves * kRows * D * 4; }
 
-template <int D, int AM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_f32_dq_kernel(AttnBwdParams p) {
-  constexpr int NC = D / 32;
-  constexpr int kStride = D * 4;
+template <typename T, int D, int AM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_rows32_dq_kernel(AttnBwdParams p) {
+  constexpr bool k16 = is16<T>::value;
+  constexpr int kStride = D * (k16 ? 2 : 4);
+  constexpr int NC = kStride / 128;      // chunks per block
+  constexpr int kOC = k16 ? 2 : 1;       // blocks of 32 columns per chunk
   __shared__ __align__(4096) unsigned char smem[bwd_smem<D>()];
   __shared__ float red[kWaves][3][kRows];
   const int tid = threadIdx.x;
@@ -729,10 +732,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int m0 = (n_rblk - 1 - mi) * kRows;
   const int L = bwd_seq_len(p, b);
   const size_t q_row0 = (size_t)(b * p.Hq + h) * N;
-  float* const dq = reinterpret_cast<float*>(p.dq) + q_row0 * D;
+  unsigned char* const dq = reinterpret_cast<unsigned char*>(p.dq) + q_row0 * kStride;
   if (m0 >= L) {
     const int rows = N - m0 < kRows ? N - m0 : kRows;
-    for (int i = tid; i < rows * (D / 4); i += 256) reinterpret_cast<f32x4*>(dq + (size_t)m0 * D)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = tid; i < rows * (kStride / 16); i += 256) reinterpret_cast<f32x4*>(dq + (size_t)m0 * kStride)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     return;
   }
   const unsigned char* kg = reinterpret_cast<const unsigned char*>(p.k) + (size_t)bkv * N * kStride;
@@ -743,17 +746,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int key_hi = p.causal ? (m0 + kRows < L ? m0 + kRows : L) : L;
   const int n_kblk = (key_hi + kRows - 1) / kRows;
   const float tau = live ? p.taus[q_row0 + qi] : INFINITY;
-  uint32_t qf[D / 2], dof[D / 2];
+  uint32_t qf[16 * NC], dof[16 * NC];
   {
     const size_t r = q_row0 + (live ? qi : L - 1);
-    load_row<D / 8>(reinterpret_cast<const unsigned char*>(p.q) + r * kStride, lh, qf);
-    load_row<D / 8>(reinterpret_cast<const unsigned char*>(p.dout) + r * kStride, lh, dof);
+    load_row<4 * NC>(reinterpret_cast<const unsigned char*>(p.q) + r * kStride, lh, qf);
+    load_row<4 * NC>(reinterpret_cast<const unsigned char*>(p.dout) + r * kStride, lh, dof);
   }
   Ring<kStride> ring(smem + wave * (kStages * kChunk), lane);
   const uint32_t rl = row_lane_of(lq, lh), cl = col_lane_of(lq, lh);
   // chunks of a block: K, V and, for the second walk, K again
   auto src = [&](int blk, int s, int st) {
-    ring.issue(s < NC || s >= 2 * NC ? kg : vg, blk * kRows, L, s < NC ? s : (s < 2 * NC ? s - NC : s - 2 * NC), st);
+    const unsigned char* g = s < NC || s >= 2 * NC ? kg : vg;
+    if (k16 && s >= 2 * NC) ring.issue_t(g, blk * kRows, L, s % NC, st);
+    else ring.issue(g, blk * kRows, L, s % NC, st);
   };
   // r = z - tau (-inf where the row may not look); false when no row of the block has a member, whose dP is then not formed
   auto block_terms = [&](int blk, auto&& next, float (&r)[16], f32x16& dp) -> bool {
@@ -761,7 +766,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) dot_chunk<D == 64>(s, next(c), rl, qf + c * 16);
+    for (int c = 0; c < NC; ++c) dot_chunk<D == 64, T>(s, next(c), rl, qf + c * 16);
     const int jb = blk * kRows + 4 * lh;
     float mx = -INFINITY;
 #pragma unroll
@@ -773,7 +778,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(NC + c);
-      if (any) dot_chunk<D == 64>(dp, a, rl, dof + c * 16);
+      if (any) dot_chunk<D == 64, T>(dp, a, rl, dof + c * 16);
     }
     return any;
   };
@@ -809,13 +814,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     p.delta[q_row0 + qi] = delta;
     p.zinv[q_row0 + qi] = zsum > 0.f ? 1.f / zsum : 0.f;
   }
-  f32x16 o[NC];
+  f32x16 o[NC][kOC];
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) o[c][i] = 0.f;
+    for (int d = 0; d < kOC; ++d)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[c][d][i] = 0.f;
   walk<3 * NC>(ring, wave, n_kblk, kWaves, src, [&](int blk, auto&& next) {
-    float r[16], dx[16];
+    float r[16], dx[16], lo[16];
     f32x16 dp;
     const bool any = block_terms(blk, next, r, dp);
 #pragma unroll
@@ -823,25 +830,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       float pr, u;
       bwd_prob<AM>(r[i], p.c0, pr, u);
       dx[i] = u > 0.f ? u * (dp[i] - delta) : 0.f;
+      if constexpr (k16) lo[i] = dx[i] - unpack_lo<T>(pack2<T>(dx[i], 0.f));
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(2 * NC + c);
-      if (any) acc_chunk(o[c], a, cl, dx);
+      if constexpr (k16) {
+        if (any) {  // the fp32 weights as two 16-bit parts
+          acc_chunk_16<T>(o[c], a, lane, dx);
+          acc_chunk_16<T>(o[c], a, lane, lo);
+        }
+      } else {
+        if (any) acc_chunk(o[c][0], a, cl, dx);
+      }
     }
   });
   __syncthreads();  // every wave is done with its ring
   const float sm = p.sm_scale;
-  combine_store<D>(o, smem, dq, m0, N, wave, lane, [&](int) { return sm; });
+  combine_store<D>(reinterpret_cast<const f32x16(&)[D / 32]>(o), smem, reinterpret_cast<T*>(dq), m0, N, wave, lane, [&](int) { return sm; });
 }
 
 // ---------------------------------------------------------------------------------------------------------
 // dK, dV: one walk over the (query block, query head) pairs of a K/V head, dV^T += dO^T P and dK^T += Q^T dX
 // ---------------------------------------------------------------------------------------------------------
-template <int D, int AM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void attn_f32_dkdv_kernel(AttnBwdParams p) {
-  constexpr int NC = D / 32;
-  constexpr int kStride = D * 4;
+template <typename T, int D, int AM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void attn_rows32_dkdv_kernel(AttnBwdParams p) {
+  constexpr bool k16 = is16<T>::value;
+  constexpr int kStride = D * (k16 ? 2 : 4);
+  constexpr int NC = kStride / 128;      // chunks per block
+  constexpr int kOC = k16 ? 2 : 1;       // blocks of 32 columns per chunk
   __shared__ __align__(4096) unsigned char smem[bwd_smem<D>()];
   __shared__ __align__(256) float scal[kWaves][4 * kRows];  // of the wave's block: tau, 1 / sum p, delta (and delta once more)
   const int tid = threadIdx.x;
@@ -854,23 +871,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   const int L = bwd_seq_len(p, b);
   const int n0 = kblk * kRows;
   const size_t kv_row0 = (size_t)bkv * N;
-  float* const dk = reinterpret_cast<float*>(p.dk) + kv_row0 * D;
-  float* const dv = reinterpret_cast<float*>(p.dv) + kv_row0 * D;
+  unsigned char* const dk = reinterpret_cast<unsigned char*>(p.dk) + kv_row0 * kStride;
+  unsigned char* const dv = reinterpret_cast<unsigned char*>(p.dv) + kv_row0 * kStride;
   if (n0 >= L) {
     const int rows = N - n0 < kRows ? N - n0 : kRows;
-    for (int i = tid; i < rows * (D / 4); i += 256) {
-      reinterpret_cast<f32x4*>(dk + (size_t)n0 * D)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-      reinterpret_cast<f32x4*>(dv + (size_t)n0 * D)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = tid; i < rows * (kStride / 16); i += 256) {
+      reinterpret_cast<f32x4*>(dk + (size_t)n0 * kStride)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      reinterpret_cast<f32x4*>(dv + (size_t)n0 * kStride)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     return;
   }
   const int kj = n0 + lq;
   const bool live = kj < L;
-  uint32_t kf[D / 2], vf[D / 2];
+  uint32_t kf[16 * NC], vf[16 * NC];
   {
     const size_t r = kv_row0 + (live ? kj : L - 1);
-    load_row<D / 8>(reinterpret_cast<const unsigned char*>(p.k) + r * kStride, lh, kf);
-    load_row<D / 8>(reinterpret_cast<const unsigned char*>(p.v) + r * kStride, lh, vf);
+    load_row<4 * NC>(reinterpret_cast<const unsigned char*>(p.k) + r * kStride, lh, kf);
+    load_row<4 * NC>(reinterpret_cast<const unsigned char*>(p.v) + r * kStride, lh, vf);
   }
   const int q_first = p.causal ? kblk : 0;            // first query block that sees the keys
   const int n_q = (L + kRows - 1) / kRows - q_first;  // query blocks per head
@@ -888,20 +905,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
       dma4((lane < 32 ? p.taus : p.zinv) + at, &scal[wave][0]);
       dma4(p.delta + at, &scal[wave][64]);
     }
-    ring.issue(base, qb * kRows, L, s % NC, st);
+    if (k16 && s >= 2 * NC) ring.issue_t(base, qb * kRows, L, s % NC, st);
+    else ring.issue(base, qb * kRows, L, s % NC, st);
   };
-  f32x16 ov[NC], ok[NC];
+  f32x16 ov[NC][kOC], ok[NC][kOC];
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) ov[c][i] = ok[c][i] = 0.f;
+    for (int d = 0; d < kOC; ++d)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) ov[c][d][i] = ok[c][d][i] = 0.f;
   walk<4 * NC>(ring, wave, n_q * group, kWaves, src, [&](int x, auto&& next) {
     const int g = x / n_q, q0 = (q_first + (x - g * n_q)) * kRows;
     f32x16 s, dp;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) dot_chunk<D == 64>(s, next(c), rl, kf + c * 16);
+    for (int c = 0; c < NC; ++c) dot_chunk<D == 64, T>(s, next(c), rl, kf + c * 16);
     // tau, 1 / sum p and delta of the lane's sixteen queries: they came in front of the block's first chunk
     auto scalars = [&](int which, float (&y)[16]) {
 #pragma unroll
@@ -930,7 +950,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(NC + c);
-      if (any) dot_chunk<D == 64>(dp, a, rl, vf + c * 16);
+      if (any) dot_chunk<D == 64, T>(dp, a, rl, vf + c * 16);
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -942,19 +962,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(2 * NC + c);
-      if (any) acc_chunk(ov[c], a, cl, w);
+      if constexpr (k16) {
+        if (any) acc_chunk_16<T>(ov[c], a, lane, w);
+      } else {
+        if (any) acc_chunk(ov[c][0], a, cl, w);
+      }
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(3 * NC + c);
-      if (any) acc_chunk(ok[c], a, cl, dx);
+      if constexpr (k16) {
+        if (any) acc_chunk_16<T>(ok[c], a, lane, dx);
+      } else {
+        if (any) acc_chunk(ok[c][0], a, cl, dx);
+      }
     }
   });
   __syncthreads();  // every wave is done with its ring
-  combine_store<D>(ov, smem, dv, n0, N, wave, lane, [](int) { return 1.f; });
+  combine_store<D>(reinterpret_cast<const f32x16(&)[D / 32]>(ov), smem, reinterpret_cast<T*>(dv), n0, N, wave, lane, [](int) { return 1.f; });
   __syncthreads();
   const float sm = p.sm_scale;
-  combine_store<D>(ok, smem, dk, n0, N, wave, lane, [&](int) { return sm; });
+  combine_store<D>(reinterpret_cast<const f32x16(&)[D / 32]>(ok), smem, reinterpret_cast<T*>(dk), n0, N, wave, lane, [&](int) { return sm; });
 }
 
 }  // namespace f32path

@@ -108,12 +108,14 @@ struct SavedLayout {
 // out, and in `saved` what a later backward needs.  Without one (`keep` is false) thresholds and tile mask share the
 // workspace's allocation.
 Tensor attn_forward(const Tensor& q, const Tensor& k, const Tensor& v, const AttnCall& c, bool keep, int keep_mode, Tensor* saved,
-                    size_t* supports_bytes) {
+                    size_t* supports_bytes, bool* has_mask = nullptr) {
   const int B = (int)q.size(0), Hq = (int)q.size(1), N = (int)q.size(2), D = (int)q.size(3), Hkv = (int)k.size(1);
   const int dt = dtype_code(q);
   require(k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type(), "q, k and v must share a dtype");
+  // (a caller that asked for supports gets the route that keeps them)
+  const bool mask = keep && ((keep_mode == KEEP_ALWAYS && dt != ADSP_F32) || adsp_attn_bwd_reads_bmask(B, Hq, Hkv, N, D, dt, c.alpha, c.causal));
   size_t sup = 0;
-  if (keep && keep_mode != KEEP_NEVER) {
+  if (mask && keep_mode != KEEP_NEVER) {
     sup = adsp_attn_supports_bytes(B, Hq, Hkv, N, D, dt);
     // "auto": at most twice the bytes of q, or 256 MiB
     const size_t most = std::max((size_t)2 * q.numel() * q.element_size(), (size_t)256 << 20);
@@ -136,7 +138,7 @@ Tensor attn_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Att
     wp = ws_bytes ? kp + align256(l.total) : nullptr;
   }
   float* taus = (float*)kp;
-  int32_t* bmask = keep && adsp_attn_bwd_reads_bmask(N, D, dt, c.alpha) ? (int32_t*)(kp + l.bmask_off) : nullptr;
+  int32_t* bmask = mask ? (int32_t*)(kp + l.bmask_off) : nullptr;
   void* supports = sup ? kp + l.supports_off : nullptr;
   void* stream = stream_of(q);
   if (c.version == 2) {
@@ -155,6 +157,7 @@ Tensor attn_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Att
   }
   if (saved) *saved = kept;
   if (supports_bytes) *supports_bytes = sup;
+  if (has_mask) *has_mask = mask;
   return out;
 }
 
@@ -162,11 +165,13 @@ struct AttnFunction : torch::autograd::Function<AttnFunction> {
   static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const AttnCall& c, int keep_mode) {
     Tensor saved;
     size_t sup = 0;
-    Tensor out = attn_forward(q, k, v, c, true, keep_mode, &saved, &sup);
+    bool mask = false;
+    Tensor out = attn_forward(q, k, v, c, true, keep_mode, &saved, &sup, &mask);
     ctx->save_for_backward({q, k, v, saved});
     ctx->saved_data["alpha"] = c.alpha;
     ctx->saved_data["causal"] = c.causal;
     ctx->saved_data["supports"] = (int64_t)sup;
+    ctx->saved_data["bmask"] = mask;
     if (c.varlen.defined()) ctx->saved_data["varlen"] = c.varlen;
     return out;
   }
@@ -190,13 +195,14 @@ struct AttnFunction : torch::autograd::Function<AttnFunction> {
     char* const sp = (char*)scratch.data_ptr();
     char* const kp = (char*)saved.data_ptr();
     void* const ws = ws_bytes ? sp + 2 * per_row : nullptr;
+    int32_t* const bmask = ctx->saved_data["bmask"].toBool() ? (int32_t*)(kp + l.bmask_off) : nullptr;
     void* const stream = stream_of(q);
     const int st =
-        l.supports ? adsp_attn_bwd_kept(q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), (float*)kp, (int32_t*)(kp + l.bmask_off),
+        l.supports ? adsp_attn_bwd_kept(q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), (float*)kp, bmask,
                                         data(c.varlen), c.varlen_bits(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), (float*)sp,
                                         (float*)(sp + per_row), B, Hq, Hkv, N, D, dt, alpha, causal, ws, ws_bytes,
                                         kp + l.supports_off, l.supports, stream)
-                   : adsp_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), (float*)kp, (int32_t*)(kp + l.bmask_off),
+                   : adsp_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), (float*)kp, bmask,
                                    data(c.varlen), c.varlen_bits(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), (float*)sp,
                                    (float*)(sp + per_row), B, Hq, Hkv, N, D, dt, alpha, causal, ws, ws_bytes, stream);
     check(st, l.supports ? "adsp_attn_bwd_kept" : "adsp_attn_bwd");

@@ -108,9 +108,10 @@ size_t adsp_attn_workspace_bytes(int B, int Hq, int Hkv, int N, int D, int dtype
 /* Number of int32 words per (batch, head) the block mask needs: n_row_blocks * words_per_row. */
 size_t adsp_attn_bmask_words(int N);
 
-/* 0 when the backward of such a call does not look at the forward's tile mask, so that a caller with no other use for it may
- * pass NULL for bmask to both (single precision at head dims 64 and 128; the forward then has less to write), else 1. */
-int adsp_attn_bwd_reads_bmask(int N, int D, int dtype, double alpha);
+/* 0 when the backward of such a call needs neither the forward's tile mask nor its supports, so that a caller with no other use
+ * for them passes NULL to both (single precision at head dims 64 and 128, and short 16-bit problems there: the call then
+ * takes the kernels made for them), else 1. */
+int adsp_attn_bwd_reads_bmask(int B, int Hq, int Hkv, int N, int D, int dtype, double alpha, int is_causal);
 
 /*
  * AdaSplash-2 forward: causal entmax-1.5 attention with GQA and right-padded variable lengths.
