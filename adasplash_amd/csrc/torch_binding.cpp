@@ -287,6 +287,13 @@ Tensor decode_forward(const Tensor& q, const Tensor& k, const Tensor& v, double 
 }
 
 bool wants_grad(const Tensor& t) { return t.requires_grad(); }
+// A dual tensor of forward-mode differentiation need not ask for a gradient; the kernels have no forward derivative, with or
+// without a graph and whatever the grad mode is.
+bool has_tangent(const Tensor& t) { return t.defined() && t._fw_grad(0).defined(); }
+void refuse_tangent(std::initializer_list<const Tensor*> inputs) {
+  for (const Tensor* t : inputs)
+    if (has_tangent(*t)) C10_THROW_ERROR(NotImplementedError, "forward-mode differentiation (jvp) of the entmax kernels is not implemented");
+}
 
 // ---- Python side ----------------------------------------------------------------------------------------------------
 const Tensor& tensor_arg(PyObject* o, const char* what) {
@@ -336,6 +343,7 @@ PyObject* py_entmax_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
     require(x.dim() > 0, "x must have at least one dimension");
     require(x.is_contiguous(), "x must be contiguous");
     require_device(x);
+    refuse_tangent({&x});
     const bool grad = at::GradMode::is_enabled() && wants_grad(x);
     pybind11::gil_scoped_release no_gil;
     return grad ? RowsFunction::apply(x, alpha, n_iter, hist, fast) : rows_forward(x, alpha, n_iter, hist, fast);
@@ -351,6 +359,7 @@ PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (a[7] != Py_None) c.varlen = tensor_arg(a[7], "varlen");
     const int keep_mode = (int)long_arg(a[8]);
     check_attention(q, k, v, c);
+    refuse_tangent({&q, &k, &v});
     const bool grad = at::GradMode::is_enabled() && (wants_grad(q) || wants_grad(k) || wants_grad(v));
     pybind11::gil_scoped_release no_gil;
     return grad ? AttnFunction::apply(q, k, v, c, keep_mode) : attn_forward(q, k, v, c, false, KEEP_NEVER, nullptr, nullptr);
@@ -369,6 +378,7 @@ PyObject* py_decode_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (a[7] != Py_None) slopes = tensor_arg(a[7], "alibi_slopes");
   if (at::GradMode::is_enabled() && (wants_grad(q) || wants_grad(k) || wants_grad(v) || (slopes.defined() && wants_grad(slopes))))
     Py_RETURN_NONE;
+  if (has_tangent(q) || has_tangent(k) || has_tangent(v) || has_tangent(slopes)) Py_RETURN_NONE;  // (the dense path says what it can do)
   Tensor out;
   {
     pybind11::gil_scoped_release no_gil;
