@@ -253,12 +253,21 @@ void check_attention(const Tensor& q, const Tensor& k, const Tensor& v, AttnCall
 }
 
 // ---- a few queries against a cache of keys --------------------------------------------------------------------------
+// What stands between a tensor and its data: batches of vmap, wrappers of functorch's gradients, subclasses with a dispatch of
+// their own, a sign that a view carries.  Torch's operators honour it; the data pointer does not.
+bool is_plain(const Tensor& t) {
+  static const c10::DispatchKeySet behind{c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Python,
+                                          c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor};
+  return !t.defined() || !t.key_set().has_any(behind);
+}
+
 // Undefined where adsp_attn_decode_fwd does not take the call: a gradient is asked for, many queries, other head dims or types, an
-// inner stride.
+// inner stride, tensors that are more than their data.
 Tensor decode_forward(const Tensor& q, const Tensor& k, const Tensor& v, double alpha, const Tensor& varlen, bool causal, bool left,
                       const Tensor& slopes) {
   const int64_t B = q.size(0), H = q.size(1), q_len = q.size(2), D = q.size(3), k_len = k.size(2);
   const auto t = q.scalar_type();
+  if (!is_plain(q) || !is_plain(k) || !is_plain(v) || !is_plain(varlen) || !is_plain(slopes)) return Tensor();
   if (!q.is_cuda() || !k.is_cuda() || !v.is_cuda() || k.device() != q.device() || v.device() != q.device()) return Tensor();
   if ((t != at::kFloat && t != at::kBFloat16 && t != at::kHalf) || k.scalar_type() != t || v.scalar_type() != t) return Tensor();
   if (q_len < 1 || q_len > 16 || (D != 32 && D != 64 && D != 128 && D != 256) || k_len < 1 || k_len > (1 << 24)) return Tensor();

@@ -47,3 +47,14 @@ def test_a_tangent_of_v_passes_through_a_decoding_step():
         t = torch.randn_like(v)
         got = fwd.unpack_dual(fn(q, k, fwd.make_dual(v, t), s)).tangent
     assert (got - fn(q, k, t, s)).abs().max().item() < 1e-4
+
+
+def test_a_decoding_step_on_tensors_that_are_more_than_their_data():
+    """vmap over v, and caches that are views with a sign (as the imaginary part of a conjugate is): the dense path's
+    operators honour both."""
+    (q, k, v, s), fn = _calls()["decode"]
+    vs = torch.stack([v, 2 * v])
+    got = torch.func.vmap(lambda x: fn(q, k, x, s))(vs)
+    assert (got - torch.stack([fn(q, k, x, s) for x in vs])).abs().max().item() < 1e-4
+    assert (fn(q, torch._neg_view(k), v, s) - fn(q, -k, v, s)).abs().max().item() < 1e-4
+    assert (fn(q, k, torch._neg_view(v), s) - fn(q, k, -v, s)).abs().max().item() < 1e-4
