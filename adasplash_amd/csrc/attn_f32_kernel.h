@@ -1,6 +1,6 @@
 // Sparse entmax attention on workgroups of 32 rows for gfx950, head dims 64 and 128: single-precision forward, dQ and dK/dV
-// kernels, and the same for short 16-bit problems (there dQ's fp32 weights are split into two 16-bit operands; dK's and dV's are
-// rounded to one, as in the other 16-bit kernels).
+// kernels, and the same for short 16-bit problems (there dQ's fp32 weights are split into two 16-bit operands, for f16 behind a
+// power of two per row; dK's and dV's are rounded to one, as in the other 16-bit kernels).
 //
 // What bounds them: the fp32 matrix pipe (v_mfma_f32_32x32x2_f32, 64 cycles) on large problems, and on
 // ordinary ones the length of a workgroup's walk over the keys, because a K/V head of N keys has only N / rows workgroups.
@@ -721,7 +721,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr int NC = kStride / 128;      // chunks per block
   constexpr int kOC = k16 ? 2 : 1;       // blocks of 32 columns per chunk
   __shared__ __align__(4096) unsigned char smem[bwd_smem<D>()];
-  __shared__ float red[kWaves][3][kRows];
+  // f16: a row's weights are scaled by a power of two before they are split, so that neither part leaves the type's range
+  constexpr bool kScaled = k16 && !elem_traits<T>::kIsBf16;
+  __shared__ float red[kWaves][kScaled ? 4 : 3][kRows];
+  __shared__ float unscale[kScaled ? kRows : 1];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
@@ -782,7 +785,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     return any;
   };
-  float zsum = 0.f, usum = 0.f, udp = 0.f;
+  float zsum = 0.f, usum = 0.f, udp = 0.f, dmax = 0.f;
   walk<2 * NC>(ring, wave, n_kblk, kWaves, src, [&](int blk, auto&& next) {
     float r[16];
     f32x16 dp;
@@ -794,15 +797,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       zsum += pr;
       usum += u;
       udp += u > 0.f ? u * dp[i] : 0.f;
+      if constexpr (kScaled) dmax = fmaxf(dmax, u > 0.f ? fabsf(dp[i]) : 0.f);
     }
   });
   zsum += __shfl_xor(zsum, 32, 64);
   usum += __shfl_xor(usum, 32, 64);
   udp += __shfl_xor(udp, 32, 64);
+  if constexpr (kScaled) dmax = fmaxf(dmax, __shfl_xor(dmax, 32, 64));
   if (lh == 0) {
     red[wave][0][lq] = zsum;
     red[wave][1][lq] = usum;
     red[wave][2][lq] = udp;
+    if constexpr (kScaled) red[wave][3][lq] = dmax;
   }
   __syncthreads();
   auto all = [&](int k) { return (red[0][k][lq] + red[1][k][lq]) + (red[2][k][lq] + red[3][k][lq]); };
@@ -810,6 +816,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   usum = all(1);
   udp = all(2);
   const float delta = usum > 0.f ? udp / usum : 0.f;
+  // u is at most 1 (to rounding) and delta is a mean of the members' dP, so |u (dP - delta)| < 2 max |dP| < 2^(e + 1) with
+  // max |dP| < 2^e: times 2^(13 - e) it stays below 2^14, and the second part's spacing, 2^-24 at the least, is 2^-38 of that.
+  // (|dP| < 2^40, as a sum of 128 products of f16 numbers; at a factor of 2^60 the spacing is 2^-84, far below what dQ resolves.)
+  int up = 0;
+  if constexpr (kScaled) {
+    dmax = fmaxf(fmaxf(red[0][3][lq], red[1][3][lq]), fmaxf(red[2][3][lq], red[3][3][lq]));
+    const int e = (int)(__builtin_bit_cast(uint32_t, dmax) >> 23) - 126;
+    up = 13 - e;
+    up = up > 60 ? 60 : (up < -60 ? -60 : up);
+  }
   if (live && wave == 0 && lh == 0) {
     p.delta[q_row0 + qi] = delta;
     p.zinv[q_row0 + qi] = zsum > 0.f ? 1.f / zsum : 0.f;
@@ -830,6 +846,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       float pr, u;
       bwd_prob<AM>(r[i], p.c0, pr, u);
       dx[i] = u > 0.f ? u * (dp[i] - delta) : 0.f;
+      if constexpr (kScaled) dx[i] = __builtin_amdgcn_ldexpf(dx[i], up);
       if constexpr (k16) lo[i] = dx[i] - unpack_lo<T>(pack2<T>(dx[i], 0.f));
     }
 #pragma unroll
@@ -845,9 +862,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
   });
+  if constexpr (kScaled) {
+    if (wave == 0 && lh == 0) unscale[lq] = __builtin_amdgcn_ldexpf(p.sm_scale, -up);
+  }
   __syncthreads();  // every wave is done with its ring
   const float sm = p.sm_scale;
-  combine_store<D>(reinterpret_cast<const f32x16(&)[D / 32]>(o), smem, reinterpret_cast<T*>(dq), m0, N, wave, lane, [&](int) { return sm; });
+  combine_store<D>(reinterpret_cast<const f32x16(&)[D / 32]>(o), smem, reinterpret_cast<T*>(dq), m0, N, wave, lane,
+                   [&](int row) { return kScaled ? unscale[row] : sm; });
 }
 
 // ---------------------------------------------------------------------------------------------------------

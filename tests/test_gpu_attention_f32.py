@@ -125,3 +125,25 @@ def test_16bit_gradients_lengths_around_blocks_and_steps(dtype, alpha, causal, H
             assert num < 2e-2 * den, name
         else:
             assert max_err(a, w) < (2e-2 if name == "out" else 4e-2 * max(1.0, scale)), name
+
+
+@pytest.mark.parametrize("scale", [0.125, 1.0])
+@pytest.mark.parametrize("alpha,causal,Hq,Hkv,D", [(1.5, True, 2, 1, 64), (1.5, True, 1, 1, 128), (1.333, False, 1, 1, 64)])
+@pytest.mark.parametrize("dout_scale", [1e-6, 1.0, 3e4])
+def test_f16_dq_for_gradients_at_the_ends_of_the_types_range(dout_scale, alpha, causal, Hq, Hkv, D, scale):
+    """dQ's weights u (dP - delta) are held to fp32: neither upstream gradients near f16's smallest numbers nor weights
+    beyond its largest (dout of 3e4 gives some of 1e5) may cost anything.  k and q are scaled against each other so that dq
+    itself is an ordinary number.  Bound on the error (2-norm, relative): rounding dq to f16 leaves at most 2^-11 of each
+    entry; thresholds and sums in fp32 add less than that again."""
+    g = torch.Generator().manual_seed(8)
+    N = 517
+    kscale = 256.0 if dout_scale < 1.0 else (1.0 if dout_scale == 1.0 else 2.0 ** -10)
+    varlen = torch.tensor([517, 130], dtype=torch.int32)
+    q = (scale / kscale * torch.randn(2, Hq, N, D, generator=g)).half()
+    k = (kscale * torch.randn(2, Hkv, N, D, generator=g)).half()
+    v = torch.randn(2, Hkv, N, D, generator=g).half()
+    dout = (dout_scale * torch.randn(2, Hq, N, D, generator=g)).clamp(-6e4, 6e4).half()
+    want = exact.dense_entmax_attention_grads(q, k, v, dout, alpha, causal, varlen)[0]
+    got = run(q, k, v, dout, varlen, alpha, causal, Hq != Hkv)[1].double().cpu()
+    assert torch.isfinite(got).all()
+    assert (got - want).norm() < 2.0 ** -10 * want.norm()
