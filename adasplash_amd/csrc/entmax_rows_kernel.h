@@ -576,11 +576,20 @@ __global__ __launch_bounds__(rows_threads<TPR>()) void entmax_rows_bwd_reg_kerne
   } while (0)
 constexpr long long kRowsMaxChunks = 16384;
 
+// HIP takes launches of fewer than 2^32 threads: whether `rows` rows of `nvec` chunks stay below it, rounded up to whole blocks.
+inline bool rows_fit_grid(long long rows, long long nvec) {
+  long long threads = 0;
+#define ADSP_ROWS_THREADS(NC, TPR) threads = (rows + rows_threads<TPR>() / TPR - 1) / (rows_threads<TPR>() / TPR) * rows_threads<TPR>()
+  ADSP_ROWS_DISPATCH(nvec, ADSP_ROWS_THREADS);
+  return threads < (1ll << 32);
+}
+
 // 0: the row's chunks are aligned and fill it; 1: it has edges; 2: neither (bases that differ in their offset from a 16-byte
-// boundary, elements off their own alignment, very short ragged rows, more chunks than the registers hold): stream it
+// boundary, elements off their own alignment, very short ragged rows, more chunks than the registers hold, more rows than a
+// launch of the register kernels holds): stream it
 template <typename T> static int rows_shape(uintptr_t a, uintptr_t b, uintptr_t c, long long rows, long long cols) {
   constexpr int kVec = elem_traits<T>::kVec;
-  if (rows >= (1ll << 31) || cols / kVec > kRowsMaxChunks) return 2;
+  if (cols / kVec > kRowsMaxChunks || rows >= (1ll << 32) || !rows_fit_grid(rows, cols / kVec)) return 2;
   if (((a | b | c) & 15) == 0 && cols % kVec == 0) return 0;
   if (((a ^ b) & 15) != 0 || ((a ^ c) & 15) != 0 || a % elem_traits<T>::kBytes != 0 || cols < 2 * kVec - 1) return 2;
   return 1;

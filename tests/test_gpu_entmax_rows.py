@@ -243,3 +243,21 @@ def test_rows_that_start_and_end_off_a_16_byte_boundary(cols, alpha, dtype, offs
     assert (dx.double().cpu() - want).abs().max().item() < tol * max(1.0, want.abs().max().item())
     for b in bufs:
         assert float(b[-1]) == 7.0 and (offset == 0 or float(b[0]) == 7.0)
+
+
+def test_more_short_ragged_rows_than_a_grid_of_row_blocks_holds():
+    """2^28 rows of 7: sixteen threads a row would be a launch of 2^32 threads, which HIP refuses; forward and backward."""
+    rows, cols = 1 << 28, 7
+    x = torch.empty(rows, cols, device=DEV).normal_().requires_grad_(True)
+    y = A.triton_entmax(x)
+    dy = torch.empty_like(y).normal_()
+    (dx,) = torch.autograd.grad(y, (x,), dy)
+    at = torch.tensor([0, 1, 15, 16, 65535, 65536, rows // 2 + 3, rows - 2, rows - 1], device=DEV)
+    xs = x.detach()[at].cpu()
+    assert max_err(y.detach()[at], exact.entmax_rows(xs, 1.5)) < 1e-4
+    u = y.detach()[at].double().cpu().sqrt()
+    g = dy[at].double().cpu()
+    assert max_err(dx[at], u * g - (u * g).sum(-1, keepdim=True) / u.sum(-1, keepdim=True) * u) < 1e-4
+    # no row is left out: probabilities add up to one, and so do gradients to zero
+    assert all((part.sum(-1) - 1).abs().max().item() < 1e-4 for part in y.detach().split(1 << 24))
+    assert all(part.sum(-1).abs().max().item() < 1e-4 for part in dx.split(1 << 24))
