@@ -7,7 +7,8 @@
 //    the keys alone fills the chip whatever the batch.
 // 2. decode_output_kernel, a workgroup per query row: the row's scores come back from L2, the few that can be in the
 //    support (z >= max - 1) go to a list in LDS, the threshold is solved on the list as in the rows kernels, and only the V rows
-//    of the support are read.
+//    of the support are read.  The list's order, and with it that of every sum over it, is the order of the threads (a prefix sum
+//    over their counts), so a call returns the same bits every time.
 // A step of 16 x 16 heads against caches of up to 4096 keys (D = 64, bf16, 84 MB of K in use): 265 us as fp32 copies of q and
 // K, a library product, ten elementwise launches, the rows kernel and a second product; 27 us now (20 us = 4.2 TB/s and 6.7 us).
 #include "entmax_rows_kernel.h"
@@ -114,9 +115,20 @@ template <typename T, int D, int AM> __global__ __launch_bounds__(256) void deco
   __shared__ float sm[32];
   __shared__ float list_z[kDecodeCap];
   __shared__ int list_key[kDecodeCap];
-  __shared__ int list_n;
+  __shared__ int counts[2][4];
   __shared__ float red[4][D];
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // Where this thread's `count` entries start in a list that the 256 threads fill in turn, behind the `n` that it holds; `n` becomes
+  // the new length.  One barrier: two calls in a row use the two halves of `counts`.
+  auto place = [&](int count, int half, int& n) {
+    const int upto = wave_prefix_sum(count);
+    if (lane == 63) counts[half][wave] = upto;
+    __syncthreads();
+    const int c0 = counts[half][0], c1 = counts[half][1], c2 = counts[half][2], c3 = counts[half][3];
+    const int at = n + upto - count + (wave > 0 ? c0 : 0) + (wave > 1 ? c1 : 0) + (wave > 2 ? c2 : 0);
+    n += (c0 + c1) + (c2 + c3);
+    return at;
+  };
   const int row = blockIdx.x, bh = row / p.q_len, b = bh / p.H, h = bh % p.H;
   int first, last;
   decode_span(p, b, first, last);
@@ -124,7 +136,6 @@ template <typename T, int D, int AM> __global__ __launch_bounds__(256) void deco
   // whole groups of four keys around [first, last): the scores kernel has written -inf at the keys outside the span
   const int c0 = first >> 2, c1 = first < last ? (last + 3) >> 2 : c0;
   const f32x4* const z4 = reinterpret_cast<const f32x4*>(zrow);
-  if (tid == 0) list_n = 0;
   // eight loads of a thread under way together; a row of up to 8192 keys is then in registers for the second look as well
   constexpr int kHold = 8;
   f32x4 held[kHold];
@@ -148,25 +159,32 @@ template <typename T, int D, int AM> __global__ __launch_bounds__(256) void deco
   for (int e = 0; e < kVec; ++e) acc[e] = 0.f;
   if (m > -INFINITY) {  // (a query that sees no key at all is a row of zeros)
     const float thr = m - 1.f;
+    int n = 0, half = 0;
     for (int from = c0; from < c1; from += kHold * 256) {
       if (c1 - c0 > kHold * 256) load_held(from);
+      int count = 0;
+#pragma unroll
+      for (int i = 0; i < kHold; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) count += held[i][e] >= thr ? 1 : 0;
+      int at = place(count, half, n);
+      half ^= 1;
 #pragma unroll
       for (int i = 0; i < kHold; ++i) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float z = held[i][e];
           if (z >= thr) {
-            const int at = atomicAdd(&list_n, 1);
             if (at < kDecodeCap) {
               list_z[at] = z;
               list_key[at] = (from + i * 256 + tid) * 4 + e;
             }
+            ++at;
           }
         }
       }
     }
     __syncthreads();
-    const int n = list_n;
     const int grp = tid / kLanes, col = tid % kLanes;
     const char* const vbase = (const char*)p.v + ((size_t)(b * p.v_sb + h * p.v_sh) + col * kVec) * elem_traits<T>::kBytes;
     auto row_of = [&](int key) { return *reinterpret_cast<const u32x4*>(vbase + key * p.v_sn * elem_traits<T>::kBytes); };
@@ -194,19 +212,19 @@ template <typename T, int D, int AM> __global__ __launch_bounds__(256) void deco
         w[c] = i < n ? prob<AM>(list_z[i] - tau, p.rows.c0) : 0.f;
         key[c] = i < n ? list_key[i] : 0;
       }
-      __syncthreads();
-      if (tid == 0) list_n = 0;
-      __syncthreads();
+      int count = 0, members = 0;
+#pragma unroll
+      for (int c = 0; c < kDecodeCap / 256; ++c) count += w[c] > 0.f ? 1 : 0;
+      int at = place(count, half, members);  // (its barrier: every thread has read its part of the list)
 #pragma unroll
       for (int c = 0; c < kDecodeCap / 256; ++c) {
         if (w[c] > 0.f) {
-          const int at = atomicAdd(&list_n, 1);
           list_z[at] = w[c];
           list_key[at] = key[c];
+          ++at;
         }
       }
       __syncthreads();
-      const int members = list_n;
       // four rows of a group under way together; a slot past the end takes the first member's row with weight zero
       for (int i = grp; i < members; i += 4 * kGroups) {
         u32x4 raw[4];

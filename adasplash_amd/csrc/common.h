@@ -103,6 +103,17 @@ __device__ __forceinline__ int wave_sum_i(int v) {
   return v;
 }
 
+// Sum over the lanes up to and including this one.
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // a prefix within every row of 16 lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row 0's total into row 1, row 2's into row 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // the first half's total into rows 2 and 3
+  return v;
+}
+
 // ---- block numbering of the dense attention kernels -------------------------------------------------------
 // Hardware block ids are dealt round-robin to the 8 XCDs (one L2 each): XCD x runs the blocks x, x + 8, ... in
 // that order, a new one whenever a slot of its 32 CUs falls free.  The K/V heads (`units`) are dealt round-robin

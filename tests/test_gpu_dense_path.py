@@ -152,3 +152,16 @@ def test_decoding_kernels(q_len, k_len, D, alpha, padding, dtype, tol):
     zero = dense.slow_entmax_attention(q.to(DEV), kd, vd, alpha=alpha, padding=padding,
                                        varlen=torch.zeros(B, dtype=torch.int64, device=DEV)) if q_len != k_len else None
     assert zero is None or (zero == 0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("q_len,k_len,scale,alpha", [(1, 3000, 1.0, 1.5), (4, 1000, 0.1, 1.5), (1, 9000, 0.3, 1.333), (2, 700, 0.02, 2.0)])
+def test_decoding_kernels_return_the_same_bits_on_every_call(q_len, k_len, scale, alpha, dtype):
+    """Lists of a few to several hundred candidates, filled by all four waves of a workgroup (9000 keys: in two passes over
+    the row): their order, and with it the order of the sums over them, is that of the threads and not of arrival."""
+    g = torch.Generator().manual_seed(q_len * 10000 + k_len)
+    q, k, v = (torch.randn(8, 16, n, 64, generator=g).to(dtype).to(DEV) for n in (q_len, k_len, k_len))
+    q = (scale * q.float()).to(dtype)
+    first = dense.slow_entmax_attention(q, k, v, alpha=alpha, is_causal=True)
+    for _ in range(20):
+        assert torch.equal(dense.slow_entmax_attention(q, k, v, alpha=alpha, is_causal=True), first)
