@@ -92,121 +92,142 @@ struct AttnCall {
   int varlen_bits() const { return !varlen.defined() ? 0 : (varlen.scalar_type() == at::kLong ? 64 : 32); }
 };
 enum KeepMode { KEEP_NEVER = 0, KEEP_ALWAYS = 1, KEEP_AUTO = 2 };
+// "auto": supports of at most twice the bytes of q, or 256 MiB
+bool keeps_supports(int mode, size_t supports, size_t q_bytes) {
+  if (mode == KEEP_NEVER || supports == 0) return false;
+  return mode == KEEP_ALWAYS || supports <= std::max(2 * q_bytes, (size_t)256 << 20);
+}
 
-// One allocation holds what the backward reads besides q, k and v: thresholds [B, Hq, N] fp32, the tile mask, and the supports
-// the forward keeps (none when `supports` is 0).
-struct SavedLayout {
-  size_t bmask_off, supports_off, total, supports;
-  SavedLayout(const Tensor& q, size_t supports_bytes) : supports(supports_bytes) {
+// What a forward leaves behind besides its output, in one allocation: thresholds [B, Hq, N] fp32, the tile mask, and the
+// supports it keeps (none when `supports` is 0).
+struct Kept {
+  Tensor buffer;
+  bool mask = false;
+  size_t supports = 0, bmask_off = 0, supports_off = 0;
+  int64_t rows = 0, mask_words = 0;
+  size_t layout(const Tensor& q) {
     const int64_t B = q.size(0), Hq = q.size(1), N = q.size(2);
-    bmask_off = align256((size_t)(B * Hq * N) * 4);
-    supports_off = align256(bmask_off + (size_t)(B * Hq) * adsp_attn_bmask_words((int)N) * 4);
-    total = supports_off + supports;
+    rows = B * Hq * N;
+    mask_words = B * Hq * (int64_t)adsp_attn_bmask_words((int)N);
+    bmask_off = align256((size_t)rows * 4);
+    supports_off = align256(bmask_off + (size_t)mask_words * 4);
+    return supports_off + supports;
   }
+  char* base() const { return (char*)buffer.data_ptr(); }
+  float* taus() const { return (float*)base(); }
+  int32_t* bmask() const { return mask ? (int32_t*)(base() + bmask_off) : nullptr; }
+  void* kept_supports() const { return supports ? base() + supports_off : nullptr; }
 };
 
-// out, and in `saved` what a later backward needs.  Without one (`keep` is false) thresholds and tile mask share the
-// workspace's allocation.
-Tensor attn_forward(const Tensor& q, const Tensor& k, const Tensor& v, const AttnCall& c, bool keep, int keep_mode, Tensor* saved,
-                    size_t* supports_bytes, bool* has_mask = nullptr) {
+// What the caller wants of a forward besides its output.
+struct Wants {
+  bool backward = false;         // what the backward reads: the tile mask where it does, and supports as the mode says
+  int keep_mode = KEEP_NEVER;
+  bool mask = false;             // the tile mask in any case
+  bool outlives = false;         // what the forward leaves outlives the call
+  unsigned long long* tile_counts = nullptr;
+};
+
+Tensor attn_forward(const Tensor& q, const Tensor& k, const Tensor& v, const AttnCall& c, const Wants& w, Kept& kept) {
   const int B = (int)q.size(0), Hq = (int)q.size(1), N = (int)q.size(2), D = (int)q.size(3), Hkv = (int)k.size(1);
   const int dt = dtype_code(q);
   require(k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type(), "q, k and v must share a dtype");
   // (a caller that asked for supports gets the route that keeps them)
-  const bool mask = keep && ((keep_mode == KEEP_ALWAYS && dt != ADSP_F32) || adsp_attn_bwd_reads_bmask(B, Hq, Hkv, N, D, dt, c.alpha, c.causal));
-  size_t sup = 0;
-  if (mask && keep_mode != KEEP_NEVER) {
-    sup = adsp_attn_supports_bytes(B, Hq, Hkv, N, D, dt);
-    // "auto": at most twice the bytes of q, or 256 MiB
-    const size_t most = std::max((size_t)2 * q.numel() * q.element_size(), (size_t)256 << 20);
-    if (keep_mode == KEEP_AUTO && sup > most) sup = 0;
+  kept.mask = w.mask || (w.backward && ((w.keep_mode == KEEP_ALWAYS && dt != ADSP_F32) ||
+                                        adsp_attn_bwd_reads_bmask(B, Hq, Hkv, N, D, dt, c.alpha, c.causal)));
+  if (kept.mask && w.backward && !w.tile_counts) {
+    const size_t sup = adsp_attn_supports_bytes(B, Hq, Hkv, N, D, dt);
+    if (keeps_supports(w.keep_mode, sup, q.numel() * q.element_size())) kept.supports = sup;
   }
   const c10::DeviceGuard guard(q.device());
-  const SavedLayout l(q, sup);
-  const size_t ws_bytes = adsp_attn_workspace_bytes(B, Hq, Hkv, N, D, dt);
+  const size_t keep_bytes = kept.layout(q), ws_bytes = adsp_attn_workspace_bytes(B, Hq, Hkv, N, D, dt);
   Tensor out = at::empty_like(q);
-  Tensor kept, ws;
-  char *kp, *wp;
-  if (keep) {
-    kept = bytes(l.total, q);
-    kp = (char*)kept.data_ptr();
+  Tensor ws;
+  void* wp = nullptr;
+  if (w.outlives) {
+    kept.buffer = bytes(keep_bytes, q);
     if (ws_bytes) ws = bytes(ws_bytes, q);
-    wp = (char*)data(ws);
-  } else {
-    kept = bytes(align256(l.total) + ws_bytes, q);
-    kp = (char*)kept.data_ptr();
-    wp = ws_bytes ? kp + align256(l.total) : nullptr;
+    wp = data(ws);
+  } else {  // nothing outlives the call: one allocation for all of it
+    kept.buffer = bytes(align256(keep_bytes) + ws_bytes, q);
+    if (ws_bytes) wp = kept.base() + align256(keep_bytes);
   }
-  float* taus = (float*)kp;
-  int32_t* bmask = mask ? (int32_t*)(kp + l.bmask_off) : nullptr;
-  void* supports = sup ? kp + l.supports_off : nullptr;
-  void* stream = stream_of(q);
+  const size_t sup = kept.supports;
+  void* const stream = stream_of(q);
   if (c.version == 2) {
-    const int st = sup ? adsp_attn_v2_fwd_keep(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), taus, bmask, data(c.varlen),
-                                               c.varlen_bits(), B, Hq, Hkv, N, D, dt, c.niter, wp, ws_bytes, supports, sup, stream)
-                       : adsp_attn_v2_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), taus, bmask, data(c.varlen),
-                                          c.varlen_bits(), B, Hq, Hkv, N, D, dt, c.niter, wp, ws_bytes, stream);
+    const int st = sup ? adsp_attn_v2_fwd_keep(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kept.taus(), kept.bmask(),
+                                               data(c.varlen), c.varlen_bits(), B, Hq, Hkv, N, D, dt, c.niter, wp, ws_bytes,
+                                               kept.kept_supports(), sup, stream)
+                       : adsp_attn_v2_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kept.taus(), kept.bmask(),
+                                          data(c.varlen), c.varlen_bits(), B, Hq, Hkv, N, D, dt, c.niter, wp, ws_bytes, stream);
     check(st, sup ? "adsp_attn_v2_fwd_keep" : "adsp_attn_v2_fwd");
   } else {
-    const int st = sup ? adsp_attn_v1_fwd_keep(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), taus, bmask, data(c.varlen),
-                                               c.varlen_bits(), B, Hq, N, D, dt, c.alpha, c.causal, c.niter, wp, ws_bytes, supports,
-                                               sup, stream)
-                       : adsp_attn_v1_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), taus, bmask, data(c.varlen),
-                                          c.varlen_bits(), B, Hq, N, D, dt, c.alpha, c.causal, c.niter, wp, ws_bytes, nullptr, stream);
+    const int st = sup ? adsp_attn_v1_fwd_keep(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kept.taus(), kept.bmask(),
+                                               data(c.varlen), c.varlen_bits(), B, Hq, N, D, dt, c.alpha, c.causal, c.niter, wp,
+                                               ws_bytes, kept.kept_supports(), sup, stream)
+                       : adsp_attn_v1_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kept.taus(), kept.bmask(),
+                                          data(c.varlen), c.varlen_bits(), B, Hq, N, D, dt, c.alpha, c.causal, c.niter, wp, ws_bytes,
+                                          w.tile_counts, stream);
     check(st, sup ? "adsp_attn_v1_fwd_keep" : "adsp_attn_v1_fwd");
   }
-  if (saved) *saved = kept;
-  if (supports_bytes) *supports_bytes = sup;
-  if (has_mask) *has_mask = mask;
   return out;
+}
+
+// dq, dk, dv from what the forward left (`bmask` and `supports` may be null)
+variable_list attn_backward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& upstream, const float* taus,
+                            const int32_t* bmask, const void* supports, size_t supports_bytes, const AttnCall& c) {
+  const Tensor dout = upstream.to(q.scalar_type()).contiguous();
+  const int B = (int)q.size(0), Hq = (int)q.size(1), N = (int)q.size(2), D = (int)q.size(3), Hkv = (int)k.size(1);
+  const int dt = dtype_code(q);
+  const c10::DeviceGuard guard(q.device());
+  Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+  const size_t per_row = align256((size_t)B * Hq * N * 4);  // delta and 1 / sum p in front of the workspace
+  const size_t ws_bytes = adsp_attn_bwd_workspace_bytes_causal(B, Hq, Hkv, N, D, dt, c.causal);
+  Tensor scratch = bytes(2 * per_row + ws_bytes, q);
+  char* const sp = (char*)scratch.data_ptr();
+  void* const ws = ws_bytes ? sp + 2 * per_row : nullptr;
+  void* const stream = stream_of(q);
+  const int st = supports_bytes
+                     ? adsp_attn_bwd_kept(q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), taus, bmask, data(c.varlen),
+                                          c.varlen_bits(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), (float*)sp,
+                                          (float*)(sp + per_row), B, Hq, Hkv, N, D, dt, c.alpha, c.causal, ws, ws_bytes, supports,
+                                          supports_bytes, stream)
+                     : adsp_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), taus, bmask, data(c.varlen),
+                                     c.varlen_bits(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), (float*)sp, (float*)(sp + per_row),
+                                     B, Hq, Hkv, N, D, dt, c.alpha, c.causal, ws, ws_bytes, stream);
+  check(st, supports_bytes ? "adsp_attn_bwd_kept" : "adsp_attn_bwd");
+  return {dq, dk, dv};
 }
 
 struct AttnFunction : torch::autograd::Function<AttnFunction> {
   static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const AttnCall& c, int keep_mode) {
-    Tensor saved;
-    size_t sup = 0;
-    bool mask = false;
-    Tensor out = attn_forward(q, k, v, c, true, keep_mode, &saved, &sup, &mask);
-    ctx->save_for_backward({q, k, v, saved});
+    Kept kept;
+    Wants wants;
+    wants.backward = wants.outlives = true;
+    wants.keep_mode = keep_mode;
+    Tensor out = attn_forward(q, k, v, c, wants, kept);
+    ctx->save_for_backward({q, k, v, kept.buffer});
     ctx->saved_data["alpha"] = c.alpha;
     ctx->saved_data["causal"] = c.causal;
-    ctx->saved_data["supports"] = (int64_t)sup;
-    ctx->saved_data["bmask"] = mask;
+    ctx->saved_data["supports"] = (int64_t)kept.supports;
+    ctx->saved_data["bmask"] = kept.mask;
     if (c.varlen.defined()) ctx->saved_data["varlen"] = c.varlen;
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list sv = ctx->get_saved_variables();
-    const Tensor &q = sv[0], &k = sv[1], &v = sv[2], &saved = sv[3];
-    const Tensor dout = grads[0].to(q.scalar_type()).contiguous();
-    const int B = (int)q.size(0), Hq = (int)q.size(1), N = (int)q.size(2), D = (int)q.size(3), Hkv = (int)k.size(1);
-    const int dt = dtype_code(q);
-    const double alpha = ctx->saved_data["alpha"].toDouble();
-    const bool causal = ctx->saved_data["causal"].toBool();
-    AttnCall c{0, alpha, causal, 0, Tensor()};
+    const Tensor &q = sv[0], &k = sv[1], &v = sv[2];
+    AttnCall c{0, ctx->saved_data["alpha"].toDouble(), ctx->saved_data["causal"].toBool(), 0, Tensor()};
     const auto it = ctx->saved_data.find("varlen");
     if (it != ctx->saved_data.end()) c.varlen = it->second.toTensor();
-    const SavedLayout l(q, (size_t)ctx->saved_data["supports"].toInt());
-    const c10::DeviceGuard guard(q.device());
-    Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
-    const size_t per_row = align256((size_t)B * Hq * N * 4);  // delta and 1 / sum p in front of the workspace
-    const size_t ws_bytes = adsp_attn_bwd_workspace_bytes_causal(B, Hq, Hkv, N, D, dt, causal);
-    Tensor scratch = bytes(2 * per_row + ws_bytes, q);
-    char* const sp = (char*)scratch.data_ptr();
-    char* const kp = (char*)saved.data_ptr();
-    void* const ws = ws_bytes ? sp + 2 * per_row : nullptr;
-    int32_t* const bmask = ctx->saved_data["bmask"].toBool() ? (int32_t*)(kp + l.bmask_off) : nullptr;
-    void* const stream = stream_of(q);
-    const int st =
-        l.supports ? adsp_attn_bwd_kept(q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), (float*)kp, bmask,
-                                        data(c.varlen), c.varlen_bits(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), (float*)sp,
-                                        (float*)(sp + per_row), B, Hq, Hkv, N, D, dt, alpha, causal, ws, ws_bytes,
-                                        kp + l.supports_off, l.supports, stream)
-                   : adsp_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), (float*)kp, bmask,
-                                   data(c.varlen), c.varlen_bits(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), (float*)sp,
-                                   (float*)(sp + per_row), B, Hq, Hkv, N, D, dt, alpha, causal, ws, ws_bytes, stream);
-    check(st, l.supports ? "adsp_attn_bwd_kept" : "adsp_attn_bwd");
-    return {dq, dk, dv, Tensor(), Tensor()};
+    Kept kept;
+    kept.mask = ctx->saved_data["bmask"].toBool();
+    kept.supports = (size_t)ctx->saved_data["supports"].toInt();
+    kept.layout(q);
+    kept.buffer = sv[3];
+    variable_list d = attn_backward(q, k, v, grads[0], kept.taus(), kept.bmask(), kept.kept_supports(), kept.supports, c);
+    d.resize(5);  // (no gradients of the call's description and the mode)
+    return d;
   }
 };
 
@@ -371,8 +392,114 @@ PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     refuse_tangent({&q, &k, &v});
     const bool grad = at::GradMode::is_enabled() && (wants_grad(q) || wants_grad(k) || wants_grad(v));
     pybind11::gil_scoped_release no_gil;
-    return grad ? AttnFunction::apply(q, k, v, c, keep_mode) : attn_forward(q, k, v, c, false, KEEP_NEVER, nullptr, nullptr);
+    if (grad) return AttnFunction::apply(q, k, v, c, keep_mode);
+    Kept kept;
+    return attn_forward(q, k, v, c, Wants(), kept);
   });
+}
+
+// The forward and the backward as plain functions, for measurements and tests: what they leave and take is in the caller's hands.
+// Shapes and types of q, k and v are the caller's business beyond what keeps the kernels inside the tensors.
+void check_plain(const Tensor& q, const Tensor& k, const Tensor& v, const AttnCall& c) {
+  require(q.dim() == 4 && k.dim() == 4 && k.sizes() == v.sizes(), "q, k and v must have shape (batch, heads, sequence, head_dim).");
+  require(k.size(0) == q.size(0) && k.size(2) == q.size(2) && k.size(3) == q.size(3) && (c.version == 2 || k.size(1) == q.size(1)),
+          "q and k do not fit each other: ", q.sizes(), " and ", k.sizes());
+  require(q.is_contiguous() && k.is_contiguous() && v.is_contiguous(), "Q, K and/or V are not contiguous.");
+  require(!c.varlen.defined() || ((c.varlen.scalar_type() == at::kInt || c.varlen.scalar_type() == at::kLong) && c.varlen.is_contiguous() &&
+                                  c.varlen.numel() == q.size(0)),
+          "varlen must be int32/int64, one entry per batch item");
+  for (const Tensor* t : {&q, &k, &v, &c.varlen}) require_device(*t);
+}
+
+// attention_forward(q, k, v, version, alpha, is_causal, niter, varlen, keep_mode or None, tile_mask, tile_counts)
+//   -> (out, taus, bmask or None, supports or None); keep_mode None: nothing is kept for a backward
+PyObject* py_attention_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  try {
+    expect_args(n, 11);
+    const Tensor &q = tensor_arg(a[0], "q"), &k = tensor_arg(a[1], "k"), &v = tensor_arg(a[2], "v");
+    AttnCall c{(int)long_arg(a[3]), double_arg(a[4]), bool_arg(a[5]), (int)long_arg(a[6]), Tensor()};
+    if (a[7] != Py_None) c.varlen = tensor_arg(a[7], "varlen");
+    Wants wants;
+    wants.outlives = true;
+    wants.backward = a[8] != Py_None;
+    if (wants.backward) wants.keep_mode = (int)long_arg(a[8]);
+    wants.mask = bool_arg(a[9]);
+    check_plain(q, k, v, c);
+    if (a[10] != Py_None) {
+      const Tensor& counts = tensor_arg(a[10], "tile_counts");
+      require_device(counts);
+      require(c.version == 1 && counts.scalar_type() == at::kLong && counts.numel() == 2 && counts.is_contiguous(),
+              "tile_counts must be two int64, with the block-mask variant");
+      wants.tile_counts = (unsigned long long*)counts.data_ptr();
+    }
+    Kept kept;
+    Tensor out, taus, bmask, supports;
+    {
+      pybind11::gil_scoped_release no_gil;
+      out = attn_forward(q, k, v, c, wants, kept);
+      const auto part = [&](size_t off, int64_t len, at::ScalarType t) { return kept.buffer.narrow(0, (int64_t)off, len).view(t); };
+      taus = part(0, kept.rows * 4, at::kFloat).view({q.size(0), q.size(1), q.size(2)});
+      if (kept.mask) bmask = part(kept.bmask_off, kept.mask_words * 4, at::kInt).view({q.size(0), q.size(1), -1});
+      if (kept.supports) supports = part(kept.supports_off, (int64_t)kept.supports, at::kByte);
+    }
+    PyObject* tuple = PyTuple_New(4);
+    if (!tuple) throw python_error();
+    Tensor* const parts[4] = {&out, &taus, &bmask, &supports};
+    for (int i = 0; i < 4; ++i) PyTuple_SET_ITEM(tuple, i, THPVariable_Wrap(*parts[i]));  // (an undefined tensor becomes None)
+    return tuple;
+  } catch (const ArgumentAssertion& e) {
+    PyErr_SetString(PyExc_AssertionError, e.what.c_str());
+    return nullptr;
+  }
+  END_HANDLE_TH_ERRORS
+}
+
+// attention_backward(q, k, v, dout, taus, bmask or None, alpha, is_causal, varlen, supports or None) -> (dq, dk, dv)
+PyObject* py_attention_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  try {
+    expect_args(n, 10);
+    const Tensor &q = tensor_arg(a[0], "q"), &k = tensor_arg(a[1], "k"), &v = tensor_arg(a[2], "v"), &dout = tensor_arg(a[3], "dout"),
+                 &taus = tensor_arg(a[4], "taus");
+    AttnCall c{2, double_arg(a[6]), bool_arg(a[7]), 0, Tensor()};
+    if (a[8] != Py_None) c.varlen = tensor_arg(a[8], "varlen");
+    Tensor bmask, supports;
+    if (a[5] != Py_None) bmask = tensor_arg(a[5], "bmask");
+    if (a[9] != Py_None) supports = tensor_arg(a[9], "supports");
+    check_plain(q, k, v, c);
+    for (const Tensor* t : std::initializer_list<const Tensor*>{&dout, &taus, &bmask, &supports}) require_device(*t);
+    require(k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type(), "q, k and v must share a dtype");
+    require(dout.sizes() == q.sizes(), "dout must have q's shape");
+    const int64_t heads = q.size(0) * q.size(1);
+    require(taus.scalar_type() == at::kFloat && taus.is_contiguous() && taus.numel() == heads * q.size(2), "taus must be what the forward returned");
+    require(!bmask.defined() || (bmask.scalar_type() == at::kInt && bmask.is_contiguous() &&
+                                 bmask.numel() == heads * (int64_t)adsp_attn_bmask_words((int)q.size(2))),
+            "bmask must be what the forward returned");
+    require(!supports.defined() || (supports.scalar_type() == at::kByte && supports.is_contiguous()), "supports must be what the forward returned");
+    variable_list d;
+    {
+      pybind11::gil_scoped_release no_gil;
+      d = attn_backward(q, k, v, dout, (const float*)taus.data_ptr(), (const int32_t*)data(bmask), data(supports),
+                        supports.defined() ? (size_t)supports.numel() : 0, c);
+    }
+    PyObject* tuple = PyTuple_New(3);
+    if (!tuple) throw python_error();
+    for (int i = 0; i < 3; ++i) PyTuple_SET_ITEM(tuple, i, THPVariable_Wrap(d[i]));
+    return tuple;
+  } catch (const ArgumentAssertion& e) {
+    PyErr_SetString(PyExc_AssertionError, e.what.c_str());
+    return nullptr;
+  }
+  END_HANDLE_TH_ERRORS
+}
+
+// keeps_supports(mode, supports_bytes, q_bytes): whether a forward keeps supports of that size for its backward
+PyObject* py_keeps_supports(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  expect_args(n, 3);
+  return PyBool_FromLong(keeps_supports((int)long_arg(a[0]), (size_t)long_arg(a[1]), (size_t)long_arg(a[2])));
+  END_HANDLE_TH_ERRORS
 }
 
 // decode_attention(q, k, v, alpha, varlen, is_causal, left_padding, slopes) -> tensor, or None where the kernels do not take the call
@@ -401,6 +528,9 @@ PyObject* py_decode_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     {"entmax_rows", (PyCFunction)(void (*)(void))py_entmax_rows, METH_FASTCALL, "alpha-entmax of the last dimension, with autograd"},
     {"attention", (PyCFunction)(void (*)(void))py_attention, METH_FASTCALL, "sparse entmax attention, with autograd"},
+    {"attention_forward", (PyCFunction)(void (*)(void))py_attention_forward, METH_FASTCALL, "the attention forward, with what it leaves behind"},
+    {"attention_backward", (PyCFunction)(void (*)(void))py_attention_backward, METH_FASTCALL, "the attention backward from what the forward left"},
+    {"keeps_supports", (PyCFunction)(void (*)(void))py_keeps_supports, METH_FASTCALL, "whether supports of a size are kept"},
     {"decode_attention", (PyCFunction)(void (*)(void))py_decode_attention, METH_FASTCALL, "a few queries against a cache of keys"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_adsp_torch", nullptr, -1, methods};
