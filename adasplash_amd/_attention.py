@@ -44,16 +44,20 @@ def _keeps(sup_bytes, q):
     return _lib.native().keeps_supports(keep_code(), sup_bytes, q.numel() * q.element_size())
 
 
-def launch_forward(q, k, v, *, version, alpha, is_causal, niter, varlen, tile_counts=None, keep_supports=False):
+def launch_forward(q, k, v, *, version, alpha, is_causal, niter, varlen, tile_counts=None, keep_supports=False, tile_mask=True):
     """Enqueue the fused forward on the current stream.  Returns ``(out, taus, bmask)``, and with ``keep_supports`` a
     fourth value: the buffer in which the forward keeps the supports it found for ``launch_backward`` (``None`` where the
     library keeps none: fp32, head dims other than 64 / 128, a caller that asks for the tile statistics, or a buffer
     beyond what ``set_keep_supports`` allows; ``keep_supports="always"`` asks for the buffer whatever the mode).
+
+    The tile mask and the supports are left by the kernels that find them; a short 16-bit call of the entry points goes
+    to others.  ``tile_mask=False`` launches what the entry points launch: without ``keep_supports`` what a call
+    without a gradient does (``bmask`` is ``None``), with it what a training step does (``bmask`` where the backward reads one).
     """
     mode = None
     if keep_supports:
         mode = 1 if keep_supports == "always" else keep_code()
-    out, taus, bmask, sup = _lib.native().attention_forward(q, k, v, version, alpha, is_causal, niter, varlen, mode, True, tile_counts)
+    out, taus, bmask, sup = _lib.native().attention_forward(q, k, v, version, alpha, is_causal, niter, varlen, mode, tile_mask, tile_counts)
     return (out, taus, bmask, sup) if keep_supports else (out, taus, bmask)
 
 

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import adasplash_amd as A
+from adasplash_amd import _attention
 from oracle import exact
 from tests.gpu_util import DEV, max_err
 
@@ -147,3 +148,27 @@ def test_f16_dq_for_gradients_at_the_ends_of_the_types_range(dout_scale, alpha, 
     got = run(q, k, v, dout, varlen, alpha, causal, Hq != Hkv)[1].double().cpu()
     assert torch.isfinite(got).all()
     assert (got - want).norm() < 2.0 ** -10 * want.norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,N,short", [(1, 8, 2, 512, True), (2, 16, 16, 2048, False)])
+def test_the_plain_functions_launch_what_the_entry_points_launch(B, Hq, Hkv, N, short, dtype):
+    """``launch_forward(tile_mask=False)``, alone and with ``keep_supports``, and ``launch_backward`` behind it: the bits of a call
+    without a gradient and of a training step.  A short 16-bit call leaves neither tile mask nor supports there, and
+    both by default."""
+    g = torch.Generator().manual_seed(9)
+    q = torch.randn(B, Hq, N, 64, generator=g).to(dtype).to(DEV)
+    k, v = (torch.randn(B, Hkv, N, 64, generator=g).to(dtype).to(DEV) for _ in range(2))
+    dout = torch.randn(B, Hq, N, 64, generator=g).to(dtype).to(DEV)
+    kw = dict(version=2, alpha=1.5, is_causal=True, niter=1, varlen=None)
+    out, taus, bmask = _attention.launch_forward(q, k, v, tile_mask=False, **kw)
+    assert bmask is None and torch.equal(out, A.adasplash_v2(q, k, v))
+    out, taus, bmask, sup = _attention.launch_forward(q, k, v, tile_mask=False, keep_supports=True, **kw)
+    reads = dtype == torch.bfloat16 and not short
+    assert (bmask is not None) == reads and (sup is not None) == reads
+    got = _attention.launch_backward(q, k, v, dout, taus, bmask, alpha=1.5, is_causal=True, varlen=None, supports=sup)
+    want_out, *want = run(q, k, v, dout, None, 1.5, True, True)
+    assert torch.equal(out, want_out) and all(torch.equal(a, b) for a, b in zip(got, want))
+    out, taus, bmask, sup = _attention.launch_forward(q, k, v, keep_supports=True, **kw)
+    assert bmask is not None and (sup is not None) == (dtype == torch.bfloat16)
+    assert max_err(out, want_out.float().cpu()) < 2e-2
