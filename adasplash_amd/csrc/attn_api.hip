@@ -368,27 +368,50 @@ static bool f32_split(int N, int D, int dtype, double alpha) {
 // N = 256: 76 -> 18 and 38 -> 31 (1 and 1/8); 2 of 512: 99 -> 24, 52 -> 32; 32/8 heads, N = 1024: 131 -> 53, 80 -> 74; 16/4
 // heads, N = 2048: 132 -> 93, 89 -> 54, 135 -> 124; 4 x 16 heads, N = 512, not causal: 67 -> 46, 47 -> 34, 95 -> 54; 32 x 16
 // heads, N = 128: 59 -> 42, 44 -> 36, 70 -> 66; beyond it 32/8 heads, N = 2048: 147 -> 132, 96 -> 100, 139 -> 236.
+// Long sequences of few heads pass that line too, and the longest workgroup's walk is then all of the time; hence the limit on N.
+// One head, D = 64 and 128 (GPU times): causal N = 4096: 147 -> 56, 103 -> 44, 171 -> 97 and 171 -> 63, 127 -> 50, 246 -> 142; N = 8192:
+// 226 -> 226, 164 -> 69, 323 -> 187 and 275 -> 268, 211 -> 81, 475 -> 290; beyond it 9472: 260 -> 253, 187 -> 79, 371 -> 243 and
+// 305 -> 333, 236 -> 94, 545 -> 322; full N = 4096: 155 -> 127, 102 -> 45, 597 -> 102 and 177 -> 167, 128 -> 51, 766 -> 144; beyond it 6144
+// with D = 128: 238 -> 252, 170 -> 68, 1137 -> 236.  (For alpha < 1.5, where supports are longer, a list now and then overflows with
+// spread 3 as well: 2 heads, N = 3015, D = 128, alpha = 1.333: 1512 -> 164, 135 -> 167, 1205 -> 113.)
 static double rows32_cost_ns(int B, int Hq, int N, bool causal) {
   const double heads = (double)B * Hq, r = (N + 31) / 32;
   return heads * (20.0 * r + 1.35 * (causal ? 0.5 * r * (r + 1.0) : r * r));
 }
 static bool rows32_16bit(int B, int Hq, int N, int D, int dtype, double alpha, bool causal) {
-  if (dtype == ADSP_F32 || (D != 64 && D != 128) || N > 65536 || !(alpha >= 1.125 && alpha <= 2.0) || !sparse_enabled()) return false;
+  if (dtype == ADSP_F32 || (D != 64 && D != 128) || !(alpha >= 1.125 && alpha <= 2.0) || !sparse_enabled()) return false;
+  if (N > (causal ? 8192 : 4096)) return false;
   const long long groups = (long long)B * Hq * ((N + 31) / 32);
   const long long most = N <= 128 ? 2048 : ((N >= 1024 || !causal) ? 1024 : 512);
   return groups <= most && rows32_cost_ns(B, Hq, N, causal) <= 66e3;
 }
 // Of those, the calls whose backward goes the same way (and whose forward then keeps nothing for it): a dK/dV workgroup walks
-// the query blocks of all heads of its group, which only few-headed problems can afford at length.  Forward and backward, us,
-// q of spread 1, 3 and 1/8: 8 heads, 4 sequences of N = 256, D = 64: 136 -> 35, 93 -> 36, 74 -> 48; 2 x 16 heads, N = 512: 158 -> 50,
-// 103 -> 46, 103 -> 55; 8 heads, N = 2048: 238 -> 131, 134 -> 100, 273 -> 122; 16/4 heads, N = 1024: 202 -> 113, 118 -> 107,
-// 285 -> 118; 32 x 16 heads, N = 128: 144 -> 95, 109 -> 90, 136 -> 120; beyond the line 2 x 16/4 heads, N = 1024: 216 -> 143,
-// 121 -> 133, 288 -> 151; 32/8 heads, D = 128: 325 -> 201, 162 -> 190.
+// the query blocks of all heads of its group, which only few-headed problems can afford at length.  Without a causal mask
+// every walk is a long one, and with D = 128 a workgroup of that kernel fills a CU, so that a second round of them is one too many
+// from walks of some 24 blocks on.  The lines lie where a call with peaked scores, which gains least, begins to be slower by more
+// than some 5 %.  Forward and backward, GPU times in us, q of spread 1, 3 and 1/8:
+//   D = 64, causal: 8 heads, 4 sequences of N = 256: 136 -> 35, 93 -> 36, 74 -> 48; 16/4 heads, N = 1024: 202 -> 113, 118 -> 107,
+//     285 -> 118; 32 x 16 heads, N = 128: 144 -> 95, 109 -> 90, 136 -> 120; at the line 12 heads, N = 2048: 242 -> 157, 135 -> 125,
+//     270 -> 156; 6/3 heads, N = 2036: 233 -> 165, 133 -> 137, 356 -> 166; one head, N = 4096: 283 -> 236, 162 -> 160, 492 -> 220;
+//     beyond it 2 x 16/4 heads, N = 1024: 216 -> 143, 121 -> 133, 288 -> 151;
+//   D = 64, full: one head, N = 3072: 214 -> 195, 135 -> 132, 702 -> 174; beyond it N = 4032: 249 -> 251, 151 -> 163, 954 -> 236;
+//     7 heads, N = 2048: 202 -> 166, 118 -> 120, 484 -> 154; 2 x 16 of 807, alpha = 1.333: 439 -> 233, 145 -> 163, 434 -> 208;
+//   D = 128, causal: 4/1 heads, N = 1024: 300 -> 158, 144 -> 151, 470 -> 170; one head, N = 3072: 344 -> 199, 188 -> 184, 621 -> 243; 16
+//     heads, N = 1502: 316 -> 183, 168 -> 172, 352 -> 209; beyond it 12 heads, N = 2048: 322 -> 220, 180 -> 206, 448 -> 246; one head,
+//     N = 4096: 389 -> 256, 216 -> 238, 820 -> 321;
+//   D = 128, full: 3 heads, N = 2048: 247 -> 198, 153 -> 139, 700 -> 173; 4 x 3 heads, N = 725: 227 -> 109, 121 -> 104, 309 -> 122; beyond
+//     it 8 heads, N = 1153, alpha = 2: 130 -> 143, 118 -> 138, 547 -> 153; 2 x 16 heads, N = 554: 219 -> 156, 128 -> 146, 254 -> 168; 16
+//     heads, N = 1082: 244 -> 230, 136 -> 216, 421 -> 260; one head, N = 3072: 272 -> 204, 170 -> 187, 1017 -> 258.
 static bool rows32_16bit_training(int B, int Hq, int Hkv, int N, int D, int dtype, double alpha, bool causal) {
   if (!rows32_16bit(B, Hq, N, D, dtype, alpha, causal)) return false;
   const double cost = rows32_cost_ns(B, Hq, N, causal);
-  const long long walk = (long long)(Hq / Hkv) * ((N + 31) / 32);
-  return walk <= 64 ? cost <= 50e3 : (walk <= 128 && cost <= 25e3);
+  const long long blocks = (N + 31) / 32, walk = (long long)(Hq / Hkv) * blocks;
+  if (!(walk <= 64 ? cost <= 50e3 : (walk <= 128 && cost <= 25e3))) return false;
+  const long long pairs = (long long)B * Hq * blocks * blocks / (causal ? 2 : 1);
+  if (D == 64) return causal || (walk <= 96 && pairs <= 16384);
+  if (causal) return N <= 3072 && pairs <= 18432;
+  const long long rounds = ((long long)B * Hkv * blocks + 255) / 256;  // (one workgroup per CU)
+  return rounds * walk <= (rounds == 1 ? 64 : 48);
 }
 
 static int attn_common(const void* q, const void* k, const void* v, void* out, float* taus, int32_t* bmask,

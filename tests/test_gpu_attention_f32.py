@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import adasplash_amd as A
-from adasplash_amd import _attention
+from adasplash_amd import _attention, _lib
 from oracle import exact
 from tests.gpu_util import DEV, max_err
 
@@ -172,3 +172,67 @@ def test_the_plain_functions_launch_what_the_entry_points_launch(B, Hq, Hkv, N, 
     out, taus, bmask, sup = _attention.launch_forward(q, k, v, keep_supports=True, **kw)
     assert bmask is not None and (sup is not None) == (dtype == torch.bfloat16)
     assert max_err(out, want_out.float().cpu()) < 2e-2
+
+
+def _untouched(nbytes):
+    return torch.full((max(nbytes, 16),), 0xA5, device=DEV, dtype=torch.uint8)
+
+
+def _short_16bit_forward(q, k, v, alpha, causal):
+    """The forward without tile mask through the C ABI, and proof that it took the kernel on 32 rows: only the others write
+    to the workspace."""
+    lib = _lib.load()
+    B, Hq, N, D = q.shape
+    Hkv, dt = k.shape[1], _lib.dtype_code(q)
+    ws = _untouched(lib.adsp_attn_workspace_bytes(B, Hq, Hkv, N, D, dt))
+    out, taus = torch.full_like(q, float("nan")), torch.empty(B, Hq, N, device=DEV)
+    head = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), taus.data_ptr(), None, None, 0)
+    stream = _lib.current_stream(q.device)
+    if causal:
+        st = lib.adsp_attn_v2_fwd(*head, B, Hq, Hkv, N, D, dt, 1, ws.data_ptr(), ws.numel(), stream)
+    else:
+        st = lib.adsp_attn_v1_fwd(*head, B, Hq, N, D, dt, alpha, 0, 10, ws.data_ptr(), ws.numel(), None, stream)
+    assert st == 0 and (ws == 0xA5).all()
+    return out, taus
+
+
+@pytest.mark.parametrize("scale", [0.125, 1.0, 3.0])
+@pytest.mark.parametrize("N,Hq,Hkv,D,alpha,causal,dtype", [
+    (8192, 1, 1, 64, 1.5, True, torch.bfloat16), (8192, 1, 1, 128, 1.5, True, torch.float16), (4095, 4, 1, 64, 1.5, True, torch.float16),
+    (1024, 16, 4, 128, 1.5, True, torch.bfloat16), (4096, 1, 1, 128, 1.5, False, torch.bfloat16), (4096, 1, 1, 64, 1.333, False, torch.float16),
+    (2048, 4, 4, 64, 2.0, False, torch.bfloat16)])
+def test_16bit_inference_on_long_sequences(N, Hq, Hkv, D, alpha, causal, dtype, scale):
+    """Walks of up to 64 steps a wave, to the longest sequences that take this route: rows around steps and blocks and at both
+    ends, thresholds and outputs.  Thresholds: fp32 sums over 16-bit products, and steps until one is below 2e-5."""
+    g = torch.Generator().manual_seed(10)
+    q = (scale * torch.randn(1, Hq, N, D, generator=g)).to(dtype).to(DEV)
+    k, v = (torch.randn(1, Hkv, N, D, generator=g).to(dtype).to(DEV) for _ in range(2))
+    out, taus = _short_16bit_forward(q, k, v, alpha, causal)
+    rows = sorted({r for r in (0, 1, 31, 32, 127, 128, 1023, 1024, N // 2 + 5, N - 33, N - 32, N - 2, N - 1) if r < N})
+    for h in {0, Hq - 1}:
+        kk = k[0, h // (Hq // Hkv)].double().cpu()
+        s = q[0, h, rows].double().cpu() @ kk.t() / D ** 0.5
+        if causal:
+            s = s.masked_fill(torch.arange(N)[None, :] > torch.tensor(rows)[:, None], float("-inf"))
+        p, tau = exact.entmax_rows(s, alpha, return_tau=True)
+        assert max_err(out[0, h, rows], p @ v[0, h // (Hq // Hkv)].double().cpu()) < 2e-2
+        assert (taus[0, h, rows].double().cpu() - tau.double().view(-1)).abs().max().item() < 5e-5 * max(1.0, scale)
+
+
+@pytest.mark.parametrize("scale", [0.125, 1.0, 3.0])
+@pytest.mark.parametrize("N,Hq,Hkv,D,alpha,causal,dtype", [
+    (4096, 1, 1, 64, 1.5, True, torch.bfloat16), (1024, 4, 1, 64, 1.5, True, torch.float16), (3072, 1, 1, 128, 1.5, True, torch.bfloat16),
+    (3072, 1, 1, 64, 1.5, False, torch.bfloat16), (2048, 3, 3, 128, 1.5, False, torch.float16), (2048, 1, 1, 64, 1.333, False, torch.bfloat16)])
+def test_16bit_gradients_on_long_sequences(N, Hq, Hkv, D, alpha, causal, dtype, scale):
+    """Training steps at the ends of the route's range, whole tensors; bounds as in the other 16-bit tests."""
+    g = torch.Generator().manual_seed(11)
+    q = (scale * torch.randn(1, Hq, N, D, generator=g)).to(dtype)
+    k, v = (torch.randn(1, Hkv, N, D, generator=g).to(dtype) for _ in range(2))
+    dout = torch.randn(1, Hq, N, D, generator=g).to(dtype)
+    assert _lib.load().adsp_attn_bwd_reads_bmask(1, Hq, Hkv, N, D, _lib.dtype_code(q), alpha, int(causal)) == 0
+    varlen = torch.tensor([N], dtype=torch.int32)  # (N need not be a power of two)
+    got = run(q, k, v, dout, varlen, alpha, causal, causal)
+    want = [exact.dense_entmax_attention(q, k, v, alpha, causal, varlen)]
+    want += list(exact.dense_entmax_attention_grads(q, k, v, dout, alpha, causal, varlen))
+    for name, a, w in zip(("out", "dq", "dk", "dv"), got, want):
+        assert max_err(a, w) < (2e-2 if name == "out" else 4e-2 * max(1.0, scale)), name

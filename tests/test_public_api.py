@@ -209,6 +209,25 @@ def test_backward_workspace_for_a_causal_call_follows_the_merge_border(monkeypat
             assert lib.adsp_attn_bwd_workspace_bytes_causal(B, Hq, Hq, N, D, _lib.ADSP_BF16, 1) == lib.adsp_attn_bwd_workspace_bytes(B, Hq, Hq, N, D, _lib.ADSP_BF16)
 
 
+def test_which_training_steps_need_no_tile_mask():
+    """Both sides of every line of the rule that sends short 16-bit training steps to the kernels on 32 rows."""
+    lib = _lib.load()
+    reads = lambda B, Hq, Hkv, N, D, causal, alpha=1.5, dt=_lib.ADSP_BF16: lib.adsp_attn_bwd_reads_bmask(B, Hq, Hkv, N, D, dt, alpha, causal)  # noqa: E731
+    # block pairs and the dK/dV kernel's walk: D = 64 causal, then full
+    assert reads(1, 12, 12, 2048, 64, 1) == 0 and reads(1, 13, 13, 2048, 64, 1) == 1
+    assert reads(1, 4, 1, 1024, 64, 1) == 0 and reads(1, 8, 1, 1024, 64, 1) == 1 and reads(1, 1, 1, 4096, 64, 1) == 0 and reads(1, 1, 1, 4128, 64, 1) == 1
+    assert reads(1, 1, 1, 3072, 64, 0) == 0 and reads(1, 1, 1, 3073, 64, 0) == 1
+    assert reads(1, 4, 4, 2048, 64, 0) == 0 and reads(1, 5, 5, 2048, 64, 0) == 1
+    # D = 128 causal, then full (up to 256 workgroups, and several rounds of them)
+    assert reads(1, 1, 1, 3072, 128, 1) == 0 and reads(1, 1, 1, 3073, 128, 1) == 1
+    assert reads(1, 9, 9, 2048, 128, 1) == 0 and reads(1, 10, 10, 2048, 128, 1) == 1
+    assert reads(1, 4, 4, 2048, 128, 0) == 0 and reads(1, 1, 1, 2049, 128, 0) == 1
+    assert reads(4, 3, 3, 725, 128, 0) == 0 and reads(1, 8, 8, 1153, 128, 0) == 1 and reads(2, 16, 16, 554, 128, 0) == 1
+    # types, head dims and powers the kernels do not serve; single precision goes there always
+    assert reads(1, 8, 8, 512, 32, 1) == 1 and reads(1, 8, 8, 512, 64, 1, 1.1) == 1
+    assert reads(8, 32, 8, 8192, 128, 1, 1.5, _lib.ADSP_F32) == 0
+
+
 def test_argument_errors_come_back_as_status_codes():
     lib = _lib.load()
     # no pointer is dereferenced and nothing is launched for these
