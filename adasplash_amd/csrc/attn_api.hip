@@ -321,7 +321,7 @@ static void launch_probe(const AttnParams& p, int D, int dtype, int am, uint32_t
   }
 }
 
-// ADSP_SPARSE=0 in the environment keeps every row block on the dense kernel (for comparisons and tests).
+// ADSP_SPARSE=0 in the environment keeps every row block of a 16-bit call on the dense kernels (for comparisons and tests).
 static bool sparse_enabled() {
   const char* e = getenv("ADSP_SPARSE");
   return !(e && strcmp(e, "0") == 0);
@@ -487,7 +487,8 @@ static int attn_common(const void* q, const void* k, const void* v, void* out, f
     return hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
   }
   if (!tile_counts && !bmask && !supports && rows32_16bit(B, Hq, N, D, dtype, alpha, is_causal != 0)) {
-    if (w.total && (!workspace || workspace_bytes < w.total || ((uintptr_t)workspace & 15) != 0)) return ADSP_ERR_WORKSPACE;  // (as below)
+    // (not touched, but asked for as below: the size query does not know the call)
+    if (w.total && (!workspace || workspace_bytes < w.total || ((uintptr_t)workspace & 15) != 0)) return ADSP_ERR_WORKSPACE;
     const int rc = dtype == ADSP_BF16 ? (D == 64 ? launch_attn_rows32_fwd_bf16_d64(p, am, s) : launch_attn_rows32_fwd_bf16_d128(p, am, s))
                                       : (D == 64 ? launch_attn_rows32_fwd_f16_d64(p, am, s) : launch_attn_rows32_fwd_f16_d128(p, am, s));
     return rc == 0 && hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;

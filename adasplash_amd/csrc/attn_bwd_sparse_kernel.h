@@ -18,7 +18,7 @@
 // held each entry's place in the lists since the sort.
 //
 // Row blocks whose supports outgrow the stream or the lists are flagged and left to attn_bwd_dq_kernel, launched
-// behind, exactly as in the forward; the kernel is persistent and draws row blocks from the same per-XCD counters.
+// behind, exactly as in the forward; the kernel is persistent and takes row blocks as the forward does (draw_item).
 #pragma once
 #include "attn_bwd_kernel.h"
 #include "attn_sparse_kernel.h"

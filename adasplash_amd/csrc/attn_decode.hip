@@ -10,7 +10,7 @@
 //    of the support are read.  The list's order, and with it that of every sum over it, is the order of the threads (a prefix sum
 //    over their counts), so a call returns the same bits every time.
 // A step of 16 x 16 heads against caches of up to 4096 keys (D = 64, bf16, 84 MB of K in use): 265 us as fp32 copies of q and
-// K, a library product, ten elementwise launches, the rows kernel and a second product; 27 us now (20 us = 4.2 TB/s and 6.7 us).
+// K, a library product, ten elementwise launches, the rows kernel and a second product; 27 us now (20 us = 4.2 TB/s and 6.9 us).
 #include "entmax_rows_kernel.h"
 #include "../../include/adasplash_hip.h"
 #include <math.h>

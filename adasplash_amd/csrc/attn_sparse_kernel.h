@@ -28,7 +28,7 @@
 //
 // The kernel is persistent: a fixed number of workgroups (one event slot each) draw row blocks from per-XCD
 // counters in the same XCD-aware order as the dense kernel, longest causal row blocks first, and help the other
-// XCDs when their own counter runs out.
+// XCDs when their own counter runs out (a launch of up to two row blocks per workgroup does without: draw_item).
 #pragma once
 #include <type_traits>
 

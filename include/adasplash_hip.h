@@ -13,7 +13,8 @@
  *   - per device, the address of the 64 MiB scratch array behind adsp_attn_v2_fwd_noalloc, looked up on
  *     that entry point's first call on the device (calls through it share the array: see there);
  *   - the environment, read on every call (comparisons, tests and profiling; unset in normal use):
- *       ADSP_SPARSE=0               every row block on the dense kernels (no sparse-support kernels)
+ *       ADSP_SPARSE=0               every row block of a 16-bit call on the dense kernels (no sparse-support kernels,
+ *                                   none of those for short calls); fp32 calls do not look at it
  *       ADSP_BWD_STREAMS=0          the sparse-support dK/dV kernel walks the scores itself instead of taking
  *                                   the dQ kernel's candidate streams
  *       ADSP_PROBE_MAX_SUPPORT=n    the support the probe lets a K/V head's longest rows have before it
@@ -101,7 +102,8 @@ int adsp_entmax_rows_bwd(const void* y, const void* dy, void* dx, int64_t rows, 
  * the work counters, row-block flags and candidate streams of the sparse-support kernel (up to 1024 slots of 51 KiB;
  * sequences of up to 65536 keys) and a one-byte (fp8 e4m3) copy of K.  The buffer must be 16-byte aligned device
  * memory; its contents need not survive between calls, and two calls that run at the same time need a buffer each.
- * For the block-mask variant pass Hq = Hkv = H.
+ * For the block-mask variant pass Hq = Hkv = H.  The size serves any call with these dimensions and is asked for in every
+ * one: a short 16-bit call without bmask and supports, whose kernel does not touch the buffer, is refused without it too.
  */
 size_t adsp_attn_workspace_bytes(int B, int Hq, int Hkv, int N, int D, int dtype);
 
