@@ -4,6 +4,8 @@
 //
 // What bounds them: the fp32 matrix pipe (v_mfma_f32_32x32x2_f32, 64 cycles) on large problems, and on
 // ordinary ones the length of a workgroup's walk over the keys, because a K/V head of N keys has only N / rows workgroups.
+// The 16-bit forward: vector issue (its products are a sixteenth as long; about 1400 vector instructions per block of 32 x 32 scores,
+// most of them insertions into the lists; matrix pipe 1-2 %, vector pipe about 50 % of the busy SIMD cycles).
 //
 // Split: a workgroup is four waves and owns 32 rows (queries; keys in the dK/dV kernel); the waves share the rows and
 // take the 32-row blocks of the other side in turn, and meet in LDS at the end of a walk.  Against 128 rows per workgroup,
