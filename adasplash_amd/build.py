@@ -63,9 +63,11 @@ def units(extra=None):
             base = [f"-DADSP_T={ty}", f"-DADSP_TAG={tag}", f"-DADSP_D={d}"]
             for multi in (0, 1):
                 out.append((f"attn_fwd_{tag}_d{d}_m{multi}", "attn_fwd_unit.hip", base + [f"-DADSP_MULTI={multi}"] + attn_flags))
-            out.append((f"attn_bwd_{tag}_d{d}", "attn_bwd_unit.hip", base))
+            if tag == "f32" or d not in (64, 128):
+                out.append((f"attn_bwd_{tag}_d{d}", "attn_bwd_unit.hip", base))
             if tag != "f32" and d in (64, 128):
                 out.append((f"attn_rows32_{tag}_d{d}", "attn_rows32_unit.hip", base))
+                out.append((f"attn_bwd16_{tag}_d{d}", "attn_bwd16_unit.hip", base + attn_flags))
                 out.append((f"attn_sparse_{tag}_d{d}", "attn_sparse_unit.hip", base + attn_flags))
                 out.append((f"attn_bwd_sparse_{tag}_d{d}", "attn_bwd_sparse_unit.hip", base + attn_flags))
     for d in (64, 128):

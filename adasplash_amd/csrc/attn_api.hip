@@ -13,7 +13,7 @@ namespace adsp {
 #define ADSP_DECL_D(tag, d)                                                      \
   int launch_attn_fwd_##tag##_d##d##_m0(const AttnParams&, int, hipStream_t);   \
   int launch_attn_fwd_##tag##_d##d##_m1(const AttnParams&, int, hipStream_t);   \
-  int launch_attn_bwd_##tag##_d##d(const AttnBwdParams&, int, int, hipStream_t);
+  int launch_attn_bwd_##tag##_d##d(const AttnBwdParams&, int, int, hipStream_t);  // (16-bit: head dims 16, 32 and 256)
 #define ADSP_DECL_TAG(tag) ADSP_DECL_D(tag, 16) ADSP_DECL_D(tag, 32) ADSP_DECL_D(tag, 64) ADSP_DECL_D(tag, 128) ADSP_DECL_D(tag, 256)
 ADSP_DECL_TAG(f32)
 ADSP_DECL_TAG(bf16)
@@ -35,24 +35,36 @@ int launch_attn_f32_fwd_d128(const AttnParams&, int, hipStream_t);
 int launch_attn_f32_bwd_d64(const AttnBwdParams&, int, hipStream_t);
 int launch_attn_f32_bwd_d128(const AttnBwdParams&, int, hipStream_t);
 
-// the same for the 16-bit types (attn_rows32_unit.hip)
-#define ADSP_DECL_ROWS32(tag, d)                                            \
-  int launch_attn_rows32_fwd_##tag##_d##d(const AttnParams&, int, hipStream_t); \
-  int launch_attn_rows32_bwd_##tag##_d##d(const AttnBwdParams&, int, hipStream_t);
-ADSP_DECL_ROWS32(bf16, 64)
-ADSP_DECL_ROWS32(bf16, 128)
-ADSP_DECL_ROWS32(f16, 64)
-ADSP_DECL_ROWS32(f16, 128)
+// 16-bit types, head dims 64 and 128: the forward on 32 rows a workgroup (attn_rows32_unit.hip), and dQ and dK/dV on all pairs
+// (attn_bwd16_unit.hip)
+#define ADSP_DECL_16(tag, d)                                                        \
+  int launch_attn_rows32_fwd_##tag##_d##d(const AttnParams&, int, hipStream_t);     \
+  int launch_attn_bwd16_##tag##_d##d(const AttnBwdParams&, int, int, bool, hipStream_t);
+ADSP_DECL_16(bf16, 64)
+ADSP_DECL_16(bf16, 128)
+ADSP_DECL_16(f16, 64)
+ADSP_DECL_16(f16, 128)
+#define ADSP_CALL_16(name, D, dtype, ...)                                                                \
+  ((dtype) == ADSP_BF16 ? ((D) == 64 ? name##_bf16_d64(__VA_ARGS__) : name##_bf16_d128(__VA_ARGS__))    \
+                        : ((D) == 64 ? name##_f16_d64(__VA_ARGS__) : name##_f16_d128(__VA_ARGS__)))
 
 typedef int (*attn_fwd_fn)(const AttnParams&, int, hipStream_t);
 typedef int (*attn_bwd_fn)(const AttnBwdParams&, int, int, hipStream_t);
 #define ADSP_FWD_ROW(tag, d) {launch_attn_fwd_##tag##_d##d##_m0, launch_attn_fwd_##tag##_d##d##_m1}
 #define ADSP_FWD_TAG(tag) {ADSP_FWD_ROW(tag, 16), ADSP_FWD_ROW(tag, 32), ADSP_FWD_ROW(tag, 64), ADSP_FWD_ROW(tag, 128), ADSP_FWD_ROW(tag, 256)}
-#define ADSP_BWD_TAG(tag) {launch_attn_bwd_##tag##_d16, launch_attn_bwd_##tag##_d32, launch_attn_bwd_##tag##_d64, launch_attn_bwd_##tag##_d128, launch_attn_bwd_##tag##_d256}
+// (the 16-bit backward at head dims 64 and 128 has kernels of its own, attn_bwd16_unit.hip)
+#define ADSP_BWD_TAG16(tag) {launch_attn_bwd_##tag##_d16, launch_attn_bwd_##tag##_d32, nullptr, nullptr, launch_attn_bwd_##tag##_d256}
 // indexed by adsp_dtype (ADSP_F32 = 0, ADSP_BF16 = 1, ADSP_F16 = 2), head dim slot, instance
 static const attn_fwd_fn kFwdTable[3][5][2] = {ADSP_FWD_TAG(f32), ADSP_FWD_TAG(bf16), ADSP_FWD_TAG(f16)};
-static const attn_bwd_fn kBwdTable[3][5] = {ADSP_BWD_TAG(f32), ADSP_BWD_TAG(bf16), ADSP_BWD_TAG(f16)};
+static const attn_bwd_fn kBwdTable[3][5] = {
+    {launch_attn_bwd_f32_d16, launch_attn_bwd_f32_d32, launch_attn_bwd_f32_d64, launch_attn_bwd_f32_d128, launch_attn_bwd_f32_d256},
+    ADSP_BWD_TAG16(bf16), ADSP_BWD_TAG16(f16)};
 static int head_dim_slot(int D) { return D == 16 ? 0 : (D == 32 ? 1 : (D == 64 ? 2 : (D == 128 ? 3 : (D == 256 ? 4 : -1)))); }
+// dQ and / or dK and dV of whatever is not left to the kernels on the supports
+static int launch_bwd_dense(const AttnBwdParams& p, int D, int dtype, int am, int which, hipStream_t s) {
+  if (dtype != ADSP_F32 && (D == 64 || D == 128)) return ADSP_CALL_16(launch_attn_bwd16, D, dtype, p, am, which, false, s);
+  return kBwdTable[dtype][head_dim_slot(D)](p, am, which, s);
+}
 
 // e4m3 copy of K for the first walk of the sparse-support forward: [B * Hkv][Npad][D] bytes in the order of K, values
 // beyond the format's range saturated, rows from N on zero.  A thread converts 16 values.  Heads the probe has marked
@@ -489,8 +501,7 @@ static int attn_common(const void* q, const void* k, const void* v, void* out, f
   if (!tile_counts && !bmask && !supports && rows32_16bit(B, Hq, N, D, dtype, alpha, is_causal != 0)) {
     // (not touched, but asked for as below: the size query does not know the call)
     if (w.total && (!workspace || workspace_bytes < w.total || ((uintptr_t)workspace & 15) != 0)) return ADSP_ERR_WORKSPACE;
-    const int rc = dtype == ADSP_BF16 ? (D == 64 ? launch_attn_rows32_fwd_bf16_d64(p, am, s) : launch_attn_rows32_fwd_bf16_d128(p, am, s))
-                                      : (D == 64 ? launch_attn_rows32_fwd_f16_d64(p, am, s) : launch_attn_rows32_fwd_f16_d128(p, am, s));
+    const int rc = ADSP_CALL_16(launch_attn_rows32_fwd, D, dtype, p, am, s);
     return rc == 0 && hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
   }
   if (dtype != ADSP_F32) {
@@ -868,8 +879,7 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
     }
   }
   if (short16) {
-    const int rc = dtype == ADSP_BF16 ? (D == 64 ? launch_attn_rows32_bwd_bf16_d64(p, am, s) : launch_attn_rows32_bwd_bf16_d128(p, am, s))
-                                      : (D == 64 ? launch_attn_rows32_bwd_f16_d64(p, am, s) : launch_attn_rows32_bwd_f16_d128(p, am, s));
+    const int rc = ADSP_CALL_16(launch_attn_bwd16, D, dtype, p, am, 3, true, s);
     return rc == 0 && hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
   }
   if (f32_split(N, D, dtype, alpha)) {
@@ -877,13 +887,13 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
     return hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
   }
   if (!sparse) {
-    if (kBwdTable[dtype][head_dim_slot(D)](p, am, 3, s) != 0) return ADSP_ERR_LAUNCH;
+    if (launch_bwd_dense(p, D, dtype, am, 3, s) != 0) return ADSP_ERR_LAUNCH;
     return hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
   }
   // dense dQ kernel on the row blocks the sparse one flagged (delta and 1 / sum p are complete behind it), then dK and
   // dV: the sparse-support kernel per (key block, query head), the dense kernel on the key blocks it flagged, and the
   // sum of the partial rows over the query heads of each K/V head
-  if (kBwdTable[dtype][head_dim_slot(D)](p, am, 1, s) != 0) return ADSP_ERR_LAUNCH;
+  if (launch_bwd_dense(p, D, dtype, am, 1, s) != 0) return ADSP_ERR_LAUNCH;
   {
     unsigned char* ws = (unsigned char*)workspace;
     p.queue2 = (uint32_t*)(ws + w.queue2_off);
@@ -900,7 +910,7 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
     if (dtype == ADSP_BF16) rc = D == 64 ? launch_attn_bwd_sparse_bf16_d64(p, am, kind, w.slots, s) : launch_attn_bwd_sparse_bf16_d128(p, am, kind, w.slots, s);
     else rc = D == 64 ? launch_attn_bwd_sparse_f16_d64(p, am, kind, w.slots, s) : launch_attn_bwd_sparse_f16_d128(p, am, kind, w.slots, s);
     if (rc != 0) return ADSP_ERR_LAUNCH;
-    if (kBwdTable[dtype][head_dim_slot(D)](p, am, 2, s) != 0) return ADSP_ERR_LAUNCH;
+    if (launch_bwd_dense(p, D, dtype, am, 2, s) != 0) return ADSP_ERR_LAUNCH;
     if (w.part_bytes && !(p.streams && Hq == Hkv)) {  // (with one query head per K/V head the kernel on the streams writes dK and dV itself)
       const long long threads = (long long)B * Hkv * N * (D / 8);
       const dim3 grid((unsigned)((threads + 255) / 256));

@@ -1,6 +1,5 @@
 // Sparse entmax attention on workgroups of 32 rows for gfx950, head dims 64 and 128: single-precision forward, dQ and dK/dV
-// kernels, and the same for short 16-bit problems (there dQ's fp32 weights are split into two 16-bit operands, for f16 behind a
-// power of two per row; dK's and dV's are rounded to one, as in the other 16-bit kernels).
+// kernels, and the forward for some 16-bit problems.
 //
 // What bounds them: the fp32 matrix pipe (v_mfma_f32_32x32x2_f32, 64 cycles) on large problems, and on
 // ordinary ones the length of a workgroup's walk over the keys, because a K/V head of N keys has only N / rows workgroups.
@@ -716,17 +715,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // ---------------------------------------------------------------------------------------------------------
 template <int D> constexpr int bwd_smem() { return kRing > kWaves * kRows * D * 4 ? kRing : kWaves * kRows * D * 4; }
 
-template <typename T, int D, int AM>
+template <int D, int AM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_rows32_dq_kernel(AttnBwdParams p) {
-  constexpr bool k16 = is16<T>::value;
-  constexpr int kStride = D * (k16 ? 2 : 4);
+  constexpr int kStride = D * 4;
   constexpr int NC = kStride / 128;      // chunks per block
-  constexpr int kOC = k16 ? 2 : 1;       // blocks of 32 columns per chunk
   __shared__ __align__(4096) unsigned char smem[bwd_smem<D>()];
-  // f16: a row's weights are scaled by a power of two before they are split, so that neither part leaves the type's range
-  constexpr bool kScaled = k16 && !elem_traits<T>::kIsBf16;
-  __shared__ float red[kWaves][kScaled ? 4 : 3][kRows];
-  __shared__ float unscale[kScaled ? kRows : 1];
+  __shared__ float red[kWaves][3][kRows];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
@@ -762,8 +756,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // chunks of a block: K, V and, for the second walk, K again
   auto src = [&](int blk, int s, int st) {
     const unsigned char* g = s < NC || s >= 2 * NC ? kg : vg;
-    if (k16 && s >= 2 * NC) ring.issue_t(g, blk * kRows, L, s % NC, st);
-    else ring.issue(g, blk * kRows, L, s % NC, st);
+    ring.issue(g, blk * kRows, L, s % NC, st);
   };
   // r = z - tau (-inf where the row may not look); false when no row of the block has a member, whose dP is then not formed
   auto block_terms = [&](int blk, auto&& next, float (&r)[16], f32x16& dp) -> bool {
@@ -771,7 +764,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) dot_chunk<D == 64, T>(s, next(c), rl, qf + c * 16);
+    for (int c = 0; c < NC; ++c) dot_chunk<D == 64, float>(s, next(c), rl, qf + c * 16);
     const int jb = blk * kRows + 4 * lh;
     float mx = -INFINITY;
 #pragma unroll
@@ -783,11 +776,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(NC + c);
-      if (any) dot_chunk<D == 64, T>(dp, a, rl, dof + c * 16);
+      if (any) dot_chunk<D == 64, float>(dp, a, rl, dof + c * 16);
     }
     return any;
   };
-  float zsum = 0.f, usum = 0.f, udp = 0.f, dmax = 0.f;
+  float zsum = 0.f, usum = 0.f, udp = 0.f;
   walk<2 * NC>(ring, wave, n_kblk, kWaves, src, [&](int blk, auto&& next) {
     float r[16];
     f32x16 dp;
@@ -799,18 +792,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       zsum += pr;
       usum += u;
       udp += u > 0.f ? u * dp[i] : 0.f;
-      if constexpr (kScaled) dmax = fmaxf(dmax, u > 0.f ? fabsf(dp[i]) : 0.f);
     }
   });
   zsum += __shfl_xor(zsum, 32, 64);
   usum += __shfl_xor(usum, 32, 64);
   udp += __shfl_xor(udp, 32, 64);
-  if constexpr (kScaled) dmax = fmaxf(dmax, __shfl_xor(dmax, 32, 64));
   if (lh == 0) {
     red[wave][0][lq] = zsum;
     red[wave][1][lq] = usum;
     red[wave][2][lq] = udp;
-    if constexpr (kScaled) red[wave][3][lq] = dmax;
   }
   __syncthreads();
   auto all = [&](int k) { return (red[0][k][lq] + red[1][k][lq]) + (red[2][k][lq] + red[3][k][lq]); };
@@ -818,29 +808,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   usum = all(1);
   udp = all(2);
   const float delta = usum > 0.f ? udp / usum : 0.f;
-  // u is at most 1 (to rounding) and delta is a mean of the members' dP, so |u (dP - delta)| < 2 max |dP| < 2^(e + 1) with
-  // max |dP| < 2^e: times 2^(13 - e) it stays below 2^14, and the second part's spacing, 2^-24 at the least, is 2^-38 of that.
-  // (|dP| < 2^40, as a sum of 128 products of f16 numbers; at a factor of 2^60 the spacing is 2^-84, far below what dQ resolves.)
-  int up = 0;
-  if constexpr (kScaled) {
-    dmax = fmaxf(fmaxf(red[0][3][lq], red[1][3][lq]), fmaxf(red[2][3][lq], red[3][3][lq]));
-    const int e = (int)(__builtin_bit_cast(uint32_t, dmax) >> 23) - 126;
-    up = 13 - e;
-    up = up > 60 ? 60 : (up < -60 ? -60 : up);
-  }
   if (live && wave == 0 && lh == 0) {
     p.delta[q_row0 + qi] = delta;
     p.zinv[q_row0 + qi] = zsum > 0.f ? 1.f / zsum : 0.f;
   }
-  f32x16 o[NC][kOC];
+  f32x16 o[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int d = 0; d < kOC; ++d)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) o[c][d][i] = 0.f;
+    for (int i = 0; i < 16; ++i) o[c][i] = 0.f;
   walk<3 * NC>(ring, wave, n_kblk, kWaves, src, [&](int blk, auto&& next) {
-    float r[16], dx[16], lo[16];
+    float r[16], dx[16];
     f32x16 dp;
     const bool any = block_terms(blk, next, r, dp);
 #pragma unroll
@@ -848,40 +826,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       float pr, u;
       bwd_prob<AM>(r[i], p.c0, pr, u);
       dx[i] = u > 0.f ? u * (dp[i] - delta) : 0.f;
-      if constexpr (kScaled) dx[i] = __builtin_amdgcn_ldexpf(dx[i], up);
-      if constexpr (k16) lo[i] = dx[i] - unpack_lo<T>(pack2<T>(dx[i], 0.f));
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(2 * NC + c);
-      if constexpr (k16) {
-        if (any) {  // the fp32 weights as two 16-bit parts
-          acc_chunk_16<T>(o[c], a, lane, dx);
-          acc_chunk_16<T>(o[c], a, lane, lo);
-        }
-      } else {
-        if (any) acc_chunk(o[c][0], a, cl, dx);
-      }
+      if (any) acc_chunk(o[c], a, cl, dx);
     }
   });
-  if constexpr (kScaled) {
-    if (wave == 0 && lh == 0) unscale[lq] = __builtin_amdgcn_ldexpf(p.sm_scale, -up);
-  }
   __syncthreads();  // every wave is done with its ring
   const float sm = p.sm_scale;
-  combine_store<D>(reinterpret_cast<const f32x16(&)[D / 32]>(o), smem, reinterpret_cast<T*>(dq), m0, N, wave, lane,
-                   [&](int row) { return kScaled ? unscale[row] : sm; });
+  combine_store<D>(o, smem, reinterpret_cast<float*>(dq), m0, N, wave, lane,
+                   [&](int) { return sm; });
 }
 
 // ---------------------------------------------------------------------------------------------------------
 // dK, dV: one walk over the (query block, query head) pairs of a K/V head, dV^T += dO^T P and dK^T += Q^T dX
 // ---------------------------------------------------------------------------------------------------------
-template <typename T, int D, int AM>
+template <int D, int AM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void attn_rows32_dkdv_kernel(AttnBwdParams p) {
-  constexpr bool k16 = is16<T>::value;
-  constexpr int kStride = D * (k16 ? 2 : 4);
+  constexpr int kStride = D * 4;
   constexpr int NC = kStride / 128;      // chunks per block
-  constexpr int kOC = k16 ? 2 : 1;       // blocks of 32 columns per chunk
   __shared__ __align__(4096) unsigned char smem[bwd_smem<D>()];
   __shared__ __align__(256) float scal[kWaves][4 * kRows];  // of the wave's block: tau, 1 / sum p, delta (and delta once more)
   const int tid = threadIdx.x;
@@ -928,23 +892,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
       dma4((lane < 32 ? p.taus : p.zinv) + at, &scal[wave][0]);
       dma4(p.delta + at, &scal[wave][64]);
     }
-    if (k16 && s >= 2 * NC) ring.issue_t(base, qb * kRows, L, s % NC, st);
-    else ring.issue(base, qb * kRows, L, s % NC, st);
+    ring.issue(base, qb * kRows, L, s % NC, st);
   };
-  f32x16 ov[NC][kOC], ok[NC][kOC];
+  f32x16 ov[NC], ok[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int d = 0; d < kOC; ++d)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) ov[c][d][i] = ok[c][d][i] = 0.f;
+    for (int i = 0; i < 16; ++i) ov[c][i] = ok[c][i] = 0.f;
   walk<4 * NC>(ring, wave, n_q * group, kWaves, src, [&](int x, auto&& next) {
     const int g = x / n_q, q0 = (q_first + (x - g * n_q)) * kRows;
     f32x16 s, dp;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) dot_chunk<D == 64, T>(s, next(c), rl, kf + c * 16);
+    for (int c = 0; c < NC; ++c) dot_chunk<D == 64, float>(s, next(c), rl, kf + c * 16);
     // tau, 1 / sum p and delta of the lane's sixteen queries: they came in front of the block's first chunk
     auto scalars = [&](int which, float (&y)[16]) {
 #pragma unroll
@@ -973,7 +934,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(NC + c);
-      if (any) dot_chunk<D == 64, T>(dp, a, rl, vf + c * 16);
+      if (any) dot_chunk<D == 64, float>(dp, a, rl, vf + c * 16);
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -985,27 +946,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(2 * NC + c);
-      if constexpr (k16) {
-        if (any) acc_chunk_16<T>(ov[c], a, lane, w);
-      } else {
-        if (any) acc_chunk(ov[c][0], a, cl, w);
-      }
+      if (any) acc_chunk(ov[c], a, cl, w);
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(3 * NC + c);
-      if constexpr (k16) {
-        if (any) acc_chunk_16<T>(ok[c], a, lane, dx);
-      } else {
-        if (any) acc_chunk(ok[c][0], a, cl, dx);
-      }
+      if (any) acc_chunk(ok[c], a, cl, dx);
     }
   });
   __syncthreads();  // every wave is done with its ring
-  combine_store<D>(reinterpret_cast<const f32x16(&)[D / 32]>(ov), smem, reinterpret_cast<T*>(dv), n0, N, wave, lane, [](int) { return 1.f; });
+  combine_store<D>(ov, smem, reinterpret_cast<float*>(dv), n0, N, wave, lane, [](int) { return 1.f; });
   __syncthreads();
   const float sm = p.sm_scale;
-  combine_store<D>(reinterpret_cast<const f32x16(&)[D / 32]>(ok), smem, reinterpret_cast<T*>(dk), n0, N, wave, lane, [&](int) { return sm; });
+  combine_store<D>(ok, smem, reinterpret_cast<float*>(dk), n0, N, wave, lane, [&](int) { return sm; });
 }
 
 }  // namespace f32path

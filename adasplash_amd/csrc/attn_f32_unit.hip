@@ -10,8 +10,8 @@ using namespace f32path;
 static dim3 grid_of(int B, int Hkv, int group, int N) { return dim3(xcd_grid((long long)B * Hkv, (long long)((N + kRows - 1) / kRows) * group)); }
 
 template <int AM> static void launch_bwd(const AttnBwdParams& p, hipStream_t s) {
-  hipLaunchKernelGGL((attn_rows32_dq_kernel<float, ADSP_D, AM>), grid_of(p.B, p.Hkv, p.Hq / p.Hkv, p.N), dim3(256), 0, s, p);
-  hipLaunchKernelGGL((attn_rows32_dkdv_kernel<float, ADSP_D, AM>), grid_of(p.B, p.Hkv, 1, p.N), dim3(256), 0, s, p);
+  hipLaunchKernelGGL((attn_rows32_dq_kernel<ADSP_D, AM>), grid_of(p.B, p.Hkv, p.Hq / p.Hkv, p.N), dim3(256), 0, s, p);
+  hipLaunchKernelGGL((attn_rows32_dkdv_kernel<ADSP_D, AM>), grid_of(p.B, p.Hkv, 1, p.N), dim3(256), 0, s, p);
 }
 template <int AM> static void launch_fwd(const AttnParams& p, hipStream_t s) {
   hipLaunchKernelGGL((attn_rows32_fwd_kernel<float, ADSP_D, AM>), grid_of(p.B, p.Hkv, p.Hq / p.Hkv, p.N), dim3(256), 0, s, p);

@@ -1,4 +1,4 @@
-// One translation unit per (16-bit type, head dim) of the kernels on 32 rows a workgroup (attn_f32_kernel.h), compiled with
+// One translation unit per (16-bit type, head dim) of the forward on 32 rows a workgroup (attn_f32_kernel.h), compiled with
 // -DADSP_T=<bf16_t|f16_t> -DADSP_TAG=<bf16|f16> -DADSP_D=<head dim>.
 #include "attn_f32_kernel.h"
 
@@ -12,20 +12,10 @@ static dim3 grid_of(int B, int Hkv, int group, int N) { return dim3(xcd_grid((lo
 template <int AM> static void launch_fwd(const AttnParams& p, hipStream_t s) {
   hipLaunchKernelGGL((attn_rows32_fwd_kernel<ADSP_T, ADSP_D, AM>), grid_of(p.B, p.Hkv, p.Hq / p.Hkv, p.N), dim3(256), 0, s, p);
 }
-template <int AM> static void launch_bwd(const AttnBwdParams& p, hipStream_t s) {
-  hipLaunchKernelGGL((attn_rows32_dq_kernel<ADSP_T, ADSP_D, AM>), grid_of(p.B, p.Hkv, p.Hq / p.Hkv, p.N), dim3(256), 0, s, p);
-  hipLaunchKernelGGL((attn_rows32_dkdv_kernel<ADSP_T, ADSP_D, AM>), grid_of(p.B, p.Hkv, 1, p.N), dim3(256), 0, s, p);
-}
 int ADSP_CAT(launch_attn_rows32_fwd_, ADSP_TAG, ADSP_D)(const AttnParams& p, int am, hipStream_t s) {
   if (am == ATT_15) launch_fwd<ATT_15>(p, s);
   else if (am == ATT_2) launch_fwd<ATT_2>(p, s);
   else launch_fwd<ATT_GEN>(p, s);
-  return 0;
-}
-int ADSP_CAT(launch_attn_rows32_bwd_, ADSP_TAG, ADSP_D)(const AttnBwdParams& p, int am, hipStream_t s) {
-  if (am == ATT_15) launch_bwd<ATT_15>(p, s);
-  else if (am == ATT_2) launch_bwd<ATT_2>(p, s);
-  else launch_bwd<ATT_GEN>(p, s);
   return 0;
 }
 }  // namespace adsp

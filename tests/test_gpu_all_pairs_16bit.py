@@ -1,0 +1,109 @@
+"""The 16-bit kernels that visit all pairs of a row (head dims 64 and 128) against the oracle, where their split can go wrong: lengths
+around a block of 32, a tile of 128 and a workgroup's rows, workgroups of 128, 64 and 32 rows, padding that holds NaN, grouped
+K/V heads, every alpha mode.
+
+Bound on the error of a whole tensor (2-norm, relative): a weight is rounded to the type before it multiplies a row, and the result
+once more, each by at most 2^-9 (bf16) or 2^-11 (f16) of itself, together at most 2^-8 or 2^-10.  alpha = 2: a key that
+rounding puts on the other side of the support's border changes its row's gradient at once, 2e-2 as in the other tests."""
+
+import os
+
+import pytest
+import torch
+
+import adasplash_amd as A
+from adasplash_amd import _lib
+from oracle import exact
+from tests.gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+UNIT = {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -11}
+
+
+def problem(B, Hq, Hkv, N, D, dtype, scale, lengths):
+    g = torch.Generator().manual_seed(12)
+    q = (scale * torch.randn(B, Hq, N, D, generator=g)).to(dtype)
+    k, v = (torch.randn(B, Hkv, N, D, generator=g).to(dtype) for _ in range(2))
+    dout = torch.randn(B, Hq, N, D, generator=g).to(dtype)
+    varlen = torch.tensor([lengths[b % len(lengths)] for b in range(B)], dtype=torch.int32)
+    return q, k, v, dout, varlen
+
+
+def check(got, q, k, v, dout, varlen, alpha, causal, items):
+    """``got``: output alone or output and gradients; compared on the given batch items, zeros behind every item's length"""
+    q, k, v, dout, vl = q[items], k[items], v[items], dout[items], varlen[items]
+    want = [exact.dense_entmax_attention(q, k, v, alpha, causal, vl)]
+    if len(got) > 1:
+        want += list(exact.dense_entmax_attention_grads(q, k, v, dout, alpha, causal, vl))
+    for name, a, w in zip(("out", "dq", "dk", "dv"), got, want):
+        assert torch.isfinite(a).all(), name
+        for b, n in enumerate(varlen.tolist()):
+            assert (a[b, :, n:] == 0).all(), name
+        err = ((a[items].double().cpu() - w.double()).norm() / w.double().norm()).item()
+        assert err < (2e-2 if alpha == 2.0 and name in ("dq", "dk") else 2 * UNIT[a.dtype]), (name, err)
+
+
+def run(q, k, v, dout, varlen, alpha, causal, train=True):
+    q, k, v = (t.clone() for t in (q, k, v))
+    for b, n in enumerate(varlen.tolist()):  # the padding may hold anything
+        for t in (q, k, v):
+            t[b, :, n:] = float("nan")
+    q, k, v = (t.to(DEV).requires_grad_(train) for t in (q, k, v))
+    vl = varlen.to(DEV)
+    if q.shape[1] != k.shape[1]:
+        out = A.adasplash_v2(q, k, v, niter=10, varlen=vl)
+    else:
+        out = A.adasplash_v1(q, k, v, alpha=alpha, is_causal=causal, niter=10, varlen=vl)
+    if not train:
+        return (out,)
+    out.backward(dout.to(DEV))
+    return out.detach(), q.grad, k.grad, v.grad
+
+
+@pytest.fixture
+def no_supports():
+    old = os.environ.get("ADSP_SPARSE")
+    os.environ["ADSP_SPARSE"] = "0"
+    yield
+    if old is None:
+        os.environ.pop("ADSP_SPARSE", None)
+    else:
+        os.environ["ADSP_SPARSE"] = old
+
+
+@pytest.mark.parametrize("scale", [0.125, 1.0])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,alpha,causal,lengths", [
+    # rows of an item, queries and keys: from 16384 workgroups of 128 rows, from 4096 of 64, below of 32
+    (1, 16, 16, 1027, 64, 1.5, True, [1027]), (1, 16, 4, 1027, 128, 1.5, True, [1027]), (2, 8, 2, 577, 64, 1.5, True, [577, 513]),
+    (6, 2, 1, 300, 128, 1.5, True, [300, 1, 31, 32, 129, 257]), (6, 2, 2, 300, 64, 1.333, False, [300, 1, 31, 32, 129, 257]),
+    (2, 8, 8, 577, 128, 1.333, False, [577, 127]), (1, 13, 13, 1283, 128, 1.5, False, [1283]), (1, 16, 16, 1030, 64, 2.0, False, [1025]),
+    (2, 8, 8, 515, 128, 2.0, False, [515, 65])])
+def test_gradients_on_all_pairs(no_supports, B, Hq, Hkv, N, D, alpha, causal, lengths, dtype, scale):
+    q, k, v, dout, varlen = problem(B, Hq, Hkv, N, D, dtype, scale, lengths)
+    got = run(q, k, v, dout, varlen, alpha, causal)
+    assert all(torch.equal(a, b) for a, b in zip(got, run(q, k, v, dout, varlen, alpha, causal)))
+    check(got, q, k, v, dout, varlen, alpha, causal, list(range(B)))
+
+
+@pytest.mark.parametrize("scale", [0.125, 1.0])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,alpha,causal,lengths", [
+    # rows of the batch: from 32768 workgroups of 128 rows, from 16384 of 64, below of 32
+    (65, 8, 8, 64, 64, 1.5, True, [64, 63, 33, 32, 1]), (33, 16, 8, 64, 128, 1.5, True, [64, 31, 2]), (40, 8, 2, 97, 64, 1.5, True, [97, 96, 65]),
+    (3, 2, 2, 415, 128, 1.333, False, [415, 385, 128]), (20, 12, 12, 99, 64, 2.0, False, [99, 34])])
+def test_gradients_of_short_problems(B, Hq, Hkv, N, D, alpha, causal, lengths, dtype, scale):
+    q, k, v, dout, varlen = problem(B, Hq, Hkv, N, D, dtype, scale, lengths)
+    assert _lib.load().adsp_attn_bwd_reads_bmask(B, Hq, Hkv, N, D, _lib.dtype_code(q), alpha, int(causal)) == 0
+    got = run(q, k, v, dout, varlen, alpha, causal)
+    assert all(torch.equal(a, b) for a, b in zip(got, run(q, k, v, dout, varlen, alpha, causal)))
+    check(got, q, k, v, dout, varlen, alpha, causal, sorted({*range(min(B, len(lengths))), B - 1}))
+
+
+def test_gradients_leave_out_what_a_causal_mask_hides(no_supports):
+    """Rows of K and V that later queries alone see may be infinite for the earlier ones."""
+    q, k, v, dout, varlen = problem(1, 2, 2, 160, 64, torch.bfloat16, 1.0, [160])
+    want = run(q[:, :, :150], k[:, :, :150], v[:, :, :150], dout[:, :, :150], torch.tensor([150], dtype=torch.int32), 1.5, True)
+    v[:, :, 150:] = float("inf")
+    dq = run(q, k, v, dout, varlen, 1.5, True)[1]
+    assert torch.isfinite(dq[:, :, :150]).all() and torch.equal(dq[:, :, :150], want[1])
