@@ -35,10 +35,11 @@ int launch_attn_f32_fwd_d128(const AttnParams&, int, hipStream_t);
 int launch_attn_f32_bwd_d64(const AttnBwdParams&, int, hipStream_t);
 int launch_attn_f32_bwd_d128(const AttnBwdParams&, int, hipStream_t);
 
-// 16-bit types, head dims 64 and 128: the forward on 32 rows a workgroup (attn_rows32_unit.hip), and dQ and dK/dV on all pairs
-// (attn_bwd16_unit.hip)
+// 16-bit types, head dims 64 and 128: the forward on 32 rows a workgroup with lists (attn_rows32_unit.hip), the one with a row's
+// scores in registers (attn_resident_unit.hip), and dQ and dK/dV on all pairs (attn_bwd16_unit.hip)
 #define ADSP_DECL_16(tag, d)                                                        \
   int launch_attn_rows32_fwd_##tag##_d##d(const AttnParams&, int, hipStream_t);     \
+  int launch_attn_resident_fwd_##tag##_d##d(const AttnParams&, int, hipStream_t);   \
   int launch_attn_bwd16_##tag##_d##d(const AttnBwdParams&, int, int, bool, hipStream_t);
 ADSP_DECL_16(bf16, 64)
 ADSP_DECL_16(bf16, 128)
@@ -397,24 +398,48 @@ static bool rows32_16bit(int B, int Hq, int N, int D, int dtype, double alpha, b
   const long long most = N <= 128 ? 2048 : ((N >= 1024 || !causal) ? 1024 : 512);
   return groups <= most && rows32_cost_ns(B, Hq, N, causal) <= 66e3;
 }
-// Of those, the calls whose backward goes the same way (and whose forward then keeps nothing for it): a dK/dV workgroup walks
-// the query blocks of all heads of its group, which only few-headed problems can afford at length.  Without a causal mask
-// every walk is a long one, and with D = 128 a workgroup of that kernel fills a CU, so that a second round of them is one too many
-// from walks of some 24 blocks on.  The lines lie where a call with peaked scores, which gains least, begins to be slower by more
-// than some 5 %.  Forward and backward, GPU times in us, q of spread 1, 3 and 1/8:
-//   D = 64, causal: 8 heads, 4 sequences of N = 256: 136 -> 35, 93 -> 36, 74 -> 48; 16/4 heads, N = 1024: 202 -> 113, 118 -> 107,
-//     285 -> 118; 32 x 16 heads, N = 128: 144 -> 95, 109 -> 90, 136 -> 120; at the line 12 heads, N = 2048: 242 -> 157, 135 -> 125,
-//     270 -> 156; 6/3 heads, N = 2036: 233 -> 165, 133 -> 137, 356 -> 166; one head, N = 4096: 283 -> 236, 162 -> 160, 492 -> 220;
-//     beyond it 2 x 16/4 heads, N = 1024: 216 -> 143, 121 -> 133, 288 -> 151;
-//   D = 64, full: one head, N = 3072: 214 -> 195, 135 -> 132, 702 -> 174; beyond it N = 4032: 249 -> 251, 151 -> 163, 954 -> 236;
-//     7 heads, N = 2048: 202 -> 166, 118 -> 120, 484 -> 154; 2 x 16 of 807, alpha = 1.333: 439 -> 233, 145 -> 163, 434 -> 208;
-//   D = 128, causal: 4/1 heads, N = 1024: 300 -> 158, 144 -> 151, 470 -> 170; one head, N = 3072: 344 -> 199, 188 -> 184, 621 -> 243; 16
-//     heads, N = 1502: 316 -> 183, 168 -> 172, 352 -> 209; beyond it 12 heads, N = 2048: 322 -> 220, 180 -> 206, 448 -> 246; one head,
-//     N = 4096: 389 -> 256, 216 -> 238, 820 -> 321;
-//   D = 128, full: 3 heads, N = 2048: 247 -> 198, 153 -> 139, 700 -> 173; 4 x 3 heads, N = 725: 227 -> 109, 121 -> 104, 309 -> 122; beyond
-//     it 8 heads, N = 1153, alpha = 2: 130 -> 143, 118 -> 138, 547 -> 153; 2 x 16 heads, N = 554: 219 -> 156, 128 -> 146, 254 -> 168; 16
-//     heads, N = 1082: 244 -> 230, 136 -> 216, 421 -> 260; one head, N = 3072: 272 -> 204, 170 -> 187, 1017 -> 258.
-static bool rows32_16bit_training(int B, int Hq, int Hkv, int N, int D, int dtype, double alpha, bool causal) {
+// blocks of 32 x 32 scores of a call, padding included
+static long long score_blocks(int B, int Hq, int N, bool causal) {
+  const long long r = (N + 31) / 32;
+  return (long long)B * Hq * (causal ? r * (r + 1) / 2 : r * r);
+}
+static bool resident_takes(int N, int D, int dtype, double alpha) {
+  return dtype != ADSP_F32 && (D == 64 || D == 128) && N <= 2048 && alpha >= 1.125 && alpha <= 2.0 && sparse_enabled();
+}
+// Whether a 16-bit forward of which nobody wants the tile mask or the supports takes the single kernel that holds its rows' scores in
+// registers (attn_resident_kernel.h).  It does the same work whatever the scores are, so the lines lie where the kernels on
+// the supports, which do less where scores are peaked and rows are long, catch up with unit spread.  Up to 512 keys never; up to 1024
+// where the chip has more than a few rounds of it; beyond, where a workgroup of sixteen waves fills a CU, after one or two.  us, the others
+// -> this kernel, q of spread 1, 3 and 1/8:
+//   16 x 12 heads, N <= 500, D = 64: 86 -> 35, 64 -> 33, 147 -> 34; 32 x 16 heads, N <= 512, D = 128: 256 -> 122, 172 -> 125, 394 -> 127;
+//   N = 1024: 8 x 8/4 heads, D = 64: 93 -> 46, 63 -> 42, 59 -> 43; 3 x 16/8, D = 128: 151 -> 56, 82 -> 52, 84 -> 52; at the line 5 x 16, D = 128,
+//     causal: 173 -> 92, 100 -> 83, 90 -> 86; 13 x 8/2, D = 128: 187 -> 114, 106 -> 98, 96 -> 102; beyond it 3 x 64/16, D = 128: 258 -> 186, 148 -> 172, 151 -> 180;
+//   N > 1024: 1750, 8/2 heads, D = 64: 38 -> 28, 30 -> 26, 51 -> 27; 7 x 2 of 1994: 43 -> 40, 34 -> 37, 60 -> 39; 4/1 of 1684, D = 128: 40 -> 26, 30 -> 25, 64 -> 28; beyond it
+//     2 x 32/8 of 1339, D = 64: 94 -> 84, 62 -> 76, 72 -> 77; 2 x 8 of 1138, D = 128: 37 -> 39, 28 -> 37, 54 -> 38.
+static bool resident_16bit(int B, int Hq, int N, int D, int dtype, double alpha, bool causal) {
+  if (!resident_takes(N, D, dtype, alpha)) return false;
+  const long long blocks = score_blocks(B, Hq, N, causal);
+  if (N <= 512) return true;
+  if (N <= 1024) return blocks <= (D == 64 ? 100000 : 55000);
+  return blocks <= (D == 64 ? 28000 : 8000);
+}
+// The training steps whose backward computes all pairs (attn_bwd16_kernel.h, dQ's weights in two parts) and whose forward keeps nothing
+// for it.  Short ones as above, at less load, and none where a dK/dV workgroup, which walks the queries of all heads of its group,
+// had more than 128 blocks of them to visit.  us, kernels on the supports -> these, q of spread 1, 3 and 1/8:
+//   N <= 512: 16 x 12 heads, N <= 500, D = 64: 210 -> 112 (spread 1); 4 x 16/8, D = 128: 252 -> 89, 149 -> 89, 138 -> 90; 8 x 32/16, D = 128: 411 -> 227, 253 -> 224,
+//     261 -> 225;
+//   N <= 1024: 8 x 8/4 heads, D = 64: 235 -> 133, 145 -> 128, 161 -> 129; 3 x 16/8, D = 128: 347 -> 177, 188 -> 169, 216 -> 166; 4 x 4, D = 128, full: 251 -> 105, 133 -> 102, 160 -> 102;
+//     beyond the line 2 x 32/16, D = 128: 361 -> 220, 195 -> 214, 250 -> 208; 11 x 4, D = 128, full, alpha = 2: 174 -> 280, 156 -> 265, 438 -> 271;
+//   N > 1024: 7 x 2 of 1994, D = 64: 228 -> 110, 135 -> 106, 179 -> 109; 2 x 8 of 1138, D = 128: 125 -> 109, 116 -> 107, 142 -> 108; beyond it 32/8 of 1173, D = 64:
+//     242 -> 161, 134 -> 156, 188 -> 157.
+// And long sequences of few heads, where the forward is that on 32 rows a workgroup: one head, N = 3000, D = 64: 144 -> 133, 130 -> 123,
+// 164 -> 154 (gradients on 32 rows a workgroup -> these kernels), N = 4096: 239 -> 225, 165 -> 155, 214 -> 201 (on the supports 283, 162, 492).
+static bool all_pairs_training(int B, int Hq, int Hkv, int N, int D, int dtype, double alpha, bool causal) {
+  if (resident_takes(N, D, dtype, alpha) && (long long)(Hq / Hkv) * ((N + 31) / 32) <= 128) {
+    const long long blocks = score_blocks(B, Hq, N, causal);
+    if (N <= 512) return true;
+    if (blocks <= (D == 64 ? (N <= 1024 ? 50000 : (causal ? 26000 : 20000)) : (!causal ? 10000 : (N <= 1024 ? 25000 : 14000)))) return true;
+  }
   if (!rows32_16bit(B, Hq, N, D, dtype, alpha, causal)) return false;
   const double cost = rows32_cost_ns(B, Hq, N, causal);
   const long long blocks = (N + 31) / 32, walk = (long long)(Hq / Hkv) * blocks;
@@ -422,7 +447,7 @@ static bool rows32_16bit_training(int B, int Hq, int Hkv, int N, int D, int dtyp
   const long long pairs = (long long)B * Hq * blocks * blocks / (causal ? 2 : 1);
   if (D == 64) return causal || (walk <= 96 && pairs <= 16384);
   if (causal) return N <= 3072 && pairs <= 18432;
-  const long long rounds = ((long long)B * Hkv * blocks + 255) / 256;  // (one workgroup per CU)
+  const long long rounds = ((long long)B * Hkv * blocks + 255) / 256;
   return rounds * walk <= (rounds == 1 ? 64 : 48);
 }
 
@@ -498,10 +523,11 @@ static int attn_common(const void* q, const void* k, const void* v, void* out, f
     if ((D == 64 ? launch_attn_f32_fwd_d64(p, am, s) : launch_attn_f32_fwd_d128(p, am, s)) != 0) return ADSP_ERR_LAUNCH;
     return hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
   }
-  if (!tile_counts && !bmask && !supports && rows32_16bit(B, Hq, N, D, dtype, alpha, is_causal != 0)) {
+  const bool resident = resident_16bit(B, Hq, N, D, dtype, alpha, is_causal != 0);
+  if (!tile_counts && !bmask && !supports && (resident || rows32_16bit(B, Hq, N, D, dtype, alpha, is_causal != 0))) {
     // (not touched, but asked for as below: the size query does not know the call)
     if (w.total && (!workspace || workspace_bytes < w.total || ((uintptr_t)workspace & 15) != 0)) return ADSP_ERR_WORKSPACE;
-    const int rc = ADSP_CALL_16(launch_attn_rows32_fwd, D, dtype, p, am, s);
+    const int rc = resident ? ADSP_CALL_16(launch_attn_resident_fwd, D, dtype, p, am, s) : ADSP_CALL_16(launch_attn_rows32_fwd, D, dtype, p, am, s);
     return rc == 0 && hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;
   }
   if (dtype != ADSP_F32) {
@@ -563,7 +589,7 @@ extern "C" size_t adsp_attn_supports_bytes(int B, int Hq, int Hkv, int N, int D,
 
 extern "C" int adsp_attn_bwd_reads_bmask(int B, int Hq, int Hkv, int N, int D, int dtype, double alpha, int is_causal) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || N <= 0) return 1;
-  return adsp::f32_split(N, D, dtype, alpha) || adsp::rows32_16bit_training(B, Hq, Hkv, N, D, dtype, alpha, is_causal != 0) ? 0 : 1;
+  return adsp::f32_split(N, D, dtype, alpha) || adsp::all_pairs_training(B, Hq, Hkv, N, D, dtype, alpha, is_causal != 0) ? 0 : 1;
 }
 
 extern "C" size_t adsp_attn_bmask_words(int N) {
@@ -822,7 +848,7 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   BwdWorkspace w = {};
 
   (void)hipGetLastError();
-  const bool short16 = !bmask && !supports && rows32_16bit_training(B, Hq, Hkv, N, D, dtype, alpha, is_causal != 0);
+  const bool short16 = !bmask && !supports && all_pairs_training(B, Hq, Hkv, N, D, dtype, alpha, is_causal != 0);
   if (dtype != ADSP_F32) {
     w = bwd_workspace(B, Hq, Hkv, N, D, dtype, is_causal ? 1 : 0);
     const size_t need = w.total;

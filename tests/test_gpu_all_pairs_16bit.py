@@ -89,6 +89,8 @@ def test_gradients_on_all_pairs(no_supports, B, Hq, Hkv, N, D, alpha, causal, le
 @pytest.mark.parametrize("scale", [0.125, 1.0])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,Hq,Hkv,N,D,alpha,causal,lengths", [
+    (70, 8, 4, 500, 64, 1.5, True, [500, 1, 255, 499, 64]), (6, 12, 12, 500, 128, 1.333, False, [500, 129]), (2, 4, 4, 1024, 64, 1.5, True, [1024, 515]),
+    (1, 2, 2, 1997, 64, 2.0, False, [1997]), (1, 4, 2, 1023, 128, 1.5, True, [1023]),
     # rows of the batch: from 32768 workgroups of 128 rows, from 16384 of 64, below of 32
     (65, 8, 8, 64, 64, 1.5, True, [64, 63, 33, 32, 1]), (33, 16, 8, 64, 128, 1.5, True, [64, 31, 2]), (40, 8, 2, 97, 64, 1.5, True, [97, 96, 65]),
     (3, 2, 2, 415, 128, 1.333, False, [415, 385, 128]), (20, 12, 12, 99, 64, 2.0, False, [99, 34])])
@@ -98,6 +100,19 @@ def test_gradients_of_short_problems(B, Hq, Hkv, N, D, alpha, causal, lengths, d
     got = run(q, k, v, dout, varlen, alpha, causal)
     assert all(torch.equal(a, b) for a, b in zip(got, run(q, k, v, dout, varlen, alpha, causal)))
     check(got, q, k, v, dout, varlen, alpha, causal, sorted({*range(min(B, len(lengths))), B - 1}))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hq,Hkv,D,alpha,causal", [(2, 1, 64, 1.5, True), (1, 1, 128, 1.5, False), (1, 1, 64, 1.333, False), (1, 1, 128, 2.0, False)])
+@pytest.mark.parametrize("N,scale", [(64, 1.0), (129, 0.125), (512, 0.125), (513, 3.0), (1024, 1.0), (1025, 0.125), (2048, 3.0)])
+def test_forward_with_resident_scores(N, scale, Hq, Hkv, D, alpha, causal, dtype):
+    """Four waves to 512 keys, eight to 1024, sixteen to 2048.  The weights are multiplied as two 16-bit parts, so that the result's
+    rounding is all that is lost, and at most as much again for thresholds and sums in fp32."""
+    lengths = [N, 1, 31, N // 2 + 1]
+    q, k, v, dout, varlen = problem(4, Hq, Hkv, N, D, dtype, scale, lengths)
+    got = run(q, k, v, dout, varlen, alpha, causal, train=False)
+    assert torch.equal(got[0], run(q, k, v, dout, varlen, alpha, causal, train=False)[0])
+    check(got, q, k, v, dout, varlen, alpha, causal, list(range(4)))
 
 
 def test_gradients_leave_out_what_a_causal_mask_hides(no_supports):
