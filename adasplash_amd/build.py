@@ -68,6 +68,7 @@ def units(extra=None):
             if tag != "f32" and d in (64, 128):
                 out.append((f"attn_rows32_{tag}_d{d}", "attn_rows32_unit.hip", base))
                 out.append((f"attn_resident_{tag}_d{d}", "attn_resident_unit.hip", base))
+                out.append((f"attn_fwd16_{tag}_d{d}", "attn_fwd16_unit.hip", base + attn_flags))
                 out.append((f"attn_bwd16_{tag}_d{d}", "attn_bwd16_unit.hip", base + attn_flags))
                 out.append((f"attn_sparse_{tag}_d{d}", "attn_sparse_unit.hip", base + attn_flags))
                 out.append((f"attn_bwd_sparse_{tag}_d{d}", "attn_bwd_sparse_unit.hip", base + attn_flags))

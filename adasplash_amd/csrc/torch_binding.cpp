@@ -153,19 +153,20 @@ Tensor attn_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Att
     if (ws_bytes) wp = kept.base() + align256(keep_bytes);
   }
   const size_t sup = kept.supports;
+  float* const taus = w.outlives ? kept.taus() : nullptr;  // (nobody reads the thresholds of a call without a gradient)
   void* const stream = stream_of(q);
   if (c.version == 2) {
-    const int st = sup ? adsp_attn_v2_fwd_keep(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kept.taus(), kept.bmask(),
+    const int st = sup ? adsp_attn_v2_fwd_keep(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), taus, kept.bmask(),
                                                data(c.varlen), c.varlen_bits(), B, Hq, Hkv, N, D, dt, c.niter, wp, ws_bytes,
                                                kept.kept_supports(), sup, stream)
-                       : adsp_attn_v2_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kept.taus(), kept.bmask(),
+                       : adsp_attn_v2_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), taus, kept.bmask(),
                                           data(c.varlen), c.varlen_bits(), B, Hq, Hkv, N, D, dt, c.niter, wp, ws_bytes, stream);
     check(st, sup ? "adsp_attn_v2_fwd_keep" : "adsp_attn_v2_fwd");
   } else {
-    const int st = sup ? adsp_attn_v1_fwd_keep(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kept.taus(), kept.bmask(),
+    const int st = sup ? adsp_attn_v1_fwd_keep(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), taus, kept.bmask(),
                                                data(c.varlen), c.varlen_bits(), B, Hq, N, D, dt, c.alpha, c.causal, c.niter, wp,
                                                ws_bytes, kept.kept_supports(), sup, stream)
-                       : adsp_attn_v1_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kept.taus(), kept.bmask(),
+                       : adsp_attn_v1_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), taus, kept.bmask(),
                                           data(c.varlen), c.varlen_bits(), B, Hq, N, D, dt, c.alpha, c.causal, c.niter, wp, ws_bytes,
                                           w.tile_counts, stream);
     check(st, sup ? "adsp_attn_v1_fwd_keep" : "adsp_attn_v1_fwd");

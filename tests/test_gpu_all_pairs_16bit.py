@@ -115,6 +115,18 @@ def test_forward_with_resident_scores(N, scale, Hq, Hkv, D, alpha, causal, dtype
     check(got, q, k, v, dout, varlen, alpha, causal, list(range(4)))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hq,Hkv,D,alpha,causal", [(2, 1, 64, 1.5, True), (1, 1, 128, 1.5, False), (1, 1, 64, 1.125, False), (1, 1, 128, 2.0, False)])
+@pytest.mark.parametrize("N,scale", [(97, 1.0), (256, 0.125), (257, 0.125), (577, 1.0), (1153, 3.0), (1300, 0.125), (2309, 0.125)])
+def test_forward_on_all_pairs(no_supports, N, scale, Hq, Hkv, D, alpha, causal, dtype):
+    """Rows that are all in the sample of 256 keys, just beyond it, and with a step on half of the tiles (from 1024 keys); without
+    a gradient and, where the output walk corrects the threshold, with one."""
+    lengths = [N, 1, 64, N // 2 + 1]
+    q, k, v, dout, varlen = problem(4, Hq, Hkv, N, D, dtype, scale, lengths)
+    for train in (False, True):
+        check(run(q, k, v, dout, varlen, alpha, causal, train), q, k, v, dout, varlen, alpha, causal, list(range(4)))
+
+
 def test_gradients_leave_out_what_a_causal_mask_hides(no_supports):
     """Rows of K and V that later queries alone see may be infinite for the earlier ones."""
     q, k, v, dout, varlen = problem(1, 2, 2, 160, 64, torch.bfloat16, 1.0, [160])
