@@ -18,13 +18,16 @@ template <int AM, int P> static void launch_dkdv(const AttnBwdParams& p, hipStre
 }
 // Parts a row's walk is split in: as few as give every CU a workgroup of 128 / parts rows.  Training, us for 1, 2 and 4 parts: 16 x 12
 // heads, N <= 500, D = 64: 112, 114, 140; 4 x 16, N = 512, D = 128: 86, 93, 131; 8 x 8, N <= 300, D = 128: 81, 71, 79; dQ's rows 32000 and dK/dV's
-// 8000 (2 x 16/4, N <= 1000, D = 64): 138, 111, 110.  Where the kernels stand in for those on the supports, which add up an item of a
-// batch in the same order whatever the batch is, so do these: the rows are those of an item then (flat scores, 32/8 heads,
-// N = 4096, D = 128: 1308, 1247 and with dQ in one part and dK/dV in two 1143; 4 x 16/4, N <= 1000, D = 128: 309, 270, 311).
+// 8000 (2 x 16/4, N <= 1000, D = 64): 138, 111, 110.
+// Where the kernels stand in for those on the supports, which add up an item of a batch in the same order whatever the batch is, so do
+// these: the rows are those of an item then, and the lines lie where a batch of sixteen does not lose what a single item gains.
+// Training, flat scores, causal, us, one part from 16384 rows of an item and two from 4096 against 8192 and 2048 (the kernels before):
+// 8 heads, N <= 1383, D = 128, 1, 4 and 16 items: 107 (137), 283 (335), 510 (474) against 105, 246, 421; 16/4 heads, N <= 2600, D = 64,
+// 1 and 4: 365 (675), 427 (711) against 426, 482; 4 heads, N <= 900, D = 128, 1 and 16: 74 (94), 323 (255) against 73, 228.
 static int parts_of(long long heads, int B, int N, bool split) {
   const long long rows = heads * N;
   if (split) return rows * B >= 256ll * 128 ? 1 : (rows * B >= 256ll * 64 ? 2 : 4);
-  return rows >= 128ll * 128 ? 1 : (rows >= 64ll * 64 ? 2 : 4);
+  return rows >= 64ll * 128 ? 1 : (rows >= 32ll * 64 ? 2 : 4);
 }
 template <int AM> static void launch(const AttnBwdParams& p, int which, bool split, hipStream_t s) {
   if (which & 1) {

@@ -74,7 +74,7 @@ def no_supports():
 @pytest.mark.parametrize("scale", [0.125, 1.0])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,Hq,Hkv,N,D,alpha,causal,lengths", [
-    # rows of an item, queries and keys: from 16384 workgroups of 128 rows, from 4096 of 64, below of 32
+    # rows of an item, queries and keys: from 8192 workgroups of 128 rows, from 2048 of 64, below of 32
     (1, 16, 16, 1027, 64, 1.5, True, [1027]), (1, 16, 4, 1027, 128, 1.5, True, [1027]), (2, 8, 2, 577, 64, 1.5, True, [577, 513]),
     (6, 2, 1, 300, 128, 1.5, True, [300, 1, 31, 32, 129, 257]), (6, 2, 2, 300, 64, 1.333, False, [300, 1, 31, 32, 129, 257]),
     (2, 8, 8, 577, 128, 1.333, False, [577, 127]), (1, 13, 13, 1283, 128, 1.5, False, [1283]), (1, 16, 16, 1030, 64, 2.0, False, [1025]),
