@@ -14,12 +14,10 @@
 // dQ takes two walks, because a row's weights need delta = (sum u dP) / (sum u) first: 10 products of 7.  dK/dV takes one.
 // kSplit: dQ's fp32 weights as two 16-bit operands, for f16 behind a power of two per row, where a problem is short enough for that.
 //
-// Measured, us, the kernels before (128 rows a workgroup, products and weights in turn; 32 rows where kSplit) -> these: D = 64,
-// 4 x 16 heads, N = 4096, causal: dQ 372 -> 365, dK/dV 471 -> 340; not causal: 1473 -> 1150 together; 8 heads, N = 8192, alpha =
-// 1.333: 1298 -> 965.  D = 128: 4 x 16 heads, N = 4096, causal: 788 -> 800, 944 -> 780, not causal: 1540 -> 1410, 1760 -> 1380; few
-// workgroups: 16/4 heads, N = 3000: 206 -> 140, 935 -> 307; 4 of 6000: 381 -> 237, 553 -> 313.  Slower where log and exp fill the vector pipe at
-// one wave a SIMD: D = 128, alpha = 1.333, 4 x 16 heads, N = 4096: 1780 -> 2050, 1930 -> 2080; with few workgroups again faster (4 of 6000: 469 -> 353,
-// 620 -> 415).  kSplit, forward included: one head, N = 3000, D = 64: 144 -> 133, N = 4096: 239 -> 225.
+// Measured, us, the kernels before (128 rows a workgroup, products and weights in turn; 32 rows where kSplit) -> these, dQ and dK/dV: D = 64,
+// 4 x 16 heads, N = 4096, causal: 372 -> 365, 471 -> 340; not causal, alpha = 1.333: 1160 -> 909, 1104 -> 705.  D = 128: the same, causal: 788 -> 800,
+// 944 -> 780, not causal: 1540 -> 1410, 1760 -> 1380, alpha = 1.333: 1793 -> 1794, 1957 -> 1531; few workgroups: 4 of 6000: 381 -> 237,
+// 553 -> 313, alpha = 1.333: 469 -> 304, 618 -> 387.  kSplit, forward included: one head, N = 3000, D = 64: 144 -> 133, N = 4096: 239 -> 225.
 #pragma once
 #include "attn_tile16.h"
 
@@ -36,7 +34,9 @@ template <int AM> __device__ __forceinline__ void weights(float s, float qs, flo
     pr = __builtin_amdgcn_fmed3f(s, 0.f, INFINITY);
     u = s > 0.f ? 1.f : 0.f;
   } else {
-    bwd_prob<AM>(s * qs, c0, pr, u);
+    const float x = __builtin_amdgcn_fmed3f(s, 0.f, INFINITY) * qs;
+    u = fast_exp2(fast_log2(x) * (c0 - 1.f));  // (0 at 0)
+    pr = u * x;
   }
 }
 template <int AM> __device__ __forceinline__ float prob_scale(float qs) { return AM == ATT_15 ? qs * qs : (AM == ATT_2 ? qs : 1.f); }
