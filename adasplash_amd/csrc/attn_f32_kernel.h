@@ -258,11 +258,8 @@ template <int AM> __device__ __forceinline__ void powers(float u, float c0, floa
     e0 = u;
     e1 = u > 0.f ? 1.f : 0.f;
   } else {
-    const bool pos = u > 0.f;
-    const float x = pos ? u : 1.f;
-    const float e = fast_exp2(fast_log2(x) * c0);
-    e0 = pos ? e : 0.f;
-    e1 = pos ? e * fast_rcp(x) : 0.f;
+    e1 = fast_exp2(fast_log2(u) * (c0 - 1.f));  // (0 at 0)
+    e0 = e1 * u;
   }
 }
 // Newton step on (sum u^c0)^(1/c0) - 1: convex and decreasing in the threshold, nearly linear where the support is settled
