@@ -21,6 +21,12 @@
 // workgroup to walks: Newton steps on (sum u^c0)^(1/c0) - 1 from the bound the lists gave, until a step is below 2e-5, and
 // an output walk.
 //
+// One such workgroup among hundreds takes the whole launch two to three times as long, and with scores of unit spread it came about by
+// chance (a row of 38 members, 14 of them in one wave's list, which 19 scores joined).  Hence the solves come sooner where a row has
+// many members (sync(): a solve costs about 1.5 us, so none is added for fewer), and a wave drops what lies below the bound before it
+// gives up.  us, q of spread 1: 2 x 8 heads, N = 1500 and 375: 126 -> 66 (65 where no list overflows); N = 2048: 187 -> 101, D = 128, 16/4 heads:
+// 288 -> 148; 4 heads, N = 8192: 776 -> 285; bf16, 2 heads, N = 4096, D = 128: 135 -> 75.  Spread 3, where nothing overflows: 82.8 -> 83.2.
+//
 // Measured (fp32, causal, forward and backward; kernels on 128 rows a workgroup -> these): 2 x 8 heads, N = 1500 and 375,
 // D = 64: 1140 -> 287 us (forward 65, dQ 128, dK/dV 108, where one walk of the longest rows is 10 us of matrix work a
 // product); flat scores 1139 -> 380; 4 x 16/4 heads, N = 1024, D = 128: 2885 -> 927.  Eight waves to the 32 rows, one
@@ -290,7 +296,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   __shared__ float t_lds[kRows], est_lds[kRows];
   __shared__ uint8_t n_lds[kWaves][2][kRows];
   __shared__ float red[2][kWaves][3][kRows];
-  __shared__ uint32_t over_flag;
+  __shared__ uint32_t over_flag, sync_lds[kWaves];  // sync_lds: how much nearer the next solve has to be
   float* const list_s = reinterpret_cast<float*>(smem + kRing);                                   // [wave][slot][row]
   uint16_t* const list_k = reinterpret_cast<uint16_t*>(smem + kRing + kWaves * kCap * kRows * 4);  // likewise
 
@@ -358,7 +364,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int srow = wave * 8 + (lane >> 3), sj = lane & 7;
   float sv[16];  // the lane's share of the row's listed scores, relative to their maximum, in z units: kK per wave
   uint32_t sslot[16];
-  float s_max = 0.f, s_tau = 0.f;
+  float s_max = 0.f, s_tau = 0.f, s_members = 0.f;  // s_members: entries above the bound, where a wave has more than 8 of any of the rows
   // kK: the lane's entries per wave's list, enough for the longest of the eight rows' lists
   auto solve_k = [&](auto kc, bool last) {
     constexpr int kK = decltype(kc)::value;
@@ -401,6 +407,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (go) s_tau = fminf(s_tau + step, 0.f);
       go = go && step > (last ? 1e-7f : 1e-3f);
     }
+    s_members = 0.f;
+    if constexpr (kK > 1) {
+      if (!last) {
+#pragma unroll
+        for (int i = 0; i < 4 * kK; ++i) s_members += sv[i] > s_tau ? 1.f : 0.f;
+        s_members = sum8(s_members);
+      }
+    }
   };
   auto solve = [&](bool last) {
     int most = 0;
@@ -422,15 +436,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (over) over_flag = 1u;
       __syncthreads();
       solve(step_no == n_steps);
-      if (step_no == 1 && n_steps > 1) {
-        // More than half of the first 128 keys in a row's support so far: its list is about to overflow.  The threshold of
-        // a row whose other keys are like these is where the walks then start (a Newton step from beyond tau ends below it).
-        float members = 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) members += sv[i] > s_tau ? 1.f : 0.f;
-        if (__builtin_amdgcn_ballot_w64(sum8(members) > 64.f) != 0ull) {
-          const int row = m0 + srow, keys = p.causal ? (row < L - 1 ? row + 1 : L) : L;
-          const float ratio = (float)keys * (1.f / 128.f);
+      int nearer = 0;
+      if (step_no < n_steps && __builtin_amdgcn_ballot_w64(s_members > 28.f) != 0ull) {
+        const auto any_above = [&](float m) -> int { return __builtin_amdgcn_ballot_w64(s_members > m) != 0ull ? 1 : 0; };
+        // (beyond 90 a list overflows anyway)
+        nearer = any_above(90.f) ? 0 : any_above(step_no <= 2 ? 48.f : 28.f) + any_above(step_no <= 2 ? 56.f : 40.f) + any_above(56.f);
+        // A list has overflowed, or more than half of the first 128 keys are in a row's support so far and it is about to.  The
+        // threshold of a row whose other keys are like these is where the walks then start (a Newton step from beyond tau ends
+        // below it).
+        if (step_no == 1 ? any_above(64.f) != 0 : (over_flag != 0u && step_no > 2)) {
+          const int row = m0 + srow, keys = p.causal ? (row < L - 1 ? row + 1 : L) : L, seen = step_no * (kWaves * kRows);
+          const float ratio = (float)keys / (float)seen;
           float e = s_tau;
           for (int it = 0; it < 6; ++it) {
             float s0 = 0.f, s1 = 0.f;
@@ -446,9 +462,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const float step = norm_step<AM>(s0, s1, c0);
             if (s0 > 0.f && s1 > 0.f) e += step;
           }
-          if (sj == 0 && keys > 128 && e < 0.f && e > s_tau) est_lds[srow] = s_max + e * inv_qs;
+          if (sj == 0 && keys > seen && e < 0.f && e > s_tau) est_lds[srow] = s_max + e * inv_qs;
         }
       }
+      if (lane == 0) sync_lds[wave] = (uint32_t)nearer;
       if (sj == 0) {
         // (the margin covers the rounding of the difference and of the product back to raw units)
         t_lds[srow] = s_max > -INFINITY ? (s_max + (s_tau - 1e-6f) * inv_qs) - 4e-7f * fabsf(s_max) : -INFINITY;
@@ -458,9 +475,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       t_raw = fmaxf(t_raw, t_lds[lq]);
       return given_up;
     };
-    // only where a wave's list of a row is more than half full; entries below the bound do no harm otherwise
-    auto compact = [&]() {
-      if (__builtin_amdgcn_ballot_w64(n_mine + __shfl_xor(n_mine, 32, 64) > kCap / 2) == 0ull) return;
+    // where a wave's list of a row is more than half full, or about to overflow; entries below the bound do no harm otherwise
+    auto compact = [&](int more_than) {
+      if (__builtin_amdgcn_ballot_w64(n_mine + __shfl_xor(n_mine, 32, 64) > more_than) == 0ull) return;
       int kept = 0;
       for (int e0 = 0; __builtin_amdgcn_ballot_w64(e0 < n_mine) != 0ull; e0 += 8) {
         float s[8];
@@ -493,10 +510,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
       for (int i = 0; i < 16; ++i) c += s[i] > t_raw ? 1 : 0;
       c = live ? c : 0;
-      const int need = n_mine + c;
-      if (__builtin_amdgcn_ballot_w64(need + __shfl_xor(need, 32, 64) > kCap) != 0ull) {
-        over = true;  // uniform over the wave
-        return;
+      auto too_many = [&]() -> bool {
+        const int need = n_mine + c;
+        return __builtin_amdgcn_ballot_w64(need + __shfl_xor(need, 32, 64) > kCap) != 0ull;
+      };
+      if (too_many()) {
+        compact(0);  // (up to half a list may lie below the bound)
+        if (too_many()) {
+          over = true;  // uniform over the wave
+          return;
+        }
       }
       const int jb = blk * kRows + 4 * lh;
 #pragma unroll
@@ -520,8 +543,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           break;
         }
         if (step_no == n_steps) break;
-        compact();
-        next_sync = step_no * 2;
+        compact(kCap / 2);
+        // Between two solves about as many scores join a list as it has members; where a row has so many that it would overflow now
+        // and then, the next solve comes sooner.  (sync_lds is written behind the next solve's first barrier at the earliest.)
+        const uint32_t nearer = __builtin_elementwise_max(__builtin_elementwise_max(sync_lds[0], sync_lds[1]), __builtin_elementwise_max(sync_lds[2], sync_lds[3]));
+        const int gap = step_no >> nearer;
+        next_sync = step_no + (gap > 0 ? gap : 1);
       }
     }
     ring.drain();

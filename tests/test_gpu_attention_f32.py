@@ -236,3 +236,26 @@ def test_16bit_gradients_on_long_sequences(N, Hq, Hkv, D, alpha, causal, dtype, 
     want += list(exact.dense_entmax_attention_grads(q, k, v, dout, alpha, causal, varlen))
     for name, a, w in zip(("out", "dq", "dk", "dv"), got, want):
         assert max_err(a, w) < (2e-2 if name == "out" else 4e-2 * max(1.0, scale)), name
+
+
+@pytest.mark.parametrize("alpha,dtype", [(1.5, torch.float32), (1.333, torch.float32), (1.125, torch.float32), (1.5, torch.bfloat16)])
+@pytest.mark.parametrize("members", [8, 20, 26, 31, 32, 33, 80, 97])
+def test_lists_that_fill_up_between_two_solves(members, alpha, dtype):
+    """Late keys of one wave (blocks 16, 20, 24, 28 of 32 keys each: the first wave's between the solves after 4 and 8 steps), so many
+    of them above all others that the wave's list of every row fits, just fits, or overflows; the keys in front of them
+    leave entries that then lie below the bound.  fp32: as everywhere here; bf16: 2^-8 of the result, its rounding and the weights'."""
+    g = torch.Generator().manual_seed(members)
+    N, D = 1031, 64
+    axis = torch.zeros(D)
+    axis[0] = 1.0
+    q = (0.3 * torch.randn(1, 1, N, D, generator=g) + 4.0 * axis).to(dtype)
+    k = torch.randn(1, 1, N, D, generator=g)
+    k[..., 0] = 0.2 * torch.randn(1, 1, N, generator=g)
+    late = [32 * (16 + 4 * (i % 4)) + i // 4 for i in range(members)]
+    k[0, 0, late, 0] = 1.0 + 0.05 * torch.randn(members, generator=g)
+    k = k.to(dtype)
+    v = torch.randn(1, 1, N, D, generator=g).to(dtype)
+    vl = torch.tensor([N], dtype=torch.int32)
+    want = exact.dense_entmax_attention(q, k, v, alpha, False, vl)
+    got = A.adasplash_v1(*(t.to(DEV) for t in (q, k, v)), alpha=alpha, is_causal=False, varlen=vl.to(DEV)).double().cpu()
+    assert (got - want).norm() <= (2e-6 if dtype == torch.float32 else 2.0 ** -8) * want.norm()
