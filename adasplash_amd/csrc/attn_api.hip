@@ -62,6 +62,10 @@ static const attn_fwd_fn kFwdTable[3][5][2] = {ADSP_FWD_TAG(f32), ADSP_FWD_TAG(b
 static const attn_bwd_fn kBwdTable[3][5] = {
     {launch_attn_bwd_f32_d16, launch_attn_bwd_f32_d32, launch_attn_bwd_f32_d64, launch_attn_bwd_f32_d128, launch_attn_bwd_f32_d256},
     ADSP_BWD_TAG16(bf16), ADSP_BWD_TAG16(f16)};
+// An alpha whose 1 / (alpha - 1) is 1 in fp32 is 2 to the kernels: the generic ones raise u = 0 to the power 1 / (alpha - 1) - 1.
+static int alpha_mode(double alpha) {
+  return alpha == 1.5 ? ATT_15 : (alpha == 2.0 || (float)(1.0 / (alpha - 1.0)) == 1.f ? ATT_2 : ATT_GEN);
+}
 static int head_dim_slot(int D) { return D == 16 ? 0 : (D == 32 ? 1 : (D == 64 ? 2 : (D == 128 ? 3 : (D == 256 ? 4 : -1)))); }
 // dQ and / or dK and dV of whatever is not left to the kernels on the supports
 static int launch_bwd_dense(const AttnBwdParams& p, int D, int dtype, int am, int which, hipStream_t s) {
@@ -489,7 +493,7 @@ static int attn_common(const void* q, const void* k, const void* v, void* out, f
   // 16-bit types.  The second and later steps run on the candidate lists of the list-carrying instance when they fit,
   // without another K walk.  Behind the sparse-support kernel (which converges fully) the dense kernel serves the
   // row blocks whose supports did not fit that kernel's lists, longer than its own: there it walks `niter` steps.
-  const int am = alpha == 1.5 ? ATT_15 : (alpha == 2.0 ? ATT_2 : ATT_GEN);
+  const int am = alpha_mode(alpha);
   const FwdWorkspace w = dtype == ADSP_F32 ? FwdWorkspace{} : fwd_workspace(B, Hq, Hkv, N, D, dtype);
   // Sparse-support kernel first (16-bit types, alpha 1.5 / 2 or any other in [1.125, 2): below that its solver on the
   // lists would need too many rounds; either entry point, no tile statistics asked for): it serves the row blocks
@@ -853,7 +857,7 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
   p.fwd_lens = nullptr;
   p.fwd_tshift = nullptr;
   p.fwd_streams = nullptr;
-  const int am = alpha == 1.5 ? ATT_15 : (alpha == 2.0 ? ATT_2 : ATT_GEN);
+  const int am = alpha_mode(alpha);
   bool sparse = false;
   BwdWorkspace w = {};
 

@@ -134,3 +134,13 @@ def test_gradients_leave_out_what_a_causal_mask_hides(no_supports):
     v[:, :, 150:] = float("inf")
     dq = run(q, k, v, dout, varlen, 1.5, True)[1]
     assert torch.isfinite(dq[:, :, :150]).all() and torch.equal(dq[:, :, :150], want[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,scale", [(300, 1.0), (2309, 0.125)])
+def test_an_alpha_that_is_two_in_single_precision(N, scale, dtype):
+    """1 / (alpha - 1) rounds to 1 in fp32, and zero to the power of zero is no weight: the bits of alpha = 2."""
+    q, k, v, dout, varlen = problem(1, 2, 2, N, 64, dtype, scale, [N - 3])
+    want = run(q, k, v, dout, varlen, 2.0, False)
+    got = run(q, k, v, dout, varlen, 2.0 - 1e-9, False)
+    assert all(torch.isfinite(a).all() and torch.equal(a, w) for a, w in zip(got, want))
