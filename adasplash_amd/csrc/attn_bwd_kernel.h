@@ -34,11 +34,9 @@ template <int AM> __device__ __forceinline__ void bwd_prob(float r, float c0, fl
     pr = __builtin_amdgcn_fmed3f(r, 0.f, INFINITY);
     u = r > 0.f ? 1.f : 0.f;
   } else {
-    const bool pos = r > 0.f;
-    const float rr = pos ? r : 1.f;
-    const float e = fast_exp2(fast_log2(rr) * c0);
-    pr = pos ? e : 0.f;
-    u = pos ? e * fast_rcp(rr) : 0.f;
+    const float x = __builtin_amdgcn_fmed3f(r, 0.f, INFINITY);
+    u = fast_exp2(fast_log2(x) * (c0 - 1.f));  // (0 at 0)
+    pr = u * x;
   }
 }
 
