@@ -180,9 +180,12 @@ __device__ __forceinline__ bool xcd_block_map(int units, int blocks, int group, 
   // returns at once.  So the heads change places behind each round, or the blocks of one long sequence among short ones all
   // fall to the same few CUs, every second one of a set of two heads.  fp32, 2 x 8 heads, N = 1500 and 375, D = 64, forward and
   // backward: 292 -> 244 us; q of spread 3: 280 -> 228.  (Places changed from block to block fall to half of the CUs as well.)
-  const int turn = gsize > 1 ? (int)((long long)blk * span / 32 % span) : 0;
-  int r = s % span + turn;
-  r = r < span ? r : r - span;
+  int r = s % span;
+  if (gsize > 1) {
+    asm volatile("; several heads");  // (a branch: the divisions are a tenth of a microsecond of the smallest calls)
+    r += (s - r) / 32 % span;
+    r = r < span ? r : r - span;
+  }
   unit = (set * g + r / group) * 8 + x;
   member = r % group;
   return true;
