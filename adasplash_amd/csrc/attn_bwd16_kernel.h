@@ -41,6 +41,9 @@ template <int AM> __device__ __forceinline__ void weights(float s, float qs, flo
 }
 template <int AM> __device__ __forceinline__ float prob_scale(float qs) { return AM == ATT_15 ? qs * qs : (AM == ATT_2 ? qs : 1.f); }
 template <int AM> __device__ __forceinline__ float u_scale(float qs) { return AM == ATT_15 ? qs : 1.f; }
+// Whether u (dP - delta) takes u_scale in front of a product instead of behind it: raw u goes up to 1 / qs (16 at D = 64, 22.6 at
+// D = 128), and f16 ends at 65504, which gradients of a few hundred reached then.  (bf16 has fp32's range.)
+template <typename T, int AM> constexpr bool kScaleFirst = AM == ATT_15 && !elem_traits<T>::kIsBf16;
 
 // ---------------------------------------------------------------------------------------------------------
 // dQ
@@ -238,6 +241,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     if constexpr (kScaled) {
       x0 = __builtin_amdgcn_ldexpf(x0, up);
       x1 = __builtin_amdgcn_ldexpf(x1, up);
+    } else if constexpr (kScaleFirst<T, AM>) {
+      x0 *= qs;
+      x1 *= qs;
     }
     w[0][i] = pack2<T>(x0, x1);
     if constexpr (kSplit) w[1][i] = pack2<T>(x0 - unpack_lo<T>(w[0][i]), x1 - unpack_hi<T>(w[0][i]));
@@ -282,7 +288,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
             });
       });
   __syncthreads();  // the tiles become the sums' scratch
-  float scale = p.sm_scale * u_scale<AM>(qs);
+  float scale = p.sm_scale;
+  if constexpr (kScaled || !kScaleFirst<T, AM>) scale *= u_scale<AM>(qs);
   if constexpr (kScaled) scale = __builtin_amdgcn_ldexpf(scale, -up);
   if constexpr (P == 1) BwdTiles<T, D>::store_rows(o, scale, smem + wave * 32 * kRow, dq, wave_row0, N, lane);
   else store_parts<T, D, P>(o, scale, smem, dq, m0, N, wave, lane);
@@ -398,7 +405,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     weights<AM>(s[2 * i], qs, p.c0, p0, u0);
     weights<AM>(s[2 * i + 1], qs, p.c0, p1, u1);
     wp[i] = pack2<T>(p0 * z[2 * i], p1 * z[2 * i + 1]);
-    wx[i] = pack2<T>(u0 * d[2 * i], u1 * d[2 * i + 1]);
+    float x0 = u0 * d[2 * i], x1 = u1 * d[2 * i + 1];
+    if constexpr (kScaleFirst<T, AM>) {
+      x0 *= qs;
+      x1 *= qs;
+    }
+    wx[i] = pack2<T>(x0, x1);
   };
   auto one = [&](int blk, const float* sc, int q0) {
     f32x16 s, d, z;
@@ -481,7 +493,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     }
   }
   __syncthreads();
-  const float scale = p.sm_scale * u_scale<AM>(qs);
+  const float scale = kScaleFirst<T, AM> ? p.sm_scale : p.sm_scale * u_scale<AM>(qs);
   if constexpr (P == 1) {
     unsigned char* const stage = smem + wave * 32 * kRow;
     BwdTiles<T, D>::store_rows(ov, 1.f, stage, dv, wave_key0, N, lane);

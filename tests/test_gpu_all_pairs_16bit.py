@@ -127,6 +127,20 @@ def test_forward_on_all_pairs(no_supports, N, scale, Hq, Hkv, D, alpha, causal, 
         check(run(q, k, v, dout, varlen, alpha, causal, train), q, k, v, dout, varlen, alpha, causal, list(range(4)))
 
 
+@pytest.mark.parametrize("supports", [True, False])
+@pytest.mark.parametrize("Hq,Hkv,D", [(2, 2, 64), (2, 1, 128)])
+@pytest.mark.parametrize("dout_scale", [1e-2, 200.0, 300.0, 1000.0])
+def test_f16_gradients_of_a_scaled_loss(request, dout_scale, Hq, Hkv, D, supports):
+    """Upstream gradients as a loss scaler makes them: of a few hundred, u (dP - delta) is within f16's range only as long as u is
+    at most 1 (it reaches some 2e4 for a spread of 1000).  The short route (dQ's weights in two parts), and the other one (one part)."""
+    if not supports:
+        request.getfixturevalue("no_supports")
+    q, k, v, dout, varlen = problem(1, Hq, Hkv, 512, D, torch.float16, 1.0, [512])
+    dout = (dout_scale * dout.float()).half()
+    got = run(q, k, v, dout, varlen, 1.5, True)
+    check(got, q, k, v, dout, varlen, 1.5, True, [0])
+
+
 def test_gradients_leave_out_what_a_causal_mask_hides(no_supports):
     """Rows of K and V that later queries alone see may be infinite for the earlier ones."""
     q, k, v, dout, varlen = problem(1, 2, 2, 160, 64, torch.bfloat16, 1.0, [160])
