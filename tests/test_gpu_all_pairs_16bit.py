@@ -141,6 +141,19 @@ def test_f16_gradients_of_a_scaled_loss(request, dout_scale, Hq, Hkv, D, support
     check(got, q, k, v, dout, varlen, 1.5, True, [0])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("spread", [0.5e-3, 1e-3, 2e-3, 4e-3])
+@pytest.mark.parametrize("N,D,causal", [(512, 128, False), (1024, 64, True), (2048, 64, False), (2048, 128, False)])
+def test_resident_scores_that_are_nearly_equal(N, D, causal, spread, dtype):
+    """alpha = 2: a weight is about 1 / N here, and so is the border's place: a threshold off by a few 1e-4 loses some of the support."""
+    q, k, v, dout, varlen = problem(1, 1, 1, N, D, dtype, spread ** 0.5, [N])
+    k = (spread ** 0.5 * k.float()).to(dtype)
+    got = run(q, k, v, dout, varlen, 2.0, causal, train=False)
+    check(got, q, k, v, dout, varlen, 2.0, causal, [0])
+    assert _lib.load().adsp_attn_bwd_reads_bmask(1, 1, 1, N, D, _lib.dtype_code(q), 2.0, int(causal)) == 0
+    check(run(q, k, v, dout, varlen, 2.0, causal), q, k, v, dout, varlen, 2.0, causal, [0])
+
+
 def test_gradients_leave_out_what_a_causal_mask_hides(no_supports):
     """Rows of K and V that later queries alone see may be infinite for the earlier ones."""
     q, k, v, dout, varlen = problem(1, 2, 2, 160, 64, torch.bfloat16, 1.0, [160])
