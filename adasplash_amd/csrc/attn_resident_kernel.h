@@ -11,9 +11,11 @@
 // of two 16-bit values, which the idle matrix pipe does for nothing (relative error for bf16: 2.3e-3 -> 1.7e-3, that of the rounded result).
 //
 // Newton's steps are taken on (sum u^c0)^(1/c0) - 1, which is convex and nearly linear, from the maximum less 1, where u is at most 1.
-// They end with one of up to 4e-4, behind which u's relative error is below 1e-6 (alpha = 1.5 and 1.333, 64 to 2048 keys, scores of spread 1e-4 to 10).
-// alpha = 2: the sum is piecewise linear and a step leaves what the keys that it puts off the support had, so it ends at 2e-3 of the mean
-// weight, which is itself 5e-4 where 2048 scores are nearly equal.
+// They end with one of up to 4e-4, behind which the weights' relative error is below 6e-6 (alpha = 1.5 and below, 64 to 2048 keys, scores of
+// spread 1e-4 to 10).  Towards alpha = 2 the sum becomes piecewise linear, a step leaves what the keys that it puts off the support had, and
+// u is itself some 5e-4 where 2048 scores are nearly equal; so a step is also asked to be small beside the mean of u: 2e-3 of it at
+// alpha = 2, 5e-3 at a generic alpha, which adds nothing up to 1.333 and a quarter of a step at 1.9 (the weights' error at 1.75, 1.9 and 1.99 without it:
+// 2.2e-4, 9e-4, 1.8e-2; with it at most 2.7e-5).
 //
 // Measured, us, the kernels on the supports or on lists -> this one, q of spread 1, 3 and 1/8: 16 x 12 heads, N <= 500, D = 64: 86 -> 35,
 // 64 -> 33, 147 -> 34; 32 x 16 heads, N <= 512, D = 128: 256 -> 122, 172 -> 125, 394 -> 127.  A first solver
@@ -188,7 +190,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4, 4))) 
       buf ^= 1;
       const float step = f32path::norm_step<AM>(s0, s1, c0);
       t = fmaxf(t + step, t_min);
-      const float near = AM == ATT_2 ? fmaxf(2e-3f * s0 * fast_rcp(s1), fmaxf(2e-6f, 1.2e-7f * fabsf(t))) : 4e-4f;
+      float near = 4e-4f;
+      if constexpr (AM != ATT_15) {
+        const float beside = (AM == ATT_2 ? 2e-3f : 5e-3f) * s0 * fast_rcp(s1), least = fmaxf(2e-6f, 1.2e-7f * fabsf(t));
+        near = fmaxf(AM == ATT_2 ? beside : fminf(beside, 4e-4f), least);
+      }
       if (__builtin_amdgcn_ballot_w64(fabsf(step) > near) == 0ull) break;  // (the same sums in every wave)
     }
     if (live && wave == 0 && lh == 0 && p.taus) p.taus[q_row0 + qi] = t;

@@ -154,6 +154,18 @@ def test_resident_scores_that_are_nearly_equal(N, D, causal, spread, dtype):
     check(run(q, k, v, dout, varlen, 2.0, causal), q, k, v, dout, varlen, 2.0, causal, [0])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("spread", [1e-3, 2e-3, 4e-3])
+@pytest.mark.parametrize("N,D,causal", [(512, 128, False), (1024, 64, True), (2048, 64, False), (2048, 128, False)])
+@pytest.mark.parametrize("alpha", [1.9, 1.99])
+def test_resident_scores_that_are_nearly_equal_close_to_two(alpha, N, D, causal, spread, dtype):
+    """The same for a generic alpha, whose sum is nearly piecewise linear.  (dQ and dK have u^(2 - alpha) of the border's keys: its
+    rounding in fp32 counts as at alpha = 2; they are not compared here.)"""
+    q, k, v, dout, varlen = problem(1, 1, 1, N, D, dtype, spread ** 0.5, [N])
+    k = (spread ** 0.5 * k.float()).to(dtype)
+    check(run(q, k, v, dout, varlen, alpha, causal, train=False), q, k, v, dout, varlen, alpha, causal, [0])
+
+
 def test_gradients_leave_out_what_a_causal_mask_hides(no_supports):
     """Rows of K and V that later queries alone see may be infinite for the earlier ones."""
     q, k, v, dout, varlen = problem(1, 2, 2, 160, 64, torch.bfloat16, 1.0, [160])
