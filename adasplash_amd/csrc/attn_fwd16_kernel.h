@@ -224,19 +224,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       s0 *= qs;
     }
   };
+  // whether Newton's step stays in fp32 (it multiplies s0 by up to itself): not with a score far above the threshold, which an
+  // unsampled key may have; the maximum less 1 is the next threshold then
+  auto in_range = [&]() -> bool { return s0 > 0.f && s0 < 1e18f && s1 > 0.f && s1 < 1e18f; };
   if (!all_sampled) {
     // a step on every second tile, where that is much more than the sample
     const int half = whole * 32 / kTR / 2;
     if (half * kTR >= 2 * kSample) {
       sums_walk(1, 2, half * 2);
       const float ratio = (float)(lim + 1) / (float)(half * kTR) * (AM == ATT_2 ? 0.9f : 1.f);
-      if (s0 > 0.f && s1 > 0.f) t += f32path::norm_step<AM>(s0 * ratio, s1 * ratio, c0);
+      if (in_range()) t += fmaxf(mx * qs - 1.f, f32path::norm_step<AM>(s0 * ratio, s1 * ratio, c0));
+      else t += fmaxf(mx * qs - 1.f, 0.f);
     }
     for (int it = 0; it < 32; ++it) {
       sums_walk(0, 1, nt);
-      // never below the row maximum less 1, where the sums of a score far above the threshold would also leave fp32
+      // never below the row maximum less 1
       float step = mx * qs - 1.f, near = 0.f;
-      if (s0 > 0.f && s0 < 1e30f && s1 > 0.f && s1 < 1e30f) {
+      if (in_range()) {
         step = fmaxf(step, f32path::norm_step<AM>(s0, s1, c0));
         near = kNear<T, AM> * s0 * fast_rcp(s1);
       }

@@ -127,6 +127,17 @@ def test_forward_on_all_pairs(no_supports, N, scale, Hq, Hkv, D, alpha, causal, 
         check(run(q, k, v, dout, varlen, alpha, causal, train), q, k, v, dout, varlen, alpha, causal, list(range(4)))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("size", [40.0, 160.0])
+def test_one_key_far_above_a_sampled_threshold(no_supports, size, D, dtype):
+    """Key 200 is in none of the blocks that the first threshold is sampled from, but in the tiles of the step on half of them: its
+    score, 25600 (D = 64) above in units of the threshold for size 160, to the power 8 and once more is beyond fp32."""
+    q, k, v, dout, varlen = problem(1, 2, 2, 1152, D, dtype, 1.0, [1152])
+    q[:], k[:, :, 200] = size, size
+    check(run(q, k, v, dout, varlen, 1.125, False, train=False), q, k, v, dout, varlen, 1.125, False, [0])
+
+
 @pytest.mark.parametrize("supports", [True, False])
 @pytest.mark.parametrize("Hq,Hkv,D", [(2, 2, 64), (2, 1, 128)])
 @pytest.mark.parametrize("dout_scale", [1e-2, 200.0, 300.0, 1000.0])
