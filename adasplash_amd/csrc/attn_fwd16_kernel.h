@@ -296,13 +296,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int n = 4 * (g % G) + k, s = n / TL::kDB, db = n % TL::kDB;
     o[db] = mfma_16bit<T>(a, u32x4{w[4 * s], w[4 * s + 1], w[4 * s + 2], w[4 * s + 3]}, o[db]);
   };
-  auto mark = [&](float before, int k0) {
-    if (bmask && __builtin_amdgcn_ballot_w64(zacc[0] > before) != 0ull && lane == 0) atomicOr(&mask_lds[k0 >> 11], 1u << ((k0 >> 6) & 31));
+  // (from the weights themselves: one below 6e-8 of the row's sum does not show in it)
+  auto any_of = [](const uint32_t (&w)[8]) -> uint32_t { return ((w[0] | w[1]) | (w[2] | w[3])) | ((w[4] | w[5]) | (w[6] | w[7])); };
+  auto mark = [&](uint32_t weights, int k0) {
+    if (bmask && __builtin_amdgcn_ballot_w64(weights != 0u) != 0ull && lane == 0) atomicOr(&mask_lds[k0 >> 11], 1u << ((k0 >> 6) & 31));
   };
   walk(
       0, 1, nt, true,
       [&](int blk, int k0) {
-        const float before = zacc[0];
         f32x16 s = zero;
         stream<G, 2>([&](int g, u32x4(&a)[4]) { tl.rows(0, blk, g, a); }, [&](int g, int k, const u32x4& a) { mul(g, k, a, s); });
         if (k0 + 31 > lim_all) hide(k0, s);
@@ -312,12 +313,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int i = 0; i < 4; ++i) add_weights(w, i);
         stream<G, 2>([&](int g, u32x4(&a)[4]) { tl.columns(1, blk, g, a); }, [&](int g, int k, const u32x4& a) { mul_v(g, k, a, w); });
-        mark(before, k0);
+        mark(any_of(w), k0);
       },
       [&](int blk, int k0) {
-        const float before = zacc[0];
         f32x16 x0 = zero, x1 = zero;
-        uint32_t w0[8], w1[8];
+        uint32_t w0[8], w1[8], any = 0u;
         constexpr int kPer = 2 / G;
         stream<4 * G, kAhead>(
             [&](int g, u32x4(&a)[4]) {
@@ -340,9 +340,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 mul_v(g, k, a, w1);  // (nothing is left for the vector pipe)
                 if (n4 < 4) add_weights(w0, n4);
                 if (n4 >= 4 * G - 4) add_weights(w1, n4 - (4 * G - 4));
+                if (n4 == 0) any = any_of(w0) | any_of(w1);
               }
             });
-        mark(before, k0);
+        mark(any, k0);
       });
   if constexpr (kTaus) {
     q0 = total(q0);

@@ -12,7 +12,7 @@ import pytest
 import torch
 
 import adasplash_amd as A
-from adasplash_amd import _lib
+from adasplash_amd import _attention, _lib
 from oracle import exact
 from tests.gpu_util import DEV
 
@@ -136,6 +136,24 @@ def test_one_key_far_above_a_sampled_threshold(no_supports, size, D, dtype):
     q, k, v, dout, varlen = problem(1, 2, 2, 1152, D, dtype, 1.0, [1152])
     q[:], k[:, :, 200] = size, size
     check(run(q, k, v, dout, varlen, 1.125, False, train=False), q, k, v, dout, varlen, 1.125, False, [0])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("far", [640, 1099])
+def test_tile_mask_has_weights_too_small_for_the_sum(no_supports, far, D):
+    """Key 0 has nearly all of the weight, key ``far`` 1e-8 of it: adding that changes nothing in fp32, but the key is a member."""
+    q, k = torch.zeros(1, 1, 1100, D), torch.zeros(1, 1, 1100, D)
+    root = D ** 0.5
+    q[..., :2] = 1.0
+    k[..., 0] = -64.0
+    k[:, :, 0] = 0.0
+    k[:, :, far, 0], k[:, :, far, 1] = -2 * root, 2e-4 * root if D == 64 else 0.0  # 1e-4 above the threshold (22.627 rounds to 22.625)
+    v = torch.randn(1, 1, 1100, D, generator=torch.Generator().manual_seed(1))
+    q, k, v = (t.to(DEV, torch.bfloat16) for t in (q, k, v))
+    bmask = _attention.launch_forward(q, k, v, version=1, alpha=1.5, is_causal=False, niter=10, varlen=None)[2].cpu()
+    want = torch.zeros_like(bmask)
+    want[:] = 1 | 1 << (far // 64)  # (one word a row block)
+    assert torch.equal(bmask, want)
 
 
 @pytest.mark.parametrize("supports", [True, False])
