@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   const int rg = wave % kRG, part = wave / kRG;
   const int N = p.N, group = p.Hq / p.Hkv, n_blk = (N + kRows - 1) / kRows;
   int bkv, mi, hg;
-  if (!xcd_block_map(p.B * p.Hkv, n_blk, group, p.causal != 0, 2ll * N * kRow, bkv, mi, hg)) return;
+  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_blk, group, p.causal != 0, 2ll * N * kRow, bkv, mi, hg)) return;
   const int b = bkv / p.Hkv, kvh = bkv % p.Hkv, h = kvh * group + hg, bh = b * p.Hq + h;
   const int m0 = (n_blk - 1 - mi) * kRows, mblk = m0 / kMaskRows;
   if (!left.takes((size_t)bh * p.n_mblk + mblk)) return;
@@ -312,7 +312,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   const int rg = wave % kRG, part = wave / kRG;
   const int N = p.N, group = p.Hq / p.Hkv, n_blk = (N + kRows - 1) / kRows;
   int bkv, nblk, member_unused;
-  if (!xcd_block_map(p.B * p.Hkv, n_blk, 1, p.causal != 0, 2ll * group * N * kRow, bkv, nblk, member_unused)) return;
+  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_blk, 1, p.causal != 0, 2ll * group * N * kRow, bkv, nblk, member_unused)) return;
   const int b = bkv / p.Hkv, kvh = bkv % p.Hkv, n0 = nblk * kRows;
   if (!left.takes((size_t)bkv * p.n_mblk + n0 / kMaskRows)) return;
   const int L = bwd_seq_len(p, b);

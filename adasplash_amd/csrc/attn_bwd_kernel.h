@@ -289,7 +289,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((dq_waves<T
   const int n_blk = (N + kBwdRows - 1) / kBwdRows;
   const int group = p.Hq / p.Hkv;
   int bkv, mi, hg;
-  if (!xcd_block_map(p.B * p.Hkv, n_blk, group, p.causal != 0, 2ll * N * D * G::kEB, bkv, mi, hg)) return;  // (K and V of a head)
+  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_blk, group, p.causal != 0, 2ll * N * D * G::kEB, bkv, mi, hg)) return;  // (K and V of a head)
   const int mblk = n_blk - 1 - mi;  // the longest causal rows first; a group's heads side by side
   const int b = bkv / p.Hkv, kvh = bkv % p.Hkv;
   const int h = kvh * group + hg;
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((BwdTiles<T
   int bkv, nblk;  // early key blocks have the most causal work and come first
   int member_unused;
   // (the key blocks of a K/V head stream q and dout of all its query heads)
-  if (!xcd_block_map(p.B * p.Hkv, (N + kBwdRows - 1) / kBwdRows, 1, p.causal != 0, 2ll * (p.Hq / p.Hkv) * N * D * G::kEB, bkv, nblk, member_unused)) return;
+  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, (N + kBwdRows - 1) / kBwdRows, 1, p.causal != 0, 2ll * (p.Hq / p.Hkv) * N * D * G::kEB, bkv, nblk, member_unused)) return;
   const int b = bkv / p.Hkv, kvh = bkv % p.Hkv;
   const int group = p.Hq / p.Hkv;
   // behind the sparse-support dK/dV kernel: only the key blocks it flagged (all of them when it stepped aside)

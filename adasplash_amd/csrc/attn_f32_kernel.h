@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
   const int N = p.N, group = p.Hq / p.Hkv, n_rblk = (N + kRows - 1) / kRows;
   int bkv, mi, hg;
-  if (!xcd_block_map(p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
+  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
   const int b = bkv / p.Hkv, kvh = bkv % p.Hkv, h = kvh * group + hg;
   const int m0 = (n_rblk - 1 - mi) * kRows;
   int L = N;
@@ -750,7 +750,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
   const int N = p.N, group = p.Hq / p.Hkv, n_rblk = (N + kRows - 1) / kRows;
   int bkv, mi, hg;
-  if (!xcd_block_map(p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
+  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
   const int b = bkv / p.Hkv, kvh = bkv % p.Hkv, h = kvh * group + hg;
   const int m0 = (n_rblk - 1 - mi) * kRows;
   const int L = bwd_seq_len(p, b);
@@ -877,7 +877,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
   const int N = p.N, group = p.Hq / p.Hkv, n_rblk = (N + kRows - 1) / kRows;
   int bkv, kblk, member_unused;
-  if (!xcd_block_map(p.B * p.Hkv, n_rblk, 1, p.causal != 0, 2ll * group * N * kStride, bkv, kblk, member_unused)) return;
+  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, 1, p.causal != 0, 2ll * group * N * kStride, bkv, kblk, member_unused)) return;
   const int b = bkv / p.Hkv, kvh = bkv % p.Hkv;
   const int L = bwd_seq_len(p, b);
   const int n0 = kblk * kRows;

@@ -45,7 +45,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
   const int N = p.N, group = p.Hq / p.Hkv, n_blk = (N + kRows - 1) / kRows;
   int bkv, mi, hg;
-  if (!xcd_block_map(p.B * p.Hkv, n_blk, group, p.causal != 0, 2ll * N * kRow, bkv, mi, hg)) return;
+  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_blk, group, p.causal != 0, 2ll * N * kRow, bkv, mi, hg)) return;
   const int b = bkv / p.Hkv, kvh = bkv % p.Hkv, h = kvh * group + hg, bh = b * p.Hq + h;
   const int mblk = n_blk - 1 - mi, m0 = mblk * kRows;
   if (!left.takes((size_t)bh * p.n_mblk + mblk)) return;

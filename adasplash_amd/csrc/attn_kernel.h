@@ -238,7 +238,7 @@ __attribute__((amdgpu_waves_per_eu(fwd_min_waves<T, D, kMulti>(), (fwd_min_waves
   const int n_mblk = (p.N + BM - 1) / BM;
   const int group = p.Hq / p.Hkv;
   int bkv, mi, hg;
-  if (!xcd_block_map(p.B * p.Hkv, n_mblk, group, p.causal != 0, 2ll * p.N * D * G::kEB, bkv, mi, hg)) return;  // (K and V of a head)
+  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_mblk, group, p.causal != 0, 2ll * p.N * D * G::kEB, bkv, mi, hg)) return;  // (K and V of a head)
   const int b = bkv / p.Hkv, kvh = bkv % p.Hkv;
   const int h = kvh * group + hg;
   const int mblk = n_mblk - 1 - mi;

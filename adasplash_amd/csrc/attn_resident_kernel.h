@@ -54,7 +54,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4, 4))) 
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
   const int N = p.N, group = p.Hq / p.Hkv, n_rblk = (N + kRows - 1) / kRows;
   int bkv, mi, hg;
-  if (!xcd_block_map(p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
+  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
   const int b = bkv / p.Hkv, kvh = bkv % p.Hkv, h = kvh * group + hg;
   const int m0 = (n_rblk - 1 - mi) * kRows;
   int L = N;

@@ -129,7 +129,7 @@ __device__ __forceinline__ int wave_prefix_sum(int v) {
 // than bring 8 MB of that, twice an XCD's L2 -- with more, the blocks of a head that are in flight together become
 // too few to share their tiles, and on long sequences that costs more than the balance gains (dK/dV kernel on
 // B=8, Hkv=8, group 4, N=8192, D=128: 10.1 ms with sets of four heads, 7.5 ms head after head).  Returns false for
-// the padding blocks of the grid (xcd_grid workgroups), else the K/V head, the block index and the member.
+// the padding blocks of the grid (xcd_grid workgroups), else the K/V head, the block index and the member.  `padded`: the batch has lengths.
 //
 // Where the heads do not divide among the XCDs, the last four, two and / or one of them are split over two, four or eight
 // XCDs each, which take its blocks in turn, before their whole heads.  (All heads' blocks in one line cut into eight equal runs
@@ -141,7 +141,7 @@ inline unsigned xcd_grid(long long units, long long inner) {
     if (units & c) per_xcd += (inner + 8 / c - 1) / (8 / c);
   return (unsigned)(per_xcd * 8);
 }
-__device__ __forceinline__ bool xcd_block_map(int units, int blocks, int group, bool balance, long long unit_bytes, int& unit, int& blk,
+__device__ __forceinline__ bool xcd_block_map(bool padded, int units, int blocks, int group, bool balance, long long unit_bytes, int& unit, int& blk,
                                               int& member) {
   const int inner = blocks * group;
   const int x = (int)(blockIdx.x & 7);
@@ -177,11 +177,13 @@ __device__ __forceinline__ bool xcd_block_map(int units, int blocks, int group, 
   const int span = gsize * group;
   blk = s / span;
   // The XCD's 32 CUs take the workgroups of a launch in order, round after round (read from the hardware's id registers), and padding
-  // returns at once.  So the heads change places behind each round, or the blocks of one long sequence among short ones all
-  // fall to the same few CUs, every second one of a set of two heads.  fp32, 2 x 8 heads, N = 1500 and 375, D = 64, forward and
-  // backward: 292 -> 244 us; q of spread 3: 280 -> 228.  (Places changed from block to block fall to half of the CUs as well.)
+  // returns at once.  So the heads of a padded batch change places behind each round, or the blocks of one long sequence among
+  // short ones all fall to the same few CUs, every second one of a set of two heads.  fp32, 2 x 8 heads, N = 1500 and 375, D = 64,
+  // forward and backward: 292 -> 244 us; q of spread 3: 280 -> 228.  (Places changed from block to block fall to half of the CUs as
+  // well.)  Without lengths the order stays: changed, training of 4 x 16 heads, N = 2048, D = 128, bf16, flat, took 620 us for 613,
+  // prefill of 4 x 16/4, N = 1024, D = 128, fp32, spread 3: 145.2 for 144.0.
   int r = s % span;
-  if (gsize > 1) {
+  if (padded && gsize > 1) {
     asm volatile("; several heads");  // (a branch: the divisions are a tenth of a microsecond of the smallest calls)
     r += (s - r) / 32 % span;
     r = r < span ? r : r - span;

@@ -57,3 +57,23 @@ def test_a_batch_equals_its_items_forward_and_backward(dense_only, B, Hq, Hkv, N
         one = run(q[b:b + 1].contiguous(), k[b:b + 1].contiguous(), v[b:b + 1].contiguous(), dout[b:b + 1].contiguous())
         for name, w, o in zip(("out", "taus", "dq", "dk", "dv"), whole, one):
             assert torch.equal(w[b], o[0]), f"{name}: batch item {b} differs from the item run alone"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,causal", [(2, 8, 8, 1024, 64, True), (5, 8, 8, 200, 64, True), (4, 16, 8, 520, 128, True), (3, 8, 8, 1000, 64, False)])
+def test_a_padded_batch_equals_its_items(dense_only, B, Hq, Hkv, N, D, causal, dtype):
+    """The same where the batch has lengths: the heads of a set then change places from round to round (sets of one, two, four and five heads)."""
+    g = torch.Generator().manual_seed(B * 1000 + N + D)
+    q, dout = (torch.randn(B, Hq, N, D, generator=g).to(DEV, dtype) for _ in range(2))
+    k, v = (torch.randn(B, Hkv, N, D, generator=g).to(DEV, dtype) for _ in range(2))
+    lens = torch.tensor([N - b * N // 5 for b in range(B)], dtype=torch.int32, device=DEV)
+
+    def run(b):
+        qq, kk, vv, dd, ll = (t[b].contiguous() for t in (q, k, v, dout, lens))
+        out, taus, bmask = _attention.launch_forward(qq, kk, vv, version=2 if causal else 1, alpha=1.5, is_causal=causal, niter=2, varlen=ll)
+        return out, *_attention.launch_backward(qq, kk, vv, dd, taus, bmask, alpha=1.5, is_causal=causal, varlen=ll)[:3]
+
+    whole = run(slice(0, B))
+    for b in range(B):
+        for name, w, o in zip(("out", "dq", "dk", "dv"), whole, run(slice(b, b + 1))):
+            assert torch.equal(w[b], o[0]), f"{name}: batch item {b} differs from the item run alone"
