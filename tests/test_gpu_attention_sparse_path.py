@@ -229,3 +229,29 @@ def test_dense_supports_go_back_to_the_dense_backward_kernels(sparse_switch):
             assert max_err(got, ref) < 4e-2
     for a, b in zip(grads[True], grads[False]):
         assert max_err(a, b.float().cpu()) < 4e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Hq,Hkv", [(16, 8), (4, 2), (1, 1)])
+def test_some_row_and_key_blocks_go_back_to_the_dense_backward_kernels(sparse_switch, Hq, Hkv, D, dtype):
+    """Peaked rows but for one block of 128, whose supports overflow: dQ of that block, and dK and dV of the keys it sees, come
+    from the dense kernels, in workgroups of 128, 64 and 32 rows (16, 4 and 1 heads), the others from those on the supports.  (With a
+    tile mask in hand no call takes the short route.)  Bound: the weights' and the result's rounding to the type."""
+    q, k, v = qkv(2, Hq, Hkv, 1200, D, dtype, seed=3, scale=3.0)
+    q[:, :, 512:640] /= 24
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(4)).to(dtype)
+    varlen = torch.tensor([1200, 1001], dtype=torch.int32)
+    want = exact.dense_entmax_attention_grads(q, k, v, dout, 1.5, True, varlen)
+    sparse_switch(True)
+    args = [t.to(DEV) for t in (q, k, v, dout)]
+    taus, bmask = forward(q, k, v, varlen)[1:]
+    grads = {}
+    for on in (True, False):
+        sparse_switch(on)
+        grads[on] = _attention.launch_backward(*args, taus, bmask, alpha=1.5, is_causal=True, varlen=varlen.to(DEV))[:3]
+        for got, ref in zip(grads[on], want):
+            err = ((got.double().cpu() - ref.double()).norm() / ref.double().norm()).item()
+            assert err < (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -10), err
+    same = [torch.equal(a, b) for a, b in zip(grads[True][0].split(128, dim=2), grads[False][0].split(128, dim=2))]
+    assert same[4] and not any(same[:4]), same
