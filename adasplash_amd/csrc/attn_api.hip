@@ -410,7 +410,7 @@ static long long score_blocks(int B, int Hq, int N, bool causal) {
   return (long long)B * Hq * (causal ? r * (r + 1) / 2 : r * r);
 }
 static bool resident_takes(int N, int D, int dtype, double alpha) {
-  return dtype != ADSP_F32 && (D == 64 || D == 128) && N <= 2048 && alpha >= 1.125 && alpha <= 2.0 && sparse_enabled();
+  return dtype != ADSP_F32 && (D == 64 || D == 128) && N <= kResidentMaxKeys && alpha >= 1.125 && alpha <= 2.0 && sparse_enabled();
 }
 // Whether a 16-bit forward of which nobody wants the tile mask or the supports takes the single kernel that holds its rows' scores in
 // registers (attn_resident_kernel.h).  It does the same work whatever the scores are, so the lines lie where the kernels on

@@ -9,6 +9,9 @@ constexpr int kBN = 64;          // keys per tile
 constexpr int kAttnBins = 8;     // histogram bins of the attention solver
 constexpr int kMaskWords = 512;  // tile-mask capacity per row block: 512 * 32 tiles * 64 keys = 1M keys
 
+// Keys whose scores the workgroups of attn_resident_kernel.h can hold: what the dispatch sends them, and what they are built for.
+constexpr int kResidentMaxKeys = 2048;
+
 enum AttnAlphaMode { ATT_15 = 0, ATT_2 = 1, ATT_GEN = 2 };
 // control words of the sparse-support forward behind the eight work counters (AttnParams::queue)
 constexpr int kCtrlFlagged = 8;     // row blocks left to the dense kernel

@@ -1,5 +1,5 @@
 // Sparse entmax attention forward for gfx950 with a row's scores resident in registers: 16-bit types, head dims 64 and 128, up to
-// kMaxKeys keys.
+// kResidentMaxKeys keys.
 //
 // What bounds it: the vector pipe (an iteration of the solver is three instructions a score, 4 cycles each, and there are four to
 // six of them; the products are a tenth of that), and on small calls the chain of load, product, solver and output itself.
@@ -31,7 +31,7 @@ using f32path::kChunk;
 using f32path::kRows;
 constexpr int kBlocks = 4;       // blocks of 32 keys a wave holds
 constexpr int kMaxWaves = 16;
-constexpr int kMaxKeys = kRows * kBlocks * kMaxWaves;
+static_assert(kRows * kBlocks * kMaxWaves == kResidentMaxKeys, "a key beyond the registers would be dropped");
 
 // u clamped to [0, 1] in the fma itself: a score is at most 1 above a threshold that is a bound
 __device__ __forceinline__ float above(float s, float qs, float minus_t) { return __builtin_amdgcn_fmed3f(fmaf(s, qs, minus_t), 0.f, 1.f); }
