@@ -116,6 +116,18 @@ def test_forward_with_resident_scores(N, scale, Hq, Hkv, D, alpha, causal, dtype
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,alpha,causal", [(64, 1.5, True), (128, 1.5, False), (64, 1.333, False), (128, 2.0, False)])
+@pytest.mark.parametrize("N,length", [(1700, 1700), (2048, 2048), (2048, 2017), (2048, 1537)])
+def test_forward_with_the_most_resident_scores(N, length, D, alpha, causal, dtype):
+    """One head, at most 4096 blocks of 32 x 32 scores: sixteen waves with up to four blocks of keys each serve it at both head dims (D = 128
+    and more than 1024 keys: up to 8000).  A training step's forward is the same."""
+    q, k, v, dout, varlen = problem(1, 1, 1, N, D, dtype, 1.0, [length])
+    got = run(q, k, v, dout, varlen, alpha, causal, train=False)
+    assert torch.equal(got[0], run(q, k, v, dout, varlen, alpha, causal)[0])
+    check(got, q, k, v, dout, varlen, alpha, causal, [0])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("Hq,Hkv,D,alpha,causal", [(2, 1, 64, 1.5, True), (1, 1, 128, 1.5, False), (1, 1, 64, 1.125, False), (1, 1, 128, 2.0, False)])
 @pytest.mark.parametrize("N,scale", [(97, 1.0), (256, 0.125), (257, 0.125), (577, 1.0), (1153, 3.0), (1300, 0.125), (2309, 0.125)])
 def test_forward_on_all_pairs(no_supports, N, scale, Hq, Hkv, D, alpha, causal, dtype):
