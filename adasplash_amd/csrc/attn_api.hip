@@ -376,17 +376,13 @@ static bool f32_split(int N, int D, int dtype, double alpha) {
   return dtype == ADSP_F32 && (D == 64 || D == 128) && N <= 65536 && alpha >= 1.125 && alpha <= 2.0;
 }
 
-// Whether a 16-bit forward of which nobody wants the tile mask or the supports takes the single kernel on 32 rows a workgroup
-// (attn_f32_kernel.h): a short problem, for which the probe, the copy of K, the sparse-support kernel's items of 128 rows and
-// the dense kernel behind it take longer than the work.  Two workgroups fit a CU: up to 512 run at once.  With flat scores,
-// where the lists overflow and each workgroup walks several times, a second round of them is one too many on causal problems
-// of a few hundred keys (16 heads, N = 256: 8 sequences 30 -> 42 us, 5 of N = 512: 40 -> 60, against 57 -> 27 and 75 -> 43
-// with unit spread), and not on longer or full ones or where a workgroup has no more than one step.  The second
-// condition is the time the work itself takes, about 20 ns a workgroup and 1.35 ns a block of 32 x 32 scores with the chip full.
-// Measured at the line, four launches -> this kernel, us for q of spread 1, 3 and 1/8: 16/4 heads, D = 128, 4 sequences of
-// N = 256: 76 -> 18 and 38 -> 31 (1 and 1/8); 2 of 512: 99 -> 24, 52 -> 32; 32/8 heads, N = 1024: 131 -> 53, 80 -> 74; 16/4
-// heads, N = 2048: 132 -> 93, 89 -> 54, 135 -> 124; 4 x 16 heads, N = 512, not causal: 67 -> 46, 47 -> 34, 95 -> 54; 32 x 16
-// heads, N = 128: 59 -> 42, 44 -> 36, 70 -> 66; beyond it 32/8 heads, N = 2048: 147 -> 132, 96 -> 100, 139 -> 236.
+// Whether a 16-bit forward of which nobody wants the tile mask or the supports, and which the kernel with resident scores does not
+// take, runs in the single kernel on 32 rows a workgroup (attn_f32_kernel.h): more than 1024 keys and few heads, for which the
+// probe, the copy of K, the sparse-support kernel's items of 128 rows and the dense kernel behind it take longer than the work.
+// Two workgroups fit a CU: up to 512 run at once, and the rule allows two rounds of them.  The second condition is the time the work
+// itself takes, about 20 ns a workgroup and 1.35 ns a block of 32 x 32 scores with the chip full.
+// Measured at the line, four launches -> this kernel, us for q of spread 1, 3 and 1/8: 16/4 heads, D = 128, N = 2048: 132 -> 93, 89 -> 54,
+// 135 -> 124; beyond it 32/8 heads: 147 -> 132, 96 -> 100, 139 -> 236.
 // Long sequences of few heads pass that line too, and the longest workgroup's walk is then all of the time; hence the limit on N.
 // One head, D = 64 and 128 (GPU times): causal N = 4096: 147 -> 56, 103 -> 44, 171 -> 97 and 171 -> 63, 127 -> 50, 246 -> 142; N = 8192:
 // 226 -> 226, 164 -> 69, 323 -> 187 and 275 -> 268, 211 -> 81, 475 -> 290; beyond it 9472: 260 -> 253, 187 -> 79, 371 -> 243 and
@@ -401,8 +397,7 @@ static bool rows32_16bit(int B, int Hq, int N, int D, int dtype, double alpha, b
   if (dtype == ADSP_F32 || (D != 64 && D != 128) || !(alpha >= 1.125 && alpha <= 2.0) || !sparse_enabled()) return false;
   if (N > (causal ? 8192 : 4096)) return false;
   const long long groups = (long long)B * Hq * ((N + 31) / 32);
-  const long long most = N <= 128 ? 2048 : ((N >= 1024 || !causal) ? 1024 : 512);
-  return groups <= most && rows32_cost_ns(B, Hq, N, causal) <= 66e3;
+  return groups <= 1024 && rows32_cost_ns(B, Hq, N, causal) <= 66e3;
 }
 // blocks of 32 x 32 scores of a call, padding included
 static long long score_blocks(int B, int Hq, int N, bool causal) {
