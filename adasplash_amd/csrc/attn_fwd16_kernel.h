@@ -12,8 +12,8 @@
 // together, the sums or weights of one between the products of the other (tile16::stream).  The weights' sum is that of the rounded
 // weights, those that the product takes (taken from the unrounded ones the error grows from 2.2e-3 to 2.3e-3).
 //
-// Measured, us, the kernel with lists (ten solver steps allowed) -> this one: 4 x 16 heads, N = 4096, not causal, alpha = 1.5, D = 64: 2240 -> 745,
-// D = 128: 3530 -> 1250; 8 heads, N = 8192, alpha = 1.333: 2860 -> 1020, 3250 -> 1200; 4 x 16, N = 4096, alpha = 2: 2280 -> 1760, 3630 -> 2770 (there
+// Measured, us, the kernel with lists (ten solver steps allowed) -> this one: 4 x 16 heads, N = 4096, not causal, alpha = 1.5, D = 64: 2240 -> 760,
+// D = 128: 3530 -> 1270; 8 heads, N = 8192, alpha = 1.333: 2860 -> 1020, 3250 -> 1200; 4 x 16, N = 4096, alpha = 2: 2280 -> 1760, 3630 -> 2770 (there
 // the sums are piecewise linear and a step halves the support at best: five to eight walks).  Against 64 bits: bf16 2.3e-3 as before, f16 4.5e-4
 // -> 2.9e-4 at N = 6000.
 #pragma once
@@ -23,9 +23,13 @@ namespace adsp {
 namespace fwd16 {
 using namespace tile16;
 
-// A walk's Newton step of x times the mean of u leaves about (c0 - 1) / 2 x^2 of it.  The last walk takes steps of up to this: an error of
-// the weights below their rounding is left then; the thresholds that a backward reads are taken a step further by the output walk's sums.
-template <typename T, int AM> constexpr float kNear = AM == ATT_15 && elem_traits<T>::kIsBf16 ? 0.06f : 0.02f;
+// A walk's Newton step of x times the mean of u leaves about (c0 - 1) / 2 (n sum u^2 / (sum u)^2 - 1) x^2 of it (n members, alpha = 1.5): half of
+// that square for flat scores, more where few keys have most of the weight.  The last walk takes steps of up to this: an error of the weights
+// below their rounding is left then; the thresholds that a backward reads are taken a step further by the output walk's sums.  bf16,
+// alpha = 1.5: with 0.06 a row whose last step was just small enough had an error of 4.2e-3 where rounding alone gives the worst of 256 row
+// blocks 3.35e-3 (8 heads, N = 4096, D = 128, q of spread 0.03 to 2); 0.04 has 3.35e-3, 0.03 the same.  us, 0.06 / 0.04 / 0.03, 4 x 16 heads, N = 4096,
+// q of spread 1/8: D = 64 699 / 712 / 732, D = 128 1190 / 1213 / 1221; spread 1/2, D = 64: 1081 / 1125 / 1144.
+template <typename T, int AM> constexpr float kNear = AM == ATT_15 && elem_traits<T>::kIsBf16 ? 0.04f : 0.02f;
 constexpr int kSample = 256;  // keys of the sample that a row's first threshold comes from
 
 template <typename T, int D, int AM, bool kTaus>

@@ -150,6 +150,24 @@ def test_one_key_far_above_a_sampled_threshold(no_supports, size, D, dtype):
     check(run(q, k, v, dout, varlen, 1.125, False, train=False), q, k, v, dout, varlen, 1.125, False, [0])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("alpha", [1.5, 1.333])
+@pytest.mark.parametrize("N", [1280, 4096])
+def test_rows_whose_last_step_is_just_small_enough(no_supports, N, alpha, D, dtype):
+    """The walks end for 128 rows together.  Here these are equal and every row block has a spread of its own, so the last steps lie all over
+    the range that the rule allows, and a row's error is that of its own threshold, not a mean.  Bound, row by row: the weight's and the
+    result's rounding, each at most a unit and half of that on average; what a step of x leaves, about x^2 relative to the weights (1.6e-3
+    for bf16), joins them as a root of squares."""
+    q, k, v, dout, varlen = problem(1, 8, 8, N, D, dtype, 1.0, [N])
+    spread = torch.logspace(-1.5, 0.3, 8 * N // 128).reshape(1, 8, N // 128, 1, 1)
+    q = (q.float().reshape(1, 8, N // 128, 128, D)[:, :, :, :1] * spread).expand(1, 8, N // 128, 128, D).reshape(q.shape).to(dtype)
+    got = run(q, k, v, dout, varlen, alpha, False, train=False)[0].double().cpu()[:, :, ::128]
+    want = exact.dense_entmax_attention(q[:, :, ::128], k, v, alpha, False, None).double()
+    err = (got - want).norm(dim=-1) / want.norm(dim=-1)
+    assert err.max() < 2 * UNIT[dtype], err.max()
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("far", [640, 1099])
 def test_tile_mask_has_weights_too_small_for_the_sum(no_supports, far, D):
