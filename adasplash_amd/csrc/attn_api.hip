@@ -732,7 +732,7 @@ static BwdWorkspace bwd_workspace(int B, int Hq, int Hkv, int N, int D, int dtyp
 }
 
 // dK, dV = sum over the query heads of a K/V head of the sparse-support kernel's fp32 partial rows; key blocks left to
-// attn_bwd_dkdv_kernel are skipped (that kernel writes them), and so are those the kernel on the streams served for all
+// attn_bwd16_dkdv_kernel are skipped (that kernel writes them), and so are those the kernel on the streams served for all
 // heads at once.  A thread adds up 8 columns of
 // one key row.  Rows past the valid length are zeros and their partial rows are not read (the key blocks that lie
 // wholly in the padding have none).
@@ -863,7 +863,7 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
     const size_t need = w.total;
     if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0)) return ADSP_ERR_WORKSPACE;
     // Sparse-support dQ kernel first (alpha 1.5 / 2): it serves the row blocks whose supports are short and flags the
-    // others for attn_bwd_dq_kernel below; the dK/dV kernel reads delta and 1 / sum p from whichever of the two wrote them.
+    // others for attn_bwd16_dq_kernel below; the dK/dV kernel reads delta and 1 / sum p from whichever of the two wrote them.
     sparse = !short16 && w.slots > 0 && (am == ATT_15 || am == ATT_2 || (alpha >= 1.125 && alpha < 2.0)) &&
              (long long)B * Hq * mblocks_of(N) < (1ll << 31) && sparse_enabled();
     if (sparse) {

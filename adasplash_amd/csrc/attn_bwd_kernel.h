@@ -1,4 +1,5 @@
-// Backward of the sparse entmax attention for gfx950: dQ kernel and dK/dV kernel.
+// Backward of the sparse entmax attention for gfx950: dQ kernel and dK/dV kernel.  fp32 at every head dim, 16-bit types at 16, 32 and
+// 256 (64 and 128: attn_bwd16_kernel.h).
 //
 // With x_ij = q_i.k_j / sqrt(D), z = (alpha-1) x, p_ij = [z_ij - tau_i]_+^(1/(alpha-1)) and u = p^(2-alpha),
 // the entmax Jacobian is diag(u) - u u^T / sum(u), hence for dP_ij = dO_i . v_j
@@ -266,9 +267,8 @@ __device__ __forceinline__ int bwd_seq_len(const AttnBwdParams& p, int b) {
 // ---------------------------------------------------------------------------------------------------------
 // dQ kernel: one block per (K/V head, query head in its group, row block of 128 queries)
 // ---------------------------------------------------------------------------------------------------------
-constexpr int kDqPlainMaxD = 128;  // largest 16-bit head dim whose unmasked blocks take the predicate-free code
-constexpr int kDqWaves64 = 3;      // waves per SIMD of the dQ kernel at 16-bit D <= 64
-template <typename T, int D> constexpr int dq_waves() { return (TileGeo<T, D>::k16 && D <= 64) ? kDqWaves64 : BwdTiles<T, D>::kMinWaves; }
+constexpr int kDqWaves32 = 3;  // waves per SIMD of the dQ kernel at 16-bit D <= 32
+template <typename T, int D> constexpr int dq_waves() { return (TileGeo<T, D>::k16 && D <= 32) ? kDqWaves32 : BwdTiles<T, D>::kMinWaves; }
 
 template <typename T, int D, int AM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((dq_waves<T, D>()), (dq_waves<T, D>() > 2 ? dq_waves<T, D>() : 2)))) void attn_bwd_dq_kernel(AttnBwdParams p) {
@@ -294,8 +294,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((dq_waves<T
   const int b = bkv / p.Hkv, kvh = bkv % p.Hkv;
   const int h = kvh * group + hg;
   const int bh = b * p.Hq + h;
-  // behind the sparse-support dQ kernel: only the row blocks it flagged (all of them when it stepped aside)
-  if (p.block_flags && p.queue[kCtrlAllDense] == 0u && (p.queue[kCtrlFlagged] == 0u || p.block_flags[(size_t)bh * n_blk + mblk] == 0)) return;
   const int L = bwd_seq_len(p, b);
   const int m0 = mblk * kBwdRows;
   const int wave_row0 = m0 + wave * 32;
@@ -383,8 +381,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((dq_waves<T
   // the wave sees in full (below the causal diagonal, inside the sequence) is "plain": no per-score predicate,
   // one fma per score instead of a compare and two selects more.  The choice is a template argument so that each
   // kind of block is one piece of straight-line code, products included.
-  // (only where the second code path fits the register budget: at D = 128 it costs spills and more than it saves)
-  constexpr bool kPlainBlocks = k16 && D <= kDqPlainMaxD;
+  // (only where the second code path fits the register budget: 16-bit types, not at D = 256)
+  constexpr bool kPlainBlocks = k16 && D <= 32;
   auto block_is_plain = [&](int kt, int kb) { return kPlainBlocks && kt * kBN + kb * 32 + 31 <= lim_all; };
   auto block_terms = [&](auto plain_c, int kt, int kb, const unsigned char* ka, const unsigned char* va, float (&r)[16],
                          f32x16& dp) {
@@ -499,10 +497,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((BwdTiles<T
   __shared__ __align__(1024) unsigned char a1[BT::kNBuf == 2 ? BT::kTile : 16];
   __shared__ __align__(1024) unsigned char b1[BT::kNBuf == 2 ? BT::kTile : 16];
   __shared__ __align__(1024) unsigned char c1[(k16 && BT::kNBuf == 2) ? BT::kTile : 16];
-  // 16-bit types with D <= 64 make one walk over the query tiles and keep both accumulators (at D = 128
-  // the two accumulators plus the K and V fragments no longer fit 256 registers); that needs dO^T and Q^T
+  // 16-bit types with D <= 32 make one walk over the query tiles and keep both accumulators (at D = 256
+  // the two accumulators plus the K and V fragments do not fit 256 registers); that needs dO^T and Q^T
   // at the same time
-  constexpr bool kFused = k16 && D <= 64;
+  constexpr bool kFused = k16 && D <= 32;
   __shared__ __align__(1024) unsigned char d0[kFused ? BT::kTile : 16];  // Q^T tile
   __shared__ __align__(1024) unsigned char d1[(kFused && BT::kNBuf == 2) ? BT::kTile : 16];
   __shared__ __align__(16) float scal0[3][kBN];  // tau, 1 / sum p, delta of the tile's queries
@@ -518,10 +516,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((BwdTiles<T
   if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, (N + kBwdRows - 1) / kBwdRows, 1, p.causal != 0, 2ll * (p.Hq / p.Hkv) * N * D * G::kEB, bkv, nblk, member_unused)) return;
   const int b = bkv / p.Hkv, kvh = bkv % p.Hkv;
   const int group = p.Hq / p.Hkv;
-  // behind the sparse-support dK/dV kernel: only the key blocks it flagged (all of them when it stepped aside)
-  if (p.kv_flags && p.queue2[kCtrlAllDense] == 0u &&
-      (p.queue2[kCtrlFlagged] == 0u || p.kv_flags[(size_t)bkv * ((N + kBwdRows - 1) / kBwdRows) + nblk] == 0))
-    return;
   const int L = bwd_seq_len(p, b);
   const int n0 = nblk * kBwdRows;
   const int wave_key0 = n0 + wave * 32;

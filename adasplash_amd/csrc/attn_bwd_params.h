@@ -20,7 +20,7 @@ struct AttnBwdParams {
   float sm_scale;  // 1 / sqrt(D)
   float c0;        // 1 / (alpha - 1)
   // the sparse-support dQ kernel and its hand-over to the dense one (null: dense kernels only), as in AttnParams
-  int32_t* block_flags;   // [B, Hq, n_mblk] 1 = row block left to attn_bwd_dq_kernel
+  int32_t* block_flags;   // [B, Hq, n_mblk] 1 = row block left to attn_bwd16_dq_kernel
   uint32_t* queue;        // control words: work counters, flagged count, "every head dense"
   uint32_t* hints;        // two words per K/V head: word 0 is 1 << 20 where the probe left the head to the dense kernels
   unsigned char* events;  // candidate streams, one slot per workgroup of the sparse kernel
@@ -28,7 +28,7 @@ struct AttnBwdParams {
   // [B, Hq, part_rows, D] when a K/V head serves several query heads (null otherwise), and per workgroup and wave 32 fp32
   // rows of dK | dV for the sums of an item that is worked off in parts; the streams are shared
   uint32_t* queue2;
-  int32_t* kv_flags;  // [B, Hkv, n_mblk] 1 = key block left to attn_bwd_dkdv_kernel
+  int32_t* kv_flags;  // [B, Hkv, n_mblk] 1 = key block left to attn_bwd16_dkdv_kernel
   float* dk_part;
   float* dv_part;
   int part_rows;  // rows per query head in dk_part / dv_part: N, or as many as the key blocks that are not merged can need

@@ -17,7 +17,7 @@
 // delta_i)) in the element type; a last pass writes the pairs into the first words of the stream's entries, which
 // held each entry's place in the lists since the sort.
 //
-// Row blocks whose supports outgrow the stream or the lists are flagged and left to attn_bwd_dq_kernel, launched
+// Row blocks whose supports outgrow the stream or the lists are flagged and left to attn_bwd16_dq_kernel, launched
 // behind, exactly as in the forward; the kernel is persistent and takes row blocks as the forward does (draw_item).
 #pragma once
 #include "attn_bwd_kernel.h"
@@ -716,7 +716,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
 // partial rows per query head that dkdv_reduce_kernel adds up over the heads of a K/V head.  The first key blocks of a
 // causal sequence lie in the supports of hundreds of queries each: when a wave's stream is half full the walk pauses,
 // the lists made so far are worked off into the partial rows, and the walk goes on.  A key block that any of its query
-// heads gives up all the same is flagged and computed, all heads, by attn_bwd_dkdv_kernel.
+// heads gives up all the same is flagged and computed, all heads, by attn_bwd16_dkdv_kernel.
 template <typename T, int D, int AM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE_WAVES, ADSP_SPARSE_WAVES))) void attn_bwd_dkdv_sparse_kernel(AttnBwdParams p) {
   using G = TileGeo<T, D>;
@@ -794,7 +794,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
       long long l = p.varlen_bits == 64 ? ((const long long*)p.varlen)[b] : (long long)((const int*)p.varlen)[b];
       L = (int)(l < 0 ? 0 : (l > N ? N : l));
     }
-    // a key block that any query head gives up goes to attn_bwd_dkdv_kernel with all its heads
+    // a key block that any query head gives up goes to attn_bwd16_dkdv_kernel with all its heads
     int32_t* const flag = p.kv_flags + ((size_t)(b * p.Hkv + kvh) * n_mblk + mblk);
     const size_t qo_base = ((size_t)(b * p.Hq + h) * N) * D;
     const size_t kv_base = ((size_t)(b * p.Hkv + kvh) * N) * D;
@@ -1234,7 +1234,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
 // dkdv_reduce_kernel; where a K/V head has a single query head the last part writes dK and dV in the element type and
 // there is no reduction.  With a causal mask the later key blocks of a sequence (dkdv_block_merged) are short: there
 // one item serves all query heads of the K/V head and writes dK and dV itself.  A key block one of whose row blocks the
-// dQ kernel gave up (no stream) is flagged for attn_bwd_dkdv_kernel with all its heads.
+// dQ kernel gave up (no stream) is flagged for attn_bwd16_dkdv_kernel with all its heads.
 template <typename T, int D, int AM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_DKDV_WAVES, ADSP_DKDV_WAVES))) void attn_bwd_dkdv_stream_kernel(AttnBwdParams p) {
   constexpr int kQuads = ADSP_DKDV_QUADS;
@@ -1318,7 +1318,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_DKDV_W
       }
       continue;
     }
-    // a key block that any query head gives up goes to attn_bwd_dkdv_kernel with all its heads
+    // a key block that any query head gives up goes to attn_bwd16_dkdv_kernel with all its heads
     int32_t* const flag = p.kv_flags + ((size_t)(b * p.Hkv + kvh) * n_mblk + mblk);
     const size_t kv_base = ((size_t)(b * p.Hkv + kvh) * N) * D;
     // the row blocks whose queries can hold the block's keys in their supports

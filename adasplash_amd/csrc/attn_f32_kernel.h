@@ -28,9 +28,9 @@
 // 288 -> 148; 4 heads, N = 8192: 776 -> 285; bf16, 2 heads, N = 4096, D = 128: 135 -> 75.  Spread 3, where nothing overflows: 82.8 -> 83.2.
 //
 // Measured (fp32, causal, forward and backward; kernels on 128 rows a workgroup -> these): 2 x 8 heads, N = 1500 and 375,
-// D = 64: 1140 -> 287 us (forward 65, dQ 128, dK/dV 108, where one walk of the longest rows is 10 us of matrix work a
+// D = 64: 1140 -> 243 us (forward 55, dQ 106, dK/dV 93, where one walk of the longest rows is 10 us of matrix work a
 // product); flat scores 1139 -> 380; 4 x 16/4 heads, N = 1024, D = 128: 2885 -> 927.  Eight waves to the 32 rows, one
-// workgroup per CU: 330 us for the first.  Where 16-bit calls come here: rows32_16bit in attn_api.hip.
+// workgroup per CU: 330 us for the first, when this took 287.  Where 16-bit calls come here: rows32_16bit in attn_api.hip.
 #pragma once
 #include "attn_bwd_kernel.h"
 
