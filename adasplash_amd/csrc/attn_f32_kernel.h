@@ -1,8 +1,17 @@
 // Sparse entmax attention on workgroups of 32 rows for gfx950, head dims 64 and 128: single-precision forward, dQ and dK/dV
 // kernels, and the forward for some 16-bit problems.
 //
-// What bounds them: the fp32 matrix pipe (v_mfma_f32_32x32x2_f32, 64 cycles) on large problems, and on
-// ordinary ones the length of a workgroup's walk over the keys, because a K/V head of N keys has only N / rows workgroups.
+// What bounds them: vector and matrix pipe together on large problems (per block of 32 x 32 scores and product of 64 columns 24 matrix
+// products of 32 cycles and about 110 vector instructions for their operands), and on ordinary ones the length of a workgroup's
+// walk over the keys, because a K/V head of N keys has only N / rows workgroups; the forward's solves beside it.
+//
+// Products: an fp32 operand is the sum of three bf16 values exactly, and six of the nine products of the parts are what fp32 can see.  On
+// the bf16 matrix pipe they take 192 cycles per 16 columns where v_mfma_f32_32x32x2_f32 takes 512, and fewer roundings: relative
+// error against 64 bits, fp32 products -> these, of output, dQ, dK, dV: N = 1500, D = 64 4.0e-7, 4.5e-7, 4.5e-7, 4.1e-7 -> 2.7e-7, 3.3e-7, 3.3e-7,
+// 2.8e-7; q of spread 3 5.6e-7, 9.3e-7, 9.4e-7, 5.6e-7 -> 4.0e-7, 6.9e-7, 7.1e-7, 4.1e-7; flat 2.2e-7 ... 3.1e-7 -> 1.5e-7 ... 1.9e-7; D = 128
+// 3.6e-7, 9.2e-7, 9.2e-7, 8.5e-7 -> 3.4e-7, 3.7e-7, 3.7e-7, 3.5e-7; V of mean 10: dQ 1.5e-6 -> 1.0e-6.  The small products have an accumulator
+// of their own: added to the sum itself, their roundings made these errors 1.2 to 2 times those of fp32 products.
+//
 // The 16-bit forward: vector issue (its products are a sixteenth as long; about 1400 vector instructions per block of 32 x 32 scores,
 // most of them insertions into the lists; matrix pipe 1-2 %, vector pipe about 50 % of the busy SIMD cycles).
 //
@@ -10,8 +19,9 @@
 // take the 32-row blocks of the other side in turn, and meet in LDS at the end of a walk.  Against 128 rows per workgroup,
 // 32 per wave, a walk is a quarter as long and there are four times as many workgroups.  A wave's operands come through a
 // ring of three 4 KB chunks ([32 rows][32 columns]) of LDS of its own, loaded two chunks ahead with direct 16-byte loads:
-// a chunk lasts 1024 cycles of matrix work, so the waves need no barrier inside a walk and no tile shared by them.  Each
-// operand block is read by one workgroup of 32 rows instead of 128, about 16 bytes per cycle and CU out of L2.
+// a chunk lasts 400 to 900 cycles of matrix and vector work, so the waves need no barrier inside a walk and no tile shared by them.  Each
+// operand block is read by one workgroup of 32 rows instead of 128, about 30 bytes per cycle and CU out of L2.  The gradients' own rows
+// lie in LDS, split once by all four waves (in registers, 33 to 192 others were spilled).
 //
 // Forward, one product per (row, key) where supports are short: tau over a subset of the keys is a lower bound of tau over
 // all of them, so a wave lists the scores above its row's bound while it walks, and after 1, 2, 4, 8, ... steps the
@@ -27,10 +37,10 @@
 // gives up.  us, q of spread 1: 2 x 8 heads, N = 1500 and 375: 126 -> 66 (65 where no list overflows); N = 2048: 187 -> 101, D = 128, 16/4 heads:
 // 288 -> 148; 4 heads, N = 8192: 776 -> 285; bf16, 2 heads, N = 4096, D = 128: 135 -> 75.  Spread 3, where nothing overflows: 82.8 -> 83.2.
 //
-// Measured (fp32, causal, forward and backward; kernels on 128 rows a workgroup -> these): 2 x 8 heads, N = 1500 and 375,
-// D = 64: 1140 -> 243 us (forward 55, dQ 106, dK/dV 93, where one walk of the longest rows is 10 us of matrix work a
-// product); flat scores 1139 -> 380; 4 x 16/4 heads, N = 1024, D = 128: 2885 -> 927.  Eight waves to the 32 rows, one
-// workgroup per CU: 330 us for the first, when this took 287.  Where 16-bit calls come here: rows32_16bit in attn_api.hip.
+// Measured (fp32, forward and backward, us; kernels on 128 rows a workgroup -> fp32 products -> these): causal, 2 x 8 heads, N = 1500 and 375,
+// D = 64: 1140 -> 242 -> 160 (forward 55 -> 50, dQ 106 -> 62, dK/dV 93 -> 61); 4 x 16/4 heads, N = 1024, D = 128: 2885 -> 930 -> 711, flat,
+// 16 heads: 1306 -> 1002; alpha = 1.333, 8 x 16 heads, N = 1024, not causal: 4818 -> 2690 -> 1794; prefill of 8 heads, N = 128: 11.4 -> 11.4.
+// Where 16-bit calls come here: rows32_16bit in attn_api.hip.
 #pragma once
 #include "attn_bwd_kernel.h"
 
@@ -86,6 +96,23 @@ template <int kStride> struct Ring {
       }
     }
   }
+  // The same in two calls, without a branch: rows() for a block, issue_rows() for each of its chunks
+  uint32_t at[4];
+  __device__ __forceinline__ void rows(int row0, int limit) {
+    const int p0 = (lane & 7) ^ (lane >> 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      int r = row0 + 8 * j + (lane >> 3);
+      r = r < limit ? r : limit - 1;
+      at[j] = (uint32_t)r * (uint32_t)kStride + (uint32_t)((p0 ^ (4 * (j & 1))) * 16);
+    }
+  }
+  __device__ __forceinline__ void issue_rows(const unsigned char* g, int c, int s) const {
+    const unsigned char* gb = uniform_ptr(g + c * 128);
+    unsigned char* l = base + s * kChunk;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dma16s(gb, at[j], l + j * 1024);
+  }
   // the same in the layout of the transposing reads (16-bit V; see BwdTiles::tsw): row r's pieces moved by 2 r
   __device__ __forceinline__ void issue_t(const unsigned char* g, int row0, int limit, int c, int s) const {
     const unsigned char* gb = uniform_ptr(g + c * 128);
@@ -124,42 +151,140 @@ template <int SEQ, typename R, typename Src> __device__ __forceinline__ uint32_t
   ring.advance();
   return a;
 }
-// The whole walk: body(blk, next) consumes a block's chunks by calls of next(0), next(1), ... in order.
-template <int SEQ, typename R, typename Src, typename Body>
+// The whole walk: body(blk, next) consumes a block's chunks by calls of next(0), next(1), ... in order.  kStarted: the caller has issued
+// the first two chunks (`start`, where first < n_blk).
+template <int SEQ, bool kStarted = false, typename R, typename Src, typename Body>
 __device__ __forceinline__ void walk(R& ring, int first, int n_blk, int step, Src&& src, Body&& body) {
   if (first >= n_blk) return;
   ring.st = 0;
-  start<SEQ>(first, n_blk, step, src);
+  if constexpr (!kStarted) start<SEQ>(first, n_blk, step, src);
   for (int blk = first; blk < n_blk; blk += step) body(blk, [&](int s) -> uint32_t { return take<SEQ>(ring, blk, s, n_blk, step, src); });
   ring.drain();
 }
 
-// acc += (chunk rows) . (the lane's own row) over the chunk's columns: f holds of the lane's row piece 2 g + lh of every pair.  kParts: a chunk's 32 products are added up from zero and the chunks' sums then, shorter chains of smaller numbers (where
-// the registers allow it).
-template <bool kParts, typename T = float> __device__ __forceinline__ void dot_chunk(f32x16& acc, uint32_t chunk, uint32_t row_lane, const uint32_t* f) {
-  if constexpr (is16<T>::value) {
-    u32x4 a[4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) a[g] = lds_read16((chunk + row_lane) ^ (g << 5));
-#pragma unroll
-    for (int g = 0; g < 4; ++g) acc = mfma_16bit<T>(a[g], u32x4{f[4 * g], f[4 * g + 1], f[4 * g + 2], f[4 * g + 3]}, acc);
-    return;
-  }
-  f32x4 a[4];
-#pragma unroll
-  for (int g = 0; g < 4; ++g) a[g] = __builtin_bit_cast(f32x4, lds_read16((chunk + row_lane) ^ (g << 5)));
-  f32x16 part;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) part[i] = kParts ? 0.f : acc[i];
-#pragma unroll
-  for (int g = 0; g < 4; ++g)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) part = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g][e], __builtin_bit_cast(float, f[g * 4 + e]), part, 0, 0, 0);
-#pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = kParts ? acc[i] + part[i] : part[i];
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+// Eight fp32 values as three bf16 parts each, whose sum is the value itself (8 + 8 + 8 bits; the first part is cut off instead of rounded, so
+// that no finite value becomes infinite): the operand of a product of 32 x 32 x 16.
+struct Split {
+  u32x4 part[3];
+};
+// x less the low (high) half of a pair of bf16 values, as a product of pairs with (-1, 0) or (0, -1): one instruction for two.  (The constants
+// are kept in scalar registers: as an operand inside the instruction -1 stands in the other half.)
+__device__ __forceinline__ float less_half(float x, uint32_t pair, uint32_t minus_one) {
+  asm("" : "+s"(minus_one));
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pair), __builtin_bit_cast(bf16x2_t, minus_one), x, false);
 }
-// o[column of the chunk][lane's row] += sum over the chunk's rows of chunk[row][column] * w[row]; w in accumulator order
-__device__ __forceinline__ void acc_chunk(f32x16& o, uint32_t chunk, uint32_t col_lane, const float (&w)[16]) {
+__device__ __forceinline__ float less_lo(float x, uint32_t pair) { return less_half(x, pair, 0x0000bf80u); }
+__device__ __forceinline__ float less_hi(float x, uint32_t pair) { return less_half(x, pair, 0xbf800000u); }
+__device__ __forceinline__ Split split8(const float* x) {
+  Split r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float x0 = x[2 * i], x1 = x[2 * i + 1];
+    const uint32_t hi = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, x1), __builtin_bit_cast(uint32_t, x0), 0x07060302u);
+    const float r0 = less_lo(x0, hi), r1 = less_hi(x1, hi);
+    const uint32_t mid = pack2<bf16_t>(r0, r1);
+    r.part[0][i] = hi;
+    r.part[1][i] = mid;
+    r.part[2][i] = pack2<bf16_t>(less_lo(r0, mid), less_hi(r1, mid));
+  }
+  return r;
+}
+// main + small += a b of fp32 operands: the six products of their parts that fp32 can see, the largest of them apart from the others (each
+// product rounds its accumulator, and the small ones' is 2^-7 of it)
+__device__ __forceinline__ void mfma_split(const Split& a, const Split& b, f32x16& main, f32x16& small) {
+  small = mfma_16bit<bf16_t>(a.part[2], b.part[0], small);
+  small = mfma_16bit<bf16_t>(a.part[0], b.part[2], small);
+  small = mfma_16bit<bf16_t>(a.part[1], b.part[1], small);
+  small = mfma_16bit<bf16_t>(a.part[1], b.part[0], small);
+  small = mfma_16bit<bf16_t>(a.part[0], b.part[1], small);
+  main = mfma_16bit<bf16_t>(a.part[0], b.part[0], main);
+}
+
+// kPairs pairs of 16-byte pieces of a row, the lane's half of each
+template <int kPairs> __device__ __forceinline__ void load_row(const unsigned char* row, int lh, uint32_t (&f)[4 * kPairs]) {
+#pragma unroll
+  for (int g = 0; g < kPairs; ++g) {
+    const u32x4 raw = *reinterpret_cast<const u32x4*>(row + 32 * g + 16 * lh);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[g * 4 + e] = raw[e];
+  }
+}
+
+// The lane's own row as the operand of products over the columns: of every chunk the pieces 2 g + lh (load_row)
+template <typename T, int NC> struct OwnRow {
+  static constexpr bool k16 = is16<T>::value;
+  uint32_t f[k16 ? 16 * NC : 1];
+  Split sp[k16 ? 1 : 2 * NC];
+  __device__ __forceinline__ void load(const unsigned char* row, int lh) {
+    if constexpr (k16) {
+      load_row<4 * NC>(row, lh, f);
+    } else {
+      uint32_t raw[16 * NC];
+      load_row<4 * NC>(row, lh, raw);
+#pragma unroll
+      for (int s = 0; s < 2 * NC; ++s) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = __builtin_bit_cast(float, raw[8 * s + e]);
+        sp[s] = split8(x);
+      }
+    }
+  }
+  __device__ __forceinline__ const Split& get(int s) const { return sp[s]; }
+};
+// The same in LDS, for kernels that have no registers for it (the workgroup's waves have the same rows): 64 lanes x 16 bytes per operand
+template <int NC> struct OwnRowLds {
+  static constexpr int kBytes = 2 * NC * 3 * 1024;
+  uint32_t at;
+  // each wave splits its share of the steps; a barrier has to come in front of the first get()
+  __device__ __forceinline__ OwnRowLds(const unsigned char* row, unsigned char* lds, int wave, int lane) : at((uint32_t)(uintptr_t)lds + lane * 16) {
+    for (int s = wave; s < 2 * NC; s += kWaves) {
+      float x[8];
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const f32x4 raw = *reinterpret_cast<const f32x4*>(row + 64 * s + 32 * g + 16 * (lane >> 5));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[4 * g + e] = raw[e];
+      }
+      const Split sp = split8(x);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4*>(lds + (s * 3 + i) * 1024 + lane * 16) = sp.part[i];
+    }
+  }
+  __device__ __forceinline__ Split get(int s) const { return Split{{lds_read16(at, (s * 3) * 1024), lds_read16(at, (s * 3 + 1) * 1024), lds_read16(at, (s * 3 + 2) * 1024)}}; }
+};
+// acc (+ small) += (rows of chunk c) . (the lane's own row) over the chunk's columns
+template <typename T, typename Own> __device__ __forceinline__ void dot_chunk(f32x16& acc, f32x16& small, uint32_t chunk, uint32_t row_lane, const Own& own, int c) {
+  u32x4 a[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) a[g] = lds_read16((chunk + row_lane) ^ (g << 5));
+  if constexpr (is16<T>::value) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const uint32_t* f = own.f + 16 * c + 4 * g;
+      acc = mfma_16bit<T>(a[g], u32x4{f[0], f[1], f[2], f[3]}, acc);
+    }
+  } else {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      float x[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t word = a[2 * s + e / 4][e % 4];  // (a bit cast of a vector's element takes the wrong one)
+        x[e] = __builtin_bit_cast(float, word);
+      }
+      mfma_split(split8(x), own.get(2 * c + s), acc, small);
+    }
+  }
+}
+// a block's sixteen weights of the lane's row, in accumulator order, as operands
+__device__ __forceinline__ void split16(const float (&w)[16], Split (&sp)[2]) {
+  sp[0] = split8(w);
+  sp[1] = split8(w + 8);
+}
+// o[x][column of the chunk][lane's row] += sum over the chunk's rows of chunk[row][column] * (weights x)[row]
+template <int kN> __device__ __forceinline__ void acc_chunk(f32x16* const (&o)[kN], uint32_t chunk, uint32_t col_lane, const Split (&w)[kN][2]) {
   float a[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
@@ -167,8 +292,21 @@ __device__ __forceinline__ void acc_chunk(f32x16& o, uint32_t chunk, uint32_t co
     const int x = (4 * ((i >> 2) & 1)) ^ ((i >> 1) & 1);
     a[i] = *(const __attribute__((address_space(3))) float*)(((chunk + col_lane) ^ (x << 4)) + (8 * (i >> 2) + (i & 3)) * 128);
   }
+  f32x16 part[kN];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) o = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], w[i], o, 0, 0, 0);
+  for (int n = 0; n < kN; ++n)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) part[n][i] = 0.f;
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const Split as = split8(a + 8 * s);
+#pragma unroll
+    for (int n = 0; n < kN; ++n) mfma_split(as, w[n][s], *o[n], part[n]);
+  }
+#pragma unroll
+  for (int n = 0; n < kN; ++n)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) (*o[n])[i] += part[n][i];
 }
 // the same for a 16-bit chunk of 64 columns (issue_t): o[0] takes columns 0 .. 31, o[1] the others
 template <typename T> __device__ __forceinline__ void acc_chunk_16(f32x16 (&o)[2], uint32_t chunk, int lane, const float (&w)[16]) {
@@ -227,16 +365,6 @@ __device__ __forceinline__ void combine_store(const f32x16 (&o)[D / 32], unsigne
     unsigned char* at_out = reinterpret_cast<unsigned char*>(out) + ((size_t)(row0 + row) * D + c * 4) * (is16<T>::value ? 2 : 4);
     if constexpr (is16<T>::value) *reinterpret_cast<u32x2*>(at_out) = u32x2{pack2<T>(s[0] * k, s[1] * k), pack2<T>(s[2] * k, s[3] * k)};
     else *reinterpret_cast<f32x4*>(at_out) = f32x4{s[0] * k, s[1] * k, s[2] * k, s[3] * k};
-  }
-}
-
-// kPairs pairs of 16-byte pieces of a row, the lane's half of each
-template <int kPairs> __device__ __forceinline__ void load_row(const unsigned char* row, int lh, uint32_t (&f)[4 * kPairs]) {
-#pragma unroll
-  for (int g = 0; g < kPairs; ++g) {
-    const u32x4 raw = *reinterpret_cast<const u32x4*>(row + 32 * g + 16 * lh);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) f[g * 4 + e] = raw[e];
   }
 }
 
@@ -328,19 +456,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int key_hi = p.causal ? (m0 + kRows < L ? m0 + kRows : L) : L;
   const int n_kblk = (key_hi + kRows - 1) / kRows;
   const float qs = p.qscale, inv_qs = 1.f / p.qscale, c0 = p.c0;
-  uint32_t qf[16 * NC];
-  load_row<4 * NC>(reinterpret_cast<const unsigned char*>(p.q) + (q_row0 + (live ? qi : L - 1)) * kStride, lh, qf);
-
   Ring<kStride> ring(smem + wave * (kStages * kChunk), lane);
   const uint32_t rl = row_lane_of(lq, lh), cl = col_lane_of(lq, lh);
-  auto src_k = [&](int blk, int s, int st) { ring.issue(kg, blk * kRows, L, s, st); };
+  auto src_k = [&](int blk, int s, int st) {
+    if (s == 0) ring.rows(blk * kRows, L);
+    ring.issue_rows(kg, s, st);
+  };
+  OwnRow<T, NC> qf;
   // scores of a block less `sub`, -inf on the keys the row may not see
   auto scores = [&](int blk, float init, auto&& next) -> f32x16 {
-    f32x16 acc;
+    f32x16 acc, small;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = init;
+    for (int i = 0; i < 16; ++i) {
+      acc[i] = init;
+      small[i] = 0.f;
+    }
 #pragma unroll
-    for (int c = 0; c < NC; ++c) dot_chunk<true, T>(acc, next(c), rl, qf + c * 16);
+    for (int c = 0; c < NC; ++c) dot_chunk<T>(acc, small, next(c), rl, qf, c);
+    if constexpr (!k16)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[i] += small[i];
     const int k0 = blk * kRows;
     if (k0 + kRows > L || (p.causal && k0 + kRows - 1 > m0)) {
       const int jb = k0 + 4 * lh;
@@ -532,6 +667,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     };
     if (wave < n_kblk) start<NC>(wave, n_kblk, kWaves, src_k);
+    qf.load(reinterpret_cast<const unsigned char*>(p.q) + (q_row0 + (live ? qi : L - 1)) * kStride, lh);
     while (true) {
       const int blk = step_no * kWaves + wave;
       if (blk < n_kblk) list_block(blk, [&](int s) -> uint32_t { return take<NC>(ring, blk, s, n_kblk, kWaves, src_k); });
@@ -715,13 +851,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (any && p.bmask && lane == 0)
       atomicOr(reinterpret_cast<uint32_t*>(p.bmask) + ((size_t)(b * p.Hq + h) * p.n_mblk + m0 / kMaskRows) * p.mask_words + (blk >> 6),
                1u << ((blk >> 1) & 31));
+    Split ws[1][2];
+    if constexpr (!k16) split16(w, ws[0]);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const uint32_t a = next(NC + c);
       if constexpr (k16) {
         if (any) acc_chunk_16<T>(o[c], a, lane, w);
       } else {
-        if (any) acc_chunk(o[c][0], a, cl, w);
+        f32x16* const to[1] = {&o[c][0]};
+        if (any) acc_chunk(to, a, cl, ws);
       }
     }
   });
@@ -735,16 +874,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// dQ: one walk for sum p, sum u, sum u dP, one for dX and dQ^T += K^T dX^T
+// dQ: one walk for sum p, sum u, sum u dP and the products of u (dP - c) and u with K
 // ---------------------------------------------------------------------------------------------------------
+// u x, 0 where u is 0, whatever x is (one instruction; the intrinsic has no builtin)
+__device__ float mul_legacy(float u, float x) __asm("llvm.amdgcn.fmul.legacy");
+__device__ __forceinline__ float times(float u, float x) { return mul_legacy(u, x); }
+
 template <int D> constexpr int bwd_smem() { return kRing > kWaves * kRows * D * 4 ? kRing : kWaves * kRows * D * 4; }
 
 template <int D, int AM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_rows32_dq_kernel(AttnBwdParams p) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void attn_rows32_dq_kernel(AttnBwdParams p) {
   constexpr int kStride = D * 4;
   constexpr int NC = kStride / 128;      // chunks per block
   __shared__ __align__(4096) unsigned char smem[bwd_smem<D>()];
   __shared__ float red[kWaves][3][kRows];
+  __shared__ __align__(16) unsigned char own_lds[2][OwnRowLds<NC>::kBytes];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
@@ -768,54 +912,89 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int lim = p.causal ? (qi < L - 1 ? qi : L - 1) : L - 1;
   const int key_hi = p.causal ? (m0 + kRows < L ? m0 + kRows : L) : L;
   const int n_kblk = (key_hi + kRows - 1) / kRows;
+  const int lim_all = p.causal ? (m0 < L - 1 ? m0 : L - 1) : L - 1;  // the smallest of the rows
   const float tau = live ? p.taus[q_row0 + qi] : INFINITY;
-  uint32_t qf[16 * NC], dof[16 * NC];
-  {
-    const size_t r = q_row0 + (live ? qi : L - 1);
-    load_row<4 * NC>(reinterpret_cast<const unsigned char*>(p.q) + r * kStride, lh, qf);
-    load_row<4 * NC>(reinterpret_cast<const unsigned char*>(p.dout) + r * kStride, lh, dof);
-  }
   Ring<kStride> ring(smem + wave * (kStages * kChunk), lane);
   const uint32_t rl = row_lane_of(lq, lh), cl = col_lane_of(lq, lh);
-  // chunks of a block: K, V and, for the second walk, K again
+  // chunks of a block: K, V and K again
   auto src = [&](int blk, int s, int st) {
-    const unsigned char* g = s < NC || s >= 2 * NC ? kg : vg;
-    ring.issue(g, blk * kRows, L, s % NC, st);
+    if (s == 0) ring.rows(blk * kRows, L);
+    ring.issue_rows(s < NC || s >= 2 * NC ? kg : vg, s % NC, st);
   };
-  // r = z - tau (-inf where the row may not look); false when no row of the block has a member, whose dP is then not formed
-  auto block_terms = [&](int blk, auto&& next, float (&r)[16], f32x16& dp) -> bool {
-    f32x16 s;
+  if (wave < n_kblk) start<3 * NC>(wave, n_kblk, kWaves, src);  // (in front of the own rows, whose split waits for their loads)
+  const size_t own = (q_row0 + (live ? qi : L - 1)) * kStride;
+  const OwnRowLds<NC> qf(reinterpret_cast<const unsigned char*>(p.q) + own, own_lds[0], wave, lane), dof(reinterpret_cast<const unsigned char*>(p.dout) + own, own_lds[1], wave, lane);
+  __syncthreads();
+  // dX = u (dP - delta) needs delta = (sum u dP) / (sum u) first; instead of a walk for it, the walk adds up u (dP - c) K and u K, of which
+  // dQ = the first less (delta - c) of the second.  c, the row's delta in its first block with members, keeps what is common to the
+  // dP of a row (dO along the mean of V) out of the sums, which would cancel there.
+  float zsum = 0.f, usum = 0.f, udp = 0.f, centre = 0.f;
+  bool centred = false;
+  f32x16 o[NC], ou[NC];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int c = 0; c < NC; ++c) dot_chunk<D == 64, float>(s, next(c), rl, qf + c * 16);
-    const int jb = blk * kRows + 4 * lh;
+    for (int i = 0; i < 16; ++i) o[c][i] = ou[c][i] = 0.f;
+  walk<3 * NC, true>(ring, wave, n_kblk, kWaves, src, [&](int blk, auto&& next) {
+    float r[16], dx[16], u[16];
+    f32x16 s, dp, small;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = dp[i] = small[i] = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) dot_chunk<float>(s, small, next(c), rl, qf, c);
     float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      r[i] = jb + 8 * (i >> 2) + (i & 3) <= lim ? fmaf(s[i], p.qscale, -tau) : -INFINITY;
-      mx = fmaxf(mx, r[i]);
+      r[i] = fmaf(s[i] + small[i], p.qscale, -tau);  // z - tau
+      small[i] = 0.f;
     }
-    const bool any = __builtin_amdgcn_ballot_w64(mx > 0.f) != 0ull;
+    if (blk * kRows + kRows - 1 > lim_all) {
+      const int jb = blk * kRows + 4 * lh;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const uint32_t a = next(NC + c);
-      if (any) dot_chunk<D == 64, float>(dp, a, rl, dof + c * 16);
+      for (int i = 0; i < 16; ++i) r[i] = jb + 8 * (i >> 2) + (i & 3) <= lim ? r[i] : -INFINITY;
     }
-    return any;
-  };
-  float zsum = 0.f, usum = 0.f, udp = 0.f;
-  walk<2 * NC>(ring, wave, n_kblk, kWaves, src, [&](int blk, auto&& next) {
-    float r[16];
-    f32x16 dp;
-    if (!block_terms(blk, next, r, dp)) return;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, r[i]);
+    if (__builtin_amdgcn_ballot_w64(mx > 0.f) == 0ull) {  // no row of the block has a member
+#pragma unroll
+      for (int c = NC; c < 3 * NC; ++c) next(c);
+      return;
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) dot_chunk<float>(dp, small, next(NC + c), rl, dof, c);
+    float bu = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      float pr, u;
-      bwd_prob<AM>(r[i], p.c0, pr, u);
+      float pr;
+      bwd_prob<AM>(r[i], p.c0, pr, u[i]);
       zsum += pr;
-      usum += u;
-      udp += u > 0.f ? u * dp[i] : 0.f;
+      bu += u[i];
+      dp[i] += small[i];
+    }
+    usum += bu;
+    if (__builtin_amdgcn_ballot_w64(!centred && bu > 0.f) != 0ull) {
+      float bd = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) bd += times(u[i], dp[i]);
+      bd += __shfl_xor(bd, 32, 64);
+      bu += __shfl_xor(bu, 32, 64);
+      if (!centred && bu > 0.f) {
+        centre = bd * fast_rcp(bu);
+        centred = true;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      dx[i] = times(u[i], dp[i] - centre);
+      udp += dx[i];
+    }
+    Split w[2][2];
+    split16(dx, w[0]);
+    split16(u, w[1]);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      f32x16* const to[2] = {&o[c], &ou[c]};
+      acc_chunk(to, next(2 * NC + c), cl, w);
     }
   });
   zsum += __shfl_xor(zsum, 32, 64);
@@ -824,40 +1003,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (lh == 0) {
     red[wave][0][lq] = zsum;
     red[wave][1][lq] = usum;
-    red[wave][2][lq] = udp;
+    red[wave][2][lq] = fmaf(centre, usum, udp);
   }
-  __syncthreads();
+  __syncthreads();  // (every wave is done with its ring, too)
   auto all = [&](int k) { return (red[0][k][lq] + red[1][k][lq]) + (red[2][k][lq] + red[3][k][lq]); };
   zsum = all(0);
   usum = all(1);
-  udp = all(2);
-  const float delta = usum > 0.f ? udp / usum : 0.f;
+  const float delta = usum > 0.f ? all(2) / usum : 0.f;
   if (live && wave == 0 && lh == 0) {
     p.delta[q_row0 + qi] = delta;
     p.zinv[q_row0 + qi] = zsum > 0.f ? 1.f / zsum : 0.f;
   }
-  f32x16 o[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) o[c][i] = 0.f;
-  walk<3 * NC>(ring, wave, n_kblk, kWaves, src, [&](int blk, auto&& next) {
-    float r[16], dx[16];
-    f32x16 dp;
-    const bool any = block_terms(blk, next, r, dp);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      float pr, u;
-      bwd_prob<AM>(r[i], p.c0, pr, u);
-      dx[i] = u > 0.f ? u * (dp[i] - delta) : 0.f;
-    }
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const uint32_t a = next(2 * NC + c);
-      if (any) acc_chunk(o[c], a, cl, dx);
-    }
-  });
-  __syncthreads();  // every wave is done with its ring
+    for (int i = 0; i < 16; ++i) o[c][i] = fmaf(centre - delta, ou[c][i], o[c][i]);
   const float sm = p.sm_scale;
   combine_store<D>(o, smem, reinterpret_cast<float*>(dq), m0, N, wave, lane,
                    [&](int) { return sm; });
@@ -872,6 +1032,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   constexpr int NC = kStride / 128;      // chunks per block
   __shared__ __align__(4096) unsigned char smem[bwd_smem<D>()];
   __shared__ __align__(256) float scal[kWaves][4 * kRows];  // of the wave's block: tau, 1 / sum p, delta (and delta once more)
+  __shared__ __align__(16) unsigned char own_lds[2][OwnRowLds<NC>::kBytes];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
@@ -894,12 +1055,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   }
   const int kj = n0 + lq;
   const bool live = kj < L;
-  uint32_t kf[16 * NC], vf[16 * NC];
-  {
-    const size_t r = kv_row0 + (live ? kj : L - 1);
-    load_row<4 * NC>(reinterpret_cast<const unsigned char*>(p.k) + r * kStride, lh, kf);
-    load_row<4 * NC>(reinterpret_cast<const unsigned char*>(p.v) + r * kStride, lh, vf);
-  }
   const int q_first = p.causal ? kblk : 0;            // first query block that sees the keys
   const int n_q = (L + kRows - 1) / kRows - q_first;  // query blocks per head
   const size_t q_head0 = (size_t)(b * p.Hq + kvh * group) * N;
@@ -916,20 +1071,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
       dma4((lane < 32 ? p.taus : p.zinv) + at, &scal[wave][0]);
       dma4(p.delta + at, &scal[wave][64]);
     }
-    ring.issue(base, qb * kRows, L, s % NC, st);
+    if (s == 0) ring.rows(qb * kRows, L);
+    ring.issue_rows(base, s % NC, st);
   };
+  if (wave < n_q * group) start<4 * NC>(wave, n_q * group, kWaves, src);
+  const size_t own = (kv_row0 + (live ? kj : L - 1)) * kStride;
+  const OwnRowLds<NC> kf(reinterpret_cast<const unsigned char*>(p.k) + own, own_lds[0], wave, lane), vf(reinterpret_cast<const unsigned char*>(p.v) + own, own_lds[1], wave, lane);
+  __syncthreads();
   f32x16 ov[NC], ok[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
     for (int i = 0; i < 16; ++i) ov[c][i] = ok[c][i] = 0.f;
-  walk<4 * NC>(ring, wave, n_q * group, kWaves, src, [&](int x, auto&& next) {
+  walk<4 * NC, true>(ring, wave, n_q * group, kWaves, src, [&](int x, auto&& next) {
     const int g = x / n_q, q0 = (q_first + (x - g * n_q)) * kRows;
-    f32x16 s, dp;
+    f32x16 s, dp, small;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
+    for (int i = 0; i < 16; ++i) s[i] = dp[i] = small[i] = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) dot_chunk<D == 64, float>(s, next(c), rl, kf + c * 16);
+    for (int c = 0; c < NC; ++c) dot_chunk<float>(s, small, next(c), rl, kf, c);
     // tau, 1 / sum p and delta of the lane's sixteen queries: they came in front of the block's first chunk
     auto scalars = [&](int which, float (&y)[16]) {
 #pragma unroll
@@ -943,39 +1103,49 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     scalars(0, tau);
     scalars(1, zi);
     scalars(2, de);
-    const bool whole = q0 + kRows <= L;
     float r[16], w[16], dx[16];
     float mx = -INFINITY;
-    const bool plain = whole && n0 + kRows <= L && (!p.causal || n0 + kRows - 1 <= q0);  // every query of the block sees every key
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int qrow = q0 + 8 * (i >> 2) + 4 * lh + (i & 3);
-      const bool see = plain || (live && qrow < L && (!p.causal || kj <= qrow));
-      r[i] = see ? fmaf(s[i], p.qscale, -tau[i]) : -INFINITY;
-      mx = fmaxf(mx, r[i]);
+      r[i] = fmaf(s[i] + small[i], p.qscale, -tau[i]);
+      small[i] = 0.f;
     }
-    const bool any = __builtin_amdgcn_ballot_w64(mx > 0.f) != 0ull;
+    if (q0 + kRows > L || n0 + kRows > L || (p.causal && n0 + kRows - 1 > q0)) {  // not every query of the block sees every key
+      const int first = live ? (p.causal ? kj : 0) : L;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const uint32_t a = next(NC + c);
-      if (any) dot_chunk<D == 64, float>(dp, a, rl, vf + c * 16);
+      for (int i = 0; i < 16; ++i) {
+        const int qrow = q0 + 8 * (i >> 2) + 4 * lh + (i & 3);
+        r[i] = (int)(qrow >= first) & (int)(qrow < L) ? r[i] : -INFINITY;
+      }
     }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, r[i]);
+    if (__builtin_amdgcn_ballot_w64(mx > 0.f) == 0ull) {
+#pragma unroll
+      for (int c = NC; c < 4 * NC; ++c) next(c);
+      return;
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) dot_chunk<float>(dp, small, next(NC + c), rl, vf, c);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       float pr, u;
       bwd_prob<AM>(r[i], p.c0, pr, u);
-      w[i] = pr > 0.f ? pr * zi[i] : 0.f;
-      dx[i] = u > 0.f ? u * (dp[i] - de[i]) : 0.f;
+      w[i] = times(pr, zi[i]);
+      dx[i] = times(u, dp[i] + small[i] - de[i]);
     }
+    Split ws[1][2];
+    split16(w, ws[0]);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      const uint32_t a = next(2 * NC + c);
-      if (any) acc_chunk(ov[c], a, cl, w);
+      f32x16* const to[1] = {&ov[c]};
+      acc_chunk(to, next(2 * NC + c), cl, ws);
     }
+    split16(dx, ws[0]);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      const uint32_t a = next(3 * NC + c);
-      if (any) acc_chunk(ok[c], a, cl, dx);
+      f32x16* const to[1] = {&ok[c]};
+      acc_chunk(to, next(3 * NC + c), cl, ws);
     }
   });
   __syncthreads();  // every wave is done with its ring

@@ -259,3 +259,35 @@ def test_lists_that_fill_up_between_two_solves(members, alpha, dtype):
     want = exact.dense_entmax_attention(q, k, v, alpha, False, vl)
     got = A.adasplash_v1(*(t.to(DEV) for t in (q, k, v)), alpha=alpha, is_causal=False, varlen=vl.to(DEV)).double().cpu()
     assert (got - want).norm() <= (2e-6 if dtype == torch.float32 else 2.0 ** -8) * want.norm()
+
+
+@pytest.mark.parametrize("alpha,causal,Hq,Hkv,D,q_scale,v_mean", [(1.5, True, 4, 2, 64, 1.0, 0.0), (1.5, True, 2, 1, 128, 3.0, 0.0), (1.5, True, 2, 2, 64, 0.125, 10.0),
+                                                                  (1.5, True, 2, 2, 128, 1.0, 10.0), (1.333, False, 2, 2, 64, 1.0, 0.0), (2.0, False, 2, 2, 128, 1.0, 0.0)])
+def test_errors_are_those_of_single_precision(alpha, causal, Hq, Hkv, D, q_scale, v_mean):
+    """Products of three-part operands, and dQ from sums around a row's first delta: 2e-6 is 17 roundings of 2^-23, about twice what products in
+    single precision show for a V of mean 10; a part that is left out costs 2^-17 = 8e-6 or more."""
+    g = torch.Generator().manual_seed(12)
+    N, varlen = 289, torch.tensor([289, 250], dtype=torch.int32)
+    q = q_scale * torch.randn(2, Hq, N, D, generator=g)
+    k, v = (torch.randn(2, Hkv, N, D, generator=g) for _ in range(2))
+    v += v_mean
+    dout = torch.randn(2, Hq, N, D, generator=g)
+    want = [exact.dense_entmax_attention(q, k, v, alpha, causal, varlen)]
+    want += list(exact.dense_entmax_attention_grads(q, k, v, dout, alpha, causal, varlen))
+    for name, a, w in zip(("out", "dq", "dk", "dv"), run(q, k, v, dout, varlen, alpha, causal, Hq != Hkv), want):
+        rel = ((a.double().cpu() - w.double()).norm() / w.double().norm()).item()
+        assert rel < 2e-6, (name, rel)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_largest_finite_values_stay_finite(D):
+    """The first of a value's three parts is cut off, not rounded: the type's largest value stays finite, and times 0 it is 0."""
+    g = torch.Generator().manual_seed(13)
+    q, k, v, dout = (torch.randn(1, 2, 128, D, generator=g) for _ in range(4))
+    q[..., 5] = 0.0
+    k[..., 5] = torch.finfo(torch.float32).max
+    got = run(q, k, v, dout, None, 1.5, True, False)
+    k[..., 5] = 0.0
+    want = run(q, k, v, dout, None, 1.5, True, False)
+    for name, a, w in zip(("out", "dk", "dv"), (got[0], got[2], got[3]), (want[0], want[2], want[3])):
+        assert torch.equal(a, w), name
