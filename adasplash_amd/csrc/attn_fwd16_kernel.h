@@ -50,14 +50,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int N = p.N, group = p.Hq / p.Hkv, n_blk = (N + kRows - 1) / kRows;
   int bkv, mi, hg;
   if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_blk, group, p.causal != 0, 2ll * N * kRow, bkv, mi, hg)) return;
-  const int b = bkv / p.Hkv, kvh = bkv % p.Hkv, h = kvh * group + hg, bh = b * p.Hq + h;
+  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.causal == 0);
+  const int b = item.b, L = item.L, kvh = bkv % p.Hkv, h = kvh * group + hg, bh = b * p.Hq + h;
+  bkv = b * p.Hkv + kvh;
   const int mblk = n_blk - 1 - mi, m0 = mblk * kRows;
   if (!left.takes((size_t)bh * p.n_mblk + mblk)) return;
-  int L = N;
-  if (p.varlen) {
-    const long long l = p.varlen_bits == 64 ? ((const long long*)p.varlen)[b] : (long long)((const int*)p.varlen)[b];
-    L = (int)(l < 0 ? 0 : (l > N ? N : l));
-  }
   const size_t q_row0 = (size_t)bh * N;
   unsigned char* const out = reinterpret_cast<unsigned char*>(p.out) + q_row0 * kRow;
   int32_t* const bmask = p.bmask ? p.bmask + ((size_t)bh * p.n_mblk + mblk) * p.mask_words : nullptr;

@@ -193,6 +193,34 @@ __device__ __forceinline__ bool xcd_block_map(bool padded, int units, int blocks
   return true;
 }
 
+// The item at place `pos` of a batch, and its length; `longest_first`: the places are in the order of the lengths.  Workgroups start in the
+// order of their numbers, and those that find no slot at first start when others end: a long sequence in that place makes a launch longer.
+// The lengths come with one load, a lane each; beyond 64 items the order is theirs, with enough workgroups for the places to even out.
+// For kernels whose blocks of a sequence cost the same (not causal) and take long: 16 x 12 heads, N <= 500, D = 64, bf16, us, the items'
+// order -> this: dK/dV 43.8 -> 37.7, dQ 39.5 -> 37.0; 8 x 16 heads, N <= 2000, flat, alpha = 1.333: forward 370 -> 346, forward and
+// backward 839 -> 782.  Causal launches, whose sets of heads run longest block first, lose (8 x 16 heads, N <= 2000, flat: 320 -> 340),
+// and so do the short workgroups of the resident forward (16 x 12 heads: 40.9 -> 43.0; 32 x 8 of 300: 25.6 -> 29.3).
+struct BatchItem {
+  int b, L;
+};
+__device__ __forceinline__ BatchItem batch_item(const void* varlen, int varlen_bits, int B, int N, int pos, bool longest_first) {
+  if (!varlen) return {pos, N};
+  auto length_of = [&](int i) -> int {
+    const long long l = varlen_bits == 64 ? ((const long long*)varlen)[i] : (long long)((const int*)varlen)[i];
+    return (int)(l < 0 ? 0 : (l > N ? N : l));
+  };
+  if (!longest_first || B > 64) return {pos, length_of(pos)};
+  const int lane = (int)(threadIdx.x & 63);
+  const int len = length_of(lane < B ? lane : B - 1);
+  int rank = lane < B ? 0 : B;
+  for (int i = 0; i < B; ++i) {
+    const int other = __builtin_amdgcn_readlane(len, i);
+    rank += (int)(other > len) | ((int)(other == len) & (int)(i < lane));
+  }
+  const int b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(rank == pos));
+  return {b, __builtin_amdgcn_readlane(len, b)};
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }

@@ -77,3 +77,23 @@ def test_a_padded_batch_equals_its_items(dense_only, B, Hq, Hkv, N, D, causal, d
     for b in range(B):
         for name, w, o in zip(("out", "dq", "dk", "dv"), whole, run(slice(b, b + 1))):
             assert torch.equal(w[b], o[0]), f"{name}: batch item {b} differs from the item run alone"
+
+
+# not causal, with lengths: the kernels on all pairs take the items longest first (equal lengths, a length of 0, 64 items, and 65, whose order stays)
+@pytest.mark.parametrize("lens,H,N", [([70, 200, 200, 0, 129, 1], 3, 200), ([1 + 37 * i % 61 for i in range(64)], 1, 64), ([1 + 37 * i % 61 for i in range(65)], 1, 64)])
+@pytest.mark.parametrize("bits", [torch.int32, torch.int64])
+def test_items_of_a_padded_batch_longest_first(dense_only, lens, H, N, bits):
+    g = torch.Generator().manual_seed(len(lens))
+    B = len(lens)
+    q, k, v, dout = (torch.randn(B, H, N, 64, generator=g).bfloat16().to(DEV) for _ in range(4))
+    varlen = torch.tensor(lens, dtype=bits, device=DEV)
+
+    def run(rows):
+        a = [t[rows].contiguous() for t in (q, k, v, dout)]
+        out, taus, bmask = _attention.launch_forward(*a[:3], version=1, alpha=1.5, is_causal=False, niter=4, varlen=varlen[rows].contiguous())
+        return out, *_attention.launch_backward(*a, taus, bmask, alpha=1.5, is_causal=False, varlen=varlen[rows].contiguous())[:3]
+
+    whole = run(slice(None))
+    for b in range(0, B, 1 if B < 10 else 7):
+        for name, w, o in zip(("out", "dq", "dk", "dv"), whole, run(slice(b, b + 1))):
+            assert torch.equal(w[b], o[0]), f"{name}: batch item {b} differs from the item run alone"
