@@ -434,13 +434,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int N = p.N, group = p.Hq / p.Hkv, n_rblk = (N + kRows - 1) / kRows;
   int bkv, mi, hg;
   if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
-  const int b = bkv / p.Hkv, kvh = bkv % p.Hkv, h = kvh * group + hg;
+  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.causal == 0);
+  const int b = item.b, L = item.L, kvh = bkv % p.Hkv, h = kvh * group + hg;
+  bkv = b * p.Hkv + kvh;
   const int m0 = (n_rblk - 1 - mi) * kRows;
-  int L = N;
-  if (p.varlen) {
-    const long long l = p.varlen_bits == 64 ? ((const long long*)p.varlen)[b] : (long long)((const int*)p.varlen)[b];
-    L = (int)(l < 0 ? 0 : (l > N ? N : l));
-  }
   const size_t q_row0 = (size_t)(b * p.Hq + h) * N;
   unsigned char* const out = reinterpret_cast<unsigned char*>(p.out) + q_row0 * kStride;
   if (m0 >= L) {
@@ -895,9 +892,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   const int N = p.N, group = p.Hq / p.Hkv, n_rblk = (N + kRows - 1) / kRows;
   int bkv, mi, hg;
   if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
-  const int b = bkv / p.Hkv, kvh = bkv % p.Hkv, h = kvh * group + hg;
+  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.causal == 0);
+  const int b = item.b, L = item.L, kvh = bkv % p.Hkv, h = kvh * group + hg;
+  bkv = b * p.Hkv + kvh;
   const int m0 = (n_rblk - 1 - mi) * kRows;
-  const int L = bwd_seq_len(p, b);
   const size_t q_row0 = (size_t)(b * p.Hq + h) * N;
   unsigned char* const dq = reinterpret_cast<unsigned char*>(p.dq) + q_row0 * kStride;
   if (m0 >= L) {
@@ -1039,8 +1037,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   const int N = p.N, group = p.Hq / p.Hkv, n_rblk = (N + kRows - 1) / kRows;
   int bkv, kblk, member_unused;
   if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, 1, p.causal != 0, 2ll * group * N * kStride, bkv, kblk, member_unused)) return;
-  const int b = bkv / p.Hkv, kvh = bkv % p.Hkv;
-  const int L = bwd_seq_len(p, b);
+  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.causal == 0);
+  const int b = item.b, L = item.L, kvh = bkv % p.Hkv;
+  bkv = b * p.Hkv + kvh;
   const int n0 = kblk * kRows;
   const size_t kv_row0 = (size_t)bkv * N;
   unsigned char* const dk = reinterpret_cast<unsigned char*>(p.dk) + kv_row0 * kStride;

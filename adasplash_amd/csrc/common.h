@@ -198,7 +198,8 @@ __device__ __forceinline__ bool xcd_block_map(bool padded, int units, int blocks
 // The lengths come with one load, a lane each; beyond 64 items the order is theirs, with enough workgroups for the places to even out.
 // For kernels whose blocks of a sequence cost the same (not causal) and take long: 16 x 12 heads, N <= 500, D = 64, bf16, us, the items'
 // order -> this: dK/dV 43.8 -> 37.7, dQ 39.5 -> 37.0; 8 x 16 heads, N <= 2000, flat, alpha = 1.333: forward 370 -> 346, forward and
-// backward 839 -> 782.  Causal launches, whose sets of heads run longest block first, lose (8 x 16 heads, N <= 2000, flat: 320 -> 340),
+// backward 839 -> 782; fp32, alpha = 1.333, 8 x 8 heads, N <= 700: 291 -> 275; 6 x 8 of 600, D = 128, alpha = 2: 255 -> 237.  Causal launches, whose sets of heads run longest block first, lose (8 x 16 heads, N <= 2000, flat: 320 -> 340;
+// fp32, D = 128: 4 x 8 heads, N <= 1100: 410 -> 444, 4 x 16/4: 704 -> 627),
 // and so do the short workgroups of the resident forward (16 x 12 heads: 40.9 -> 43.0; 32 x 8 of 300: 25.6 -> 29.3).
 struct BatchItem {
   int b, L;

@@ -81,11 +81,11 @@ def test_a_padded_batch_equals_its_items(dense_only, B, Hq, Hkv, N, D, causal, d
 
 # not causal, with lengths: the kernels on all pairs take the items longest first (equal lengths, a length of 0, 64 items, and 65, whose order stays)
 @pytest.mark.parametrize("lens,H,N", [([70, 200, 200, 0, 129, 1], 3, 200), ([1 + 37 * i % 61 for i in range(64)], 1, 64), ([1 + 37 * i % 61 for i in range(65)], 1, 64)])
-@pytest.mark.parametrize("bits", [torch.int32, torch.int64])
-def test_items_of_a_padded_batch_longest_first(dense_only, lens, H, N, bits):
+@pytest.mark.parametrize("bits,dtype", [(torch.int32, torch.bfloat16), (torch.int64, torch.bfloat16), (torch.int32, torch.float32)])
+def test_items_of_a_padded_batch_longest_first(dense_only, lens, H, N, bits, dtype):
     g = torch.Generator().manual_seed(len(lens))
     B = len(lens)
-    q, k, v, dout = (torch.randn(B, H, N, 64, generator=g).bfloat16().to(DEV) for _ in range(4))
+    q, k, v, dout = (torch.randn(B, H, N, 64, generator=g).to(dtype).to(DEV) for _ in range(4))
     varlen = torch.tensor(lens, dtype=bits, device=DEV)
 
     def run(rows):
