@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
 
     __syncthreads();  // the previous row block is done with LDS and with s_item
     if (tid == 0) {
-      const int got = draw_item(p.queue, per_xcd, total, &s_draw);
+      const int got = draw_item(p.queue, per_xcd, total, p.causal && (!p.varlen || p.B == 1) ? group * n_mblk : 0, &s_draw);
       s_item = got;
       s_skip = 0;
       if (got >= 0) {  // the K/V head of the row block, as decoded below
@@ -761,7 +761,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
 
     __syncthreads();  // the previous row block is done with LDS and with s_item
     if (tid == 0) {
-      const int got = draw_item(p.queue2, per_xcd, total, &s_draw);
+      const int got = draw_item(p.queue2, per_xcd, total, 0, &s_draw);
       s_item = got;
       s_skip = 0;
       if (got >= 0) {  // the K/V head of the row block, as decoded below
@@ -1264,7 +1264,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_DKDV_W
   for (;;) {
     __syncthreads();  // the previous item is done with s_item
     if (tid == 0) {
-      const int got = draw_item(p.queue2, per_xcd, total, &s_draw);
+      const int got = draw_item(p.queue2, per_xcd, total, 0, &s_draw);
       s_item = got;
       s_skip = 0;
       if (got >= 0) {  // the K/V head of the key block, as decoded below: marked dense by the probe?

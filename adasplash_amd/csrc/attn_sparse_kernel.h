@@ -138,16 +138,27 @@ __device__ __forceinline__ bool sparse_steps_aside(const uint32_t* hints, const 
 // which about 85).  So with up to two items per workgroup each takes the items of its own number -- the second ones in
 // reverse, the longest items coming first -- and no counter is touched.  (First items by number in a long launch too, or a
 // look at a counter before it is incremented: 1-2 % slower at 16384 items.)
+// A causal launch of at most one item per workgroup has all of them under way at once, and what counts is that every CU has about the same
+// to do: the items of an XCD's heads (`inner` each, longest first; 0: not causal, or of different lengths) are taken block by block over the heads, and every second
+// round over the XCD's 32 CUs backwards, so that the CU with the longest item of one round has the shortest of the next.  us, head after
+// head -> this: forward of 16 heads, N = 4096, D = 64: 189 -> 174, 2 x 16, N = 2048: 129 -> 120, 8 heads, N = 8192, D = 128: 298 -> 288, 2 x 8/4, N = 4096:
+// 190 -> 185; forward and backward 363 -> 345, 282 -> 270, 575 -> 562, 448 -> 441.  Padded batches, whose heads' blocks are not the same length, now
+// and then lose (4 x 8 heads, N <= 3900, D = 128: 187 -> 196).
 // `drawn` is in LDS (0 in front of the first call) and everything else is formed anew on every call -- the empty asm hides
 // that it repeats --: the kernels have no registers to spare for it between two draws.
-__device__ __forceinline__ int draw_item(uint32_t* queue, int per_xcd, int total, int* drawn) {
+__device__ __forceinline__ int draw_item(uint32_t* queue, int per_xcd, int total, int inner, int* drawn) {
   uint32_t bid = blockIdx.x, per_part = gridDim.x >> 3;
   asm volatile("" : "+s"(bid), "+s"(per_part));
   const int own = (int)(bid & 7u), n = (int)per_part;
   int k = *drawn, got = -1;
   if (2 * n >= per_xcd) {  // k: items taken
     for (; k < 2 && got < 0; ++k) {
-      const int i = k == 0 ? (int)(bid >> 3) : 2 * n - 1 - (int)(bid >> 3);
+      int i = k == 0 ? (int)(bid >> 3) : 2 * n - 1 - (int)(bid >> 3);
+      if (inner > 0 && n >= per_xcd && i < per_xcd && per_xcd * 8 == total && per_xcd % inner == 0) {
+        const int heads = per_xcd / inner, round = i & ~31, end = round + 32 < per_xcd ? round + 32 : per_xcd;
+        const int place = i & 32 ? end - 1 - (i - round) : i;
+        i = place % heads * inner + place / heads;
+      }
       const int logical = own * per_xcd + i;
       if (i < per_xcd && logical < total) got = logical;
     }
@@ -242,7 +253,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
 
     __syncthreads();  // the previous row block is done with LDS and with s_item
     if (tid == 0) {
-      const int got = draw_item(p.queue, per_xcd, total, &s_draw);
+      const int got = draw_item(p.queue, per_xcd, total, p.causal && (!p.varlen || p.B == 1) ? group * n_mblk : 0, &s_draw);
       s_item = got;
       s_giveup[0] = 0u;
       s_giveup[1] = 0u;

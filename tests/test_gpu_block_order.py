@@ -97,3 +97,21 @@ def test_items_of_a_padded_batch_longest_first(dense_only, lens, H, N, bits, dty
     for b in range(0, B, 1 if B < 10 else 7):
         for name, w, o in zip(("out", "dq", "dk", "dv"), whole, run(slice(b, b + 1))):
             assert torch.equal(w[b], o[0]), f"{name}: batch item {b} differs from the item run alone"
+
+
+# at most one row block per workgroup of the kernels on the supports, two or three heads per XCD, a last round over the CUs that is not full
+@pytest.mark.parametrize("B,Hq,Hkv,N,D", [(2, 8, 8, 1024, 64), (3, 8, 8, 2048, 64), (2, 16, 8, 2048, 128)])
+def test_a_batch_equals_its_items_on_the_supports(B, Hq, Hkv, N, D):
+    g = torch.Generator().manual_seed(B + N)
+    q, dout = (torch.randn(B, Hq, N, D, generator=g).bfloat16().to(DEV) for _ in range(2))
+    k, v = (torch.randn(B, Hkv, N, D, generator=g).bfloat16().to(DEV) for _ in range(2))
+
+    def run(rows):
+        a = [t[rows].contiguous() for t in (q, k, v, dout)]
+        out, taus, bmask = _attention.launch_forward(*a[:3], version=2, alpha=1.5, is_causal=True, niter=2, varlen=None)
+        return out, taus, *_attention.launch_backward(*a, taus, bmask, alpha=1.5, is_causal=True, varlen=None)[:3]
+
+    whole = run(slice(None))
+    for b in range(B):
+        for name, w, o in zip(("out", "taus", "dq", "dk", "dv"), whole, run(slice(b, b + 1))):
+            assert torch.equal(w[b], o[0]), f"{name}: batch item {b} differs from the item run alone"
