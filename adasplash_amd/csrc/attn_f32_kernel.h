@@ -407,6 +407,52 @@ template <int AM> __device__ __forceinline__ float norm_step(float s0, float s1,
   return (g - 1.f) * s0 * fast_rcp(g * s1);
 }
 
+// Blocks of a causal launch, longest first over all heads of an XCD by what they walk (a padded batch's lengths included; empty blocks come
+// last).  `two`: of the kernels of which two workgroups run on a CU at a time, a launch that is under way at once has its second round over the XCD's 32 CUs
+// backwards, so that the CU with the longest block of the first has the shortest of the second.  In longer launches blocks go where one ends, and
+// every second round backwards costs: 4 x 16/4 heads, N = 1024, D = 128: 717 -> 792 us.
+// us, order of xcd_block_map -> this, forward and backward, D = 64: 2 x 8 heads, N = 1500 and 375: 159.0 -> 156.8; 2 x 8 of 1024: 121.6 -> 116.7;
+// 8 of 2048: 211 -> 202; 8 x 8, N <= 700: 141 -> 118; 4 x 16 of N <= 1024, forward: 72.6 -> 62.3; D = 128: 4 x 8, N <= 1100: 415 -> 262; 4 x 16/4, N <= 1024:
+// 584 -> 558.
+// For up to 2048 keys and eight heads per XCD, a lane per length and per head, with the heads' operands in 8 MB as in xcd_block_map.
+// `keys`: a block of keys is the longer the earlier it is.  False: the launch is not of this kind.
+__device__ __forceinline__ bool longest_first(const void* varlen, int varlen_bits, int B, int Hkv, int N, int group, bool causal, long long unit_bytes, bool keys, bool two,
+                                              int& bkv, int& rblk, int& member) {
+  const int n = (N + kRows - 1) / kRows, heads = B * Hkv / 8, x = (int)(blockIdx.x & 7);
+  if (!causal || n > 64 || (B * Hkv) % 8 != 0 || heads > 8 || heads * unit_bytes > (8ll << 20)) return false;
+  const int lane = (int)(threadIdx.x & 63);
+  int len = 0;  // blocks of head `lane` that are not empty; they are as long as 1, 2, ..., len
+  if (lane < heads) len = (batch_item(varlen, varlen_bits, B, N, (lane * 8 + x) / Hkv, false).L + kRows - 1) / kRows;
+  int longer = 0;  // blocks longer than `lane`
+  for (int u = 0; u < heads; ++u) {
+    const int more = __builtin_amdgcn_readlane(len, u) - lane;
+    longer += more > 0 ? more : 0;
+  }
+  const int total = __builtin_amdgcn_readlane(longer, 0) * group;
+  int s = (int)(blockIdx.x >> 3), u = 0;
+  if (s < total) {
+    if (two && total <= 64 && s >= 32) s = 31 + total - s;
+    const int t = 63 - __builtin_clzll(__builtin_amdgcn_ballot_w64(longer * group > s));  // the block is t + 1 long
+    const int j = s - (t < 63 ? __builtin_amdgcn_readlane(longer, t < 63 ? t + 1 : 63) * group : 0);
+    member = j % group;
+    unsigned long long with = __builtin_amdgcn_ballot_w64(len > t);
+    for (int k = j / group; k > 0; --k) with &= with - 1;
+    u = __builtin_ctzll(with);
+    rblk = keys ? __builtin_amdgcn_readlane(len, u) - 1 - t : t;
+  } else {
+    s -= total;
+    member = s % group;
+    int k = s / group, have = __builtin_amdgcn_readlane(len, 0);
+    while (u < heads - 1 && k >= n - have) {
+      k -= n - have;
+      have = __builtin_amdgcn_readlane(len, ++u);
+    }
+    rblk = have + k;
+  }
+  bkv = u * 8 + x;
+  return true;
+}
+
 // ---------------------------------------------------------------------------------------------------------
 // forward
 // ---------------------------------------------------------------------------------------------------------
@@ -432,8 +478,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
   const int N = p.N, group = p.Hq / p.Hkv, n_rblk = (N + kRows - 1) / kRows;
-  int bkv, mi, hg;
-  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
+  int bkv, mi, hg, rblk;
+  if (!k16 && longest_first(p.varlen, p.varlen_bits, p.B, p.Hkv, N, group, p.causal != 0, 2ll * N * kStride, false, true, bkv, rblk, hg)) mi = n_rblk - 1 - rblk;
+  else if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
   const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.causal == 0);
   const int b = item.b, L = item.L, kvh = bkv % p.Hkv, h = kvh * group + hg;
   bkv = b * p.Hkv + kvh;
@@ -890,8 +937,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
   const int N = p.N, group = p.Hq / p.Hkv, n_rblk = (N + kRows - 1) / kRows;
-  int bkv, mi, hg;
-  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
+  int bkv, mi, hg, rblk;
+  if (longest_first(p.varlen, p.varlen_bits, p.B, p.Hkv, N, group, p.causal != 0, 2ll * N * kStride, false, D == 64, bkv, rblk, hg)) mi = n_rblk - 1 - rblk;
+  else if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
   const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.causal == 0);
   const int b = item.b, L = item.L, kvh = bkv % p.Hkv, h = kvh * group + hg;
   bkv = b * p.Hkv + kvh;
@@ -1036,7 +1084,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
   const int N = p.N, group = p.Hq / p.Hkv, n_rblk = (N + kRows - 1) / kRows;
   int bkv, kblk, member_unused;
-  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, 1, p.causal != 0, 2ll * group * N * kStride, bkv, kblk, member_unused)) return;
+  if (!longest_first(p.varlen, p.varlen_bits, p.B, p.Hkv, N, 1, p.causal != 0, 2ll * group * N * kStride, true, D == 64, bkv, kblk, member_unused) &&
+      !xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, 1, p.causal != 0, 2ll * group * N * kStride, bkv, kblk, member_unused)) return;
   const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.causal == 0);
   const int b = item.b, L = item.L, kvh = bkv % p.Hkv;
   bkv = b * p.Hkv + kvh;

@@ -115,3 +115,32 @@ def test_a_batch_equals_its_items_on_the_supports(B, Hq, Hkv, N, D):
     for b in range(B):
         for name, w, o in zip(("out", "taus", "dq", "dk", "dv"), whole, run(slice(b, b + 1))):
             assert torch.equal(w[b], o[0]), f"{name}: batch item {b} differs from the item run alone"
+
+
+# fp32, causal: blocks longest first over an XCD's heads, against heads run alone, which take the general order (one and eight heads per XCD, 64 blocks, 64
+# blocks that are not empty and more, lengths of 0, a part of a block and equal ones)
+@pytest.mark.parametrize("lens,Hq,Hkv,N,D", [([70, 200, 0], 16, 8, 200, 64), ([2048], 8, 8, 2048, 64), ([1024, 1024], 8, 8, 1024, 64), ([33, 1, 300, 300], 16, 16, 300, 64),
+                                             ([700, 64, 511], 16, 8, 700, 128)])
+@pytest.mark.parametrize("bits", [None, torch.int32, torch.int64])
+def test_causal_blocks_longest_first(lens, Hq, Hkv, N, D, bits):
+    if bits is None and N & (N - 1):
+        pytest.skip("without lengths N is a power of two")
+    g = torch.Generator().manual_seed(N)
+    B, group = len(lens), Hq // Hkv
+    q, dout = (torch.randn(B, Hq, N, D, generator=g).to(DEV) for _ in range(2))
+    k, v = (torch.randn(B, Hkv, N, D, generator=g).to(DEV) for _ in range(2))
+    varlen = None if bits is None else torch.tensor(lens, dtype=bits, device=DEV)
+
+    def run(rows, heads):
+        qh = slice(heads.start * group, heads.stop * group)
+        a = [t[rows, h].contiguous() for t, h in ((q, qh), (k, heads), (v, heads), (dout, qh))]
+        vl = None if varlen is None else varlen[rows].contiguous()
+        out, taus, bmask = _attention.launch_forward(*a[:3], version=2, alpha=1.5, is_causal=True, niter=2, varlen=vl)
+        return out, *_attention.launch_backward(*a, taus, bmask, alpha=1.5, is_causal=True, varlen=vl)[:3]
+
+    whole = run(slice(None), slice(0, Hkv))
+    for b in range(B):
+        for h in (0, Hkv // 2, Hkv - 1):
+            for name, w, o in zip(("out", "dq", "dk", "dv"), whole, run(slice(b, b + 1), slice(h, h + 1))):
+                n = o.shape[1]
+                assert torch.equal(w[b, h * n:(h + 1) * n], o[0]), f"{name}: item {b}, head {h}"
