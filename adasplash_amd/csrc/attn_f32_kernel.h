@@ -283,8 +283,8 @@ __device__ __forceinline__ void split16(const float (&w)[16], Split (&sp)[2]) {
   sp[0] = split8(w);
   sp[1] = split8(w + 8);
 }
-// o[x][column of the chunk][lane's row] += sum over the chunk's rows of chunk[row][column] * (weights x)[row]
-template <int kN> __device__ __forceinline__ void acc_chunk(f32x16* const (&o)[kN], uint32_t chunk, uint32_t col_lane, const Split (&w)[kN][2]) {
+// o[x][column of the chunk][lane's row] += sum over the chunk's rows of chunk[row][column] * (weights x)[row]; kShift: o[0] -= shift o[1] before it
+template <bool kShift = false, int kN> __device__ __forceinline__ void acc_chunk(f32x16* const (&o)[kN], uint32_t chunk, uint32_t col_lane, const Split (&w)[kN][2], float shift = 0.f) {
   float a[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
@@ -296,7 +296,7 @@ template <int kN> __device__ __forceinline__ void acc_chunk(f32x16* const (&o)[k
 #pragma unroll
   for (int n = 0; n < kN; ++n)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) part[n][i] = 0.f;
+    for (int i = 0; i < 16; ++i) part[n][i] = kShift && n == 0 ? -shift * (*o[kN - 1])[i] : 0.f;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     const Split as = split8(a + 8 * s);
@@ -920,6 +920,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // ---------------------------------------------------------------------------------------------------------
 // dQ: one walk for sum p, sum u, sum u dP and the products of u (dP - c) and u with K
 // ---------------------------------------------------------------------------------------------------------
+// x of a row's two lanes, added up
+__device__ __forceinline__ float both_lanes(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __builtin_bit_cast(float, r[0]) + __builtin_bit_cast(float, r[1]);
+}
 // u x, 0 where u is 0, whatever x is (one instruction; the intrinsic has no builtin)
 __device__ float mul_legacy(float u, float x) __asm("llvm.amdgcn.fmul.legacy");
 __device__ __forceinline__ float times(float u, float x) { return mul_legacy(u, x); }
@@ -972,10 +978,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   const OwnRowLds<NC> qf(reinterpret_cast<const unsigned char*>(p.q) + own, own_lds[0], wave, lane), dof(reinterpret_cast<const unsigned char*>(p.dout) + own, own_lds[1], wave, lane);
   __syncthreads();
   // dX = u (dP - delta) needs delta = (sum u dP) / (sum u) first; instead of a walk for it, the walk adds up u (dP - c) K and u K, of which
-  // dQ = the first less (delta - c) of the second.  c, the row's delta in its first block with members, keeps what is common to the
-  // dP of a row (dO along the mean of V) out of the sums, which would cancel there.
+  // dQ = the first less (delta - c) of the second.  c is the row's delta over the wave's blocks so far, moved in front of a block that brings as much
+  // u as there was when it was last moved: what is added up around one c weighs no more than the keys whose delta c is, and roundings of the size
+  // of u |dP - c| stay within a small multiple of those of the terms u (dP - delta) themselves.  (With c kept from a wave's first member, whatever its weight, they
+  // do not: a V row of 1000 times the norm with u = 2^-10, 300 members: relative error of dQ 5.7e-5, as here 1.2e-7; K of mean 4: 1.4e-3, 9.7e-7.)
+  // The sums so far go over to the new c by o -= shift ou: at head dim 128, where they lie in accumulation registers that the vector pipe does not
+  // reach, as the start of the small products' sum.  us, 4 x 16/4 heads, N = 1024, forward and backward: 735 -> 694; D = 64, 2 x 8, N = 1500 and 375: 157.6, that way 160.2.
+  constexpr bool kShiftInPart = D != 64;
   float zsum = 0.f, usum = 0.f, udp = 0.f, centre = 0.f;
-  bool centred = false;
+  float mark = 0x1p-100f;  // sum u when c was last moved (below it, it has no delta worth a division)
   f32x16 o[NC], ou[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c)
@@ -1008,7 +1019,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) dot_chunk<float>(dp, small, next(NC + c), rl, dof, c);
-    float bu = 0.f;
+    float bu = 0.f, bd = 0.f, shift = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       float pr;
@@ -1016,23 +1027,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
       zsum += pr;
       bu += u[i];
       dp[i] += small[i];
+      dx[i] = times(u[i], dp[i] - centre);
+      bd += dx[i];
     }
-    usum += bu;
-    if (__builtin_amdgcn_ballot_w64(!centred && bu > 0.f) != 0ull) {
-      float bd = 0.f;
+    const float us = both_lanes(usum + bu);
+    const bool moves = us >= 2.f * mark;
+    if (__builtin_amdgcn_ballot_w64(moves) != 0ull) {
+      const float ud = both_lanes(udp + bd);
+      shift = moves ? ud * fast_rcp(us) : 0.f;
+      mark = moves ? us : mark;
+      centre += shift;
+      udp = fmaf(-shift, usum, udp);
+      bd = 0.f;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) bd += times(u[i], dp[i]);
-      bd += __shfl_xor(bd, 32, 64);
-      bu += __shfl_xor(bu, 32, 64);
-      if (!centred && bu > 0.f) {
-        centre = bd * fast_rcp(bu);
-        centred = true;
+      for (int i = 0; i < 16; ++i) {
+        dx[i] = times(u[i], dp[i] - centre);
+        bd += dx[i];
       }
     }
+    usum += bu;
+    udp += bd;
+    if constexpr (!kShiftInPart) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      dx[i] = times(u[i], dp[i] - centre);
-      udp += dx[i];
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[c][i] = fmaf(-shift, ou[c][i], o[c][i]);
     }
     Split w[2][2];
     split16(dx, w[0]);
@@ -1040,7 +1059,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       f32x16* const to[2] = {&o[c], &ou[c]};
-      acc_chunk(to, next(2 * NC + c), cl, w);
+      acc_chunk<kShiftInPart>(to, next(2 * NC + c), cl, w, shift);
     }
   });
   zsum += __shfl_xor(zsum, 32, 64);

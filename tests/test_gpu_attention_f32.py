@@ -4,6 +4,8 @@ workgroup from the lists to walks) and that do not, padding that holds NaN, grou
 
 Tolerance 1e-4 as in the other single-precision tests of forward and backward."""
 
+import math
+
 import pytest
 import torch
 
@@ -259,6 +261,56 @@ def test_lists_that_fill_up_between_two_solves(members, alpha, dtype):
     want = exact.dense_entmax_attention(q, k, v, alpha, False, vl)
     got = A.adasplash_v1(*(t.to(DEV) for t in (q, k, v)), alpha=alpha, is_causal=False, varlen=vl.to(DEV)).double().cpu()
     assert (got - want).norm() <= (2e-6 if dtype == torch.float32 else 2.0 ** -8) * want.norm()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("norm", [1.0, 100.0, 1000.0])
+def test_dq_of_an_outlying_row_of_v_that_is_barely_a_member(D, norm):
+    """Key 0 is the only member of its block and wave's first, with u = 2^-10 of 300 members, and its V row is `norm` times the others'.  u is exact (q has one
+    column, tau is given as 1, and u is what fp32 makes of scores that it holds exactly), so what is left is dP, delta and the sums: 2e-6 as
+    below; a dQ whose sums are taken around that key's dP is off by 5e-5 and more (K has a mean of 1, which makes them large)."""
+    g = torch.Generator().manual_seed(14)
+    N, members = 512, 300
+    n, left = torch.zeros(N, dtype=torch.int64), (1 << 20) - 1  # u in units of 2^-10: sum u^2 = 1
+    n[0] = 1
+    at = (torch.randperm(N - 128, generator=g)[:members] + 128).tolist()
+    for i, j in enumerate(at):
+        n[j] = math.isqrt(left) if i >= members - 8 else max(1, int(math.sqrt(left / (members - i)) * (0.7 + 0.6 * torch.rand((), generator=g).item())))
+        left -= int(n[j]) ** 2
+    z = torch.where(n > 0, 1.0 + n / 1024, -torch.ones(N))
+    q = torch.zeros(1, 1, N, D)
+    q[..., 0] = 16.0
+    k, v, dout = (torch.randn(1, 1, N, D, generator=g) for _ in range(3))
+    k += 1.0
+    k[0, 0, :, 0] = z * (D / 64) ** 0.5  # (exact at head dim 64 only)
+    v[:, :, 0] *= norm
+    qscale = torch.tensor(0.5 * D ** -0.5, dtype=torch.float32).double()
+    u = ((16.0 * k[0, 0, :, 0].double()) * qscale - 1.0).float().double().clamp_min(0.0)
+    dp = dout[0, 0].double() @ v[0, 0].double().t()
+    want = (u * (dp - (dp @ u / u.sum())[:, None])) @ k[0, 0].double() / D ** 0.5
+    a = [t.to(DEV) for t in (q, k, v, dout)]
+    _, taus, bmask = _attention.launch_forward(*a[:3], version=1, alpha=1.5, is_causal=False, niter=4, varlen=None)
+    got = _attention.launch_backward(*a, torch.ones_like(taus), bmask, alpha=1.5, is_causal=False, varlen=None)[0][0, 0].double().cpu()
+    assert (got - want).norm() <= 2e-6 * want.norm()
+
+
+@pytest.mark.parametrize("alpha,causal,D", [(1.5, True, 64), (1.5, False, 128), (1.333, False, 64), (2.0, False, 64)])
+@pytest.mark.parametrize("tails,k_mean", [(1.5, 0.0), (0.0, 3.0), (1.5, 3.0)])
+def test_errors_with_heavy_tails_and_a_common_part_of_k(alpha, causal, D, tails, k_mean):
+    """V rows whose norms have heavy tails (dP differs from block to block), and K with a mean, which cancels in dQ as the weights' derivatives add up to
+    0: 2e-6 as below, times the K that cancels over the K that does not."""
+    g = torch.Generator().manual_seed(15)
+    N = 512
+    q, k, v, dout = (torch.randn(1, 2, N, D, generator=g) for _ in range(4))
+    if tails:
+        v *= torch.rand(1, 2, N, 1, generator=g) ** (-1.0 / tails)
+    k += k_mean
+    want = [exact.dense_entmax_attention(q, k, v, alpha, causal)]
+    want += list(exact.dense_entmax_attention_grads(q, k, v, dout, alpha, causal))
+    bound = 2e-6 * max(1.0, k_mean)
+    for name, a, w in zip(("out", "dq", "dk", "dv"), run(q, k, v, dout, None, alpha, causal, False), want):
+        rel = ((a.double().cpu() - w.double()).norm() / w.double().norm()).item()
+        assert rel < bound, (name, rel)
 
 
 @pytest.mark.parametrize("alpha,causal,Hq,Hkv,D,q_scale,v_mean", [(1.5, True, 4, 2, 64, 1.0, 0.0), (1.5, True, 2, 1, 128, 3.0, 0.0), (1.5, True, 2, 2, 64, 0.125, 10.0),
