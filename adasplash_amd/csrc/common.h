@@ -196,15 +196,18 @@ __device__ __forceinline__ bool xcd_block_map(bool padded, int units, int blocks
 // The item at place `pos` of a batch, and its length; `longest_first`: the places are in the order of the lengths.  Workgroups start in the
 // order of their numbers, and those that find no slot at first start when others end: a long sequence in that place makes a launch longer.
 // The lengths come with one load, a lane each; beyond 64 items the order is theirs, with enough workgroups for the places to even out.
-// For kernels whose blocks of a sequence cost the same (not causal) and take long: 16 x 12 heads, N <= 500, D = 64, bf16, us, the items'
-// order -> this: dK/dV 43.8 -> 37.7, dQ 39.5 -> 37.0; 8 x 16 heads, N <= 2000, flat, alpha = 1.333: forward 370 -> 346, forward and
-// backward 839 -> 782; fp32, alpha = 1.333, 8 x 8 heads, N <= 700: 291 -> 275; 6 x 8 of 600, D = 128, alpha = 2: 255 -> 237.  Causal launches, whose sets of heads run longest block first, lose (8 x 16 heads, N <= 2000, flat: 320 -> 340;
-// fp32, D = 128: 4 x 8 heads, N <= 1100: 410 -> 444, 4 x 16/4: 704 -> 627),
-// and so do the short workgroups of the resident forward (16 x 12 heads: 40.9 -> 43.0; 32 x 8 of 300: 25.6 -> 29.3).
+// Head u of a batch runs on XCD u % 8, so with fewer than eight K/V heads an item has some of the XCDs only: every second round of items over the
+// XCDs goes backwards, or the same XCDs have the longer items of every round.  us, the items' order (three batches with the same lengths) ->
+// plainly longest first -> this: forward of 4 x 4 heads, N <= 1500, D = 64, bf16: 46, 54, 68 -> 55 -> 43 to 46; 5 x 4 of 700, D = 128, f16, alpha = 1.333,
+// training: 111, 122, 122 -> 108 to 111 -> 91 to 94; 8 x 4 of 3000, flat, forward: 190, 147, 132 -> 134 -> 116 to 123.
+// For kernels whose blocks of a sequence cost the same (not causal) and take long: 16 x 12 heads, N <= 500, D = 64, bf16, training: 112 to 115 -> 108 to 110;
+// 8 x 16 heads, N <= 2000, flat, alpha = 1.333: forward 370 -> 346, forward and backward 839 -> 782; 16 x 4 heads: 539 to 571 -> 476; fp32, alpha = 1.333,
+// 8 x 8 heads, N <= 700: 291 -> 275; 6 x 8 of 600, D = 128, alpha = 2: 255 -> 237.  Causal launches, whose sets of heads run longest block first, lose
+// (8 x 16 heads, N <= 2000, flat, bf16: 320 -> 340), and so do the short workgroups of the resident forward (16 x 12 heads: 40.9 -> 43.0; 32 x 8 of 300: 25.6 -> 29.3).
 struct BatchItem {
   int b, L;
 };
-__device__ __forceinline__ BatchItem batch_item(const void* varlen, int varlen_bits, int B, int N, int pos, bool longest_first) {
+__device__ __forceinline__ BatchItem batch_item(const void* varlen, int varlen_bits, int B, int N, int pos, int Hkv, bool longest_first) {
   if (!varlen) return {pos, N};
   auto length_of = [&](int i) -> int {
     const long long l = varlen_bits == 64 ? ((const long long*)varlen)[i] : (long long)((const int*)varlen)[i];
@@ -218,6 +221,9 @@ __device__ __forceinline__ BatchItem batch_item(const void* varlen, int varlen_b
     const int other = __builtin_amdgcn_readlane(len, i);
     rank += (int)(other > len) | ((int)(other == len) & (int)(i < lane));
   }
+  const int c = Hkv & 1 ? 8 : Hkv & 2 ? 4 : Hkv & 4 ? 2 : 1;  // places after which the heads are back at the first XCD
+  const int row = pos & -c;
+  if ((row & c) != 0 && row + c <= B) pos = 2 * row + c - 1 - pos;
   const int b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(rank == pos));
   return {b, __builtin_amdgcn_readlane(len, b)};
 }
