@@ -42,6 +42,8 @@
 // 16 heads: 1306 -> 1002; alpha = 1.333, 8 x 16 heads, N = 1024, not causal: 4818 -> 2690 -> 1794; prefill of 8 heads, N = 128: 11.4 -> 11.4.
 // Where 16-bit calls come here: rows32_16bit in attn_api.hip.
 #pragma once
+#include <cfloat>
+
 #include "attn_bwd_kernel.h"
 
 namespace adsp {
@@ -283,8 +285,9 @@ __device__ __forceinline__ void split16(const float (&w)[16], Split (&sp)[2]) {
   sp[0] = split8(w);
   sp[1] = split8(w + 8);
 }
-// o[x][column of the chunk][lane's row] += sum over the chunk's rows of chunk[row][column] * (weights x)[row]; kShift: o[0] -= shift o[1] before it
-template <bool kShift = false, int kN> __device__ __forceinline__ void acc_chunk(f32x16* const (&o)[kN], uint32_t chunk, uint32_t col_lane, const Split (&w)[kN][2], float shift = 0.f) {
+// o[x][column of the chunk][lane's row] += sum over the chunk's rows of chunk[row][column] * (weights x)[row]; kShift: o[0] -= shift o[1] before it; kInf: an infinite
+// sum stays what it is, whatever the small products (NaN, where an operand is infinite)
+template <bool kShift = false, bool kInf = false, int kN> __device__ __forceinline__ void acc_chunk(f32x16* const (&o)[kN], uint32_t chunk, uint32_t col_lane, const Split (&w)[kN][2], float shift = 0.f) {
   float a[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
@@ -306,7 +309,7 @@ template <bool kShift = false, int kN> __device__ __forceinline__ void acc_chunk
 #pragma unroll
   for (int n = 0; n < kN; ++n)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) (*o[n])[i] += part[n][i];
+    for (int i = 0; i < 16; ++i) (*o[n])[i] += kInf ? __builtin_amdgcn_fmed3f(part[n][i], -FLT_MAX, FLT_MAX) : part[n][i];
 }
 // the same for a 16-bit chunk of 64 columns (issue_t): o[0] takes columns 0 .. 31, o[1] the others
 template <typename T> __device__ __forceinline__ void acc_chunk_16(f32x16 (&o)[2], uint32_t chunk, int lane, const float (&w)[16]) {
@@ -517,9 +520,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) dot_chunk<T>(acc, small, next(c), rl, qf, c);
-    if constexpr (!k16)
+    if constexpr (!k16) {
+      // An infinite operand's other parts are NaN, and so are its small products: beside an infinite sum they have no say, or a row with a score of +inf
+      // (tau = +inf, output and gradients 0) would lose that key.  (Scores of -inf and NaN drop out of every comparison alike.)
+      float top = acc[0];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) top = fmaxf(top, acc[i]);
+      if (__builtin_amdgcn_ballot_w64(top == INFINITY) != 0ull) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) small[i] = acc[i] == INFINITY ? 0.f : small[i];
+      }
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[i] += small[i];
+    }
     const int k0 = blk * kRows;
     if (k0 + kRows > L || (p.causal && k0 + kRows - 1 > m0)) {
       const int jb = k0 + 4 * lh;
@@ -904,7 +917,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (any) acc_chunk_16<T>(o[c], a, lane, w);
       } else {
         f32x16* const to[1] = {&o[c][0]};
-        if (any) acc_chunk(to, a, cl, ws);
+        if (any) acc_chunk<false, true>(to, a, cl, ws);
       }
     }
   });

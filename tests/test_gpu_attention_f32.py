@@ -11,6 +11,7 @@ import torch
 
 import adasplash_amd as A
 from adasplash_amd import _attention, _lib
+from adasplash_amd.adasplash_block_mask import tile_sparsity
 from oracle import exact
 from tests.gpu_util import DEV, max_err
 
@@ -329,6 +330,48 @@ def test_errors_are_those_of_single_precision(alpha, causal, Hq, Hkv, D, q_scale
     for name, a, w in zip(("out", "dq", "dk", "dv"), run(q, k, v, dout, varlen, alpha, causal, Hq != Hkv), want):
         rel = ((a.double().cpu() - w.double()).norm() / w.double().norm()).item()
         assert rel < 2e-6, (name, rel)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("scale", [1.0, 0.05])  # of q: lists that hold, and that overflow
+@pytest.mark.parametrize("side,value,times", [("k", -math.inf, 1.0), ("k", math.inf, 1.0), ("k", math.nan, 1.0), ("q", math.inf, 1.0), ("k", -3e38, 100.0), ("k", 3e38, 100.0)])
+def test_scores_that_are_not_finite(D, scale, side, value, times):
+    """An infinite or NaN operand, and products beyond the type's range: as the kernels on 128 rows a workgroup, which form them in single precision.  A row with a
+    score of +inf is 0, as are its gradients; keys of score -inf or NaN have no weight and no gradients."""
+    g = torch.Generator().manual_seed(16)
+    N = 256
+    q, k, v, dout = (torch.randn(1, 2, N, D, generator=g) for _ in range(4))
+    q *= scale
+    q[..., 5], k[..., 5] = (times, 0.0) if side == "k" else (0.0, 1.0)
+    at = slice(17, None, 40)
+    (k if side == "k" else q)[:, :, at, 5] = value
+    want = tile_sparsity(*(t.to(DEV) for t in (q, k, v)), alpha=1.5)[0]
+    out, dq, dk, dv = run(q, k, v, dout, None, 1.5, False, False)
+    assert torch.isfinite(want).all() and max_err(out, want.cpu()) < TOL
+    top = value == math.inf or value > 1e38
+    assert bool((out[:, :, at] == 0).all()) == top
+    if top and side == "k":
+        assert (dq == 0).all() and (dk == 0).all() and (dv == 0).all()
+    elif side == "q":
+        assert (dq[:, :, at] == 0).all() and torch.isfinite(dv).all()
+    else:
+        assert (dk[:, :, at] == 0).all() and (dv[:, :, at] == 0).all() and torch.isfinite(dk).all() and torch.isfinite(dv).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("scale", [1.0, 0.05])
+def test_an_infinite_value_stays_in_its_column(D, scale):
+    """V with an infinite entry: infinite in the rows that have the key, and nowhere but in its column."""
+    g = torch.Generator().manual_seed(17)
+    q, k, v = (torch.randn(1, 2, 256, D, generator=g) for _ in range(3))
+    q *= scale
+    p = exact.entmax_rows(exact.attention_scores(q, k, False)[0], 1.5)[..., 17]
+    want = exact.dense_entmax_attention(q, k, v, 1.5)
+    v[:, :, 17, 3] = math.inf
+    out = A.adasplash_v1(*(t.to(DEV) for t in (q, k, v)), alpha=1.5, is_causal=False).cpu()
+    assert (out[..., 3][p > 1e-6] == math.inf).all()
+    keep = [c for c in range(D) if c != 3]
+    assert max_err(out[..., keep], want[..., keep]) < TOL
 
 
 @pytest.mark.parametrize("D", [64, 128])
