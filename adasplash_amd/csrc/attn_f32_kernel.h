@@ -417,12 +417,16 @@ template <int AM> __device__ __forceinline__ float norm_step(float s0, float s1,
 // us, order of xcd_block_map -> this, forward and backward, D = 64: 2 x 8 heads, N = 1500 and 375: 159.0 -> 156.8; 2 x 8 of 1024: 121.6 -> 116.7;
 // 8 of 2048: 211 -> 202; 8 x 8, N <= 700: 141 -> 118; 4 x 16 of N <= 1024, forward: 72.6 -> 62.3; D = 128: 4 x 8, N <= 1100: 415 -> 262; 4 x 16/4, N <= 1024:
 // 584 -> 558.
+// Without lengths xcd_block_map goes by the same order over sets of heads of 256 blocks.  From two such sets on theirs, whose K and V are fewer, is the faster one:
+// this -> theirs, forward and backward, D = 64: 8 x 16/8 heads, N = 1024: 681 -> 667; 8 x 32/8 of 512: 421 -> 415; 8 x 8 of 2048: 1181 -> 1167; below, where a set is
+// left that is not whole, this one is: 6 x 8 of 2048, forward: 221, theirs 228.
 // For up to 2048 keys and eight heads per XCD, a lane per length and per head, with the heads' operands in 8 MB as in xcd_block_map.
 // `keys`: a block of keys is the longer the earlier it is.  False: the launch is not of this kind.
 __device__ __forceinline__ bool longest_first(const void* varlen, int varlen_bits, int B, int Hkv, int N, int group, bool causal, long long unit_bytes, bool keys, bool two,
                                               int& bkv, int& rblk, int& member) {
   const int n = (N + kRows - 1) / kRows, heads = B * Hkv / 8, x = (int)(blockIdx.x & 7);
   if (!causal || n > 64 || (B * Hkv) % 8 != 0 || heads > 8 || heads * unit_bytes > (8ll << 20)) return false;
+  if (!varlen && heads * n * group >= 512) return false;
   const int lane = (int)(threadIdx.x & 63);
   int len = 0;  // blocks of head `lane` that are not empty; they are as long as 1, 2, ..., len
   if (lane < heads) len = (batch_item(varlen, varlen_bits, B, N, (lane * 8 + x) / Hkv, Hkv, false).L + kRows - 1) / kRows;

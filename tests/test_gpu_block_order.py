@@ -120,13 +120,14 @@ def test_a_batch_equals_its_items_on_the_supports(B, Hq, Hkv, N, D):
 
 
 # fp32, causal: blocks longest first over an XCD's heads, against heads run alone, which take the general order (one and eight heads per XCD, 64 blocks, 64
-# blocks that are not empty and more, lengths of 0, a part of a block and equal ones)
-@pytest.mark.parametrize("lens,Hq,Hkv,N,D", [([70, 200, 0], 16, 8, 200, 64), ([2048], 8, 8, 2048, 64), ([1024, 1024], 8, 8, 1024, 64), ([33, 1, 300, 300], 16, 16, 300, 64),
-                                             ([700, 64, 511], 16, 8, 700, 128)])
-@pytest.mark.parametrize("bits", [None, torch.int32, torch.int64])
-def test_causal_blocks_longest_first(lens, Hq, Hkv, N, D, bits):
-    if bits is None and N & (N - 1):
-        pytest.skip("without lengths N is a power of two")
+# blocks that are not empty and more, lengths of 0, a part of a block and equal ones; without lengths, where N is a power of two: launches that are
+# under way at once, and longer ones that the general order divides evenly and does not)
+LENGTHS_CAUSAL = [([70, 200, 0], 16, 8, 200, 64), ([2048], 8, 8, 2048, 64), ([1024, 1024], 8, 8, 1024, 64), ([33, 1, 300, 300], 16, 16, 300, 64), ([700, 64, 511], 16, 8, 700, 128)]
+WHOLE_CAUSAL = [([2048], 8, 8, 2048, 64), ([1024, 1024], 8, 8, 1024, 64), ([512] * 8, 32, 8, 512, 64), ([1024] * 8, 8, 8, 1024, 64), ([2048] * 6, 8, 8, 2048, 64)]
+
+
+@pytest.mark.parametrize("bits,lens,Hq,Hkv,N,D", [(bits, *c) for bits in (torch.int32, torch.int64) for c in LENGTHS_CAUSAL] + [(None, *c) for c in WHOLE_CAUSAL])
+def test_causal_blocks_longest_first(bits, lens, Hq, Hkv, N, D):
     g = torch.Generator().manual_seed(N)
     B, group = len(lens), Hq // Hkv
     q, dout = (torch.randn(B, Hq, N, D, generator=g).to(DEV) for _ in range(2))
