@@ -195,32 +195,34 @@ __device__ __forceinline__ bool xcd_block_map(bool padded, int units, int blocks
 
 // The item at place `pos` of a batch, and its length; `longest_first`: the places are in the order of the lengths.  Workgroups start in the
 // order of their numbers, and those that find no slot at first start when others end: a long sequence in that place makes a launch longer.
-// The lengths come with one load, a lane each; beyond 64 items the order is theirs, with enough workgroups for the places to even out.
 // Head u of a batch runs on XCD u % 8, so with fewer than eight K/V heads an item has some of the XCDs only: every second round of items over the
 // XCDs goes backwards, or the same XCDs have the longer items of every round.  us, the items' order (three batches with the same lengths) ->
 // plainly longest first -> this: forward of 4 x 4 heads, N <= 1500, D = 64, bf16: 46, 54, 68 -> 55 -> 43 to 46; 5 x 4 of 700, D = 128, f16, alpha = 1.333,
 // training: 111, 122, 122 -> 108 to 111 -> 91 to 94; 8 x 4 of 3000, flat, forward: 190, 147, 132 -> 134 -> 116 to 123.
-// For kernels whose blocks of a sequence cost the same (not causal) and take long: 16 x 12 heads, N <= 500, D = 64, bf16, training: 112 to 115 -> 108 to 110;
-// 8 x 16 heads, N <= 2000, flat, alpha = 1.333: forward 370 -> 346, forward and backward 839 -> 782; 16 x 4 heads: 539 to 571 -> 476; fp32, alpha = 1.333,
+// For kernels whose blocks of a sequence cost the same (not causal) and take long: 16 x 12 heads, N <= 500, D = 64, bf16, training: 113 to 116 -> 107 to 109;
+// 8 x 16 heads, N <= 2000, flat, alpha = 1.333: forward 370 -> 346, forward and backward 839 -> 782; 16 x 4 heads: 548 to 589 -> 494; fp32, alpha = 1.333,
 // 8 x 8 heads, N <= 700: 291 -> 275; 6 x 8 of 600, D = 128, alpha = 2: 255 -> 237.  Causal launches, whose sets of heads run longest block first, lose
 // (8 x 16 heads, N <= 2000, flat, bf16: 320 -> 340), and so do the short workgroups of the resident forward (16 x 12 heads: 40.9 -> 43.0; 32 x 8 of 300: 25.6 -> 29.3).
+// And launches of many rounds of workgroups (`per_cu` at a time on a CU), where the end is a small part and items of different lengths side by side do better than of
+// the same; the more so, the more items: training, D = 128: 32 x 16 heads, N <= 500, bf16 (8 rounds): 489, 505, 499 -> 535; 60 x 8 of 400 (7.5): 365 -> 416; 16 x 16 of 1500, flat
+// (12): 1442, 1467, 1431 -> 1464; fp32 32 x 16 of 300 (20): 827 -> 901; at the lines 16 x 8 of 500, fp32 (8): 470, 460, 453 -> 452; 20 x 16 of 300, bf16 (3.75): 164, 157, 166 -> 154;
+// 32 x 8 of 500, D = 64 (2): 131, 134, 132 -> 126.  A few heads, which the items' order shares out unevenly, gain in any number: 50 x 2 of 600, fp32: 268, 250, 264 -> 244.
 struct BatchItem {
   int b, L;
 };
-__device__ __forceinline__ BatchItem batch_item(const void* varlen, int varlen_bits, int B, int N, int pos, int Hkv, bool longest_first) {
+__device__ __forceinline__ BatchItem batch_item(const void* varlen, int varlen_bits, int B, int N, int pos, int Hkv, bool longest_first, int per_cu) {
   if (!varlen) return {pos, N};
   auto length_of = [&](int i) -> int {
     const long long l = varlen_bits == 64 ? ((const long long*)varlen)[i] : (long long)((const int*)varlen)[i];
     return (int)(l < 0 ? 0 : (l > N ? N : l));
   };
-  if (!longest_first || B > 64) return {pos, length_of(pos)};
+  const bool few_rounds = gridDim.x <= (B <= 16 ? 8u : B <= 24 ? 4u : 2u) * 256u * (uint32_t)per_cu, few_heads = Hkv % 8 != 0 && B * Hkv <= 128;
+  if (!longest_first || B > 64 || !(few_rounds || few_heads)) return {pos, length_of(pos)};
   const int lane = (int)(threadIdx.x & 63);
   const int len = length_of(lane < B ? lane : B - 1);
-  int rank = lane < B ? 0 : B;
-  for (int i = 0; i < B; ++i) {
-    const int other = __builtin_amdgcn_readlane(len, i);
-    rank += (int)(other > len) | ((int)(other == len) & (int)(i < lane));
-  }
+  const int key = lane < B ? len * 64 + 63 - lane : -1;  // (the length, and of equal ones the earlier; lengths are below 2^24)
+  int rank = 0;
+  for (int i = 0; i < B; ++i) rank += __builtin_amdgcn_readlane(key, i) > key ? 1 : 0;
   const int c = Hkv & 1 ? 8 : Hkv & 2 ? 4 : Hkv & 4 ? 2 : 1;  // places after which the heads are back at the first XCD
   const int row = pos & -c;
   if ((row & c) != 0 && row + c <= B) pos = 2 * row + c - 1 - pos;

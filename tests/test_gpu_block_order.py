@@ -80,8 +80,10 @@ def test_a_padded_batch_equals_its_items(dense_only, B, Hq, Hkv, N, D, causal, d
 
 
 # not causal, with lengths: the kernels on all pairs take the items longest first (equal lengths, a length of 0, 64 items, and 65, whose order stays), every
-# second round over the XCDs backwards (rounds of eight items, four, two and one; a last round that is whole and one that is not)
+# second round over the XCDs backwards (rounds of eight items, four, two and one; a last round that is whole and one that is not), and keep their order in launches
+# of many workgroups (20 x 24 heads and 30 x 24, on both sides of the line for the fp32 gradients)
 @pytest.mark.parametrize("lens,H,N", [([70, 200, 200, 0, 129, 1], 3, 200), ([70, 200, 33, 0, 129, 1, 64], 4, 200), ([70, 200, 33, 0, 129, 1, 64, 150], 6, 200), ([70, 150, 33, 20], 8, 150),
+                                      ([1 + 37 * i % 61 for i in range(20)], 24, 64), ([1 + 37 * i % 61 for i in range(30)], 24, 64),
                                       ([1 + 37 * i % 61 for i in range(19)], 1, 64), ([1 + 37 * i % 61 for i in range(64)], 1, 64), ([1 + 37 * i % 61 for i in range(65)], 1, 64)])
 @pytest.mark.parametrize("bits,dtype", [(torch.int32, torch.bfloat16), (torch.int64, torch.bfloat16), (torch.int32, torch.float32)])
 def test_items_of_a_padded_batch_longest_first(dense_only, lens, H, N, bits, dtype):
