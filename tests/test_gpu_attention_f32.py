@@ -317,8 +317,8 @@ def test_errors_with_heavy_tails_and_a_common_part_of_k(alpha, causal, D, tails,
 @pytest.mark.parametrize("alpha,causal,Hq,Hkv,D,q_scale,v_mean", [(1.5, True, 4, 2, 64, 1.0, 0.0), (1.5, True, 2, 1, 128, 3.0, 0.0), (1.5, True, 2, 2, 64, 0.125, 10.0),
                                                                   (1.5, True, 2, 2, 128, 1.0, 10.0), (1.333, False, 2, 2, 64, 1.0, 0.0), (2.0, False, 2, 2, 128, 1.0, 0.0)])
 def test_errors_are_those_of_single_precision(alpha, causal, Hq, Hkv, D, q_scale, v_mean):
-    """Products of three-part operands, and dQ from sums around a row's first delta: 2e-6 is 17 roundings of 2^-23, about twice what products in
-    single precision show for a V of mean 10; a part that is left out costs 2^-17 = 8e-6 or more."""
+    """Products of three-part operands, and dQ from sums around a row's running delta: 2e-6 is 17 roundings of 2^-23, about twice what products in
+    single precision show for a V of mean 10; a product with a third part that is left out costs about 5e-6 of a score."""
     g = torch.Generator().manual_seed(12)
     N, varlen = 289, torch.tensor([289, 250], dtype=torch.int32)
     q = q_scale * torch.randn(2, Hq, N, D, generator=g)
@@ -386,3 +386,23 @@ def test_largest_finite_values_stay_finite(D):
     want = run(q, k, v, dout, None, 1.5, True, False)
     for name, a, w in zip(("out", "dk", "dv"), (got[0], got[2], got[3]), (want[0], want[2], want[3])):
         assert torch.equal(a, w), name
+    keep = [c for c in range(D) if c != 5]  # (column 5 of dQ is sums of the largest value, in which u K overflows)
+    assert torch.equal(got[1][..., keep], want[1][..., keep])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("small,exponent", [("dout", -100), ("v", -100), ("q", -100), ("dout", -116), ("v", -116), ("q", -116)])
+def test_small_magnitudes(D, small, exponent):
+    """Operands whose third part reaches below bf16's smallest number, 2^-133, lose it: up to 2^-134 of a value, 2^-18 of one of 2^-116 and nothing above 2^-110.
+    2e-6 as above, and twice that."""
+    g = torch.Generator().manual_seed(18)
+    t = dict(zip(("q", "k", "v", "dout"), (torch.randn(1, 2, 256, D, generator=g) for _ in range(4))))
+    t[small] *= 2.0 ** exponent
+    if small == "q":
+        t["k"] *= 2.0 ** -exponent  # the scores stay what they are
+    a = list(t.values())
+    want = [exact.dense_entmax_attention(*a[:3], 1.5, True)] + list(exact.dense_entmax_attention_grads(*a, 1.5, True))
+    bound = 2e-6 + (2 * 2.0 ** (-134 - exponent) if exponent < -110 else 0.0)
+    for name, got, w in zip(("out", "dq", "dk", "dv"), run(*a, None, 1.5, True, False), want):
+        rel = ((got.double().cpu() - w).norm() / w.norm()).item()
+        assert rel < bound, (name, rel)
