@@ -5,12 +5,13 @@
 // products of 32 cycles and about 110 vector instructions for their operands), and on ordinary ones the length of a workgroup's
 // walk over the keys, because a K/V head of N keys has only N / rows workgroups; the forward's solves beside it.
 //
-// Products: an fp32 operand is the sum of three bf16 values exactly, and six of the nine products of the parts are what fp32 can see.  On
-// the bf16 matrix pipe they take 192 cycles per 16 columns where v_mfma_f32_32x32x2_f32 takes 512, and fewer roundings: relative
-// error against 64 bits, fp32 products -> these, of output, dQ, dK, dV: N = 1500, D = 64 4.0e-7, 4.5e-7, 4.5e-7, 4.1e-7 -> 2.7e-7, 3.3e-7, 3.3e-7,
-// 2.8e-7; q of spread 3 5.6e-7, 9.3e-7, 9.4e-7, 5.6e-7 -> 4.0e-7, 6.9e-7, 7.1e-7, 4.1e-7; flat 2.2e-7 ... 3.1e-7 -> 1.5e-7 ... 1.9e-7; D = 128
-// 3.6e-7, 9.2e-7, 9.2e-7, 8.5e-7 -> 3.4e-7, 3.7e-7, 3.7e-7, 3.5e-7; V of mean 10: dQ 1.5e-6 -> 1.0e-6.  The small products have an accumulator
-// of their own: added to the sum itself, their roundings made these errors 1.2 to 2 times those of fp32 products.
+// Products: an fp32 operand from 2^-110 on is the sum of three bf16 values exactly (below, the third part is rounded to bf16's smallest number, 2^-133: 2^-18 of
+// 2^-116), and six of the nine products of the parts are formed.  The three that are left out are 2^-22 of a product at most, and a small part of fp32's rounding on
+// average.  On the bf16 matrix pipe the six take 192 cycles per 16 columns where v_mfma_f32_32x32x2_f32 takes 512, and round less often: relative
+// error against 64 bits, fp32 products -> these, of output, dQ, dK, dV: N = 1500, D = 64 4.0e-7, 4.5e-7, 4.5e-7, 4.0e-7 -> 2.7e-7, 3.3e-7, 3.2e-7, 2.8e-7;
+// q of spread 3 5.6e-7, 9.4e-7, 9.5e-7, 5.7e-7 -> 3.9e-7, 6.7e-7, 6.9e-7, 4.0e-7; flat 2.1e-7 ... 3.1e-7 -> 1.4e-7 ... 1.9e-7; D = 128
+// 3.7e-7, 9.2e-7, 9.2e-7, 8.5e-7 -> 3.4e-7, 3.6e-7, 3.6e-7, 3.5e-7; dQ with a V of mean 10: 1.5e-6 -> 1.1e-6, a K of mean 10: 2.7e-6 -> 1.8e-6.  The small products
+// have an accumulator of their own: added to the sum itself, their roundings made these errors 1.2 to 2 times those of fp32 products.
 //
 // The 16-bit forward: vector issue (its products are a sixteenth as long; about 1400 vector instructions per block of 32 x 32 scores,
 // most of them insertions into the lists; matrix pipe 1-2 %, vector pipe about 50 % of the busy SIMD cycles).
@@ -38,8 +39,8 @@
 // 288 -> 148; 4 heads, N = 8192: 776 -> 285; bf16, 2 heads, N = 4096, D = 128: 135 -> 75.  Spread 3, where nothing overflows: 82.8 -> 83.2.
 //
 // Measured (fp32, forward and backward, us; kernels on 128 rows a workgroup -> fp32 products -> these): causal, 2 x 8 heads, N = 1500 and 375,
-// D = 64: 1140 -> 242 -> 160 (forward 55 -> 50, dQ 106 -> 62, dK/dV 93 -> 61); 4 x 16/4 heads, N = 1024, D = 128: 2885 -> 930 -> 711, flat,
-// 16 heads: 1306 -> 1002; alpha = 1.333, 8 x 16 heads, N = 1024, not causal: 4818 -> 2690 -> 1794; prefill of 8 heads, N = 128: 11.4 -> 11.4.
+// D = 64: 1140 -> 241 -> 158 (forward 50, dQ 62, dK/dV 58), flat 316 -> 201; 4 x 16/4 heads, N = 1024, D = 128: 2885 -> 928 -> 700; alpha = 1.333, 8 x 16 heads,
+// N = 1024, not causal: 4818 -> 2686 -> 1800; prefill of 8 heads, N = 128: 11.4 -> 11.3.
 // Where 16-bit calls come here: rows32_16bit in attn_api.hip.
 #pragma once
 #include <cfloat>
@@ -165,7 +166,7 @@ __device__ __forceinline__ void walk(R& ring, int first, int n_blk, int step, Sr
 }
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-// Eight fp32 values as three bf16 parts each, whose sum is the value itself (8 + 8 + 8 bits; the first part is cut off instead of rounded, so
+// Eight fp32 values as three bf16 parts each, whose sum is the value itself from 2^-110 on (8 + 8 + 8 bits; the first part is cut off instead of rounded, so
 // that no finite value becomes infinite): the operand of a product of 32 x 32 x 16.
 struct Split {
   u32x4 part[3];
@@ -192,7 +193,7 @@ __device__ __forceinline__ Split split8(const float* x) {
   }
   return r;
 }
-// main + small += a b of fp32 operands: the six products of their parts that fp32 can see, the largest of them apart from the others (each
+// main + small += a b of fp32 operands: the six largest of the nine products of their parts, the largest of them apart from the others (each
 // product rounds its accumulator, and the small ones' is 2^-7 of it)
 __device__ __forceinline__ void mfma_split(const Split& a, const Split& b, f32x16& main, f32x16& small) {
   small = mfma_16bit<bf16_t>(a.part[2], b.part[0], small);
@@ -415,8 +416,8 @@ template <int AM> __device__ __forceinline__ float norm_step(float s0, float s1,
 // backwards, so that the CU with the longest block of the first has the shortest of the second.  In longer launches blocks go where one ends, and
 // every second round backwards costs: 4 x 16/4 heads, N = 1024, D = 128: 717 -> 792 us.
 // us, order of xcd_block_map -> this, forward and backward, D = 64: 2 x 8 heads, N = 1500 and 375: 159.0 -> 156.8; 2 x 8 of 1024: 121.6 -> 116.7;
-// 8 of 2048: 211 -> 202; 8 x 8, N <= 700: 141 -> 118; 4 x 16 of N <= 1024, forward: 72.6 -> 62.3; D = 128: 4 x 8, N <= 1100: 415 -> 262; 4 x 16/4, N <= 1024:
-// 584 -> 558.
+// 8 of 2048: 211 -> 202; with lengths, three batches each: 8 x 8, N <= 700: 151, 152, 134 -> 125; 4 x 16, N <= 1024, forward: 69, 73, 72 -> 62; 8 x 8 of 2000: 613 -> 572; D = 128: 4 x 8,
+// N <= 1100: 407, 397, 396 -> 255; 8 x 8 of 1000: 510, 524, 458 -> 411; 4 x 16/4, N <= 1024: 519, 573, 631 -> 507, 544, 612; in long launches of many items it can lose: 32 x 8/2, N <= 900: 1616 -> 1644.
 // Without lengths xcd_block_map goes by the same order over sets of heads of 256 blocks.  From two such sets on theirs, whose K and V are fewer, is the faster one:
 // this -> theirs, forward and backward, D = 64: 8 x 16/8 heads, N = 1024: 681 -> 667; 8 x 32/8 of 512: 421 -> 415; 8 x 8 of 2048: 1181 -> 1167; below, where a set is
 // left that is not whole, this one is: 6 x 8 of 2048, forward: 221, theirs 228.
