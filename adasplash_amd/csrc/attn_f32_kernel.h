@@ -1037,7 +1037,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) dot_chunk<float>(dp, small, next(NC + c), rl, dof, c);
-    float bu = 0.f, bd = 0.f, shift = 0.f;
+    float bu = 0.f, shift = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       float pr;
@@ -1045,23 +1045,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
       zsum += pr;
       bu += u[i];
       dp[i] += small[i];
-      dx[i] = times(u[i], dp[i] - centre);
-      bd += dx[i];
     }
     const float us = both_lanes(usum + bu);
     const bool moves = us >= 2.f * mark;
     if (__builtin_amdgcn_ballot_w64(moves) != 0ull) {
+      float bd = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) bd += times(u[i], dp[i] - centre);
       const float ud = both_lanes(udp + bd);
       shift = moves ? ud * fast_rcp(us) : 0.f;
       mark = moves ? us : mark;
       centre += shift;
       udp = fmaf(-shift, usum, udp);
-      bd = 0.f;
+    }
+    float bd = 0.f;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        dx[i] = times(u[i], dp[i] - centre);
-        bd += dx[i];
-      }
+    for (int i = 0; i < 16; ++i) {
+      dx[i] = times(u[i], dp[i] - centre);
+      bd += dx[i];
     }
     usum += bu;
     udp += bd;
@@ -1071,6 +1072,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[c][i] = fmaf(-shift, ou[c][i], o[c][i]);
     }
+    // (alpha = 2: what follows, taken up among the weights, had 23 registers spilled instead of 16.  us, forward and backward, 6 x 8 heads, N <= 600, D = 64: 130.5 ->
+    // 127.5; at the other alphas the parts of one block among the weights of it are the faster way: 2 x 8 heads, N = 1500 and 375: 162.2 against 164.7.)
+    if constexpr (AM == ATT_2) __builtin_amdgcn_sched_barrier(0);
     Split w[2][2];
     split16(dx, w[0]);
     split16(u, w[1]);
