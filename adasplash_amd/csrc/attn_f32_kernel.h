@@ -515,9 +515,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     ring.issue_rows(kg, s, st);
   };
   OwnRow<T, NC> qf;
-  // scores of a block less `sub`, -inf on the keys the row may not see
-  auto scores = [&](int blk, float init, auto&& next) -> f32x16 {
-    f32x16 acc, small;
+  // scores of a block plus `init`, -inf on the keys the row may not see, and the largest of the lane's (kTop)
+  auto scores = [&](auto kTop, int blk, float init, float& top, auto&& next) -> f32x16 {
+    f32x16 acc, small, main;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       acc[i] = init;
@@ -525,24 +525,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) dot_chunk<T>(acc, small, next(c), rl, qf, c);
-    if constexpr (!k16) {
-      // An infinite operand's other parts are NaN, and so are its small products: beside an infinite sum they have no say, or a row with a score of +inf
-      // (tau = +inf, output and gradients 0) would lose that key.  (Scores of -inf and NaN drop out of every comparison alike.)
-      float top = acc[0];
-#pragma unroll
-      for (int i = 1; i < 16; ++i) top = fmaxf(top, acc[i]);
-      if (__builtin_amdgcn_ballot_w64(top == INFINITY) != 0ull) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) small[i] = acc[i] == INFINITY ? 0.f : small[i];
-      }
+    main = acc;
+    if constexpr (!k16)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[i] += small[i];
-    }
     const int k0 = blk * kRows;
     if (k0 + kRows > L || (p.causal && k0 + kRows - 1 > m0)) {
       const int jb = k0 + 4 * lh;
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[i] = jb + 8 * (i >> 2) + (i & 3) <= lim ? acc[i] : -INFINITY;
+    }
+    if constexpr (kTop) {
+      top = acc[0];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) top = k16 ? fmaxf(top, acc[i]) : __builtin_elementwise_maximum(top, acc[i]);
+      // An infinite operand's other parts are NaN, and so are its small products: beside an infinite sum they have no say, or a row with a score of +inf
+      // (tau = +inf, output and gradients 0) would lose that key.  (Scores of -inf and NaN drop out of every comparison alike.)  The maximum that is
+      // wanted anyway shows NaN (v_maximum3_f32 hands it on); a maximum of the main sums for it, in front of the small ones, cost us, forward: 2 x 8
+      // heads, N = 1500 and 375, D = 64: 50.4 against 49.9; of spread 3 34.9, 34.4; alpha = 1.333, 8 x 16 heads, N = 1024: 900, 892 (no test at all: 49.2, 33.9, 884).
+      if constexpr (!k16) {
+        if (__builtin_amdgcn_ballot_w64(top != top) != 0ull) {
+          top = -INFINITY;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            acc[i] = acc[i] != acc[i] && main[i] == INFINITY ? INFINITY : acc[i];
+            top = fmaxf(top, acc[i]);
+          }
+        }
+      }
     }
     return acc;
   };
@@ -698,10 +708,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __syncthreads();  // over_flag is clear
     // (as walk() does it, with the loads of the coming step under way across a solve)
     auto list_block = [&](int blk, auto&& next) {
-      const f32x16 s = scores(blk, 0.f, next);
-      float bm = s[0];
-#pragma unroll
-      for (int i = 1; i < 16; ++i) bm = fmaxf(bm, s[i]);
+      float bm;
+      const f32x16 s = scores(std::true_type{}, blk, 0.f, bm, next);
       if (over || __builtin_amdgcn_ballot_w64(live && bm > t_raw) == 0ull) return;
       int c = 0;
 #pragma unroll
@@ -853,10 +861,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   for (int it = 0; it < 24; ++it) {
     float a0 = 0.f, a1 = 0.f, mx = -INFINITY;
     walk<NC>(ring, wave, n_kblk, kWaves, src_k, [&](int blk, auto&& next) {
-      const f32x16 s = scores(blk, -t, next);
+      float bm;
+      const f32x16 s = scores(std::true_type{}, blk, -t, bm, next);
+      mx = fmaxf(mx, bm);
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        mx = fmaxf(mx, s[i]);
         float e0, e1;
         powers<AM>(fmaxf(s[i], 0.f) * qs, c0, e0, e1);
         a0 += e0;
@@ -898,7 +907,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     else ring.issue(vg, blk * kRows, L, s - NC, st);
   };
   walk<2 * NC>(ring, wave, n_kblk, kWaves, src_kv, [&](int blk, auto&& next) {
-    const f32x16 s = scores(blk, -t, next);
+    float unused;
+    const f32x16 s = scores(std::false_type{}, blk, -t, unused, next);  // (a row with a score of +inf has no finite t, and no weights)
     float w[16];
     float bs = 0.f;
 #pragma unroll
