@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   const int N = p.N, group = p.Hq / p.Hkv, n_blk = (N + kRows - 1) / kRows;
   int bkv, mi, hg;
   if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_blk, group, p.causal != 0, 2ll * N * kRow, bkv, mi, hg)) return;
-  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.Hkv, p.causal == 0, D == 64 ? 2 : 1);
+  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.Hkv, n_blk * group, p.causal == 0, D == 64 ? 2 : 1);
   const int b = item.b, L = item.L, kvh = bkv % p.Hkv, h = kvh * group + hg, bh = b * p.Hq + h;
   bkv = b * p.Hkv + kvh;
   const int m0 = (n_blk - 1 - mi) * kRows, mblk = m0 / kMaskRows;
@@ -314,7 +314,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   const int N = p.N, group = p.Hq / p.Hkv, n_blk = (N + kRows - 1) / kRows;
   int bkv, nblk, member_unused;
   if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_blk, 1, p.causal != 0, 2ll * group * N * kRow, bkv, nblk, member_unused)) return;
-  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.Hkv, p.causal == 0, D == 64 ? 2 : 1);
+  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.Hkv, n_blk, p.causal == 0, D == 64 ? 2 : 1);
   const int b = item.b, L = item.L, kvh = bkv % p.Hkv, n0 = nblk * kRows;
   bkv = b * p.Hkv + kvh;
   if (!left.takes((size_t)bkv * p.n_mblk + n0 / kMaskRows)) return;

@@ -430,7 +430,7 @@ __device__ __forceinline__ bool longest_first(const void* varlen, int varlen_bit
   if (!varlen && heads * n * group >= 512) return false;
   const int lane = (int)(threadIdx.x & 63);
   int len = 0;  // blocks of head `lane` that are not empty; they are as long as 1, 2, ..., len
-  if (lane < heads) len = (batch_item(varlen, varlen_bits, B, N, (lane * 8 + x) / Hkv, Hkv, false, 1).L + kRows - 1) / kRows;
+  if (lane < heads) len = (batch_item(varlen, varlen_bits, B, N, (lane * 8 + x) / Hkv, Hkv, 0, false, 1).L + kRows - 1) / kRows;
   int longer = 0;  // blocks longer than `lane`
   for (int u = 0; u < heads; ++u) {
     const int more = __builtin_amdgcn_readlane(len, u) - lane;
@@ -489,7 +489,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   int bkv, mi, hg, rblk;
   if (!k16 && longest_first(p.varlen, p.varlen_bits, p.B, p.Hkv, N, group, p.causal != 0, 2ll * N * kStride, false, true, bkv, rblk, hg)) mi = n_rblk - 1 - rblk;
   else if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
-  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.Hkv, p.causal == 0, 2);
+  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.Hkv, n_rblk * group, p.causal == 0, 2);
   const int b = item.b, L = item.L, kvh = bkv % p.Hkv, h = kvh * group + hg;
   bkv = b * p.Hkv + kvh;
   const int m0 = (n_rblk - 1 - mi) * kRows;
@@ -974,7 +974,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   int bkv, mi, hg, rblk;
   if (longest_first(p.varlen, p.varlen_bits, p.B, p.Hkv, N, group, p.causal != 0, 2ll * N * kStride, false, D == 64, bkv, rblk, hg)) mi = n_rblk - 1 - rblk;
   else if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, group, p.causal != 0, 2ll * N * kStride, bkv, mi, hg)) return;
-  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.Hkv, p.causal == 0, D == 64 ? 2 : 1);
+  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.Hkv, n_rblk * group, p.causal == 0, D == 64 ? 2 : 1);
   const int b = item.b, L = item.L, kvh = bkv % p.Hkv, h = kvh * group + hg;
   bkv = b * p.Hkv + kvh;
   const int m0 = (n_rblk - 1 - mi) * kRows;
@@ -1137,7 +1137,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   int bkv, kblk, member_unused;
   if (!longest_first(p.varlen, p.varlen_bits, p.B, p.Hkv, N, 1, p.causal != 0, 2ll * group * N * kStride, true, D == 64, bkv, kblk, member_unused) &&
       !xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_rblk, 1, p.causal != 0, 2ll * group * N * kStride, bkv, kblk, member_unused)) return;
-  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.Hkv, p.causal == 0, D == 64 ? 2 : 1);
+  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.Hkv, n_rblk, p.causal == 0, D == 64 ? 2 : 1);
   const int b = item.b, L = item.L, kvh = bkv % p.Hkv;
   bkv = b * p.Hkv + kvh;
   const int n0 = kblk * kRows;

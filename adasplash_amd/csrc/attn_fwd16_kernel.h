@@ -50,7 +50,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int N = p.N, group = p.Hq / p.Hkv, n_blk = (N + kRows - 1) / kRows;
   int bkv, mi, hg;
   if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_blk, group, p.causal != 0, 2ll * N * kRow, bkv, mi, hg)) return;
-  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.Hkv, p.causal == 0, 2);
+  const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.Hkv, n_blk * group, p.causal == 0, 2);
   const int b = item.b, L = item.L, kvh = bkv % p.Hkv, h = kvh * group + hg, bh = b * p.Hq + h;
   bkv = b * p.Hkv + kvh;
   const int mblk = n_blk - 1 - mi, m0 = mblk * kRows;

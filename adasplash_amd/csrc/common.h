@@ -203,20 +203,22 @@ __device__ __forceinline__ bool xcd_block_map(bool padded, int units, int blocks
 // 8 x 16 heads, N <= 2000, flat, alpha = 1.333: forward 370 -> 346, forward and backward 839 -> 782; 16 x 4 heads: 548 to 589 -> 494; fp32, alpha = 1.333,
 // 8 x 8 heads, N <= 700: 291 -> 275; 6 x 8 of 600, D = 128, alpha = 2: 255 -> 237.  Causal launches, whose sets of heads run longest block first, lose
 // (8 x 16 heads, N <= 2000, flat, bf16: 320 -> 340), and so do the short workgroups of the resident forward (16 x 12 heads: 40.9 -> 43.0; 32 x 8 of 300: 25.6 -> 29.3).
-// And launches of many rounds of workgroups (`per_cu` at a time on a CU), where the end is a small part and items of different lengths side by side do better than of
+// And launches of many rounds of workgroups (`blocks` per K/V head, `per_cu` at a time on a CU), where the end is a small part and items of different lengths side by side do better than of
 // the same; the more so, the more items: training, D = 128: 32 x 16 heads, N <= 500, bf16 (8 rounds): 489, 505, 499 -> 535; 60 x 8 of 400 (7.5): 365 -> 416; 16 x 16 of 1500, flat
 // (12): 1442, 1467, 1431 -> 1464; fp32 32 x 16 of 300 (20): 827 -> 901; at the lines 16 x 8 of 500, fp32 (8): 470, 460, 453 -> 452; 20 x 16 of 300, bf16 (3.75): 164, 157, 166 -> 154;
 // 32 x 8 of 500, D = 64 (2): 131, 134, 132 -> 126.  A few heads, which the items' order shares out unevenly, gain in any number: 50 x 2 of 600, fp32: 268, 250, 264 -> 244.
 struct BatchItem {
   int b, L;
 };
-__device__ __forceinline__ BatchItem batch_item(const void* varlen, int varlen_bits, int B, int N, int pos, int Hkv, bool longest_first, int per_cu) {
-  if (!varlen) return {pos, N};
+__device__ __forceinline__ BatchItem batch_item(const void* varlen, int varlen_bits, int B, int N, int pos, int Hkv, int blocks, bool longest_first, int per_cu) {
+  // (What only padded batches need stands behind the other code, and the number of workgroups is formed here: gridDim would bring 256 bytes of hidden arguments to
+  // every launch.  Forward of 8 heads, N = 128, fp32, which starts from cold instruction lines: 12.2 -> 12.05 us; 4 x 16/4 heads, N = 1024, D = 128: 138.2 -> 137.0.)
+  if (__builtin_expect(!varlen, 1)) return {pos, N};
   auto length_of = [&](int i) -> int {
     const long long l = varlen_bits == 64 ? ((const long long*)varlen)[i] : (long long)((const int*)varlen)[i];
     return (int)(l < 0 ? 0 : (l > N ? N : l));
   };
-  const bool few_rounds = gridDim.x <= (B <= 16 ? 8u : B <= 24 ? 4u : 2u) * 256u * (uint32_t)per_cu, few_heads = Hkv % 8 != 0 && B * Hkv <= 128;
+  const bool few_rounds = (uint32_t)(B * Hkv) * (uint32_t)blocks <= (B <= 16 ? 8u : B <= 24 ? 4u : 2u) * 256u * (uint32_t)per_cu, few_heads = Hkv % 8 != 0 && B * Hkv <= 128;
   if (!longest_first || B > 64 || !(few_rounds || few_heads)) return {pos, length_of(pos)};
   const int lane = (int)(threadIdx.x & 63);
   const int len = length_of(lane < B ? lane : B - 1);
