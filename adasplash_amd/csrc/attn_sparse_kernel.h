@@ -176,11 +176,12 @@ __device__ __forceinline__ int draw_item(uint32_t* queue, int per_xcd, int total
   return got;
 }
 
-template <typename T, int D> struct SparseGeo {
+// KP: waves that share 32 rows, each with a part of the keys (see attn_fwd_sparse_kernel).  The backward's kernels have KP = 1.
+template <typename T, int D, int KP = 1> struct SparseGeo {
   using G = TileGeo<T, D>;
-  static constexpr int kNW = 4;
+  static constexpr int kNW = 4;  // sets of 32 rows
   static constexpr int kBM = 32 * kNW;
-  static constexpr int kThreads = 64 * kNW;
+  static constexpr int kThreads = 64 * kNW * KP;
   // K stages during the walks, with the waves' event rings behind them; afterwards the whole array holds the
   // candidate lists.  Two stages of 16-bit tiles: 39 KB, four workgroups per CU (one wave of each per SIMD); three
   // stages (52 KB at head dim 128, three workgroups per CU) measured slower.  The fp8 tiles of the first walk are
@@ -191,21 +192,23 @@ template <typename T, int D> struct SparseGeo {
   static constexpr int kK8Tile = kBN * kK8Row;
   static constexpr int kK8Loads = kK8Tile / 1024;
   static constexpr int kMinLds = 39 * 1024;  // (1 KB left for the small arrays)
-  static constexpr int kLds = kStages * G::kKTile + 4608 > kMinLds ? kStages * G::kKTile + 4608 : kMinLds;  // rings of >= 32 events
-  static constexpr int kWaveLds = kLds / kNW;
+  static constexpr int kLds1 = kStages * G::kKTile + 4608 > kMinLds ? kStages * G::kKTile + 4608 : kMinLds;  // rings of >= 32 events
+  static constexpr int kLds = KP * kLds1;
+  static constexpr int kWaveLds = kLds / kNW;  // of a set of rows
+  static constexpr int kRingsAt = KP * kStages * G::kKTile;
   // candidates per wave: scores (fp32) and keys (16 bits: the path serves up to 65536 keys) in two arrays, then the
   // rows' counters, offsets and 1 / sum
-  static constexpr int kListCapRaw = (kWaveLds - 512) / 6 / 8 * 8;
+  static constexpr int kListCapRaw = (kLds1 / kNW - 512) / 6 / 8 * 8;  // (the same for every KP: the same row blocks fit)
   static constexpr int kListCap = kListCapRaw > kSparseStreamCap ? kSparseStreamCap : kListCapRaw;
-  static constexpr int kRingBytes = (kLds - kStages * G::kKTile) / kNW;
+  static constexpr int kRingBytes = (kLds1 - kStages * G::kKTile) / kNW;
   static constexpr int kRing = kRingBytes / 36 > 192 ? 192 : kRingBytes / 36;  // events: 8 scores and a tag
   static_assert(kRing >= 32, "half a wave can bring 32 events at once");
 };
 
-template <typename T, int D, int AM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE_WAVES, ADSP_SPARSE_WAVES))) void attn_fwd_sparse_kernel(AttnParams p) {
+template <typename T, int D, int AM, int KP>
+__global__ __launch_bounds__(256 * KP) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE_WAVES, ADSP_SPARSE_WAVES))) void attn_fwd_sparse_kernel(AttnParams p) {
   using G = TileGeo<T, D>;
-  using SG = SparseGeo<T, D>;
+  using SG = SparseGeo<T, D, KP>;
   using KS = Swz<G::kKRow>;
   using KS8 = Swz<SG::kK8Row>;
   static_assert(G::k16, "16-bit element types only");
@@ -217,9 +220,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
   // a lane ran out of event slots, or a wave out of list room.  Two words: the walks write the one of the tile's
   // parity and read the other one behind the next barrier, so no wave can read a word another one is still setting
   __shared__ uint32_t s_giveup[2];
+  __shared__ int s_len[KP > 1 ? NW * KP : 1];  // the streams' lengths (KP > 1)
   extern __shared__ uint32_t mask_out[];  // p.mask_words words: key tiles that hold a non-zero probability
 
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int wave_id = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int wave = KP > 1 ? wave_id % NW : wave_id;  // the set of rows
+  const int part = KP > 1 ? wave_id / NW : 0;        // the part of the keys
   const int N = p.N;
   const int n_mblk = (N + BM - 1) / BM;
   const int group = p.Hq / p.Hkv;
@@ -309,6 +315,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
       continue;
     }
     const int nt = p.causal ? (row_hi + kBN - 1) / kBN : (L + kBN - 1) / kBN;
+    const int n_steps = KP > 1 ? (nt + KP - 1) / KP : nt;  // of a walk
+    const int kt0 = part * n_steps;                        // the wave's tiles: kt0 .. kt0 + nt_w - 1
+    const int nt_w = KP > 1 ? (nt - kt0 < n_steps ? (nt - kt0 > 0 ? nt - kt0 : 0) : n_steps) : nt;
     const int lim = p.causal ? (qi < L - 1 ? qi : L - 1) : L - 1;
     const int wave_row0 = m0 + wave * 32;
     const bool live = qi < L;
@@ -359,21 +368,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
         }
       }
     };
-    // body(kt, tile) over all key tiles of the row block; stops when a lane gave up.  The K tiles go through a ring of
+    // body(step, kt, tile) over the wave's key tiles of the row block; stops when a lane gave up.  The K tiles go through a ring of
     // kStages LDS buffers: the load of tile t + kStages - 1 is issued behind the barrier that opens tile t (every wave
-    // is done with tile t - 1, whose buffer it takes) and has kStages - 1 tile times to arrive.
+    // is done with tile t - 1, whose buffer it takes) and has kStages - 1 tile times to arrive.  (KP > 1: a buffer holds a tile
+    // of each part of the keys, loaded by the waves that read it.)
     // (stages_c, tile_c, per_c: the ring's depth, the bytes of a tile and the loads per wave and tile, as constants)
     auto walk = [&](auto stages_c, auto tile_c, auto per_c, auto&& issue, auto&& body) {
       constexpr int kStages = decltype(stages_c)::value, kTile = decltype(tile_c)::value, kPer = decltype(per_c)::value;
+      unsigned char* const bufs = lds_all + part * kTile;
       __syncthreads();
 #pragma unroll
       for (int s = 0; s < kStages - 1; ++s)
-        if (s < nt) issue(lds_all + s * kTile, s);
+        if (s < nt_w) issue(bufs + s * (KP * kTile), kt0 + s);
       int stage = 0;  // buffer of tile cur
-      for (int cur = 0; cur < nt; ++cur) {
+      for (int cur = 0; cur < n_steps; ++cur) {
         // this wave's share of tile cur has landed: everything but the loads issued after it (those of the tiles in
         // between; stores issued after it only make the wait longer than needed)
-        if (cur + kStages - 1 <= nt) {
+        if (cur + kStages - 1 <= nt_w) {
           if constexpr (kStages == 2) __builtin_amdgcn_s_waitcnt(0x0f70);
           else __builtin_amdgcn_s_waitcnt(0x0f70 | ((kStages - 2) * kPer));
         } else {
@@ -382,9 +393,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
         __syncthreads();
         if (s_giveup[(cur + 1) & 1]) break;  // set while the previous tile was worked on
         const int pre = cur + kStages - 1;
-        if (pre < nt) issue(lds_all + (stage == 0 ? kStages - 1 : stage - 1) * kTile, pre);
+        if (pre < nt_w) issue(bufs + (stage == 0 ? kStages - 1 : stage - 1) * (KP * kTile), kt0 + pre);
         __builtin_amdgcn_sched_barrier(0);
-        body(cur, lds_all + stage * kTile);
+        if (KP == 1 || cur < nt_w) body(cur, kt0 + cur, bufs + stage * (KP * kTile));
         stage = stage + 1 == kStages ? 0 : stage + 1;
       }
     };
@@ -481,7 +492,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
     // position in the block (4 bits); unsigned comparisons order the words by their sums.  Words whose sum field is
     // 0 (nothing seen, or only masked scores) stand for no key.
     // A flat score distribution (a support of hundreds of keys) shows early: most block maxima lie close to the
-    // running maximum.  Tiles 6 .. 11 are counted; if more than half of their (lane, block) maxima lie within 1/4 (in
+    // running maximum.  Tiles 6 .. 11 (of each part) are counted; if more than half of their (lane, block) maxima lie within 1/4 (in
     // z) of the lane's running maximum, the row block is given up before the walk is over.  A heuristic that only
     // decides which kernel does the work.
     uint32_t t1 = 0u, t2 = 0u, t3 = 0u, t4 = 0u;
@@ -494,7 +505,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
     };
     int near_cnt = 0;
     const uint32_t near_d = (uint32_t)fminf(0.25f * inv_qs * 16.f * aqk, 8191.f) << 15;
-    walk(std::integral_constant<int, SG::kStages8>{}, std::integral_constant<int, SG::kK8Tile>{}, std::integral_constant<int, kK8Per>{}, issue_k8, [&](int kt, const unsigned char* kt_lds) {
+    walk(std::integral_constant<int, SG::kStages8>{}, std::integral_constant<int, SG::kK8Tile>{}, std::integral_constant<int, kK8Per>{}, issue_k8, [&](int step, int kt, const unsigned char* kt_lds) {
       for_tile8(kt, kt_lds, [&](const f32x16& s0, const f32x16& s1) {
         float m0v = fmaxf(s0[0], s0[1]), m1v = fmaxf(s1[0], s1[1]);
 #pragma unroll
@@ -507,10 +518,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
         const uint32_t k1 = (((b1 >> 9) & 0x3fffu) << 15) | ((b1 & 15u) | ((uint32_t)(2 * kt + 1) << 4));
         keep_top(k0);
         keep_top(k1);
-        if (kt >= 6 && kt < 12) {
+        if (step >= 6 && step < 12) {
           const uint32_t near = t1 > near_d ? t1 - near_d : 0u;
           near_cnt += __builtin_popcountll(__builtin_amdgcn_ballot_w64(live && k0 > near)) + __builtin_popcountll(__builtin_amdgcn_ballot_w64(live && k1 > near));
-          if (kt == 11 && near_cnt > 6 * 128 / 2 && lane == 0) s_giveup[1] = 1u;
+          if (step == 11 && near_cnt > 6 * 128 / 2 && lane == 0) s_giveup[1] = 1u;
         }
       });
     });
@@ -541,19 +552,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
     // product m the A operand's row i is the key that row i chose as its m-th (a lane fetches its slice of that key's
     // row from memory), so the diagonal of S^T holds the wanted scores, bit for bit those the second walk will see
     // ----------------------------------------------------------------------------------------------------------------
+    // (KP = 2: a wave scores the two best keys of each of its lanes, the row's eight meet in LDS)
     float r[8];
     {
+      constexpr int kR = 4 / KP;  // keys a lane has scored
       // The rows of the chosen keys are gathered into LDS the way the walks' tiles get there: per product m the wave
       // loads a 32-row "tile" whose row i is the key that row i chose as its m-th, with 1 KB DMA instructions (a
       // group of kC lanes per key row: whole rows, coalesced), and reads the A fragments from it as from a K tile.
       const uint32_t u[4] = {t1, t2, t3, t4};
       constexpr int kRowsPer = 64 / KS::kC;   // key rows per 1 KB DMA instruction
       constexpr int kInstr = 32 / kRowsPer;   // instructions per gathered tile
-      uint32_t* const ktab = reinterpret_cast<uint32_t*>(lds_all + SG::kStages * G::kKTile + wave * SG::kRingBytes);  // [8][kRowsPer][kInstr]
-      unsigned char* const gtile = lds_all + wave * (32 * G::kKRow);
-      bool okm[4], okp[4];
+      uint32_t* const ktab = reinterpret_cast<uint32_t*>(lds_all + SG::kRingsAt + wave_id * SG::kRingBytes);  // [2 kR][kRowsPer][kInstr]
+      unsigned char* const gtile = lds_all + wave_id * (32 * G::kKRow);
+      bool okm[kR], okp[kR];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < kR; ++i) {
         const uint32_t w = u[i];
         okm[i] = (w >> 15) != 0u;
         uint32_t key = ((w >> 4) & 0x7ffu) * 32u + 8u * ((w & 15u) >> 2) + (w & 3u) + 4u * (uint32_t)lh;
@@ -561,7 +574,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
         // scores of the row's own keys bound its threshold)
         okm[i] = okm[i] && (int)key <= lim;
         key = okm[i] ? key : 0u;
-        ktab[(4 * lh + i) * 32 + (lq % kRowsPer) * kInstr + lq / kRowsPer] = key;
+        ktab[(kR * lh + i) * 32 + (lq % kRowsPer) * kInstr + lq / kRowsPer] = key;
         okp[i] = __shfl_xor((int)okm[i], 32, 64) != 0;
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -570,8 +583,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
       const bool diag_here = lh == ((lq >> 2) & 1);  // and which of the row's two lanes holds it
       const unsigned char* kg = uniform_ptr(kglob);
       const int grow = lane / KS::kC, gslot = lane % KS::kC;
+      float mine[2 * kR];
 #pragma unroll
-      for (int m = 0; m < 8; ++m) {
+      for (int m = 0; m < 2 * kR; ++m) {
         uint32_t keys[kInstr];
 #pragma unroll
         for (int j = 0; j < kInstr; j += 4) {
@@ -602,14 +616,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
         for (int i = 1; i < 16; ++i) d = diag == i ? acc[i] : d;
         const float other = __shfl_xor(d, 32, 64);
         d = diag_here ? d : other;
-        const bool ok = ((m < 4) == (lh == 0)) ? okm[m & 3] : okp[m & 3];
-        r[m] = ok ? d : -INFINITY;
+        const bool ok = ((m < kR) == (lh == 0)) ? okm[m % kR] : okp[m % kR];
+        mine[m] = ok ? d : -INFINITY;
+      }
+      if constexpr (KP == 1) {
+#pragma unroll
+        for (int m = 0; m < 8; ++m) r[m] = mine[m];
+      } else {
+        static_assert(KP == 2 && SG::kRingBytes >= 1024, "the values lie behind the table, in the ring's place");
+        f32x4* const meet = reinterpret_cast<f32x4*>(lds_all + SG::kRingsAt + wave * SG::kRingBytes + 512);
+        constexpr int kOther = NW * SG::kRingBytes / 16;  // from a wave's values to those of the other part's wave
+        if (lh == 0) meet[part * kOther + lq] = f32x4{mine[0], mine[1], mine[2], mine[3]};
+        __syncthreads();
+        const f32x4 x0 = meet[lq], x1 = meet[kOther + lq];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          r[m] = x0[m];
+          r[4 + m] = x1[m];
+        }
       }
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the last fragment reads are done before the tiles of walk 2 arrive
     }
     float lo_raw;
     {
-      const float rmax = fmaxf(r[0], r[4]);
+      float rmax = fmaxf(r[0], r[4]);
+      if constexpr (KP > 1) rmax = fmaxf(rmax, fmaxf(r[2], r[6]));
       float t = rmax - inv_qs;
       const float target = (AM == ATT_15) ? inv_qs * inv_qs : inv_qs;
 #pragma unroll 1
@@ -653,15 +684,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
     // ring in LDS (slots are handed out with a ballot: no atomics).  When the ring is full the wave empties it, one
     // event per lane: the positive entries go to the wave's candidate stream in global memory as (score - lo, key and
     // row) pairs, compact and in bursts, so the tile loop rarely waits for a store.
-    float* const ring = reinterpret_cast<float*>(lds_all + SG::kStages * G::kKTile + wave * SG::kRingBytes);
+    float* const ring = reinterpret_cast<float*>(lds_all + SG::kRingsAt + wave_id * SG::kRingBytes);
     uint32_t* const ring_tag = reinterpret_cast<uint32_t*>(ring + SG::kRing * 8);
     // (kept for the backward, the stream has a place of its own per row block and wave)
     const size_t stream_id = ((size_t)(b * p.Hq + h) * n_mblk + mblk) * NW + wave;
     uint2* const stream = p.save_streams ? reinterpret_cast<uint2*>(p.save_streams) + stream_id * (size_t)kSparseStreamCap
                                          : reinterpret_cast<uint2*>(p.events) + ((size_t)blockIdx.x * NW + wave) * (size_t)kSparseStreamCap;
+    // (KP = 2: the second part's wave fills the row set's place from its end.  Together the two hold kListCap entries at most, which
+    // is asked when both are complete; where they have more, what one has written over the other's is not read.)
+    auto place = [&](int e) -> int { return KP > 1 && part ? kSparseStreamCap - 1 - e : e; };
     int ring_n = 0, stream_n = 0;  // wave-uniform
-    // (kt: the tile being worked on; a stream that fills faster than the tiles go by will not last: give up early)
-    auto flush = [&](int parity, int kt) {
+    // (step: of the walk; a stream that fills faster than the tiles go by will not last: give up early)
+    auto flush = [&](int parity, int step) {
       for (int e0 = 0; e0 < ring_n; e0 += 64) {
         const int e = e0 + lane;
         const bool has = e < ring_n;
@@ -677,19 +711,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
         for (int i = 0; i < 4; ++i) c += (w0[i] > 0.f ? 1 : 0) + (w1[i] > 0.f ? 1 : 0);
         const int incl = wave_scan_i(c);
         const int total_c = __builtin_amdgcn_readlane(incl, 63);
-        if (stream_n + total_c > SG::kListCap || (long long)(stream_n + total_c) * nt > (long long)SG::kListCap * (kt + 16)) {
+        if (stream_n + total_c > SG::kListCap || (long long)(stream_n + total_c) * nt_w > (long long)SG::kListCap * (step + 16)) {
           if (lane == 0) s_giveup[parity] = 1u;
         } else {
           // producer lane = tag & 63: row (tag & 31), key half (tag >> 5) & 1; half block (tag >> 6) & 3 of tile tag >> 8
           const uint32_t key0 = (tag >> 8) * kBN + ((tag >> 6) & 3u) * 16 + 4 * ((tag >> 5) & 1u);
           const uint32_t rowbits = (tag & 31u) << 20;
-          uint2* dst = stream + stream_n + (incl - c);
+          uint2* dst = stream + place(stream_n + (incl - c));
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
             const float x = i < 4 ? w0[i & 3] : w1[i & 3];
             if (x > 0.f) {
               *dst = uint2{__builtin_bit_cast(uint32_t, x), (key0 + 8 * (i >> 2) + (i & 3)) | rowbits};
-              ++dst;
+              dst += KP > 1 && part ? -1 : 1;
             }
           }
           stream_n += total_c;
@@ -697,34 +731,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
       }
       ring_n = 0;
     };
-    // the lanes of `m` (those of them for which `mine` holds put their half block) take consecutive ring slots
-    auto put = [&](unsigned long long m, bool mine, const f32x16& s, int first, uint32_t tag, int kt) {
-      const int c = __builtin_popcountll(m);
-      if (ring_n + c > SG::kRing) flush(kt & 1, kt);
-      if (mine) {
-        const int slot = ring_n + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-        f32x4 w0 = {s[first], s[first + 1], s[first + 2], s[first + 3]};
-        f32x4 w1 = {s[first + 4], s[first + 5], s[first + 6], s[first + 7]};
-        *reinterpret_cast<f32x4*>(ring + slot * 8) = w0;
-        *reinterpret_cast<f32x4*>(ring + slot * 8 + 4) = w1;
-        ring_tag[slot] = (tag << 6) | (uint32_t)lane;
-      }
-      ring_n += c;
-    };
-    auto collect = [&](const f32x16& s, int first, float hmax, uint32_t tag, int kt) {
-      const unsigned long long m = __builtin_amdgcn_ballot_w64(hmax > 0.f);
-      if (m != 0ull) {
-        if (__builtin_popcountll(m) <= SG::kRing) {
-          put(m, hmax > 0.f, s, first, tag, kt);
-        } else {  // more events than the ring holds at once (the first tiles of a sequence): in two halves
-          put(m & 0xffffffffull, hmax > 0.f && lane < 32, s, first, tag, kt);
-          put(m & ~0xffffffffull, hmax > 0.f && lane >= 32, s, first, tag, kt);
-        }
-      }
-    };
     // One decision per tile: the four half blocks' events are counted together; when they fit the ring (after a flush
     // if need be) every lane writes its events at slots known from the four ballots, without further tests.  A tile
-    // with more events than the ring holds (the first tiles of a sequence) goes through in eight parts.
+    // with more events than the ring holds (rows of some hundred keys) goes through block by block, and where a block has
+    // more (the first tiles of a sequence) in eight parts.
     auto put_at = [&](unsigned long long m, bool mine, const f32x16& s, int first, uint32_t tag, int base) {
       if (mine) {
         const int slot = base + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
@@ -735,7 +745,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
         ring_tag[slot] = (tag << 6) | (uint32_t)lane;
       }
     };
-    walk(std::integral_constant<int, SG::kStages>{}, std::integral_constant<int, G::kKTile>{}, std::integral_constant<int, kKPer>{}, issue_k, [&](int kt, const unsigned char* kt_lds) {
+    walk(std::integral_constant<int, SG::kStages>{}, std::integral_constant<int, G::kKTile>{}, std::integral_constant<int, kKPer>{}, issue_k, [&](int step_w, int kt, const unsigned char* kt_lds) {
       for_tile(kt, kt_lds, -lo_raw, [&](const f32x16& s0, const f32x16& s1) {
         float h00 = s0[0], h01 = s0[8], h10 = s1[0], h11 = s1[8];
 #pragma unroll
@@ -750,23 +760,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
         const int c0 = __builtin_popcountll(m0), c1 = __builtin_popcountll(m1), c2 = __builtin_popcountll(m2), c3 = __builtin_popcountll(m3);
         const int E = c0 + c1 + c2 + c3;
         if (E != 0) {
-          int step = E <= SG::kRing ? -1 : 0;
+          // -1: all at once; -3, -2: the first block, the second; 0 .. 7: the eighths
+          constexpr bool kByBlock = SG::kRing < 128;  // (rings that hold any block's events are rarely short of room: the longer code is 1 % slower)
+          int step = E <= SG::kRing ? -1 : (kByBlock && c0 + c1 <= SG::kRing && c2 + c3 <= SG::kRing ? -3 : 0);
           do {
             unsigned long long sub = 0ull;
-            int need = E;
+            int need = !kByBlock || step == -1 ? E : (step == -3 ? c0 + c1 : c2 + c3);
             if (step >= 0) {
               const int hb = step >> 1;
               sub = hb == 0 ? m0 : hb == 1 ? m1 : hb == 2 ? m2 : m3;
               sub &= (step & 1) ? ~0xffffffffull : 0xffffffffull;
               need = __builtin_popcountll(sub);
             }
-            if (ring_n + need > SG::kRing) flush(kt & 1, kt);
+            if (ring_n + need > SG::kRing) flush(step_w & 1, step_w);
             if (step < 0) {
-              put_at(m0, h00 > 0.f, s0, 0, (uint32_t)(kt * 4 + 0), ring_n);
-              put_at(m1, h01 > 0.f, s0, 8, (uint32_t)(kt * 4 + 1), ring_n + c0);
-              put_at(m2, h10 > 0.f, s1, 0, (uint32_t)(kt * 4 + 2), ring_n + c0 + c1);
-              put_at(m3, h11 > 0.f, s1, 8, (uint32_t)(kt * 4 + 3), ring_n + c0 + c1 + c2);
-              step = 8;
+              if (!kByBlock || step != -2) {
+                put_at(m0, h00 > 0.f, s0, 0, (uint32_t)(kt * 4 + 0), ring_n);
+                put_at(m1, h01 > 0.f, s0, 8, (uint32_t)(kt * 4 + 1), ring_n + c0);
+              }
+              if (!kByBlock || step != -3) {
+                const int base = !kByBlock || step == -1 ? ring_n + c0 + c1 : ring_n;
+                put_at(m2, h10 > 0.f, s1, 0, (uint32_t)(kt * 4 + 2), base);
+                put_at(m3, h11 > 0.f, s1, 8, (uint32_t)(kt * 4 + 3), base + c2);
+              }
+              step = kByBlock && step == -3 ? -2 : 8;
             } else {
               const int hb = step >> 1;
               if ((sub >> lane) & 1ull) {
@@ -788,10 +805,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
         }
       });
     });
-    flush(0, nt);
+    flush(0, nt_w);
     __builtin_amdgcn_s_waitcnt(0x0f70);  // the wave's stream is in memory before it reads it back
+    if constexpr (KP > 1) {
+      if (lane == 0) s_len[wave_id] = stream_n;
+    }
     __syncthreads();                      // every wave has left the K tiles: LDS becomes the lists
-    if (s_giveup[0] | s_giveup[1]) {
+    bool too_long = false;
+    if constexpr (KP > 1) {
+#pragma unroll
+      for (int w = 0; w < NW; ++w) too_long = too_long || s_len[w] + s_len[NW + w] > SG::kListCap;
+    }
+    if ((s_giveup[0] | s_giveup[1]) || too_long) {
       if (tid == 0) {
         *flag = 1;
         atomicAdd(&p.queue[kCtrlFlagged], 1u);
@@ -810,7 +835,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
     uint32_t* const row_cnt = reinterpret_cast<uint32_t*>(wave_lds + SG::kListCap * 6);     // 32 counters
     uint32_t* const row_start = row_cnt + 32;                                                // 33 offsets
     float* const row_inv = reinterpret_cast<float*>(row_start + 33);                         // 32 x 1 / sum p
-    if (lane < 32) row_cnt[lane] = 0u;
+    // (KP = 2: each part's wave counts and places its own entries, the first part's in front of the second's, so that a list's
+    // order does not depend on which wave is first)
+    uint32_t* const own_cnt = KP > 1 && part ? row_cnt + 128 : row_cnt;
+    if (lane < 32) own_cnt[lane] = 0u;
     {
       constexpr int kPer = (SG::kListCap + 63) / 64;
       uint2 ent[kPer];
@@ -819,16 +847,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
       for (int j = 0; j < kPer; ++j) {
         const int e = j * 64 + lane;
         ent[j] = uint2{0u, 0u};
-        if (e < stream_n) ent[j] = stream[e];
+        if (e < stream_n) ent[j] = stream[place(e)];
       }
 #pragma unroll
       for (int j = 0; j < kPer; ++j) {
         const int e = j * 64 + lane;
         pos[j] = 0u;
-        if (e < stream_n) pos[j] = atomicAdd(&row_cnt[(ent[j].y >> 20) & 31u], 1u);
+        if (e < stream_n) pos[j] = atomicAdd(&own_cnt[(ent[j].y >> 20) & 31u], 1u);
+      }
+      if constexpr (KP > 1) {
+        __syncthreads();
+        if (part && p.save_streams) {  // kept for the backward: behind the first part's, in the order of the keys
+          const int first = s_len[wave];
+#pragma unroll
+          for (int j = 0; j < kPer; ++j) {
+            const int e = j * 64 + lane;
+            if (e < stream_n) stream[first + e] = ent[j];
+          }
+        }
       }
       {
-        const int c = lane < 32 ? (int)row_cnt[lane] : 0;
+        int c = lane < 32 ? (int)row_cnt[lane] : 0;
+        if constexpr (KP > 1) c += lane < 32 ? (int)row_cnt[128 + lane] : 0;
         const int incl = wave_scan_i(c);
         if (lane < 32) row_start[lane] = (uint32_t)(incl - c);
         if (lane == 31) row_start[32] = (uint32_t)incl;
@@ -837,7 +877,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
       for (int j = 0; j < kPer; ++j) {
         const int e = j * 64 + lane;
         if (e < stream_n) {
-          const uint32_t at = row_start[(ent[j].y >> 20) & 31u] + pos[j];
+          uint32_t at = row_start[(ent[j].y >> 20) & 31u] + pos[j];
+          if (KP > 1 && part) at += row_cnt[(ent[j].y >> 20) & 31u];
           lval[at] = __builtin_bit_cast(float, ent[j].x);
           lkey[at] = (uint16_t)(ent[j].y & 0xffffu);
           // the tile mask takes every candidate's tile: a superset of the tiles with a non-zero probability by the few
@@ -849,7 +890,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
     }
 
     // ---- threshold: Newton from the left on the row's candidates (its two lanes take alternate entries) -----------
-    const int row_lo = (int)row_start[lq], row_end = (int)row_start[lq + 1];
+    // (KP = 2: each wave has half of the rows from here on, four lanes a row)
+    constexpr int kRowsW = 32 / KP, kLanes = 2 * KP;
+    const int row = KP > 1 ? kRowsW * part + (lane & (kRowsW - 1)) : lq, sub = KP > 1 ? lane / kRowsW : lh;
+    if constexpr (KP > 1) __syncthreads();  // the lists are complete
+    const int row_lo = (int)row_start[row], row_end = (int)row_start[row + 1];
     float t = 0.f;  // threshold minus lo, raw units
     {
       const float target = (AM == ATT_15) ? inv_qs * inv_qs : inv_qs;
@@ -860,14 +905,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
       const int max_len = (int)wave_max((float)(row_end - row_lo));
       for (int it = 0; it < (AM == ATT_GEN ? 96 : 24); ++it) {
         float a0 = 0.f, a1 = 0.f;
-        for (int o = 0; o < max_len; o += 8) {
-          const int e0 = row_lo + lh + o;
+        for (int o = 0; o < max_len; o += 4 * kLanes) {
+          const int e0 = row_lo + sub + o;
           const int e0r = e0 < SG::kListCap ? e0 : SG::kListCap;
           float x[4];
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const float raw = lval[e0r + 2 * j];
-            x[j] = e0 + 2 * j < row_end ? raw : -INFINITY;
+            const float raw = lval[e0r + kLanes * j];
+            x[j] = e0 + kLanes * j < row_end ? raw : -INFINITY;
           }
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
@@ -886,6 +931,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
             }
           }
         }
+        if constexpr (KP > 1) {
+          a0 += __shfl_xor(a0, 16, 64);
+          a1 += __shfl_xor(a1, 16, 64);
+        }
         a0 += __shfl_xor(a0, 32, 64);
         a1 += __shfl_xor(a1, 32, 64);
         const float step = (AM == ATT_15) ? (a0 - target) / (2.f * a1) : (AM == ATT_2) ? (a0 - target) / a1 : (a0 - 1.f) * inv_qs / (p.c0 * a1);
@@ -896,7 +945,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
     }
     // scores -> probabilities (not yet normalised): the row's first lane rewrites its list in place, keeping only the
     // support; 1 / sum per row
-    {
+    if constexpr (KP > 1) {  // (the row's four lanes together, four entries a turn, all rows alike: what a lane keeps goes behind what
+                             // the lanes in front of it keep)
+      const int max_len = (int)wave_max((float)(row_end - row_lo));
+      const unsigned long long one = 0x0001000100010001ull;  // the row's lanes
+      float psum = 0.f;
+      int w = row_lo;
+      for (int o = 0; o < max_len; o += kLanes) {
+        const int e = row_lo + o + sub;
+        const bool has = e < row_end;
+        const float u = has ? lval[e] - t : 0.f;
+        const uint16_t key = has ? lkey[e] : (uint16_t)0;
+        const unsigned long long m = (__builtin_amdgcn_ballot_w64(u > 0.f) >> (lane & 15)) & one;
+        if (u > 0.f) {
+          const float pv = (AM == ATT_15) ? u * u : (AM == ATT_2) ? u : fast_exp2(p.c0 * fast_log2(u * qs));
+          const int at = w + __builtin_popcountll(m & ((1ull << (16 * sub)) - 1ull));
+          lval[at] = __builtin_bit_cast(float, pack2<T>(pv, 0.f));
+          lkey[at] = key;
+          psum += pv;
+        }
+        w += __builtin_popcountll(m);
+      }
+      psum += __shfl_xor(psum, 16, 64);
+      psum += __shfl_xor(psum, 32, 64);
+      const float lo_row = __shfl(lo_raw, row, 64);
+      if (sub == 0) {
+        const int qr = wave_row0 + row;
+        row_cnt[row] = (uint32_t)(w - row_lo);
+        row_inv[row] = (qr < L && psum > 0.f) ? 1.f / psum : 0.f;
+        if (qr < L && p.taus) p.taus[(size_t)(b * p.Hq + h) * N + qr] = (lo_row + t) * qs;
+        if (qr < L && p.save_tshift) p.save_tshift[(size_t)(b * p.Hq + h) * N + qr] = t;
+      }
+    } else {
       float psum = 0.f;
       int w = row_lo;
       if (lh == 0) {
@@ -935,21 +1015,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
       unsigned char* obase = reinterpret_cast<unsigned char*>(p.out) + (qo_base + (size_t)wave_row0 * D) * 2 + col * 16;
       // The rows are served kGroups at a time and a round lasts as long as its longest support: rows in the order of
       // their supports' sizes, longest first, keep the rows of a round alike.
-      uint8_t* const order = reinterpret_cast<uint8_t*>(row_inv + 32);
+      uint8_t* const order = reinterpret_cast<uint8_t*>(row_inv + 32) + kRowsW * part;
       {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
         int rank = 0;
-        const int mine = lane < 32 ? (int)row_cnt[lane] : 0;
-        for (int o = 0; o < 32; ++o) {
-          const int c = (int)row_cnt[o];
+        const int row0 = kRowsW * part;
+        const int mine = lane < kRowsW ? (int)row_cnt[row0 + lane] : 0;
+        for (int o = 0; o < kRowsW; ++o) {
+          const int c = (int)row_cnt[row0 + o];
           rank += (c > mine || (c == mine && o < lane)) ? 1 : 0;
         }
-        if (lane < 32) order[rank] = (uint8_t)lane;
+        if (lane < kRowsW) order[rank] = (uint8_t)(row0 + lane);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
       }
-      for (int r0 = 0; r0 < 32; r0 += kGroups) {
+      for (int r0 = 0; r0 < kRowsW; r0 += kGroups) {
         const int r = (int)order[r0 + grp];
         const int e_lo = (int)row_start[r], e_hi = e_lo + (int)row_cnt[r];
         float acc[8];
@@ -989,7 +1070,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
     __syncthreads();  // every wave's tile marks are in
     if (bmask_out)
       for (int i = tid; i < p.mask_words; i += SG::kThreads) bmask_out[i] = (int32_t)mask_out[i];
-    if (p.save_lens && lane == 0) p.save_lens[stream_id] = (uint16_t)stream_n;
+    if (p.save_lens && lane == 0 && part == 0) p.save_lens[stream_id] = (uint16_t)(KP > 1 ? s_len[wave] + s_len[NW + wave] : stream_n);
     if (tid == 0) {
       *flag = 0;
       if (p.save_flags) p.save_flags[(size_t)(b * p.Hq + h) * n_mblk + mblk] = 1;
@@ -998,9 +1079,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADSP_SPARSE
 }
 
 // Workgroups to launch: as many as fit the device at once (each owns one event slot), at most `max_slots`.
-template <typename T, int D, int AM> static int launch_attn_sparse_one(const AttnParams& p, int max_slots, hipStream_t s) {
-  using SG = SparseGeo<T, D>;
-  auto kern = attn_fwd_sparse_kernel<T, D, AM>;
+template <typename T, int D, int AM, int KP> static int launch_attn_sparse_one(const AttnParams& p, int max_slots, hipStream_t s) {
+  using SG = SparseGeo<T, D, KP>;
+  auto kern = attn_fwd_sparse_kernel<T, D, AM, KP>;
   static int per_cu = 0, n_cu = 0;  // (one device family per process: gfx950)
   const size_t dyn = (size_t)p.mask_words * sizeof(uint32_t);
   if (per_cu == 0) {
@@ -1019,10 +1100,22 @@ template <typename T, int D, int AM> static int launch_attn_sparse_one(const Att
   return 0;
 }
 
+// Two waves share 32 rows (KP = 2) in launches of up to 512 row blocks: two workgroups of eight waves a CU are then all of them at
+// once, where one wave for 32 rows leaves a CU eight waves and the launch lasts as long as the chain of stages of its longest item,
+// of which KP = 2 halves each.  us, KP = 1 -> 2, whole forwards, causal unless noted: 32/8 heads, N = 2048, D = 128, q of spread 1 and 3: 120 -> 100,
+// 92 -> 79; 16/8, N = 4096, D = 128: 184 -> 137; 8, N = 8192, D = 64: 575 -> 499 with the gradients; 2 x 16 of up to 2000, D = 64: 113 -> 87; 16, N = 4096, D = 64,
+// alpha = 2, full: 119 -> 102.  Beyond the line KP = 1 has its waves side by side anyway: 2 x 32/8, N = 2048, D = 128: 171 -> 214, 3 x 16, N = 2048, D = 64:
+// 122 -> 133, 16, N = 8192, D = 64: 597 -> 616 (f16).
 template <typename T, int D> static int launch_attn_sparse(const AttnParams& p, int am, int max_slots, hipStream_t s) {
-  if (am == ATT_15) return launch_attn_sparse_one<T, D, ATT_15>(p, max_slots, s);
-  if (am == ATT_2) return launch_attn_sparse_one<T, D, ATT_2>(p, max_slots, s);
-  if (am == ATT_GEN) return launch_attn_sparse_one<T, D, ATT_GEN>(p, max_slots, s);
+  if ((long long)p.B * p.Hq * p.n_mblk <= 512) {
+    if (am == ATT_15) return launch_attn_sparse_one<T, D, ATT_15, 2>(p, max_slots, s);
+    if (am == ATT_2) return launch_attn_sparse_one<T, D, ATT_2, 2>(p, max_slots, s);
+    if (am == ATT_GEN) return launch_attn_sparse_one<T, D, ATT_GEN, 2>(p, max_slots, s);
+  } else {
+    if (am == ATT_15) return launch_attn_sparse_one<T, D, ATT_15, 1>(p, max_slots, s);
+    if (am == ATT_2) return launch_attn_sparse_one<T, D, ATT_2, 1>(p, max_slots, s);
+    if (am == ATT_GEN) return launch_attn_sparse_one<T, D, ATT_GEN, 1>(p, max_slots, s);
+  }
   return 2;
 }
 

@@ -255,3 +255,36 @@ def test_some_row_and_key_blocks_go_back_to_the_dense_backward_kernels(sparse_sw
             assert err < (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -10), err
     same = [torch.equal(a, b) for a, b in zip(grads[True][0].split(128, dim=2), grads[False][0].split(128, dim=2))]
     assert same[4] and not any(same[:4]), same
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,N,D,alpha,causal,lens", [
+    (1, 2, 64, 64, 1.5, True, None),             # one tile: the second part of the keys is empty
+    (3, 3, 190, 128, 1.5, True, [190, 1, 129]),  # three tiles: two and one
+    (2, 2, 577, 64, 1.333, False, [577, 65]),
+    (2, 4, 1100, 128, 1.5, True, [1100, 1025]),  # more candidates a tile than a wave's ring holds
+    (1, 3, 2048, 128, 2.0, False, [2001]),
+    (1, 8, 4096, 64, 1.5, True, None),
+])
+def test_two_waves_or_one_for_32_rows(dtype, B, H, N, D, alpha, causal, lens):
+    """Up to 512 row blocks two waves share 32 rows, beyond them one wave has them: the same problem by itself and as the first
+    item of a batch that crosses the line.  Thresholds are solved to rounding on either side: a few units of fp32's last place in scores of a
+    size of up to ten; outputs differ by roundings of the type, at most two of them."""
+    q, k, v = qkv(B, H, H, N, D, dtype, seed=N + D)
+    varlen = torch.tensor(lens or [N] * B, dtype=torch.int32)
+    version = 1 if alpha != 1.5 or not causal else 2
+    out, tau, _ = forward(q, k, v, varlen, version, alpha, causal)
+    assert torch.equal(out, forward(q, k, v, varlen, version, alpha, causal)[0])
+    copies = 512 // (B * H * ((N + 127) // 128)) + 1
+    many = [x.repeat(copies, 1, 1, 1) for x in (q, k, v)]
+    out_b, tau_b, _ = forward(*many, varlen.repeat(copies), version, alpha, causal)
+    for b in range(B):
+        L = int(varlen[b])
+        assert (out[b, :, L:] == 0).all() and (out_b[b, :, L:] == 0).all()
+        assert (tau[b, :, :L] - tau_b[b, :, :L]).abs().max().item() < 1e-5
+        ulp = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+        assert ((out[b].float() - out_b[b].float()).abs() <= 2 * ulp * (out_b[b].float().abs() + 0.25)).all()
+        rows = sorted({r for r in (0, 1, 31, 32, 63, 64, 127, 128, 700, L // 2, L - 2, L - 1) if 0 <= r < L})
+        for h in (0, H - 1):
+            want = oracle_rows_of_attention(q, k, v, b, h, rows, alpha, causal, L)
+            assert max_err(out[b, h, rows], want) < 2e-2 and max_err(out_b[b, h, rows], want) < 2e-2
