@@ -4,9 +4,13 @@
 // What bounds it: matrix and vector pipe together, at the 1.8 - 1.9 GHz that their power leaves (a block of 32 x 32 scores takes two to
 // four products of 34 cycles a walk and three vector instructions a score).  So the number of walks over the keys is what counts.
 //
-// A row's threshold starts from a sample of 256 keys held in registers, where Newton's steps cost no memory; one step on every
-// second tile corrects the sampling error, and one or two on all tiles finish it (a step squares what is left; flat scores: two and
-// a half walks and the output's).  The output walk's own sums take the threshold that a backward reads one step further.
+// A row's threshold starts from a sample of 256 keys held in registers.  alpha = 1.5: from the sample's mean and spread, as if the scores were
+// normal, unless the sample contradicts it; the walks' steps know the members' number and the density where they end (set_step), so that one leaves the
+// cube of what there was, at the four instructions a score that the sums and the maximum took.  Where a row has hundreds of members, a quarter of the
+// tiles corrects the start, the others give a threshold, and the quarter's sums there go together with the others', moved as far
+// (move_sums): one and a quarter walks and the output's.  Fewer members: walks over all tiles until a step is small, mostly two; a wave whose rows are done
+// no longer takes part.  Other alphas: Newton's steps on the sample, one on every second tile, one or two on all tiles (a step squares what is left).
+// The output walk's own sums take the threshold that a backward reads one step further.
 //
 // Split: four waves of 32 rows, tiles of K (and V in the output walk) through two stages of LDS, two workgroups a CU; two blocks of a tile go
 // together, the sums or weights of one between the products of the other (tile16::stream).  The weights' sum is that of the rounded
@@ -16,6 +20,9 @@
 // D = 128: 3530 -> 1270; 8 heads, N = 8192, alpha = 1.333: 2860 -> 1020, 3250 -> 1200; 4 x 16, N = 4096, alpha = 2: 2280 -> 1760, 3630 -> 2770 (there
 // the sums are piecewise linear and a step halves the support at best: five to eight walks).  Against 64 bits: bf16 2.3e-3 as before, f16 4.5e-4
 // -> 2.9e-4 at N = 6000.
+// alpha = 1.5, Newton's steps (sample, half, two and more walks) -> this, the same errors: 4 x 16 heads, N = 4096, not causal, q of spread 1/8 and 1/2: D = 64 724 -> 583,
+// 1151 -> 851, D = 128 1254 -> 973, 1957 -> 1425; 2 x 16 heads of up to 1100, 2100, 3000 and 9000, D = 64, 1/8: 49.7 -> 48.7, 98.2 -> 97.5, 151.5 -> 131, 1035 -> 764,
+// 1/2: 74.5 -> 68.9, 151 -> 145, 235 -> 197, 1547 -> 1186.  Rows of one key far above thousands of others had errors of up to 3.3e-2 and have 4e-3.
 #pragma once
 #include "attn_tile16.h"
 
@@ -23,13 +30,42 @@ namespace adsp {
 namespace fwd16 {
 using namespace tile16;
 
-// A walk's Newton step of x times the mean of u leaves about (c0 - 1) / 2 (n sum u^2 / (sum u)^2 - 1) x^2 of it (n members, alpha = 1.5): half of
-// that square for flat scores, more where few keys have most of the weight.  The last walk takes steps of up to this: an error of the weights
-// below their rounding is left then; the thresholds that a backward reads are taken a step further by the output walk's sums.  bf16,
-// alpha = 1.5: with 0.06 a row whose last step was just small enough had an error of 4.2e-3 where rounding alone gives the worst of 256 row
-// blocks 3.35e-3 (8 heads, N = 4096, D = 128, q of spread 0.03 to 2); 0.04 has 3.35e-3, 0.03 the same.  us, 0.06 / 0.04 / 0.03, 4 x 16 heads, N = 4096,
-// q of spread 1/8: D = 64 699 / 712 / 732, D = 128 1190 / 1213 / 1221; spread 1/2, D = 64: 1081 / 1125 / 1144.
-template <typename T, int AM> constexpr float kNear = AM == ATT_15 && elem_traits<T>::kIsBf16 ? 0.04f : 0.02f;
+// The last walk takes steps of up to this times (sum u^2 / sum u) -- alpha = 1.5: times the mean of u, see near_of --: an error of the weights below
+// their rounding is left then; the thresholds that a backward reads are taken a step further by the output walk's sums.  A walk's Newton step of x times the mean of u leaves about (c0 - 1) / 2 (n sum u^2 / (sum u)^2 - 1)
+// x^2 of it (n members), set_step a twentieth of x^3.  With Newton's steps, bf16, alpha = 1.5, and 0.06 a row whose last step was just
+// small enough had an error of 4.2e-3 where rounding alone gives the worst of 256 row blocks 3.35e-3 (8 heads, N = 4096, D = 128, q of spread 0.03 to 2); 0.04 had
+// 3.35e-3: some 1e-3 of the mean of u left.  set_step leaves as much behind 0.22 of the mean of u where there are 256 members (f16: a sixth of it behind 0.15); with fewer they are
+// further apart, and a member that changes counts for more.  The parts' sums are moved by up to 2.5 times that where
+// the sums are as a normal distribution's upper part has them and keys are left to become members, otherwise by 1.5 times (by 2.5 always: rows of two clusters of scores, or of one key far above the others,
+// up to 4.7e-3 and 2e-2; by 2: 584 -> 645 us, D = 64).
+template <typename T, int AM> constexpr float kNear = AM == ATT_15 ? (elem_traits<T>::kIsBf16 ? 0.22f : 0.15f) : 0.02f;
+// alpha = 1.5: steps from the sums of u^2 and u and the members' number.  With the same members the sum of u^2 is a parabola in the threshold; the
+// members that change are few, near u = 0, and their density there follows from the three sums (members_density: exact for u distributed evenly
+// and exponentially, and within 2 % for the upper part of a normal distribution).  What a step of x times the mean of u leaves of it, root of
+// mean square and the most of 256 rows of 575 members: x = 0.2: 2e-4 and 6e-4, 0.3: 5e-4 and 2e-3 (Newton's on the norm 9e-3 and 2e-2); of 62 members: 5e-4
+// and 2e-3, 1.5e-3 and 4e-3.  Where the parabola has no root nearby Newton's step on the norm is taken.
+__device__ __forceinline__ float members_density(float s0, float s1, float n) {
+  const float shape = n * s0 * fast_rcp(s1 * s1);
+  return n * n * fast_rcp(s1) * __builtin_amdgcn_fmed3f(fmaf(0.75f, shape, -0.5f), 0.f, 1.5f);
+}
+__device__ __forceinline__ float set_step(float s0, float s1, float n, float c0) {
+  const float disc = fmaf(s1, s1, -n * (s0 - 1.f));
+  if (!(disc > 0.25f * s1 * s1)) return f32path::norm_step<ATT_15>(s0, s1, c0);
+  const float root = __builtin_amdgcn_sqrtf(disc), x = (s0 - 1.f) * fast_rcp(s1 + root);
+  return x * (1.f - fminf(members_density(s0, s1, n) * x * x * fast_rcp(6.f * root), 0.4f));  // (far away the density is another)
+}
+// the sums `by` further up
+__device__ __forceinline__ void move_sums(float by, float& s0, float& s1, float& n) {
+  const float d = members_density(s0, s1, n);
+  s0 = fmaf(by, fmaf(by, fmaf(by, d * (-1.f / 3.f), n), -2.f * s1), s0);
+  s1 = fmaf(by, fmaf(by, 0.5f * d, -n), s1);
+  n = fmaf(-by, d, n);
+}
+// Where the threshold of n keys of normally distributed scores lies (alpha = 1.5), in spreads above their mean: n s^2 ((1 + a^2) Q(a) - a phi(a)) = 1,
+// within 0.15 from n s^2 = 0.2 to 5000.
+__device__ __forceinline__ float normal_threshold(float ns2) {
+  return ns2 < 0.7f ? -__builtin_amdgcn_sqrtf(fmaxf(fast_rcp(ns2) - 1.f, 0.f)) : __builtin_amdgcn_sqrtf(fmaf(1.8f, fast_log2(ns2), 1.7f)) - 1.87f;
+}
 constexpr int kSample = 256;  // keys of the sample that a row's first threshold comes from
 
 template <typename T, int D, int AM, bool kTaus>
@@ -39,6 +75,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr int kRow = TL::kRow, kRows = kMaskRows, kBlk = kTR / 32, G = TL::kG;
   constexpr int kAhead = D == 64 ? 2 : 1;  // (registers)
   constexpr int kSampleTiles = kSample / kTR, NS = kSample / 32;
+  constexpr bool kSet = AM == ATT_15;  // steps with the members' number (set_step)
   __shared__ __align__(1024) unsigned char smem[4 * TL::kBytes];  // two stages of a K and a V tile
   __shared__ uint32_t more_flag[4];
   extern __shared__ uint32_t mask_lds[];  // the tile mask of the row block, where one is asked for
@@ -90,6 +127,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int n_key_blk = (key_hi + 31) / 32;
   const bool all_sampled = n_key_blk * 32 <= kSample;
   float t;  // in z units
+  bool flat = false;  // hundreds of members, alpha = 1.5
   {
     auto block_of = [&](int x) { return all_sampled ? x : (int)((long long)x * whole / (kSample / 32)); };  // block x of the sample
 #pragma unroll
@@ -107,7 +145,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __syncthreads();
     stream<NS * G, kAhead>([&](int g, u32x4(&a)[4]) { tl.rows(g / G / kBlk, g / G % kBlk, g % G, a); },
                       [&](int g, int k, const u32x4& a) { s[g / G] = mfma_16bit<T>(a, piece<D>(qf, 4 * (g % G) + k), s[g / G]); });
-    float mx = -INFINITY;
+    float mx = -INFINITY, m1 = 0.f, m2 = 0.f;
     if (all_sampled) {
 #pragma unroll
       for (int x = 0; x < NS; ++x) hide(x * 32, s[x]);
@@ -115,27 +153,73 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int x = 0; x < NS; ++x)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[x][i]);
+      for (int i = 0; i < 16; ++i) {
+        mx = fmaxf(mx, s[x][i]);
+        if constexpr (kSet) {
+          m1 += s[x][i];
+          m2 = fmaf(s[x][i], s[x][i], m2);
+        }
+      }
     mx = top(mx);
     // From above its root alpha = 2's sum, of few keys, throws a step far below: its sample aims at three times the sum.
     const float ratio = all_sampled ? 1.f : (float)(lim + 1) * (AM == ATT_2 ? 1.f / (3 * kSample) : 1.f / kSample);
     const float t_min = fmaf(mx, qs, -1.f);
     t = t_min;
+    float spread = 0.f;
+    bool keep = false, far_out = false;  // some ten members of the sample at most are to be expected
+    if constexpr (kSet) {
+      if (!all_sampled) {  // (as if the scores were normal: two steps less than from t_min)
+        const float mean = total(m1) * (qs / kSample), var = fmaxf(fmaf(-mean, mean, total(m2) * (qs * qs / kSample)), 0.f);
+        const float a = normal_threshold(var * (float)(lim + 1)), guess = fmaf(a, spread = __builtin_amdgcn_sqrtf(var), mean);
+        far_out = a > 1.7f;
+        keep = guess > t_min && guess < t_min + 1.f + (far_out ? spread : 0.f);  // (with the sample's maximum in view)
+        t = keep ? guess : t_min;
+      }
+    }
+    float many = 0.f;  // members that the sample makes out
     for (int it = 0; it < 16; ++it) {
-      float s0 = 0.f, s1 = 0.f;
+      float s0 = 0.f, s1 = 0.f, step;
+      if constexpr (kSet) {
+        // (below the threshold the difference's sign shows; u of up to a sample's rounding above 1 is no harm)
+        uint32_t below = 0u, signs = 0u;
 #pragma unroll
-      for (int x = 0; x < NS; ++x)
+        for (int x = 0; x < NS; ++x) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) add_powers<AM>(__builtin_amdgcn_fmed3f(fmaf(s[x][i], qs, -t), 0.f, 1.f), c0, s0, s1);
-      const float step = f32path::norm_step<AM>(total(s0) * ratio, total(s1) * ratio, c0);
+          for (int i = 0; i < 16; ++i) {
+            const float d = fmaf(s[x][i], qs, -t), u = fmaxf(d, 0.f);
+            s0 = fmaf(u, u, s0);
+            s1 += u;
+            signs = __builtin_amdgcn_alignbit(signs, __builtin_bit_cast(uint32_t, d), 31);
+          }
+          if (x & 1) below += __builtin_popcount(signs);
+        }
+        s0 = total(s0) * ratio;
+        s1 = total(s1) * ratio;
+        const float n = total((float)(NS * 16 - (int)below)) * ratio;
+        // (the set's steps come from either side of the threshold; Newton's, from below, end in any case)
+        step = it < 6 ? set_step(s0, s1, n, c0) : f32path::norm_step<AM>(s0, s1, c0);
+        many = n;
+        // (the sample's own error is as large as the guess's: one that the sample does not contradict stays)
+        if (it == 0) keep = keep && (s1 > 0.f ? fabsf(step) <= (far_out ? spread : s0 * fast_rcp(s1)) : far_out);
+        step = keep ? 0.f : (s1 > 0.f ? step : t_min - t);
+      } else {
+#pragma unroll
+        for (int x = 0; x < NS; ++x)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) add_powers<AM>(__builtin_amdgcn_fmed3f(fmaf(s[x][i], qs, -t), 0.f, 1.f), c0, s0, s1);
+        step = f32path::norm_step<AM>(total(s0) * ratio, total(s1) * ratio, c0);
+      }
       t = fmaxf(t + step, t_min);
       if (__builtin_amdgcn_ballot_w64(fabsf(step) > (all_sampled ? 2e-4f : 2e-2f)) == 0ull) break;
     }
+    flat = many >= 224.f;
   }
 
-  // ---- walks over the tiles first, first + step, ... below n ----
+  // ---- walks over the tiles next(-1), next of that, ... below n ----
   // pair(block) for two of the wave's blocks of a tile that all of its rows see in full, else one(block, its first key)
-  auto walk = [&](int first, int step, int n, bool with_v, auto&& one, auto&& pair) {
+  bool idle = false;  // the wave's rows are done: it loads its share of the tiles for the others
+  auto walk = [&](auto&& next, int n, bool with_v, auto&& one, auto&& pair) {
+    const int first = next(-1);
     __syncthreads();
     int st = 0;
     auto issue = [&](int s, int x) {
@@ -143,10 +227,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (with_v) tl.issue(vg, x * kTR, L, smem + s * 2 * TL::kBytes + TL::kBytes, wave, lane);
     };
     if (first < n) issue(0, first);
-    for (int cur = first; cur < n; cur += step) {
+    for (int cur = first, nxt; cur < n; cur = nxt) {
+      nxt = next(cur);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
-      if (cur + step < n) issue(st ^ 1, cur + step);
+      if (nxt < n) issue(st ^ 1, nxt);
+      if (!idle)
 #pragma unroll
       for (int x = 0; x < kBlk; x += 2) {
         const int k0 = cur * kTR + x * 32;
@@ -169,22 +255,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     if (st) tl.move(-2u * TL::kBytes);
   };
+  auto every = [](int cur) { return cur + 1; };
   auto mul = [&](int g, int k, const u32x4& a, f32x16& s) { s = mfma_16bit<T>(a, piece<D>(qf, 4 * (g % G) + k), s); };
 
-  // sums of u^c0 and u^(c0 - 1) above t, and the maximum less t, over the tiles; in raw units of u for alpha = 1.5 and 2
-  float s0, s1, mx;
-  auto sums_walk = [&](int first, int step, int n) {
+  // sums of u^c0 and u^(c0 - 1) above t, and their number (alpha = 1.5) or the maximum less t, over the tiles; in raw units of u for
+  // alpha = 1.5 and 2.  A score's sign goes into a word with those of the block's others, and the words' ones are counted.
+  float s0 = 0.f, s1 = 0.f, mx = -INFINITY, members = 0.f;
+  auto sums_walk = [&](auto&& next, int n) {
+    const float k0 = s0, k1 = s1, kn = members;
     s0 = s1 = 0.f;
     mx = -INFINITY;
+    uint32_t signs = 0u;
+    int count = 0;
     const f32x16 from_t = splat(-t * inv_qs);
     f32x16 late = splat(-INFINITY);
     auto add = [&](float x) {
-      mx = fmaxf(mx, x);
-      if constexpr (AM == ATT_15) {
+      if constexpr (kSet) {
         const float u = __builtin_amdgcn_fmed3f(x, 0.f, INFINITY);
         s0 = fmaf(u, u, s0);
         s1 += u;
-      } else if constexpr (AM == ATT_2) {
+        signs = __builtin_amdgcn_alignbit(signs, __builtin_bit_cast(uint32_t, x), 31);
+        return;
+      }
+      mx = fmaxf(mx, x);
+      if constexpr (AM == ATT_2) {
         s0 += __builtin_amdgcn_fmed3f(x, 0.f, INFINITY);
         s1 += x > 0.f ? 1.f : 0.f;
       } else {
@@ -193,13 +287,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     };
     constexpr int kPer = 4 / G;  // values of a block per product of another
     walk(
-        first, step, n, false,
+        next, n, false,
         [&](int blk, int k0) {
           f32x16 s = from_t;
           stream<G, 2>([&](int g, u32x4(&a)[4]) { tl.rows(0, blk, g, a); }, [&](int g, int k, const u32x4& a) { mul(g, k, a, s); });
           if (k0 + 31 > lim_all) hide(k0, s);
 #pragma unroll
           for (int i = 0; i < 16; ++i) add(s[i]);
+          if constexpr (kSet) count += 16 - __builtin_popcount(signs & 0xffffu);
         },
         [&](int blk, int) {
           f32x16 x0 = from_t, x1 = from_t;
@@ -211,47 +306,128 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
                              for (int i = 0; i < kPer; ++i) add(g < G ? late[n4 * kPer + i] : x0[n4 * kPer + i]);
                            });
+          if constexpr (kSet) count += 32 - __builtin_popcount(signs);
           late = x1;
         });
 #pragma unroll
     for (int i = 0; i < 16; ++i) add(late[i]);
     s0 = total(s0);
     s1 = total(s1);
-    mx = top(mx);
+    if constexpr (kSet) members = total((float)(count + 16 - __builtin_popcount(signs & 0xffffu)));
+    else mx = top(mx);
     if constexpr (AM == ATT_15) {
       s0 *= qs * qs;
       s1 *= qs;
     } else if constexpr (AM == ATT_2) {
       s0 *= qs;
     }
+    if (idle) {
+      s0 = k0;
+      s1 = k1;
+      members = kn;
+    }
   };
-  // whether Newton's step stays in fp32 (it multiplies s0 by up to itself): not with a score far above the threshold, which an
+  // whether a step stays in fp32 (it multiplies s0 by up to itself): not with a score far above the threshold, which an
   // unsampled key may have; the maximum less 1 is the next threshold then
   auto in_range = [&]() -> bool { return s0 > 0.f && s0 < 1e18f && s1 > 0.f && s1 < 1e18f; };
+  auto step_of = [&](float ratio, bool set) -> float {
+    if constexpr (kSet) return set ? set_step(s0 * ratio, s1 * ratio, members * ratio, c0) : f32path::norm_step<AM>(s0 * ratio, s1 * ratio, c0);
+    else return f32path::norm_step<AM>(s0 * ratio, s1 * ratio, c0);
+  };
+  auto near_of = [&]() -> float {  // (few members have no density to go by)
+    if constexpr (kSet) return kNear<T, AM> * s1 * fast_rcp(members) * __builtin_amdgcn_sqrtf(fminf(members * (1.f / 256.f), 1.f));
+    else return kNear<T, AM> * s0 * fast_rcp(s1);
+  };
+  auto any_wave = [&](bool mine) -> bool {  // of a lane of the workgroup
+    __syncthreads();
+    const bool any = __builtin_amdgcn_ballot_w64(mine) != 0ull;
+    if (lane == 0) more_flag[wave] = any ? 1u : 0u;
+    __syncthreads();
+    return (more_flag[0] | more_flag[1] | more_flag[2] | more_flag[3]) != 0u;
+  };
+  float last_step = 0.f;
   if (!all_sampled) {
-    // a step on every second tile, where that is much more than the sample
-    const int half = whole * 32 / kTR / 2;
-    if (half * kTR >= 2 * kSample) {
-      sums_walk(1, 2, half * 2);
-      const float ratio = (float)(lim + 1) / (float)(half * kTR) * (AM == ATT_2 ? 0.9f : 1.f);
-      if (in_range()) t += fmaxf(mx * qs - 1.f, f32path::norm_step<AM>(s0 * ratio, s1 * ratio, c0));
-      else t += fmaxf(mx * qs - 1.f, 0.f);
-    }
-    for (int it = 0; it < 32; ++it) {
-      sums_walk(0, 1, nt);
-      // never below the row maximum less 1
-      float step = mx * qs - 1.f, near = 0.f;
-      if (in_range()) {
-        step = fmaxf(step, f32path::norm_step<AM>(s0, s1, c0));
-        near = kNear<T, AM> * s0 * fast_rcp(s1);
+    bool done = false;
+    if constexpr (kSet) {
+      // A step on every fourth tile (the first part), one on the others, and one on all of them: the first part's sums at the threshold
+      // that the second part gave, and the second's, which are known for the one before, moved there.  From 1792 keys on (at 1700 the quarter is too
+      // few keys and the walk over all follows all the same: 68 us against 64); with fewer than some hundred members likewise (N = 4096, D = 64, q of spread 1/4: 800
+      // against 727).
+      const int n_first = whole * 32 / kTR / 4 * 4;  // tiles 1, 5, 9, .. below it are the first part
+      if (n_first * kTR >= 7 * kSample && !any_wave(live && !flat)) {
+        auto first_part = [](int cur) { return cur < 0 ? 1 : cur + 4; };
+        auto second_part = [&](int cur) { return cur + 1 + ((cur & 3) == 0 && cur < n_first ? 1 : 0); };
+        const int first_keys = n_first / 4 * kTR;
+        const float keys = (float)(lim + 1);
+        sums_walk(first_part, n_first);
+        if (in_range()) t += step_of(keys / (float)first_keys, true);
+        sums_walk(second_part, nt);
+        bool ok = in_range();
+        if (!any_wave(live && !ok)) {
+          const float by = step_of(keys / (float)((lim + 1) - first_keys), true);
+          const float shape = members * s0 * fast_rcp(s1 * s1);
+          ok = fabsf(by) <= (shape > 1.35f && shape < 2.f && members < 0.9f * (keys - (float)first_keys) ? 2.5f : 1.5f) * near_of();
+          float r0 = s0, r1 = s1, rn = members;
+          move_sums(by, r0, r1, rn);
+          if (live) t += by;
+          sums_walk(first_part, n_first);
+          s0 += r0;
+          s1 += r1;
+          members += rn;
+          ok = ok && in_range();
+          if (ok) {
+            last_step = step_of(1.f, true);
+            ok = fabsf(last_step) <= near_of();
+            if (live) t += last_step;
+          }
+          done = !any_wave(live && !ok);
+        }
       }
-      if (live) t += step;
-      const bool more = __builtin_amdgcn_ballot_w64(live && fabsf(step) > fmaxf(near, 2e-6f)) != 0ull;
-      if (lane == 0) more_flag[wave] = more ? 1u : 0u;
-      __syncthreads();
-      const uint32_t any = more_flag[0] | more_flag[1] | more_flag[2] | more_flag[3];
-      if (any == 0u) break;
+    } else {
+      // a step on every second tile, where that is much more than the sample
+      const int half = whole * 32 / kTR / 2;
+      if (half * kTR >= 2 * kSample) {
+        sums_walk([](int cur) { return cur + 2; }, half * 2);  // (1, 3, ..)
+        const float ratio = (float)(lim + 1) / (float)(half * kTR) * (AM == ATT_2 ? 0.9f : 1.f);
+        if (in_range()) t += fmaxf(mx * qs - 1.f, step_of(ratio, false));
+        else t += fmaxf(mx * qs - 1.f, 0.f);
+      }
     }
+    for (int it = 0; it < 32 && !done; ++it) {
+      sums_walk(every, nt);
+      if constexpr (kSet) {
+        if (any_wave(!idle && live && !in_range())) {
+          mx = -INFINITY;
+          auto maximum = [&](int blk, int k0) {
+            f32x16 s = splat(-t * inv_qs);
+            stream<G, 2>([&](int g, u32x4(&a)[4]) { tl.rows(0, blk, g, a); }, [&](int g, int k, const u32x4& a) { mul(g, k, a, s); });
+            if (k0 + 31 > lim_all) hide(k0, s);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
+          };
+          walk(every, nt, false, maximum, [&](int blk, int k0) {
+            maximum(blk, k0);
+            maximum(blk + 1, k0 + 32);
+          });
+          mx = top(mx);
+        }
+      }
+      if (!idle) {
+        float step, near = 0.f;
+        if (in_range()) {
+          step = step_of(1.f, it < 6);
+          if constexpr (!kSet) step = fmaxf(step, mx * qs - 1.f);  // (never below the row maximum less 1)
+          near = near_of();
+        } else {
+          step = mx * qs - 1.f;
+        }
+        if (live) t += step;
+        last_step = step;
+        idle = __builtin_amdgcn_ballot_w64(live && fabsf(step) > fmaxf(near, 2e-6f)) == 0ull;
+      }
+      if (!any_wave(!idle)) break;
+    }
+    idle = false;
   }
 
   // ---- output ----
@@ -266,7 +442,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   f32x16 zero;
 #pragma unroll
   for (int i = 0; i < 16; ++i) zero[i] = 0.f;
-  float q0 = 0.f, q1 = 0.f;  // the sums at t, for the threshold that is kept
+  // The sums at t, for the threshold that is kept.  alpha = 1.5: that of u^2 is the rounded weights' (some 1e-4 off, which moves the
+  // threshold by as much of the mean of u), that of u the last walk's less the step, without an instruction a score.
+  float q0 = 0.f, q1 = 0.f;
   auto prob = [&](float x) -> float {
     // (within 1 but for the last step's remainder)
     const float u = __builtin_amdgcn_fmed3f(fmaf(x, qs, -t), 0.f, 1.f);
@@ -281,7 +459,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       e1 = fast_exp2(fast_log2(u) * (c0 - 1.f));  // (0 at 0)
       pr = e1 * u;
     }
-    if constexpr (kTaus) {
+    if constexpr (kTaus && !kSet) {
       q0 += pr;
       q1 += e1;
       asm volatile("" : "+v"(q0), "+v"(q1));  // (else the compiler gathers the terms of a block, in 36 registers)
@@ -303,7 +481,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (bmask && __builtin_amdgcn_ballot_w64(weights != 0u) != 0ull && lane == 0) atomicOr(&mask_lds[k0 >> 11], 1u << ((k0 >> 6) & 31));
   };
   walk(
-      0, 1, nt, true,
+      every, nt, true,
       [&](int blk, int k0) {
         f32x16 s = zero;
         stream<G, 2>([&](int g, u32x4(&a)[4]) { tl.rows(0, blk, g, a); }, [&](int g, int k, const u32x4& a) { mul(g, k, a, s); });
@@ -346,13 +524,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             });
         mark(any, k0);
       });
+  const float zsum = total(zacc[0]);
   if constexpr (kTaus) {
-    q0 = total(q0);
-    q1 = total(q1);
+    q0 = kSet ? zsum : total(q0);
+    q1 = kSet ? s1 - members * last_step : total(q1);
     if (!all_sampled && q0 > 0.f && q1 > 0.f) t += f32path::norm_step<AM>(q0, q1, c0);
     if (live && lh == 0) p.taus[q_row0 + qi] = t;
   }
-  const float zsum = total(zacc[0]);
   const float inv = live && zsum > 0.f ? 1.f / zsum : 0.f;
   __syncthreads();  // the tiles become the sums' scratch
   BwdTiles<T, D>::store_rows(o, inv, smem + wave * 32 * kRow, out, wave_row0, N, lane);
