@@ -77,18 +77,23 @@ static int launch_bwd_dense(const AttnBwdParams& p, int D, int dtype, int am, in
 // beyond the format's range saturated, rows from N on zero.  A thread converts 16 values.  Heads the probe has marked
 // as dense are skipped (`hints`: two words per head).  The values are multiplied by the head's power of two first
 // (`w1_scales`, from the probe).
+// What bounds it is memory: tiles that lie wholly behind a sequence's length, which no walk reads, are left out (8 x 8 heads, N <= 8192, D = 128: 32 -> 22 us).
 // (the first walk's operands lie on a grid of 1/16, see attn_sparse_kernel.h)
 #define G16(x) (((x) * ak + 786432.f) - 786432.f)
 template <typename T>
 __global__ __launch_bounds__(256) void k8_layout_kernel(const uint16_t* __restrict__ k, unsigned char* __restrict__ k8, int N,
-                                                       int Npad, int D, const uint32_t* hints, const float* w1_scales) {
+                                                       int Npad, int D, int Hkv, const void* varlen, int varlen_bits,
+                                                       const uint32_t* hints, const float* w1_scales) {
   const size_t head = blockIdx.y;
+  long long L = N;
+  if (varlen) L = varlen_bits == 64 ? ((const long long*)varlen)[head / Hkv] : (long long)((const int*)varlen)[head / Hkv];
   if (hints[2 * head] >= (1u << 20)) return;
   const float ak = w1_scales[4 * head + 1];
   const int per_row = D / 16;
   const long long id = (long long)blockIdx.x * 256 + threadIdx.x;
   if (id >= (long long)Npad * per_row) return;
   const int row = (int)(id / per_row), c = (int)(id % per_row);
+  if (row / kBN * kBN >= L) return;
   u32x4 out = {0u, 0u, 0u, 0u};
   if (row < N) {
     const uint16_t* src = k + (head * (size_t)N + row) * D + c * 16;
@@ -554,9 +559,9 @@ static int attn_common(const void* q, const void* k, const void* v, void* out, f
       const dim3 k8_grid((unsigned)(((long long)p.Npad * (D / 16) + 255) / 256), (unsigned)(B * Hkv));
       launch_probe(p, D, dtype, am, nullptr, nullptr, s);
       if (dtype == ADSP_BF16) {
-        hipLaunchKernelGGL(k8_layout_kernel<bf16_t>, k8_grid, dim3(256), 0, s, (const uint16_t*)k, ws + w.k8_off, N, p.Npad, D, (const uint32_t*)p.hints, (const float*)p.w1_scales);
+        hipLaunchKernelGGL(k8_layout_kernel<bf16_t>, k8_grid, dim3(256), 0, s, (const uint16_t*)k, ws + w.k8_off, N, p.Npad, D, Hkv, varlen, varlen_bits, (const uint32_t*)p.hints, (const float*)p.w1_scales);
       } else {
-        hipLaunchKernelGGL(k8_layout_kernel<f16_t>, k8_grid, dim3(256), 0, s, (const uint16_t*)k, ws + w.k8_off, N, p.Npad, D, (const uint32_t*)p.hints, (const float*)p.w1_scales);
+        hipLaunchKernelGGL(k8_layout_kernel<f16_t>, k8_grid, dim3(256), 0, s, (const uint16_t*)k, ws + w.k8_off, N, p.Npad, D, Hkv, varlen, varlen_bits, (const uint32_t*)p.hints, (const float*)p.w1_scales);
       }
       int rc = dtype == ADSP_BF16 ? (D == 64 ? launch_attn_sparse_bf16_d64(p, am, w.slots, s) : launch_attn_sparse_bf16_d128(p, am, w.slots, s))
                                   : (D == 64 ? launch_attn_sparse_f16_d64(p, am, w.slots, s) : launch_attn_sparse_f16_d128(p, am, w.slots, s));
