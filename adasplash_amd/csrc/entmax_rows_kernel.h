@@ -4,9 +4,9 @@
 // from HBM exactly once (16-byte loads, the whole row then lives in registers), the threshold is solved on the
 // few entries that can be in the support, and the result is written once.  A row that does not start or end on a
 // 16-byte boundary (an odd number of columns) keeps aligned 16-byte accesses for its inner part; the up to
-// fifteen bytes at either end are an extra register slot of the row's first two lanes, read and written element by element
+// fifteen bytes at either end are an extra register slot of the row's first sixteen lanes, an element each, and the chunks are dealt out from a 128-byte line on
 // (fp32 [2048, 32001] forward and backward: 665 us when such rows took the streaming kernels, which re-read the row per
-// pass with 4-byte accesses, 196 us = 5.4 TB/s now; [1024, 65536]: 1003 and 198 us).  Rows longer than the registers of
+// pass with 4-byte accesses, 196 us with the edges in two lanes, 183 us = 5.7 TB/s now; [1024, 65536]: 1003 and 195 us).  Rows longer than the registers of
 // 1024 threads hold take a streaming variant that re-reads the row (from L2) per pass.  Semantics follow
 // adasplash/triton_entmax_v2.py:363-536.
 #pragma once
@@ -207,26 +207,35 @@ template <int K> struct ListRow {
 template <int TPR> constexpr int rows_threads() { return TPR > 256 ? TPR : 256; }
 
 // A row as the threads that share it see it: `nvec` aligned 16-byte chunks from element `head` on, and with EDGE the elements
-// in front of and behind them: the row's first lane holds the front ones, its second lane the ones at the end.
+// in front of and behind them, one to a lane: the row's first lanes hold the front ones, those from the ninth on the ones at the end (two lanes with up to seven
+// each took a load and a store an element: of the figures below, bf16, 16384 x 8191 104.5 -> 91.4).  With EDGE the lanes' places start
+// `lead` chunks in front of the first, on a 128-byte line: a wave's load or store then takes whole lines, where one that starts and ends inside a line
+// costs that line twice.  `places`: how many the row's lanes have.  us, forward and backward, chunk 0 in the first lane and two lanes with all edge
+// elements -> this: fp32, 2048 x 32001: 97.8, 96.4 -> 89.4, 93.5; 32768 x 2047: 95.5, 98 -> 86.8, 95; bf16, 16384 x 8191: 104.2, 112 -> 87.9, 94.7; 2048 x 50000: 75.3, 78.2 -> 71.2,
+// 73.3; 32768 x 1000: 31, 36.6 -> 24.5, 26.6.
 template <typename T, bool EDGE> struct RowSpan {
   size_t base;       // index of the row's first element
   long long nvec;
+  int lead;          // (0 without EDGE, and where the row has no place to spare)
   int head;          // elements in front of the chunks (0 without EDGE)
-  long long e0;      // this lane's edge elements: index in the row, and count
-  int en;
-  __device__ __forceinline__ RowSpan(const void* x, long long row, long long cols, int t_in_row) {
+  long long e0;      // this lane's edge element: index in the row
+  bool edge;         // whether it has one
+  __device__ __forceinline__ RowSpan(const void* x, long long row, long long cols, int t_in_row, int places) {
     constexpr int kVec = elem_traits<T>::kVec;
     base = (size_t)row * cols;
     head = 0;
+    lead = 0;
     e0 = 0;
-    en = 0;
+    edge = false;
     if constexpr (EDGE) {
       const uint32_t addr = (uint32_t)(uintptr_t)x + (uint32_t)base * elem_traits<T>::kBytes;
       head = (int)((0u - addr) & 15u) / elem_traits<T>::kBytes;
       nvec = (cols - head) / kVec;  // (at least one: the dispatch asks for 2 kVec - 1 columns and more)
       const int tail = (int)(cols - head - nvec * kVec);
-      e0 = t_in_row == 0 ? 0 : cols - tail;
-      en = t_in_row == 0 ? head : (t_in_row == 1 ? tail : 0);
+      e0 = t_in_row < 8 ? t_in_row : cols - tail + (t_in_row - 8);
+      edge = t_in_row < head || (t_in_row >= 8 && t_in_row < 8 + tail);
+      lead = (int)((addr + (uint32_t)head * elem_traits<T>::kBytes) >> 4) & 7;
+      lead = nvec + lead <= places ? lead : 0;
     } else {
       nvec = cols / kVec;
     }
@@ -237,16 +246,8 @@ template <typename T, bool EDGE> struct RowSpan {
   __device__ __forceinline__ u32x4* chunks(void* y) const {
     return reinterpret_cast<u32x4*>(reinterpret_cast<char*>(y) + (base + head) * elem_traits<T>::kBytes);
   }
-  // the lane's edge elements of `x`, `fill` where it has none
-  __device__ __forceinline__ void load_edge(const void* x, float fill, float (&v)[elem_traits<T>::kVec]) const {
-#pragma unroll
-    for (int e = 0; e < elem_traits<T>::kVec; ++e) v[e] = fill;
-    if (en > 0) {
-#pragma unroll
-      for (int e = 0; e < elem_traits<T>::kVec - 1; ++e)
-        if (e < en) v[e] = load_elem<T>(x, base + e0 + e);
-    }
-  }
+  // the lane's edge element of `x`, `fill` where it has none
+  __device__ __forceinline__ float load_edge(const void* x, float fill) const { return edge ? load_elem<T>(x, base + e0) : fill; }
 };
 
 template <typename T, int AM, int NCHUNK, int TPR, bool EDGE>
@@ -265,8 +266,9 @@ __global__ __launch_bounds__(rows_threads<TPR>()) __attribute__((amdgpu_waves_pe
   // past the last row simply leaves (no block-level barrier is used in that configuration).
   if (row >= p.rows) return;
 
-  const RowSpan<T, EDGE> span(p.x, row, p.cols, t_in_row);
+  const RowSpan<T, EDGE> span(p.x, row, p.cols, t_in_row, NCHUNK * TPR);
   const long long nvec = span.nvec;
+  const int t_place = t_in_row - span.lead;
   const u32x4* xrow = span.chunks(p.x);
   u32x4* yrow = span.chunks(p.y);
 
@@ -276,13 +278,13 @@ __global__ __launch_bounds__(rows_threads<TPR>()) __attribute__((amdgpu_waves_pe
   } r;
 #pragma unroll
   for (int c = 0; c < NCHUNK; ++c) {
-    long long vi = (long long)c * TPR + t_in_row;
-    r.valid[c] = vi < nvec;
-    // a lane past the row end re-reads the row's last chunk and ignores it: no branch between the loads
+    long long vi = (long long)c * TPR + t_place;
+    r.valid[c] = EDGE ? (unsigned long long)vi < (unsigned long long)nvec : vi < nvec;
+    // a lane outside the row re-reads the row's last chunk and ignores it: no branch between the loads
     r.raw[c] = __builtin_nontemporal_load(xrow + (r.valid[c] ? vi : nvec - 1));
   }
-  float ev[kVec];
-  if constexpr (EDGE) span.load_edge(p.x, -INFINITY, ev);
+  float ev = -INFINITY;
+  if constexpr (EDGE) ev = span.load_edge(p.x, -INFINITY);
   if (t_in_row == 0) cand_n[r_in_blk] = 0;
 
   // pass 1: per-chunk and row maxima, in the input's own units
@@ -317,10 +319,7 @@ __global__ __launch_bounds__(rows_threads<TPR>()) __attribute__((amdgpu_waves_pe
     cmax[c] = r.valid[c] ? cm : -INFINITY;
     xm = fmaxf(xm, cmax[c]);
   }
-  if constexpr (EDGE) {
-#pragma unroll
-    for (int e = 0; e < kVec; ++e) xm = fmaxf(xm, ev[e]);
-  }
+  if constexpr (EDGE) xm = fmaxf(xm, ev);
   xm = row_max<TPR>(xm, sm);  // (TPR >= 256: its barriers also publish cand_n = 0)
   if constexpr (elem_traits<T>::kIsBf16) xm = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, xm) & 0xffff0000u);
 
@@ -340,12 +339,9 @@ __global__ __launch_bounds__(rows_threads<TPR>()) __attribute__((amdgpu_waves_pe
     }
   }
   if constexpr (EDGE) {
-#pragma unroll
-    for (int e = 0; e < kVec - 1; ++e) {
-      if (e < span.en && ev[e] >= x_thr) {
-        const int idx = atomicAdd(&cand_n[r_in_blk], 1);
-        if (idx < kCap) cand[r_in_blk][idx] = ev[e] * p.scale;
-      }
+    if (span.edge && ev >= x_thr) {
+      const int idx = atomicAdd(&cand_n[r_in_blk], 1);
+      if (idx < kCap) cand[r_in_blk][idx] = ev * p.scale;
     }
   }
   if constexpr (TPR > 64) __syncthreads();
@@ -385,7 +381,7 @@ __global__ __launch_bounds__(rows_threads<TPR>()) __attribute__((amdgpu_waves_pe
 #pragma unroll
   for (int c = 0; c < NCHUNK; ++c) {
     if (r.valid[c]) {
-      long long vi = (long long)c * TPR + t_in_row;
+      long long vi = (long long)c * TPR + t_place;
       u32x4 o = {0u, 0u, 0u, 0u};
       if (cmax[c] * p.scale > tau) {
         if constexpr (kVec == 4) {
@@ -403,9 +399,7 @@ __global__ __launch_bounds__(rows_threads<TPR>()) __attribute__((amdgpu_waves_pe
     }
   }
   if constexpr (EDGE) {
-#pragma unroll
-    for (int e = 0; e < kVec - 1; ++e)
-      if (e < span.en) store_elem<T>(p.y, span.base + span.e0 + e, prob<AM>(ev[e] * p.scale - tau, p.c0));
+    if (span.edge) store_elem<T>(p.y, span.base + span.e0, prob<AM>(ev * p.scale - tau, p.c0));
   }
 }
 
@@ -474,8 +468,9 @@ __global__ __launch_bounds__(rows_threads<TPR>()) void entmax_rows_bwd_reg_kerne
   const int t_in_row = tid % TPR, r_in_blk = tid / TPR;
   const long long row = (long long)blockIdx.x * kRowsPerBlock + r_in_blk;
   if (row >= rows) return;  // TPR >= 256: the whole block; TPR == 64: a wave, and no block barrier is used
-  const RowSpan<T, EDGE> span(y, row, cols, t_in_row);
+  const RowSpan<T, EDGE> span(y, row, cols, t_in_row, NCHUNK * TPR);
   const long long nvec = span.nvec;
+  const int t_place = t_in_row - span.lead;
   const u32x4* yrow = span.chunks(y);
   const u32x4* grow = span.chunks(dy);
   u32x4* xrow = span.chunks(dx);
@@ -486,8 +481,8 @@ __global__ __launch_bounds__(rows_threads<TPR>()) void entmax_rows_bwd_reg_kerne
   // all the loads of a row are in flight together
 #pragma unroll
   for (int c = 0; c < NCHUNK; ++c) {
-    const long long vi = (long long)c * TPR + t_in_row;
-    valid[c] = vi < nvec;
+    const long long vi = (long long)c * TPR + t_place;
+    valid[c] = EDGE ? (unsigned long long)vi < (unsigned long long)nvec : vi < nvec;
     yr[c] = __builtin_nontemporal_load(yrow + (valid[c] ? vi : nvec - 1));
   }
 #pragma unroll
@@ -496,18 +491,18 @@ __global__ __launch_bounds__(rows_threads<TPR>()) void entmax_rows_bwd_reg_kerne
   // line per wave instead of a kilobyte of HBM traffic) so that these loads need no branch either
   if constexpr (kKeepDy) {
 #pragma unroll
-    for (int c = 0; c < NCHUNK; ++c) gr[c] = __builtin_nontemporal_load(grow + (live[c] ? (long long)c * TPR + t_in_row : 0ll));
+    for (int c = 0; c < NCHUNK; ++c) gr[c] = __builtin_nontemporal_load(grow + (live[c] ? (long long)c * TPR + t_place : 0ll));
   }
-  float ey[kVec], eg[kVec];
+  float ey = 0.f, eg = 0.f;
   if constexpr (EDGE) {
-    span.load_edge(y, 0.f, ey);
-    span.load_edge(dy, 0.f, eg);
+    ey = span.load_edge(y, 0.f);
+    eg = span.load_edge(dy, 0.f);
   }
   float s[2] = {0.f, 0.f};
 #pragma unroll
   for (int c = 0; c < NCHUNK; ++c) {
     if (live[c]) {
-      const u32x4 g = kKeepDy ? gr[kKeepDy ? c : 0] : grow[(long long)c * TPR + t_in_row];
+      const u32x4 g = kKeepDy ? gr[kKeepDy ? c : 0] : grow[(long long)c * TPR + t_place];
 #pragma unroll
       for (int e = 0; e < kVec; ++e) {
         const float u = bwd_u<AM>(chunk_elem<T>(yr[c], e), cf);
@@ -517,12 +512,9 @@ __global__ __launch_bounds__(rows_threads<TPR>()) void entmax_rows_bwd_reg_kerne
     }
   }
   if constexpr (EDGE) {
-#pragma unroll
-    for (int e = 0; e < kVec - 1; ++e) {
-      const float u = bwd_u<AM>(ey[e], cf);
-      s[0] = fmaf(u, eg[e], s[0]);
-      s[1] += u;
-    }
+    const float u = bwd_u<AM>(ey, cf);
+    s[0] = fmaf(u, eg, s[0]);
+    s[1] += u;
   }
   row_sum<TPR, 2>(s, sm);
   const float q = s[1] > 0.f ? s[0] / s[1] : 0.f;
@@ -531,7 +523,7 @@ __global__ __launch_bounds__(rows_threads<TPR>()) void entmax_rows_bwd_reg_kerne
     if (valid[c]) {
       u32x4 o = {0u, 0u, 0u, 0u};
       if (live[c]) {
-        const u32x4 g = kKeepDy ? gr[kKeepDy ? c : 0] : grow[(long long)c * TPR + t_in_row];
+        const u32x4 g = kKeepDy ? gr[kKeepDy ? c : 0] : grow[(long long)c * TPR + t_place];
         if constexpr (kVec == 4) {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
@@ -543,13 +535,11 @@ __global__ __launch_bounds__(rows_threads<TPR>()) void entmax_rows_bwd_reg_kerne
                             bwd_u<AM>(chunk_elem<T>(yr[c], 2 * e + 1), cf) * (chunk_elem<T>(g, 2 * e + 1) - q));
         }
       }
-      __builtin_nontemporal_store(o, xrow + (long long)c * TPR + t_in_row);
+      __builtin_nontemporal_store(o, xrow + (long long)c * TPR + t_place);
     }
   }
   if constexpr (EDGE) {
-#pragma unroll
-    for (int e = 0; e < kVec - 1; ++e)
-      if (e < span.en) store_elem<T>(dx, span.base + span.e0 + e, bwd_u<AM>(ey[e], cf) * (eg[e] - q));
+    if (span.edge) store_elem<T>(dx, span.base + span.e0, bwd_u<AM>(ey, cf) * (eg - q));
   }
 }
 
@@ -584,13 +574,20 @@ inline bool rows_fit_grid(long long rows, long long nvec) {
   return threads < (1ll << 32);
 }
 
-// 0: the row's chunks are aligned and fill it; 1: it has edges; 2: neither (bases that differ in their offset from a 16-byte
+// The places that rows of `nvec` chunks ask for: where they do not start on a line, up to seven more, in front of the first chunk.  Rows of a few
+// hundred bytes do without where they have none to spare (32768 rows, bf16, 249 columns: 13.7 us with, 9.8 without; fp32, 125: 8.6, 7.7; beyond the line bf16,
+// 1019: 26.0, 30.1; fp32, 505: 23.6, 27.4).
+constexpr long long kRowsShort = 64;
+inline long long rows_places(long long rows, long long nvec, int shape) { return shape == 1 && nvec > kRowsShort && rows_fit_grid(rows, nvec + 7) ? nvec + 7 : nvec; }
+
+// 0: the rows' chunks are aligned and fill them, and the rows start on 128-byte lines or are short; 1: they have edges, or start inside a line; 2: neither (bases that differ in their offset from a 16-byte
 // boundary, elements off their own alignment, very short ragged rows, more chunks than the registers hold, more rows than a
 // launch of the register kernels holds): stream it
 template <typename T> static int rows_shape(uintptr_t a, uintptr_t b, uintptr_t c, long long rows, long long cols) {
   constexpr int kVec = elem_traits<T>::kVec;
   if (cols / kVec > kRowsMaxChunks || rows >= (1ll << 32) || !rows_fit_grid(rows, cols / kVec)) return 2;
-  if (((a | b | c) & 15) == 0 && cols % kVec == 0) return 0;
+  const bool whole = ((a | b | c) & 15) == 0 && cols % kVec == 0;
+  if (whole && (cols / kVec <= kRowsShort || (((a | b | c) & 127) == 0 && cols * elem_traits<T>::kBytes % 128 == 0))) return 0;
   if (((a ^ b) & 15) != 0 || ((a ^ c) & 15) != 0 || a % elem_traits<T>::kBytes != 0 || cols < 2 * kVec - 1) return 2;
   return 1;
 }
@@ -609,7 +606,7 @@ template <typename T, int AM> static void launch_fwd(const RowsParams& p, hipStr
     if (shape == 0) hipLaunchKernelGGL((entmax_rows_reg_kernel<T, AM, NC, TPR, false>), grid, block, 0, s, p);              \
     else hipLaunchKernelGGL((entmax_rows_reg_kernel<T, AM, NC, TPR, true>), grid, block, 0, s, p);                          \
   } while (0)
-  ADSP_ROWS_DISPATCH(p.cols / elem_traits<T>::kVec, ADSP_ROWS_FWD);
+  ADSP_ROWS_DISPATCH(rows_places(p.rows, p.cols / elem_traits<T>::kVec, shape), ADSP_ROWS_FWD);
 }
 
 template <typename T, int AM>
@@ -627,7 +624,7 @@ static void launch_bwd(const void* y, const void* dy, void* dx, long long rows, 
     if (shape == 0) hipLaunchKernelGGL((entmax_rows_bwd_reg_kernel<T, AM, NC, TPR, false>), grid, block, 0, s, y, dy, dx, rows, cols, cf); \
     else hipLaunchKernelGGL((entmax_rows_bwd_reg_kernel<T, AM, NC, TPR, true>), grid, block, 0, s, y, dy, dx, rows, cols, cf);      \
   } while (0)
-  ADSP_ROWS_DISPATCH(cols / elem_traits<T>::kVec, ADSP_ROWS_BWD);
+  ADSP_ROWS_DISPATCH(rows_places(rows, cols / elem_traits<T>::kVec, shape), ADSP_ROWS_BWD);
 }
 
 }  // namespace adsp

@@ -245,6 +245,35 @@ def test_rows_that_start_and_end_off_a_16_byte_boundary(cols, alpha, dtype, offs
         assert float(b[-1]) == 7.0 and (offset == 0 or float(b[0]) == 7.0)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("alpha", [1.5, 1.333])
+@pytest.mark.parametrize("chunks", [64, 65, 121, 122, 128, 249, 250, 1017, 1020, 2043, 4090, 8186, 16378, 16384])
+@pytest.mark.parametrize("extra", [0, 1, -1])
+def test_rows_that_start_inside_a_line(chunks, extra, alpha, dtype):
+    """Whole and ragged rows around the lengths where the places in front of a row's first 16-byte chunk, up to its 128-byte line, take it to the
+    next kernel or are not there, on buffers that start one chunk behind a line, forward and backward; nothing outside is touched.
+    Tolerances as in the tests above."""
+    from adasplash_amd import _lib
+    per = 16 // torch.empty(0, dtype=dtype).element_size()
+    rows, cols = 9, chunks * per + extra
+    g = torch.Generator().manual_seed(cols)
+    x0 = (3 * torch.randn(rows, cols, generator=g)).to(dtype)
+    dy0 = torch.randn(rows, cols, generator=g).to(dtype)
+    bufs = [torch.full((rows * cols + 2 * per,), 7.0, device=DEV, dtype=dtype) for _ in range(4)]
+    x, y, dy, dx = (b[per:per + rows * cols].view(rows, cols) for b in bufs)
+    x.copy_(x0)
+    dy.copy_(dy0)
+    lib, stream = _lib.load(), _lib.current_stream(x.device)
+    assert lib.adsp_entmax_rows_fwd(x.data_ptr(), y.data_ptr(), rows, cols, _lib.dtype_code(x), alpha, 2, 1, 0, stream) == 0
+    assert lib.adsp_entmax_rows_bwd(y.data_ptr(), dy.data_ptr(), dx.data_ptr(), rows, cols, _lib.dtype_code(x), alpha, stream) == 0
+    assert max_err(y, exact.entmax_rows(x0, alpha)) < tol_for(dtype, alpha)
+    want = _rows_backward_reference(y, dy0, alpha)
+    tol = (1e-5 if alpha == 1.5 else 1e-4) if dtype == torch.float32 else 1e-2
+    assert (dx.double().cpu() - want).abs().max().item() < tol * max(1.0, want.abs().max().item())
+    for b in bufs:
+        assert (b[:per] == 7.0).all() and (b[per + rows * cols:] == 7.0).all()
+
+
 def test_more_short_ragged_rows_than_a_grid_of_row_blocks_holds():
     """2^28 rows of 7: sixteen threads a row would be a launch of 2^32 threads, which HIP refuses; forward and backward."""
     rows, cols = 1 << 28, 7
