@@ -74,37 +74,50 @@ static int launch_bwd_dense(const AttnBwdParams& p, int D, int dtype, int am, in
 }
 
 // e4m3 copy of K for the first walk of the sparse-support forward: [B * Hkv][Npad][D] bytes in the order of K, values
-// beyond the format's range saturated, rows from N on zero.  A thread converts 16 values.  Heads the probe has marked
-// as dense are skipped (`hints`: two words per head).  The values are multiplied by the head's power of two first
-// (`w1_scales`, from the probe).
-// What bounds it is memory: tiles that lie wholly behind a sequence's length, which no walk reads, are left out (8 x 8 heads, N <= 8192, D = 128: 32 -> 22 us).
-// (the first walk's operands lie on a grid of 1/16, see attn_sparse_kernel.h)
-#define G16(x) (((x) * ak + 786432.f) - 786432.f)
-template <typename T>
-__global__ __launch_bounds__(256) void k8_layout_kernel(const uint16_t* __restrict__ k, unsigned char* __restrict__ k8, int N,
-                                                       int Npad, int D, int Hkv, const void* varlen, int varlen_bits,
-                                                       const uint32_t* hints, const float* w1_scales) {
-  const size_t head = blockIdx.y;
-  long long L = N;
-  if (varlen) L = varlen_bits == 64 ? ((const long long*)varlen)[head / Hkv] : (long long)((const int*)varlen)[head / Hkv];
-  if (hints[2 * head] >= (1u << 20)) return;
-  const float ak = w1_scales[4 * head + 1];
-  const int per_row = D / 16;
-  const long long id = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (id >= (long long)Npad * per_row) return;
-  const int row = (int)(id / per_row), c = (int)(id % per_row);
-  if (row / kBN * kBN >= L) return;
-  u32x4 out = {0u, 0u, 0u, 0u};
-  if (row < N) {
-    const uint16_t* src = k + (head * (size_t)N + row) * D + c * 16;
-    const u32x4 lo = *reinterpret_cast<const u32x4*>(src), hi = *reinterpret_cast<const u32x4*>(src + 8);
-#pragma unroll
-    for (int e = 0; e < 4; e += 2) {
-      out[e >> 1] = cvt_e4m3_pair(G16(unpack_lo<T>(lo[e + 1])), G16(unpack_hi<T>(lo[e + 1])), cvt_e4m3_pair(G16(unpack_lo<T>(lo[e])), G16(unpack_hi<T>(lo[e])), 0u, false), true);
-      out[2 + (e >> 1)] = cvt_e4m3_pair(G16(unpack_lo<T>(hi[e + 1])), G16(unpack_hi<T>(hi[e + 1])), cvt_e4m3_pair(G16(unpack_lo<T>(hi[e])), G16(unpack_hi<T>(hi[e])), 0u, false), true);
+// beyond the format's range saturated, rows from N on zero.  The values are multiplied by the head's power of two first
+// (`ak`, from the probe) and lie on the first walk's grid of 1/16 (see attn_sparse_kernel.h).
+// A thread converts 16 values at a time: element `id` of the head's rows.
+template <typename T, int D>
+struct K8Copy {
+  const u32x4* src;  // the head's rows, 8 values a piece
+  u32x4* dst;
+  long long rows, n;  // of K; of the copy: whole tiles of the sequence's length
+  u32x4 lo, hi;
+  __device__ K8Copy(const uint16_t* k, unsigned char* k8, size_t head, int N, int Npad, int L)
+      : src(reinterpret_cast<const u32x4*>(k + head * (size_t)N * D)), dst(reinterpret_cast<u32x4*>(k8 + head * (size_t)Npad * D)),
+        rows((long long)N * (D / 16)), n((long long)((L + kBN - 1) / kBN * kBN) * (D / 16)) {}
+  __device__ void load(long long id) {
+    lo = hi = u32x4{0u, 0u, 0u, 0u};
+    if (id < n && id < rows) {
+      lo = src[2 * id];
+      hi = src[2 * id + 1];
     }
   }
-  *reinterpret_cast<u32x4*>(k8 + (head * (size_t)Npad + row) * D + c * 16) = out;
+  __device__ void store(long long id, float ak) const {
+    if (id >= n) return;
+    auto on_grid = [ak](float x) { return (x * ak + 786432.f) - 786432.f; };
+    u32x4 out;
+#pragma unroll
+    for (int e = 0; e < 4; e += 2) {
+      out[e >> 1] = cvt_e4m3_pair(on_grid(unpack_lo<T>(lo[e + 1])), on_grid(unpack_hi<T>(lo[e + 1])), cvt_e4m3_pair(on_grid(unpack_lo<T>(lo[e])), on_grid(unpack_hi<T>(lo[e])), 0u, false), true);
+      out[2 + (e >> 1)] = cvt_e4m3_pair(on_grid(unpack_lo<T>(hi[e + 1])), on_grid(unpack_hi<T>(hi[e + 1])), cvt_e4m3_pair(on_grid(unpack_lo<T>(hi[e])), on_grid(unpack_hi<T>(hi[e])), 0u, false), true);
+    }
+    dst[id] = out;
+  }
+};
+
+// The copy by itself, behind the probe: a thread to 16 values.  Heads the probe has marked as dense are skipped.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void k8_layout_kernel(AttnParams p) {
+  const int u = blockIdx.y;
+  long long L = p.N;
+  if (p.varlen) L = p.varlen_bits == 64 ? ((const long long*)p.varlen)[u / p.Hkv] : (long long)((const int*)p.varlen)[u / p.Hkv];
+  L = L < 0 ? 0 : (L > p.N ? p.N : L);
+  if (p.hints[2 * u] >= (1u << 20)) return;
+  K8Copy<T, D> copy(reinterpret_cast<const uint16_t*>(p.k), const_cast<unsigned char*>(p.k8), (size_t)u, p.N, p.Npad, (int)L);
+  const long long id = (long long)blockIdx.x * 256 + threadIdx.x;
+  copy.load(id);
+  copy.store(id, p.w1_scales[4 * u + 1]);
 }
 
 static int npad_of(int N) { return (N + kBN - 1) / kBN * kBN; }
@@ -126,81 +139,70 @@ static int mask_words_of(int N) { return ((N + kBN - 1) / kBN + 31) / 32; }
 // them.  The prediction only decides which kernel does the work (a row block it gets wrong is caught by the kernel's
 // own checks), and it depends on the inputs alone: the same call takes the same way every time.
 //
-// What bounds it is latency, one workgroup per K/V head in front of the real work: the sampled keys' rows are all under way
-// before the query rows are waited for, and the length whose predicted support just fits comes from the support point instead
+// What bounds it is latency, one workgroup per K/V head in front of the real work: the sampled keys' rows and the query rows are
+// all under way at once, and the length whose predicted support just fits comes from the support point instead
 // of the other way round -- a lane takes an a, n(a) = 1 / (mass above a per key) and support n(a) Q(a) are closed forms that
 // grow with a, and a second look between the two neighbouring lanes refines it (bisecting a for 64 lengths
 // took 14 rounds, each an integral of 32 terms at a generic alpha).  192 heads, D = 64: 10.7 -> 6.7 us a launch.
 //
-// In front of a backward it clears the control words and flags of the dK/dV kernels as well (`ctrl2`, `kv_flags`).
+// (all 256 threads; `first`: writes what it finds; `share` as in the kernel below, written by thread 0)
 template <typename T, int D>
-__global__ __launch_bounds__(256) void attn_probe_kernel(AttnParams p, int am, uint32_t* ctrl2, int32_t* kv_flags) {
-  __shared__ __align__(16) float qrows[4][D];
+__device__ __forceinline__ void probe_head(const AttnParams& p, int am, int u, int L, bool first, float* share) {
   __shared__ float red[4][2][4];
   __shared__ float ksum[4];
-  const int u = blockIdx.x, tid = threadIdx.x;
-  const int units = p.B * p.Hkv;
-  uint32_t* const ctrl = p.queue;
+  const int tid = threadIdx.x;
   const int b = u / p.Hkv, kvh = u % p.Hkv, group = p.Hq / p.Hkv;
-  int L = p.N;
-  if (p.varlen) {
-    long long l = p.varlen_bits == 64 ? ((const long long*)p.varlen)[b] : (long long)((const int*)p.varlen)[b];
-    L = (int)(l < 0 ? 0 : (l > p.N ? p.N : l));
-  }
-  if (u == 0 && tid < 11) ctrl[tid] = 0u;
-  if (u == 0 && tid < 2) ctrl[64 + 2 * units + tid] = 0u;
-  if (tid < 2) ctrl[64 + 2 * u + tid] = 0u;
-  if (ctrl2 && u == 0 && tid < 11) ctrl2[tid] = 0u;
-  if (kv_flags) {
-    const int n_mblk = (p.N + kMaskRows - 1) / kMaskRows;
-    for (int i = tid; i < n_mblk; i += 256) kv_flags[(size_t)u * n_mblk + i] = 0;
-  }
-  if (p.save_flags)  // supports kept for the backward: no row block of this K/V head has a valid stream yet
-    for (int i = tid; i < group * p.n_mblk; i += 256) p.save_flags[(size_t)(b * p.Hq + kvh * group) * p.n_mblk + i] = 0;
-  if (p.w1_scales && tid < 4) p.w1_scales[4 * u + tid] = tid < 2 ? 1.f : (tid == 2 ? INFINITY : 0.f);
   if (L < 256) return;  // short sequences: finding out in the kernel costs little
-  int rows[4];
+  // Lanes side by side read a row's pieces of 16 bytes, so a load is whole lines; the sums over a row's lanes leave each lane with one
+  // key's scores.  (A row to a lane made each load 64 lines, which several workgroups on a CU pay for one after another: 64 heads, D = 128, 11.7 -> 9.4 us a launch; with the copy of 32 workgroups a head 6 us less.)
+  constexpr int P = D / 8;  // pieces of a row, and loads of 64 / P rows a wave
+  const int lane = tid & 63, piece = lane % P;
+  const int last_row = L - 1 - 3 * (L / 16);
+  const int span = (p.causal ? last_row + 1 : L);
+  const u32x4* kg = reinterpret_cast<const u32x4*>(p.k) + (size_t)(b * p.Hkv + kvh) * p.N * P + piece;
+  u32x4 kw[P], qw[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) rows[j] = L - 1 - j * (L / 16);
-  const int span = (p.causal ? rows[3] + 1 : L);
-  const int key = (int)(((long long)tid * span) / 256);
-  const u32x4* krow = reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p.k) + ((size_t)(b * p.Hkv + kvh) * p.N + key) * D);
-  u32x4 kw[D / 8];
+  for (int i = 0; i < P; ++i) kw[i] = kg[(size_t)(((long long)((tid & ~63) + i * (64 / P) + lane / P) * span) / 256) * P];
+  const u32x4* qg = reinterpret_cast<const u32x4*>(p.q) + (size_t)(b * p.Hq + kvh * group) * p.N * P + piece;
 #pragma unroll
-  for (int c = 0; c < D / 8; ++c) kw[c] = krow[c];
-  const uint16_t* qbase = reinterpret_cast<const uint16_t*>(p.q) + ((size_t)(b * p.Hq + kvh * group) * p.N) * D;
-#pragma unroll
-  for (int x = 0; x < 4 * D / 256; ++x) {
-    const int i = x * 256 + tid, j = i / D;
-    const uint32_t w = qbase[(size_t)(L - 1 - j * (L / 16)) * D + i % D];
-    qrows[j][i % D] = elem_traits<T>::kIsBf16 ? bf16_bits_to_float(w) : f16_bits_to_float(w);
-  }
-  __syncthreads();
-  float dot[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < 4; ++j) qw[j] = qg[(size_t)(L - 1 - j * (L / 16)) * P];
+  float dot[P][4];
   float ksq = 0.f;
 #pragma unroll
-  for (int c = 0; c < D / 8; ++c) {
-    __builtin_amdgcn_sched_barrier(0);  // (all of the query rows' LDS reads ahead of the first product would not fit the registers)
+  for (int i = 0; i < P; ++i) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dot[i][j] = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float lo = unpack_lo<T>(kw[c][e]), hi = unpack_hi<T>(kw[c][e]);
+      const float lo = unpack_lo<T>(kw[i][e]), hi = unpack_hi<T>(kw[i][e]);
       ksq = fmaf(lo, lo, fmaf(hi, hi, ksq));
 #pragma unroll
-      for (int j = 0; j < 4; ++j) dot[j] = fmaf(lo, qrows[j][8 * c + 2 * e], fmaf(hi, qrows[j][8 * c + 2 * e + 1], dot[j]));
+      for (int j = 0; j < 4; ++j) dot[i][j] = fmaf(lo, unpack_lo<T>(qw[j][e]), fmaf(hi, unpack_hi<T>(qw[j][e]), dot[i][j]));
     }
   }
 #pragma unroll
+  for (int h = P / 2; h > 0; h >>= 1) {
+    const bool upper = (lane & h) != 0;
+#pragma unroll
+    for (int i = 0; i < h; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float keep = upper ? dot[i + h][j] : dot[i][j], give = upper ? dot[i][j] : dot[i + h][j];
+        dot[i][j] = keep + __shfl_xor(give, h, 64);
+      }
+  }
+#pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const float z = dot[j] * p.qscale;
+    const float z = dot[0][j] * p.qscale;
     const float s1 = wave_sum(z), s2 = wave_sum(z * z);
-    if ((tid & 63) == 0) {
+    if (lane == 0) {
       red[tid >> 6][0][j] = s1;
       red[tid >> 6][1][j] = s2;
     }
   }
   {
     const float ks = wave_sum(ksq);
-    if ((tid & 63) == 0) ksum[tid >> 6] = ks;
+    if (lane == 0) ksum[tid >> 6] = ks;
   }
   __syncthreads();
   if (tid == 0 && p.w1_scales) {
@@ -215,8 +217,11 @@ __global__ __launch_bounds__(256) void attn_probe_kernel(AttnParams p, int am, u
       float ak = exp2f(rintf(log2f(8.f / (sqrtf((float)D) * k_rms))));
       ak = fminf(fmaxf(ak, 0x1p-40f), 0x1p40f);
       float aq = fminf(fmaxf(a / ak, 0x1p-40f), 0x1p40f);
-      p.w1_scales[4 * u] = aq;
-      p.w1_scales[4 * u + 1] = ak;
+      if (first) {
+        p.w1_scales[4 * u] = aq;
+        p.w1_scales[4 * u + 1] = ak;
+      }
+      share[0] = ak;
     }
   }
   if (tid >= 64) return;
@@ -278,8 +283,66 @@ __global__ __launch_bounds__(256) void attn_probe_kernel(AttnParams p, int am, u
   // lists outweighs the walks saved, and a launch split between the two kernels took 15 % longer than the dense kernel
   // alone.)  A marked head: the copy of K skips it and the sparse-support kernels leave its row blocks to the dense ones.
   const bool fits_all = n_fit >= (float)L;
-  if (p.w1_scales) p.w1_scales[4 * u + 2] = fits_all ? INFINITY : 0.f;
-  if (!fits_all) ctrl[64 + 2 * u] = 1u << 20;
+  if (p.w1_scales && first) p.w1_scales[4 * u + 2] = fits_all ? INFINITY : 0.f;
+  if (!fits_all) {
+    if (first) p.queue[64 + 2 * u] = 1u << 20;
+    share[1] = 1.f;
+  }
+}
+
+// In front of a backward it clears the control words and flags of the dK/dV kernels as well (`ctrl2`, `kv_flags`).
+//
+// COPY, in front of a forward: gridDim.y workgroups look at a head, each to the same result, the first of them writes it, and
+// all of them go on with the e4m3 copy of the head's K (none where the head is marked; tiles that lie wholly behind a
+// sequence's length, which no walk reads, are left out).  A launch and the
+// wait for the probe's end are saved by that; where and how it is worth it: launch_probe_as.
+template <typename T, int D, bool COPY>
+__global__ __launch_bounds__(256) void attn_probe_kernel(AttnParams p, int am, uint32_t* ctrl2, int32_t* kv_flags) {
+  __shared__ float share[2];  // COPY: k's scale; nonzero where the head is marked
+  const int u = blockIdx.x, tid = threadIdx.x;
+  const int units = p.B * p.Hkv;
+  uint32_t* const ctrl = p.queue;
+  const int b = u / p.Hkv, kvh = u % p.Hkv, group = p.Hq / p.Hkv;
+  const bool first = !COPY || blockIdx.y == 0;
+  int L = p.N;
+  if (p.varlen) {
+    long long l = p.varlen_bits == 64 ? ((const long long*)p.varlen)[b] : (long long)((const int*)p.varlen)[b];
+    L = (int)(l < 0 ? 0 : (l > p.N ? p.N : l));
+  }
+  if (first) {
+    if (u == 0 && tid < 11) ctrl[tid] = 0u;
+    if (u == 0 && tid < 2) ctrl[64 + 2 * units + tid] = 0u;
+    if (tid < 2) ctrl[64 + 2 * u + tid] = 0u;
+    if (ctrl2 && u == 0 && tid < 11) ctrl2[tid] = 0u;
+    if (kv_flags) {
+      const int n_mblk = (p.N + kMaskRows - 1) / kMaskRows;
+      for (int i = tid; i < n_mblk; i += 256) kv_flags[(size_t)u * n_mblk + i] = 0;
+    }
+    if (p.save_flags)  // supports kept for the backward: no row block of this K/V head has a valid stream yet
+      for (int i = tid; i < group * p.n_mblk; i += 256) p.save_flags[(size_t)(b * p.Hq + kvh * group) * p.n_mblk + i] = 0;
+    if (p.w1_scales && tid < 4) p.w1_scales[4 * u + tid] = tid < 2 ? 1.f : (tid == 2 ? INFINITY : 0.f);
+  }
+  if constexpr (COPY) {
+    K8Copy<T, D> copy(reinterpret_cast<const uint16_t*>(p.k), const_cast<unsigned char*>(p.k8), (size_t)u, p.N, p.Npad, L);
+    long long id = (long long)blockIdx.y * 256 + tid;
+    copy.load(id);  // (under way while the probe works)
+    if (tid == 0) {
+      share[0] = 1.f;
+      share[1] = 0.f;
+    }
+    probe_head<T, D>(p, am, u, L, first, share);
+    __syncthreads();
+    const float ak = share[0];
+    if (share[1] != 0.f) return;
+    const long long step = (long long)gridDim.y * 256;
+    for (; id - tid < copy.n; id += step) {
+      K8Copy<T, D> now = copy;
+      copy.load(id + step);
+      now.store(id, ak);
+    }
+  } else {
+    probe_head<T, D>(p, am, u, L, true, share);
+  }
 }
 
 // Workspace of the forward for the 16-bit types, for the head dims the sparse-support kernel serves: its work
@@ -333,15 +396,40 @@ __global__ __launch_bounds__(256) void fill_zero_kernel(int32_t* x, long long n)
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) x[i] = 0;
 }
 
-// the kernel for the head dims the sparse-support kernels serve
-static void launch_probe(const AttnParams& p, int D, int dtype, int am, uint32_t* ctrl2, int32_t* kv_flags, hipStream_t s) {
-  const dim3 grid((unsigned)(p.B * p.Hkv));
-  if (dtype == ADSP_BF16) {
-    if (D == 64) hipLaunchKernelGGL((attn_probe_kernel<bf16_t, 64>), grid, dim3(256), 0, s, p, am, ctrl2, kv_flags);
-    else hipLaunchKernelGGL((attn_probe_kernel<bf16_t, 128>), grid, dim3(256), 0, s, p, am, ctrl2, kv_flags);
+// The probe, and in front of a forward (COPY) the e4m3 copy of K, for the head dims the sparse-support kernels serve.
+constexpr long long kCopyPieces = 4096;  // pieces of 256 threads x 16 values that the probe's own workgroups copy
+template <typename T, int D, bool COPY>
+static void launch_probe_as(const AttnParams& p, int am, uint32_t* ctrl2, int32_t* kv_flags, hipStream_t s) {
+  const long long units = (long long)p.B * p.Hkv;
+  if constexpr (COPY) {
+    const long long pieces = ((long long)p.Npad * (D / 16) + 255) / 256;
+    // Up to 32 MiB of K the probe's workgroups copy it.  About one to a CU: looking at a head again costs each of them the sample's loads (2 x 32/8
+    // heads, N = 2048, D = 128: forward 150 us with the copy behind the probe, 146.5 with 256 workgroups, 147.2 with 512, 152 with 1024), and more, to
+    // what a CU holds, once eight pieces and more are left to each.  The forward, copy behind the probe against this: 32/8 heads, N = 2048, D = 128
+    // 98.4 -> 93.6; 8 heads, N = 4096, D = 64 116.4 -> 113.0; 4 x 16 heads 329 -> 326 (16 MiB).  For larger K the copy
+    // wants more bytes in flight than these workgroups have: 4 x 16 heads, N = 4096, D = 128 (64 MiB) 304 -> 309; 8 x 8 heads, N <= 8192 2223 -> 2250.
+    if (units * pieces <= kCopyPieces) {
+      long long parts = (255 + units) / units;
+      const long long more = pieces / 8 < 768 / units ? pieces / 8 : 768 / units;
+      parts = parts > more ? parts : more;
+      parts = parts < pieces ? parts : pieces;
+      hipLaunchKernelGGL((attn_probe_kernel<T, D, true>), dim3((unsigned)units, (unsigned)parts), dim3(256), 0, s, p, am, ctrl2, kv_flags);
+      return;
+    }
+    hipLaunchKernelGGL((attn_probe_kernel<T, D, false>), dim3((unsigned)units), dim3(256), 0, s, p, am, ctrl2, kv_flags);
+    hipLaunchKernelGGL((k8_layout_kernel<T, D>), dim3((unsigned)pieces, (unsigned)units), dim3(256), 0, s, p);
   } else {
-    if (D == 64) hipLaunchKernelGGL((attn_probe_kernel<f16_t, 64>), grid, dim3(256), 0, s, p, am, ctrl2, kv_flags);
-    else hipLaunchKernelGGL((attn_probe_kernel<f16_t, 128>), grid, dim3(256), 0, s, p, am, ctrl2, kv_flags);
+    hipLaunchKernelGGL((attn_probe_kernel<T, D, false>), dim3((unsigned)units), dim3(256), 0, s, p, am, ctrl2, kv_flags);
+  }
+}
+template <bool COPY>
+static void launch_probe(const AttnParams& p, int D, int dtype, int am, uint32_t* ctrl2, int32_t* kv_flags, hipStream_t s) {
+  if (dtype == ADSP_BF16) {
+    if (D == 64) launch_probe_as<bf16_t, 64, COPY>(p, am, ctrl2, kv_flags, s);
+    else launch_probe_as<bf16_t, 128, COPY>(p, am, ctrl2, kv_flags, s);
+  } else {
+    if (D == 64) launch_probe_as<f16_t, 64, COPY>(p, am, ctrl2, kv_flags, s);
+    else launch_probe_as<f16_t, 128, COPY>(p, am, ctrl2, kv_flags, s);
   }
 }
 
@@ -556,13 +644,7 @@ static int attn_common(const void* q, const void* k, const void* v, void* out, f
         p.save_tshift = (float*)(sp + sl.tshift_off);
         p.save_streams = sp + sl.streams_off;
       }
-      const dim3 k8_grid((unsigned)(((long long)p.Npad * (D / 16) + 255) / 256), (unsigned)(B * Hkv));
-      launch_probe(p, D, dtype, am, nullptr, nullptr, s);
-      if (dtype == ADSP_BF16) {
-        hipLaunchKernelGGL(k8_layout_kernel<bf16_t>, k8_grid, dim3(256), 0, s, (const uint16_t*)k, ws + w.k8_off, N, p.Npad, D, Hkv, varlen, varlen_bits, (const uint32_t*)p.hints, (const float*)p.w1_scales);
-      } else {
-        hipLaunchKernelGGL(k8_layout_kernel<f16_t>, k8_grid, dim3(256), 0, s, (const uint16_t*)k, ws + w.k8_off, N, p.Npad, D, Hkv, varlen, varlen_bits, (const uint32_t*)p.hints, (const float*)p.w1_scales);
-      }
+      launch_probe<true>(p, D, dtype, am, nullptr, nullptr, s);
       int rc = dtype == ADSP_BF16 ? (D == 64 ? launch_attn_sparse_bf16_d64(p, am, w.slots, s) : launch_attn_sparse_bf16_d128(p, am, w.slots, s))
                                   : (D == 64 ? launch_attn_sparse_f16_d64(p, am, w.slots, s) : launch_attn_sparse_f16_d128(p, am, w.slots, s));
       if (rc != 0) return ADSP_ERR_LAUNCH;
@@ -910,7 +992,7 @@ static int attn_bwd_impl(const void* q, const void* k, const void* v, const void
       pp.queue = p.queue;
       pp.hints = p.hints;
       pp.probe_max_support = probe_max_support();
-      launch_probe(pp, D, dtype, am, (uint32_t*)(ws + w.queue2_off), (int32_t*)(ws + w.kvflags_off), s);
+      launch_probe<false>(pp, D, dtype, am, (uint32_t*)(ws + w.queue2_off), (int32_t*)(ws + w.kvflags_off), s);
       int rc;
       if (dtype == ADSP_BF16) {
         rc = D == 64 ? launch_attn_bwd_sparse_bf16_d64(p, am, 0, w.slots, s) : launch_attn_bwd_sparse_bf16_d128(p, am, 0, w.slots, s);

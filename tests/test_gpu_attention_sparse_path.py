@@ -288,3 +288,29 @@ def test_two_waves_or_one_for_32_rows(dtype, B, H, N, D, alpha, causal, lens):
         for h in (0, H - 1):
             want = oracle_rows_of_attention(q, k, v, b, h, rows, alpha, causal, L)
             assert max_err(out[b, h, rows], want) < 2e-2 and max_err(out_b[b, h, rows], want) < 2e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,N,D,causal,lens", [
+    (4, 32, 700, 64, True, [700, 256, 255, 1]),  # two workgroups a head, eleven pieces; sequences the probe does not look at
+    (2, 20, 1990, 128, False, [1990, 1025]),     # eight of eight pieces
+    (1, 9, 8192, 64, True, None),                # 29, of four and five
+])
+def test_k_copied_by_the_probe_or_behind_it(dtype, B, H, N, D, causal, lens):
+    """Up to 32 MiB of K the probe's workgroups copy it to 8 bits, beyond that a kernel of its own: the same problem by itself and as the
+    first item of a batch that crosses the line (both with more than 512 row blocks).  The copy is the same bytes either way, and so is all that follows."""
+    q, k, v = qkv(B, H, H, N, D, dtype, seed=N + D)
+    q[:, 1] *= 0.02  # flat: left to the dense kernel where the probe looks
+    k[:, 2] *= 8.0
+    varlen = torch.tensor(lens or [N] * B, dtype=torch.int32)
+    version = 2 if causal else 1
+    out, tau, _ = forward(q, k, v, varlen, version, 1.5, causal)
+    copies = 2 ** 25 // (q.numel() * q.element_size()) + 1
+    out_b, tau_b, _ = forward(*[x.repeat(copies, 1, 1, 1) for x in (q, k, v)], varlen.repeat(copies), version, 1.5, causal)
+    for b in range(B):
+        L = int(varlen[b])
+        assert torch.equal(out[b], out_b[b]) and torch.equal(out[b], out_b[b - B])
+        assert torch.equal(tau[b, :, :L], tau_b[b, :, :L])
+        rows = sorted({0, L // 3, L - 1})
+        for h in (1, 2, H - 1):
+            assert max_err(out[b, h, rows], oracle_rows_of_attention(q, k, v, b, h, rows, 1.5, causal, L)) < 2e-2
