@@ -456,9 +456,22 @@ static bool bwd_streams_enabled() {
 // With a causal mask the kernel on the dQ kernel's streams serves the key blocks from this share (in 256ths) of a
 // sequence on with one item for all query heads of a K/V head (attn_bwd_dkdv_stream_kernel).  ADSP_DKDV_MERGE256 in the
 // environment overrides it (0: every key block per query head, with partial rows; for comparisons and tests).
-static int dkdv_merge256() {
+// Where the line lies: in units of the first key block's item, whose queries are a head's all, the longest merged item is
+// group * (1 - share), and a workgroup's part of the launch (two of them a CU) half of the row blocks / 512.  Merging saves partial rows, so it
+// starts as early as it can without an item that takes longer than the rest of the launch, or than the first key block's, which is there anyway; not before
+// 80 / 256, where long launches do best.  Training steps with 80 / 256 against
+// this, D = 128: 32/8 heads, N = 2048 346 -> 320 us, 16/4, N = 4096 456 -> 413, 32/8, N = 8192 1266 -> 1255; D = 64: 2 x 16/2, N = 2048 396 -> 246, 2 x 16/1, N = 4096
+// 906 -> 434, 4 x 16/4, N <= 1500 286 -> 252.  (224 throughout: 4 x 32/8, N <= 3000, D = 128 945 -> 983, which this leaves at 80.)
+static int dkdv_merge256(int B, int Hq, int Hkv, int N) {
   const char* e = getenv("ADSP_DKDV_MERGE256");
-  int v = e ? atoi(e) : 80;
+  int v = 80;
+  if (e) {
+    v = atoi(e);
+  } else {
+    const double part = (double)B * Hq * mblocks_of(N) / 1024.0, longest = part > 1.0 ? part : 1.0;
+    const double share = 256.0 * (1.0 - longest * Hkv / Hq);
+    if (share > v) v = (int)share;
+  }
   return v < 0 ? 0 : (v > 256 ? 256 : v);
 }
 
@@ -803,7 +816,7 @@ static BwdWorkspace bwd_workspace(int B, int Hq, int Hkv, int N, int D, int dtyp
     w.part_off = align256(w.scratch_off + (size_t)slots * 4 * 32 * 2 * D * 4);
     // (with one query head per K/V head the kernel on the streams writes dK and dV itself: no partial rows; with a
     // causal mask it does so for the key blocks it merges, and the others start in front of N * merge256 / 256)
-    w.merge256 = (bwd_streams_enabled() && causal && Hq != Hkv) ? dkdv_merge256() : 0;
+    w.merge256 = (bwd_streams_enabled() && causal && Hq != Hkv) ? dkdv_merge256(B, Hq, Hkv, N) : 0;
     w.part_rows = N;
     if (w.merge256 > 0) {
       const long long bound = ((long long)N * w.merge256 + 255) / 256;

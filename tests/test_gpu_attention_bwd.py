@@ -210,6 +210,23 @@ def test_dkdv_from_the_dq_kernels_streams_and_from_its_own_walk(alpha, causal, B
         assert max_err(a, b.float().cpu(), report=False) < grad_tol(dtype)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,dtype,lens", [
+    (2, 8, 2, 1100, 64, torch.bfloat16, [1100, 700]),
+    (1, 16, 1, 1000, 128, torch.float16, [1000]),
+    (3, 4, 2, 129, 128, torch.bfloat16, [129, 128, 1]),
+])
+def test_merge_border_of_short_launches(monkeypatch, B, Hq, Hkv, N, D, dtype, lens):
+    """The border that a short launch gets by default (three quarters of the sequence and more for these groups, half for two heads): the oracle's
+    gradients, and those of the border at 80 / 256 up to the order of fp32 sums and one rounding."""
+    varlen = torch.tensor(lens, dtype=torch.int32)
+    monkeypatch.delenv("ADSP_DKDV_MERGE256", raising=False)
+    got, want = run_case(1.5, True, B, Hq, Hkv, N, D, dtype, varlen=varlen, version=2, seed=12)
+    check(got, want, dtype)
+    monkeypatch.setenv("ADSP_DKDV_MERGE256", "80")
+    for a, b in zip(got, run_case(1.5, True, B, Hq, Hkv, N, D, dtype, varlen=varlen, version=2, seed=12)[0]):
+        assert max_err(a, b.float().cpu(), report=False) < 0.25 * grad_tol(dtype)
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,N,D,dtype,lens,with_oracle,scale", [
     (2, 8, 2, 1024, 64, torch.bfloat16, [1024, 700], True, 1.0),   # 4 heads x 1024 rows: one 16-bit list entry names any of them
     (1, 4, 1, 3000, 128, torch.float16, [2777], True, 1.0),

@@ -209,6 +209,19 @@ def test_backward_workspace_for_a_causal_call_follows_the_merge_border(monkeypat
             assert lib.adsp_attn_bwd_workspace_bytes_causal(B, Hq, Hq, N, D, _lib.ADSP_BF16, 1) == lib.adsp_attn_bwd_workspace_bytes(B, Hq, Hq, N, D, _lib.ADSP_BF16)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,N,m256", [
+    (1, 32, 8, 2048, 192), (1, 16, 4, 8192, 192), (1, 16, 4, 8320, 190),    # up to 1024 row blocks: as long as the first key block's item
+    (2, 16, 1, 4096, 240), (2, 16, 2, 2048, 224), (1, 32, 8, 8192, 128),
+    (1, 4, 2, 2048, 128), (4, 16, 8, 4096, 80), (8, 32, 8, 8192, 80), (64, 32, 8, 8192, 80),
+])
+def test_merge_border_of_short_launches(monkeypatch, B, Hq, Hkv, N, m256):
+    """Without ADSP_DKDV_MERGE256 the border lies at 80 / 256, or so that a merged item is no longer than a workgroup's part of the launch."""
+    monkeypatch.delenv("ADSP_DKDV_MERGE256", raising=False)
+    got = _lib.load().adsp_attn_bwd_workspace_bytes_causal(B, Hq, Hkv, N, 64, _lib.ADSP_BF16, 1)
+    monkeypatch.setenv("ADSP_DKDV_MERGE256", str(m256))
+    assert got == _lib.load().adsp_attn_bwd_workspace_bytes_causal(B, Hq, Hkv, N, 64, _lib.ADSP_BF16, 1)
+
+
 def test_which_training_steps_need_no_tile_mask():
     """Both sides of every line of the rule that sends short 16-bit training steps to the kernels on 32 rows."""
     lib = _lib.load()
