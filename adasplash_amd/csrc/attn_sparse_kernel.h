@@ -518,6 +518,9 @@ __global__ __launch_bounds__(256 * KP) __attribute__((amdgpu_waves_per_eu(ADSP_S
       t3 = n3;
       t4 = n4;
     };
+    // (KP = 2: as many tiles of a row block are through after half the steps.  The maximum of fewer keys is lower and more lie near it: two thirds instead of
+    // half.  2 x 16 heads, N = 1024, D = 128, alpha = 2, flat, whose parts have eight steps: training 282 us with one wave, 330 without this, 272 with it.)
+    constexpr int kFlat = 6 / KP, kFlatCnt = KP == 1 ? 6 * 128 / 2 : 3 * 128 * 2 / 3;
     int near_cnt = 0;
     const uint32_t near_d = (uint32_t)fminf(0.25f * inv_qs * 16.f * aqk, 8191.f) << 15;
     walk(std::integral_constant<int, SG::kStages8>{}, std::integral_constant<int, SG::kK8Tile>{}, std::integral_constant<int, kK8Per>{}, issue_k8, [&](int step, int kt, const unsigned char* kt_lds) {
@@ -533,10 +536,10 @@ __global__ __launch_bounds__(256 * KP) __attribute__((amdgpu_waves_per_eu(ADSP_S
         const uint32_t k1 = (((b1 >> 9) & 0x3fffu) << 15) | ((b1 & 15u) | ((uint32_t)(2 * kt + 1) << 4));
         keep_top(k0);
         keep_top(k1);
-        if (step >= 6 && step < 12) {
+        if (step >= kFlat && step < 2 * kFlat) {
           const uint32_t near = t1 > near_d ? t1 - near_d : 0u;
           near_cnt += __builtin_popcountll(__builtin_amdgcn_ballot_w64(live && k0 > near)) + __builtin_popcountll(__builtin_amdgcn_ballot_w64(live && k1 > near));
-          if (step == 11 && near_cnt > 6 * 128 / 2 && lane == 0) s_giveup[1] = 1u;
+          if (step == 2 * kFlat - 1 && near_cnt > kFlatCnt && lane == 0) s_giveup[1] = 1u;
         }
       });
     });
@@ -566,10 +569,12 @@ __global__ __launch_bounds__(256 * KP) __attribute__((amdgpu_waves_per_eu(ADSP_S
     // ---- the scores of the row's eight chosen keys from the 16-bit inputs: both lanes of a row hold half of its query and read the same half of the
     // chosen key, two-term dot products add them up.  (The diagonal of a matrix product had the same scores for 256 cycles of the matrix
     // pipe a key, and as many instructions to pick them: 8 x 32/8 heads, N <= 8192, D = 128: 2296 -> 2258 us; what is left is the rows' way out of L2.) ----
-    // (KP = 2: a wave scores the two best keys of each of its lanes, the row's eight meet in LDS)
-    float r[8];
+    // (KP = 2: a wave scores the three best keys of each of its lanes, the row's twelve meet in LDS.  Two of each of the four lanes are a worse choice than
+    // four of each of two: the candidates were 8 % more, and row blocks whose lists were nearly full with one wave overflowed: 4 heads, N = 16184, D = 64, a training step 659 us with one wave, 1898 with two keys a lane, 533 with three.)
+    constexpr int kChosen = KP == 1 ? 8 : 12;
+    float r[kChosen];
     {
-      constexpr int kR = 4 / KP;  // keys a lane has scored
+      constexpr int kR = kChosen / 2 / KP;  // keys a lane has scored
       // The rows of the chosen keys are gathered into LDS the way the walks' tiles get there: per product m the wave
       // loads a 32-row "tile" whose row i is the key that row i chose as its m-th, with 1 KB DMA instructions (a
       // group of kC lanes per key row: whole rows, coalesced), and reads the A fragments from it as from a K tile.
@@ -632,31 +637,34 @@ __global__ __launch_bounds__(256 * KP) __attribute__((amdgpu_waves_per_eu(ADSP_S
 #pragma unroll
         for (int m = 0; m < 8; ++m) r[m] = mine[m];
       } else {
-        static_assert(KP == 2 && SG::kRingBytes >= 1024, "the values lie behind the table, in the ring's place");
-        f32x4* const meet = reinterpret_cast<f32x4*>(lds_all + SG::kRingsAt + wave * SG::kRingBytes + 512);
-        constexpr int kOther = NW * SG::kRingBytes / 16;  // from a wave's values to those of the other part's wave
-        if (lh == 0) meet[part * kOther + lq] = f32x4{mine[0], mine[1], mine[2], mine[3]};
-        __syncthreads();
-        const f32x4 x0 = meet[lq], x1 = meet[kOther + lq];
+        constexpr int kTable = 2 * kR * 32 * 4;  // bytes
+        static_assert(KP == 2 && SG::kRingBytes >= 2 * kTable, "the values lie behind the table, in the ring's place");
+        float* const meet = reinterpret_cast<float*>(lds_all + SG::kRingsAt + wave * SG::kRingBytes + kTable);  // [2 kR][32]
+        constexpr int kOther = NW * SG::kRingBytes / 4;  // from a wave's values to those of the other part's wave
+        if (lh == 0) {
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          r[m] = x0[m];
-          r[4 + m] = x1[m];
+          for (int m = 0; m < 2 * kR; ++m) meet[part * kOther + m * 32 + lq] = mine[m];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < 2 * kR; ++m) {
+          r[m] = meet[m * 32 + lq];
+          r[2 * kR + m] = meet[kOther + m * 32 + lq];
         }
       }
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the last fragment reads are done before the tiles of walk 2 arrive
     }
     float lo_raw;
     {
-      float rmax = fmaxf(r[0], r[4]);
-      if constexpr (KP > 1) rmax = fmaxf(rmax, fmaxf(r[2], r[6]));
+      float rmax = fmaxf(r[0], r[kChosen / 2]);  // (a lane's best is its first)
+      if constexpr (KP > 1) rmax = fmaxf(rmax, fmaxf(r[kChosen / 4], r[kChosen * 3 / 4]));
       float t = rmax - inv_qs;
       const float target = (AM == ATT_15) ? inv_qs * inv_qs : inv_qs;
 #pragma unroll 1
       for (int it = 0; it < 8; ++it) {
         float a0 = 0.f, a1 = 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < kChosen; ++i) {
           const float u = fmaxf(r[i] - t, 0.f);
           if constexpr (AM == ATT_15) {
             a0 = fmaf(u, u, a0);

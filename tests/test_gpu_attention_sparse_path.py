@@ -290,6 +290,18 @@ def test_two_waves_or_one_for_32_rows(dtype, B, H, N, D, alpha, causal, lens):
             assert max_err(out[b, h, rows], want) < 2e-2 and max_err(out_b[b, h, rows], want) < 2e-2
 
 
+@pytest.mark.parametrize("H,N,D", [(4, 16184, 64), (3, 16384, 128)])
+def test_two_waves_keep_what_one_wave_keeps(H, N, D):
+    """Long rows whose candidates nearly fill the lists (32 rows of 20 members and more): with two waves the bound has to be as close as with one, or row blocks
+    are given up that would fit.  A row block's flag in the kept supports says that it was served; heads the probe leaves to the dense kernel have none."""
+    q, k, v = qkv(1, H, H, N, D, torch.float16, seed=1)
+    sup = _attention.launch_forward(q.to(DEV), k.to(DEV), v.to(DEV), version=2, alpha=1.5, is_causal=True, niter=1,
+                                    varlen=torch.tensor([N], dtype=torch.int32, device=DEV), keep_supports="always")[3]
+    served = sup.view(torch.uint8)[:H * ((N + 127) // 128) * 4].view(torch.int32).view(H, -1) != 0
+    taken = served.any(1)
+    assert taken.any() and served[taken].all(), (~served).sum(1).tolist()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,H,N,D,causal,lens", [
     (4, 32, 700, 64, True, [700, 256, 255, 1]),  # two workgroups a head, eleven pieces; sequences the probe does not look at
