@@ -212,7 +212,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       t = fmaxf(t + step, t_min);
       if (__builtin_amdgcn_ballot_w64(fabsf(step) > (all_sampled ? 2e-4f : 2e-2f)) == 0ull) break;
     }
-    flat = many >= 224.f;
+    // (f16's last step has to be smaller, and unless a third of the keys are members a quarter's is too far off for it, so that a walk over all follows: 4 x 16 heads, N = 2048, D = 64, not
+    // causal, q of spread 1/8 (a quarter of the keys): 225 us with the parts, 188 without; of spread 1/32 (three quarters) 158 and 184; 16 heads, N = 8192, spread 1/32 (two fifths) 526 and 657)
+    flat = many >= (elem_traits<T>::kIsBf16 ? 224.f : fmaxf(224.f, 0.3f * (float)(lim + 1)));
   }
 
   // ---- walks over the tiles next(-1), next of that, ... below n ----
