@@ -70,21 +70,6 @@ template <> __device__ __forceinline__ void dot2_chunk<f16_t>(float (&acc)[8], u
   ADSP_DOT2_CHUNK("v_dot2c_f32_f16");
 }
 #undef ADSP_DOT2_CHUNK
-// acc[i] += a[i].lo * b[i].lo + a[i].hi * b[i].hi for two 16-byte chunks of a row each, as one block for the same reason
-template <typename T> __device__ __forceinline__ void dot2_rows(float (&acc)[4], u32x4 a0, u32x4 b0, u32x4 a1, u32x4 b1);
-#define ADSP_DOT2_ROWS(OP)                                                                                              \
-  asm volatile(OP " %0, %4, %8\n\t" OP " %1, %5, %9\n\t" OP " %2, %6, %10\n\t" OP " %3, %7, %11\n\t"               \
-               OP " %0, %12, %16\n\t" OP " %1, %13, %17\n\t" OP " %2, %14, %18\n\t" OP " %3, %15, %19\n\ts_nop 3" \
-               : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3])                                                \
-               : "v"(a0[0]), "v"(a0[1]), "v"(a0[2]), "v"(a0[3]), "v"(b0[0]), "v"(b0[1]), "v"(b0[2]), "v"(b0[3]),       \
-                 "v"(a1[0]), "v"(a1[1]), "v"(a1[2]), "v"(a1[3]), "v"(b1[0]), "v"(b1[1]), "v"(b1[2]), "v"(b1[3]))
-template <> __device__ __forceinline__ void dot2_rows<bf16_t>(float (&acc)[4], u32x4 a0, u32x4 b0, u32x4 a1, u32x4 b1) {
-  ADSP_DOT2_ROWS("v_dot2c_f32_bf16");
-}
-template <> __device__ __forceinline__ void dot2_rows<f16_t>(float (&acc)[4], u32x4 a0, u32x4 b0, u32x4 a1, u32x4 b1) {
-  ADSP_DOT2_ROWS("v_dot2c_f32_f16");
-}
-#undef ADSP_DOT2_ROWS
 
 // two 16-byte chunks of e4m3 values as one operand of the fp8 MFMA (64 values of k per lane pair)
 typedef int i32x8 __attribute__((ext_vector_type(8)));
@@ -507,7 +492,7 @@ __global__ __launch_bounds__(256 * KP) __attribute__((amdgpu_waves_per_eu(ADSP_S
     // position in the block (4 bits); unsigned comparisons order the words by their sums.  Words whose sum field is
     // 0 (nothing seen, or only masked scores) stand for no key.
     // A flat score distribution (a support of hundreds of keys) shows early: most block maxima lie close to the
-    // running maximum.  Tiles 6 .. 11 (of each part) are counted; if more than half of their (lane, block) maxima lie within 1/4 (in
+    // running maximum.  Tiles 6 .. 11 (KP = 2: steps 3 .. 5 of each part) are counted; if more than half (KP = 2: two thirds) of their (lane, block) maxima lie within 1/4 (in
     // z) of the lane's running maximum, the row block is given up before the walk is over.  A heuristic that only
     // decides which kernel does the work.
     uint32_t t1 = 0u, t2 = 0u, t3 = 0u, t4 = 0u;
@@ -556,7 +541,7 @@ __global__ __launch_bounds__(256 * KP) __attribute__((amdgpu_waves_per_eu(ADSP_S
 #if ADSP_SPARSE_STOP == 1
     continue;
 #endif
-    // ---- lower bound of the row's threshold from its eight kept values (raw score units) --------------------
+    // ---- lower bound of the row's threshold from the scores of its chosen keys (raw score units) ------------
     // f(t) = qs^2 sum (r - t)_+^2 - 1 (alpha 1.5) or qs sum (r - t)_+ - 1 (alpha 2) is convex and decreasing and
     // f(max - 1 / qs) >= 0, so Newton from there approaches the subset's root from the left and never passes it.
     // ---- Q fragments of the 16-bit products ----------------------------------------------------------------------
@@ -566,9 +551,11 @@ __global__ __launch_bounds__(256 * KP) __attribute__((amdgpu_waves_per_eu(ADSP_S
 #pragma unroll
       for (int e = 0; e < 4; ++e) qf[ks * 4 + e] = live ? raw[e] : 0u;
     }
-    // ---- the scores of the row's eight chosen keys from the 16-bit inputs: both lanes of a row hold half of its query and read the same half of the
-    // chosen key, two-term dot products add them up.  (The diagonal of a matrix product had the same scores for 256 cycles of the matrix
-    // pipe a key, and as many instructions to pick them: 8 x 32/8 heads, N <= 8192, D = 128: 2296 -> 2258 us; what is left is the rows' way out of L2.) ----
+    // ---- the scores of the row's chosen keys (eight; KP = 2: twelve) from the 16-bit inputs, with the products of the second walk: in
+    // product m the A operand's row i is the key that row i chose as its m-th (a lane fetches its slice of that key's
+    // row from memory), so the diagonal of S^T holds the wanted scores, added up as the second walk adds them.  (Dot products of two terms took
+    // 2 % less of a large forward, 8 x 32/8 heads, N <= 8192, D = 128: 2258 us against 2296, but add in another order, and where large terms cancel no
+    // margin of the score's own size covers that: a bound above the threshold loses members.) ----
     // (KP = 2: a wave scores the three best keys of each of its lanes, the row's twelve meet in LDS.  Two of each of the four lanes are a worse choice than
     // four of each of two: the candidates were 8 % more, and row blocks whose lists were nearly full with one wave overflowed: 4 heads, N = 16184, D = 64, a training step 659 us with one wave, 1898 with two keys a lane, 533 with three.)
     constexpr int kChosen = KP == 1 ? 8 : 12;
@@ -598,6 +585,8 @@ __global__ __launch_bounds__(256 * KP) __attribute__((amdgpu_waves_per_eu(ADSP_S
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
+      const int diag = ((lq >> 3) << 2) | (lq & 3);  // which of the lane's 16 values of a block belongs to key lq of the block,
+      const bool diag_here = lh == ((lq >> 2) & 1);  // and which of the row's two lanes holds it
       const unsigned char* kg = uniform_ptr(kglob);
       const int grow = lane / KS::kC, gslot = lane % KS::kC;
       float mine[2 * kR];
@@ -618,18 +607,21 @@ __global__ __launch_bounds__(256 * KP) __attribute__((amdgpu_waves_per_eu(ADSP_S
           dma16s(kg, keys[j] * (uint32_t)G::kKRow + (uint32_t)((gslot ^ KS::sw(rr)) << 4), gtile + j * 1024);
         }
         __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the gathered tile is in LDS (this wave's own loads)
-        float acc[4] = {0.f, 0.f, 0.f, 0.f};
+        f32x16 acc;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
         uint32_t ka = (uint32_t)(uintptr_t)gtile + k_lane;
         asm volatile("" : "+v"(ka));
         u32x4 af[D / 16];
 #pragma unroll
         for (int ks = 0; ks < D / 16; ++ks) af[ks] = lds_read16(ka ^ (ks << 5));
 #pragma unroll
-        for (int ks = 0; ks < D / 16; ks += 2)
-          dot2_rows<T>(acc, af[ks], u32x4{qf[ks * 4], qf[ks * 4 + 1], qf[ks * 4 + 2], qf[ks * 4 + 3]}, af[ks + 1],
-                       u32x4{qf[ks * 4 + 4], qf[ks * 4 + 5], qf[ks * 4 + 6], qf[ks * 4 + 7]});
-        float d = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-        d += __shfl_xor(d, 32, 64);
+        for (int ks = 0; ks < D / 16; ++ks) acc = mfma_16bit<T>(af[ks], u32x4{qf[ks * 4], qf[ks * 4 + 1], qf[ks * 4 + 2], qf[ks * 4 + 3]}, acc);
+        float d = acc[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) d = diag == i ? acc[i] : d;
+        const float other = __shfl_xor(d, 32, 64);
+        d = diag_here ? d : other;
         const bool ok = ((m < kR) == (lh == 0)) ? okm[m % kR] : okp[m % kR];
         mine[m] = ok ? d : -INFINITY;
       }
@@ -684,9 +676,10 @@ __global__ __launch_bounds__(256 * KP) __attribute__((amdgpu_waves_per_eu(ADSP_S
         const float step = (AM == ATT_15) ? (a0 - target) / (2.f * a1) : (AM == ATT_2) ? (a0 - target) / a1 : (a0 - 1.f) * inv_qs / (p.c0 * a1);
         t += (a1 > 0.f && step > 0.f) ? step : 0.f;
       }
-      // the margin covers the rounding of the iteration and what the chosen keys' scores differ from the second walk's, which adds them up in another
-      // order; rows past the valid length take no part in walk 2
-      lo_raw = t - (1e-5f * inv_qs + 4e-6f * fabsf(rmax));
+      // the margin covers the rounding of the iteration, and for scores whose terms do not cancel by orders of magnitude that the second walk's sums start
+      // at -lo and the chosen keys' at 0 (terms of +-48^2 beside scores of some ten, D = 128: all rows; with +-64^2 one row of 80000 ends at lo, with +-256^2 one
+      // of 800, off by no more than their scores' own rounding); rows past the valid length take no part in walk 2
+      lo_raw = t - (1e-5f * inv_qs + 1e-6f * fabsf(rmax));
       // (a row none of whose chosen keys could be used -- its first walk's sums left the tags' range -- has no bound:
       // the row block goes to the dense kernel; the second walk stops at its first tile)
       if (live && !(rmax > -INFINITY)) s_giveup[1] = 1u;

@@ -290,6 +290,35 @@ def test_two_waves_or_one_for_32_rows(dtype, B, H, N, D, alpha, causal, lens):
             assert max_err(out[b, h, rows], want) < 2e-2 and max_err(out_b[b, h, rows], want) < 2e-2
 
 
+def kept(sup, H, N):
+    """Of supports kept for one batch item: which row blocks were served, and the rows' thresholds less their bounds (raw scores)."""
+    at = lambda n: (n + 255) // 256 * 256
+    items = H * ((N + 127) // 128)
+    first = at(at(4 * items) + 8 * items)
+    raw = sup.view(torch.uint8)
+    return raw[:4 * items].view(torch.int32).view(H, -1) != 0, raw[first:first + 4 * H * N].view(torch.float32).view(H, N)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H", [2, 40])  # two waves to 32 rows, and one
+def test_the_bound_is_below_the_threshold_where_large_terms_cancel(dtype, H):
+    """Scores of some ten with two terms of +-48^2 that cancel.  The bound comes from some keys' scores, summed as the second walk sums: summed in another order
+    they differ by 48^2 * 2^-24 and more, and a bound above the threshold leaves the row's solution on it.  Thresholds against 64 bits: eight
+    roundings of sums of 48^2, in units of z."""
+    N, D = 2048, 128
+    q, k, v = qkv(1, H, H, N, D, dtype, seed=5)
+    q *= 3
+    q[..., 0], q[..., 2], k[..., 0], k[..., 2] = 48.0, 48.0, 48.0, -48.0
+    _, tau, _, sup = _attention.launch_forward(q.to(DEV), k.to(DEV), v.to(DEV), version=2, alpha=1.5, is_causal=True, niter=1,
+                                               varlen=torch.tensor([N], dtype=torch.int32, device=DEV), keep_supports="always")
+    served, above = kept(sup, H, N)
+    assert served.all()
+    assert (above > 0).all(), int((above <= 0).sum())
+    for h in (0, H - 1):
+        _, _, want, _ = exact.dense_entmax_attention(q[:, h:h + 1], k[:, h:h + 1], v[:, h:h + 1], 1.5, True, None, return_aux=True)
+        assert (tau[0, h].double().cpu() - want[0, 0]).abs().max().item() < 8 * 48 ** 2 * 2.0 ** -24 * 0.5 / D ** 0.5
+
+
 @pytest.mark.parametrize("H,N,D", [(4, 16184, 64), (3, 16384, 128)])
 def test_two_waves_keep_what_one_wave_keeps(H, N, D):
     """Long rows whose candidates nearly fill the lists (32 rows of 20 members and more): with two waves the bound has to be as close as with one, or row blocks
