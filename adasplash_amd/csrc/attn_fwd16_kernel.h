@@ -347,7 +347,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __syncthreads();
     return (more_flag[0] | more_flag[1] | more_flag[2] | more_flag[3]) != 0u;
   };
-  float last_step = 0.f;
   if (!all_sampled) {
     bool done = false;
     if constexpr (kSet) {
@@ -378,9 +377,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           members += rn;
           ok = ok && in_range();
           if (ok) {
-            last_step = step_of(1.f, true);
-            ok = fabsf(last_step) <= near_of();
-            if (live) t += last_step;
+            const float step = step_of(1.f, true);
+            ok = fabsf(step) <= near_of();
+            if (live) t += step;
           }
           done = !any_wave(live && !ok);
         }
@@ -424,7 +423,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           step = mx * qs - 1.f;
         }
         if (live) t += step;
-        last_step = step;
         idle = __builtin_amdgcn_ballot_w64(live && fabsf(step) > fmaxf(near, 2e-6f)) == 0ull;
       }
       if (!any_wave(!idle)) break;
@@ -444,8 +442,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   f32x16 zero;
 #pragma unroll
   for (int i = 0; i < 16; ++i) zero[i] = 0.f;
-  // The sums at t, for the threshold that is kept.  alpha = 1.5: that of u^2 is the rounded weights' (some 1e-4 off, which moves the
-  // threshold by as much of the mean of u), that of u the last walk's less the step, without an instruction a score.
+  // The sums at t, in fp32, for the threshold that is kept.  (From the rounded weights' sum it would be off by up to 2e-3 of the mean of u in bf16: roundings cancel
+  // neither over a few members nor over equal ones.)
   float q0 = 0.f, q1 = 0.f;
   auto prob = [&](float x) -> float {
     // (within 1 but for the last step's remainder)
@@ -461,7 +459,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       e1 = fast_exp2(fast_log2(u) * (c0 - 1.f));  // (0 at 0)
       pr = e1 * u;
     }
-    if constexpr (kTaus && !kSet) {
+    if constexpr (kTaus) {
       q0 += pr;
       q1 += e1;
       asm volatile("" : "+v"(q0), "+v"(q1));  // (else the compiler gathers the terms of a block, in 36 registers)
@@ -528,8 +526,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       });
   const float zsum = total(zacc[0]);
   if constexpr (kTaus) {
-    q0 = kSet ? zsum : total(q0);
-    q1 = kSet ? s1 - members * last_step : total(q1);
+    q0 = total(q0);
+    q1 = total(q1);
     if (!all_sampled && q0 > 0.f && q1 > 0.f) t += f32path::norm_step<AM>(q0, q1, c0);
     if (live && lh == 0) p.taus[q_row0 + qi] = t;
   }

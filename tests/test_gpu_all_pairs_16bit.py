@@ -191,6 +191,27 @@ def test_thresholds_of_scores_that_are_not_normal(no_supports, scores, N, D, dty
     assert err.max() < 3 * UNIT[dtype], err.max()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("N", [300, 1100, 2309])
+@pytest.mark.parametrize("scores", ["normal", "equal", "few values"])
+def test_kept_thresholds_of_few_equal_and_many_members(no_supports, scores, N, D, dtype):
+    """The threshold that a backward reads is a factor on all of a row's weights.  Rows of one member up to all keys; against 64 bits, relative to the mean of u:
+    fp32 sums of N terms (N / 2 * 2^-24 at most) and what a last step leaves, 5e-3 at most, of which a step on the output walk's sums leaves the square."""
+    g = torch.Generator().manual_seed(N)
+    x = {"normal": torch.randn(N, generator=g), "equal": torch.ones(N), "few values": (8 * torch.rand(N, generator=g)).floor() / 8}[scores]
+    q, k, v, _, _ = problem(1, 1, 1, N, D, dtype, 1.0, [N])
+    q.zero_()
+    q[0, 0, :, 0] = torch.logspace(-1, 2, N).to(dtype)
+    k[0, 0, :, 0] = x.to(dtype)
+    tau = _attention.launch_forward(q.to(DEV), k.to(DEV), v.to(DEV), version=1, alpha=1.5, is_causal=False, niter=10, varlen=None)[1][0, 0].double().cpu()
+    rows = torch.arange(0, N, 3)
+    _, p, want, _ = exact.dense_entmax_attention(q[:, :, rows], k, v, 1.5, False, None, return_aux=True)
+    u = p[0, 0].double().sqrt()
+    err = (tau[rows] - want[0, 0].double()).abs() / (u.sum(1) / (u > 0).sum(1))
+    assert err.max() < N / 2 * 2.0 ** -24 + 2 * 5e-3 ** 2, err.max()
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("far", [640, 1099])
 def test_tile_mask_has_weights_too_small_for_the_sum(no_supports, far, D):
