@@ -431,6 +431,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 
   // ---- output ----
+  if (!live) t = INFINITY;  // rows behind the sequence's end are copies of its last, with thresholds that no walk has moved: no weights and no marks of theirs
   if (bmask)
     for (int i = tid; i < p.mask_words; i += 256) mask_lds[i] = 0u;
   f32x16 o[TL::kDB];

@@ -212,6 +212,22 @@ def test_kept_thresholds_of_few_equal_and_many_members(no_supports, scores, N, D
     assert err.max() < N / 2 * 2.0 ** -24 + 2 * 5e-3 ** 2, err.max()
 
 
+@pytest.mark.parametrize("alpha", [1.5, 1.333])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("key", [40, 300, 1030])
+def test_tile_mask_has_no_marks_of_rows_behind_the_end(no_supports, key, D, alpha):
+    """One key has all of the weight, and no first threshold's sample sees it.  The last row block has 76 rows, the others behind it
+    are loaded as copies of the last one and take no part in the walks."""
+    q, k = torch.zeros(1, 1, 1100, D), torch.zeros(1, 1, 1100, D)
+    q[..., 0] = 1.0
+    k[..., 0] = -64.0
+    k[:, :, key, 0] = 0.0
+    v = torch.randn(1, 1, 1100, D, generator=torch.Generator().manual_seed(1))
+    q, k, v = (t.to(DEV, torch.bfloat16) for t in (q, k, v))
+    bmask = _attention.launch_forward(q, k, v, version=1, alpha=alpha, is_causal=False, niter=10, varlen=None)[2].cpu()
+    assert (bmask == 1 << (key // 64)).all(), bmask
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("far", [640, 1099])
 def test_tile_mask_has_weights_too_small_for_the_sum(no_supports, far, D):
