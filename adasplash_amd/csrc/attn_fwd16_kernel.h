@@ -5,7 +5,7 @@
 // four products of 34 cycles a walk and three vector instructions a score).  So the number of walks over the keys is what counts.
 //
 // A row's threshold starts from a sample of 256 keys held in registers.  alpha = 1.5: from the sample's mean and spread, as if the scores were
-// normal, unless the sample contradicts it; the walks' steps know the members' number and the density where they end (set_step), so that one leaves the
+// normal, unless the sample contradicts it, then from the sample's own solution; the walks' steps know the members' number and the density where they end (set_step), so that one leaves the
 // cube of what there was, at the four instructions a score that the sums and the maximum took.  Where a row has hundreds of members, a quarter of the
 // tiles corrects the start, the others give a threshold, and the quarter's sums there go together with the others', moved as far
 // (move_sums): one and a quarter walks and the output's.  Fewer members: walks over all tiles until a step is small, mostly two; a wave whose rows are done
@@ -20,9 +20,10 @@
 // D = 128: 3530 -> 1270; 8 heads, N = 8192, alpha = 1.333: 2860 -> 1020, 3250 -> 1200; 4 x 16, N = 4096, alpha = 2: 2280 -> 1760, 3630 -> 2770 (there
 // the sums are piecewise linear and a step halves the support at best: five to eight walks).  Against 64 bits: bf16 2.3e-3 as before, f16 4.5e-4
 // -> 2.9e-4 at N = 6000.
-// alpha = 1.5, Newton's steps (sample, half, two and more walks) -> this, the same errors: 4 x 16 heads, N = 4096, not causal, q of spread 1/8 and 1/2: D = 64 724 -> 583,
-// 1151 -> 851, D = 128 1254 -> 973, 1957 -> 1425; 2 x 16 heads of up to 1100, 2100, 3000 and 9000, D = 64, 1/8: 49.7 -> 48.7, 98.2 -> 97.5, 151.5 -> 131, 1035 -> 764,
-// 1/2: 74.5 -> 68.9, 151 -> 145, 235 -> 197, 1547 -> 1186.  Rows of one key far above thousands of others had errors of up to 3.3e-2 and have 4e-3.
+// alpha = 1.5, Newton's steps (sample, half, two and more walks) -> this, 32 heads, N = 4096, not causal, scores (z) of spread 1/16, 1/8 and 1/4: D = 64 normal 379 -> 333, 490 ->
+// 403, 624 -> 519, even 374 -> 287, 382 -> 292, 370 -> 303, rising along the keys 359 -> 270, 361 -> 277, 358 -> 372; D = 128, 1/16 and 1/4: normal 662 -> 520, 931 -> 793, even 604 -> 463,
+// 599 -> 499.  Slower: a tenth of the keys in a cluster above the others, 1/4: 373 -> 423, log-normal 481 -> 532.  With a first threshold by the normal distribution wherever no key of
+// the sample was above it: even, 1/8 and 1/4: 686 and 670, D = 128, 1/4: 1044.  Rows of one key far above thousands of others had errors of up to 3.3e-2 and have 4e-3.
 #pragma once
 #include "attn_tile16.h"
 
@@ -41,7 +42,8 @@ using namespace tile16;
 template <typename T, int AM> constexpr float kNear = AM == ATT_15 ? (elem_traits<T>::kIsBf16 ? 0.22f : 0.15f) : 0.02f;
 // alpha = 1.5: steps from the sums of u^2 and u and the members' number.  With the same members the sum of u^2 is a parabola in the threshold; the
 // members that change are few, near u = 0, and their density there follows from the three sums (members_density: exact for u distributed evenly
-// and exponentially, and within 2 % for the upper part of a normal distribution).  What a step of x times the mean of u leaves of it, root of
+// and exponentially; for a normal distribution above a threshold 0.4 spreads over its mean and more within 2.5 %, at the mean 7 % too high, half a spread below it 18 %, a
+// spread below it 44 %: there most keys are members and few change).  What a step of x times the mean of u leaves of it, root of
 // mean square and the most of 256 rows of 575 members: x = 0.2: 2e-4 and 6e-4, 0.3: 5e-4 and 2e-3 (Newton's on the norm 9e-3 and 2e-2); of 62 members: 5e-4
 // and 2e-3, 1.5e-3 and 4e-3.  Where the parabola has no root nearby Newton's step on the norm is taken.
 __device__ __forceinline__ float members_density(float s0, float s1, float n) {
@@ -62,9 +64,9 @@ __device__ __forceinline__ void move_sums(float by, float& s0, float& s1, float&
   n = fmaf(-by, d, n);
 }
 // Where the threshold of n keys of normally distributed scores lies (alpha = 1.5), in spreads above their mean: n s^2 ((1 + a^2) Q(a) - a phi(a)) = 1,
-// within 0.15 from n s^2 = 0.2 to 5000.
+// within 0.16 from n s^2 = 0.2 to 20000, where the two pieces meet (0.03 from 2 on).
 __device__ __forceinline__ float normal_threshold(float ns2) {
-  return ns2 < 0.7f ? -__builtin_amdgcn_sqrtf(fmaxf(fast_rcp(ns2) - 1.f, 0.f)) : __builtin_amdgcn_sqrtf(fmaf(1.8f, fast_log2(ns2), 1.7f)) - 1.87f;
+  return ns2 < 0.82f ? -__builtin_amdgcn_sqrtf(fmaxf(fast_rcp(ns2) - 1.f, 0.f)) : __builtin_amdgcn_sqrtf(fmaf(1.8f, fast_log2(ns2), 1.7f)) - 1.87f;
 }
 constexpr int kSample = 256;  // keys of the sample that a row's first threshold comes from
 
@@ -129,7 +131,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   float t;  // in z units
   bool flat = false;  // hundreds of members, alpha = 1.5
   {
-    auto block_of = [&](int x) { return all_sampled ? x : (int)((long long)x * whole / (kSample / 32)); };  // block x of the sample
+    // block x of the sample (alpha = 1.5: in the middle of its eighth of the keys, for scores that rise or fall along the sequence)
+    auto block_of = [&](int x) { return all_sampled ? x : (int)((kSet ? (2ll * x + 1) * whole / 2 : (long long)x * whole) / (kSample / 32)); };
 #pragma unroll
     for (int i = 0; i < kSampleTiles; ++i)
       tl.issue_blocks(kg, [&](int r) {
@@ -172,7 +175,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const float mean = total(m1) * (qs / kSample), var = fmaxf(fmaf(-mean, mean, total(m2) * (qs * qs / kSample)), 0.f);
         const float a = normal_threshold(var * (float)(lim + 1)), guess = fmaf(a, spread = __builtin_amdgcn_sqrtf(var), mean);
         far_out = a > 1.7f;
-        keep = guess > t_min && guess < t_min + 1.f + (far_out ? spread : 0.f);  // (with the sample's maximum in view)
+        keep = guess > t_min && guess < t_min + 1.f;  // (below the sample's maximum)
         t = keep ? guess : t_min;
       }
     }
@@ -199,8 +202,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         // (the set's steps come from either side of the threshold; Newton's, from below, end in any case)
         step = it < 6 ? set_step(s0, s1, n, c0) : f32path::norm_step<AM>(s0, s1, c0);
         many = n;
-        // (the sample's own error is as large as the guess's: one that the sample does not contradict stays)
-        if (it == 0) keep = keep && (s1 > 0.f ? fabsf(step) <= (far_out ? spread : s0 * fast_rcp(s1)) : far_out);
+        // (the sample's own error is as large as the guess's: one that the sample does not contradict stays.  Far out a guess above the sample's
+        // solution, or without a key of the sample above it, may lie where no key is -- scores with an upper end -- and costs walks until it is found: there the
+        // sample's own solution is taken.)
+        if (it == 0) keep = keep && s1 > 0.f && (far_out ? step >= 0.f && step <= spread : fabsf(step) <= s0 * fast_rcp(s1));
         step = keep ? 0.f : (s1 > 0.f ? step : t_min - t);
       } else {
 #pragma unroll
@@ -260,10 +265,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   auto every = [](int cur) { return cur + 1; };
   auto mul = [&](int g, int k, const u32x4& a, f32x16& s) { s = mfma_16bit<T>(a, piece<D>(qf, 4 * (g % G) + k), s); };
 
-  // sums of u^c0 and u^(c0 - 1) above t, and their number (alpha = 1.5) or the maximum less t, over the tiles; in raw units of u for
-  // alpha = 1.5 and 2.  A score's sign goes into a word with those of the block's others, and the words' ones are counted.
+  // sums of u^c0 and u^(c0 - 1) above t, their number (alpha = 1.5) and the maximum less t (alpha = 1.5: only `with_top`), over the tiles; in raw
+  // units of u for alpha = 1.5 and 2.  A score's sign goes into a word with those of the block's others, and the words' ones are counted.
   float s0 = 0.f, s1 = 0.f, mx = -INFINITY, members = 0.f;
-  auto sums_walk = [&](auto&& next, int n) {
+  auto sums_walk = [&](auto with_top, auto&& next, int n) {
+    constexpr bool kTop = !kSet || decltype(with_top)::value;
     const float k0 = s0, k1 = s1, kn = members;
     s0 = s1 = 0.f;
     mx = -INFINITY;
@@ -272,15 +278,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const f32x16 from_t = splat(-t * inv_qs);
     f32x16 late = splat(-INFINITY);
     auto add = [&](float x) {
+      if constexpr (kTop) mx = fmaxf(mx, x);
       if constexpr (kSet) {
         const float u = __builtin_amdgcn_fmed3f(x, 0.f, INFINITY);
         s0 = fmaf(u, u, s0);
         s1 += u;
         signs = __builtin_amdgcn_alignbit(signs, __builtin_bit_cast(uint32_t, x), 31);
-        return;
-      }
-      mx = fmaxf(mx, x);
-      if constexpr (AM == ATT_2) {
+      } else if constexpr (AM == ATT_2) {
         s0 += __builtin_amdgcn_fmed3f(x, 0.f, INFINITY);
         s1 += x > 0.f ? 1.f : 0.f;
       } else {
@@ -316,7 +320,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     s0 = total(s0);
     s1 = total(s1);
     if constexpr (kSet) members = total((float)(count + 16 - __builtin_popcount(signs & 0xffffu)));
-    else mx = top(mx);
+    if constexpr (kTop) mx = top(mx);
     if constexpr (AM == ATT_15) {
       s0 *= qs * qs;
       s1 *= qs;
@@ -360,9 +364,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         auto second_part = [&](int cur) { return cur + 1 + ((cur & 3) == 0 && cur < n_first ? 1 : 0); };
         const int first_keys = n_first / 4 * kTR;
         const float keys = (float)(lim + 1);
-        sums_walk(first_part, n_first);
+        sums_walk(std::false_type{}, first_part, n_first);
         if (in_range()) t += step_of(keys / (float)first_keys, true);
-        sums_walk(second_part, nt);
+        sums_walk(std::false_type{}, second_part, nt);
         bool ok = in_range();
         if (!any_wave(live && !ok)) {
           const float by = step_of(keys / (float)((lim + 1) - first_keys), true);
@@ -371,7 +375,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           float r0 = s0, r1 = s1, rn = members;
           move_sums(by, r0, r1, rn);
           if (live) t += by;
-          sums_walk(first_part, n_first);
+          sums_walk(std::false_type{}, first_part, n_first);
           s0 += r0;
           s1 += r1;
           members += rn;
@@ -388,41 +392,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       // a step on every second tile, where that is much more than the sample
       const int half = whole * 32 / kTR / 2;
       if (half * kTR >= 2 * kSample) {
-        sums_walk([](int cur) { return cur + 2; }, half * 2);  // (1, 3, ..)
+        sums_walk(std::true_type{}, [](int cur) { return cur + 2; }, half * 2);  // (1, 3, ..)
         const float ratio = (float)(lim + 1) / (float)(half * kTR) * (AM == ATT_2 ? 0.9f : 1.f);
         if (in_range()) t += fmaxf(mx * qs - 1.f, step_of(ratio, false));
         else t += fmaxf(mx * qs - 1.f, 0.f);
       }
     }
+    // The first walk over all keys takes the maximum as well (an instruction a score): the threshold is at least that less 1, which is what brings rows of
+    // a few keys far above the sample near it, and where a row goes that a step has thrown above all of its keys.
+    float low = 0.f;  // that bound, less t
     for (int it = 0; it < 32 && !done; ++it) {
-      sums_walk(every, nt);
       if constexpr (kSet) {
-        if (any_wave(!idle && live && !in_range())) {
-          mx = -INFINITY;
-          auto maximum = [&](int blk, int k0) {
-            f32x16 s = splat(-t * inv_qs);
-            stream<G, 2>([&](int g, u32x4(&a)[4]) { tl.rows(0, blk, g, a); }, [&](int g, int k, const u32x4& a) { mul(g, k, a, s); });
-            if (k0 + 31 > lim_all) hide(k0, s);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
-          };
-          walk(every, nt, false, maximum, [&](int blk, int k0) {
-            maximum(blk, k0);
-            maximum(blk + 1, k0 + 32);
-          });
-          mx = top(mx);
-        }
+        if (it == 0) sums_walk(std::true_type{}, every, nt);
+        else sums_walk(std::false_type{}, every, nt);
+      } else {
+        sums_walk(std::true_type{}, every, nt);
       }
       if (!idle) {
-        float step, near = 0.f;
+        if (!kSet || it == 0) low = mx * qs - 1.f;
+        float step = low, near = 0.f;
         if (in_range()) {
-          step = step_of(1.f, it < 6);
-          if constexpr (!kSet) step = fmaxf(step, mx * qs - 1.f);  // (never below the row maximum less 1)
+          step = fmaxf(step, step_of(1.f, it < 6));
           near = near_of();
-        } else {
-          step = mx * qs - 1.f;
         }
         if (live) t += step;
+        low -= step;
         idle = __builtin_amdgcn_ballot_w64(live && fabsf(step) > fmaxf(near, 2e-6f)) == 0ull;
       }
       if (!any_wave(!idle)) break;

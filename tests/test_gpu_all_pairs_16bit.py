@@ -191,6 +191,32 @@ def test_thresholds_of_scores_that_are_not_normal(no_supports, scores, N, D, dty
     assert err.max() < 3 * UNIT[dtype], err.max()
 
 
+@pytest.mark.parametrize("scores", ["even", "rising"])
+def test_scores_with_an_upper_end_take_no_longer_than_normal_ones(no_supports, scores):
+    """Normal scores of spread 1/4 (about 70 members of 4096 keys) take about three walks over the keys in front of the output's, even ones of that spread (400 members)
+    two at most.  A start above all keys, where a normal distribution would have its members, took six: 1.35 to 1.4 times as long as the normal ones.
+    Bound: 1.15, for the clock's wandering."""
+    N, H, D = 4096, 32, 64
+    g = torch.Generator().manual_seed(3)
+    times = {}
+    for name in ("normal", scores):
+        x = {"normal": torch.randn(1, H, N, D, generator=g), "even": torch.rand(1, H, N, D, generator=g), "rising": (torch.arange(N) / N)[:, None].expand(1, H, N, D)}[name]
+        k = ((x - x.mean(2, keepdim=True)) / x.std(2, keepdim=True)).bfloat16().to(DEV)
+        q = torch.nn.functional.one_hot(torch.arange(N) % D, D).expand(1, H, N, D).mul(0.25 / 0.5 * D ** 0.5).bfloat16().to(DEV)  # (z: half of the scaled score)
+        v = torch.randn(1, H, N, D, generator=g).bfloat16().to(DEV)
+        took = []
+        for _ in range(8):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(4):
+                A.adasplash_v1(q, k, v, alpha=1.5, is_causal=False, niter=10)
+            end.record()
+            end.synchronize()
+            took.append(start.elapsed_time(end))
+        times[name] = min(took)
+    assert times[scores] < 1.15 * times["normal"], times
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("N", [300, 1100, 2309])
