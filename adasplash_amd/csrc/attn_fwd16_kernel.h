@@ -9,7 +9,7 @@
 // cube of what there was, at the four instructions a score that the sums and the maximum took.  Where a row has hundreds of members, a quarter of the
 // tiles corrects the start, the others give a threshold, and the quarter's sums there go together with the others', moved as far
 // (move_sums): one and a quarter walks and the output's.  Fewer members: walks over all tiles until a step is small, mostly two; a wave whose rows are done
-// no longer takes part.  Other alphas: Newton's steps on the sample, one on every second tile, one or two on all tiles (a step squares what is left).
+// no longer takes part.  The output walk checks what the steps left (kOff).  Other alphas: Newton's steps on the sample, one on every second tile, one or two on all tiles (a step squares what is left).
 // The output walk's own sums take the threshold that a backward reads one step further.
 //
 // Split: four waves of 32 rows, tiles of K (and V in the output walk) through two stages of LDS, two workgroups a CU; two blocks of a tile go
@@ -40,6 +40,13 @@ using namespace tile16;
 // the sums are as a normal distribution's upper part has them and keys are left to become members, otherwise by 1.5 times (by 2.5 always: rows of two clusters of scores, or of one key far above the others,
 // up to 4.7e-3 and 2e-2; by 2: 584 -> 645 us, D = 64).
 template <typename T, int AM> constexpr float kNear = AM == ATT_15 ? (elem_traits<T>::kIsBf16 ? 0.22f : 0.15f) : 0.02f;
+// What a density misjudges shows in the output walk's own sum of u^2, taken in fp32: where rows of a last step beyond kSure times (sum u^2 / sum u), or of sums that were
+// moved, have it kOff and more from 1, Newton's step from there is taken and the output walk done again, twice at most.  Scores of few values, whose members come and go
+// by hundreds (600 sets of 4 to 48 values, N = 1100 to 4096, a model of the kernel): the worst row's weights off by 4.0e-3 without this, bf16 1.4e-3 and f16 2.6e-4 with it, 1.5e-3 and 2.3e-4
+// with Newton's steps and the smaller limits.  Scores without such steps seldom need it.  32 heads, N = 4096, not causal, us without and with: D = 64 normal scores of spread 1/16 355 and 360, 1/4 481 and 489,
+// even 289 and 302, on 25 values 375 and 465; D = 128 normal 522 and 551, 764 and 767; N = 2048, D = 64, 1/16, where all row blocks run at once, 102 and 113.
+template <typename T> constexpr float kSure = elem_traits<T>::kIsBf16 ? 0.04f : 0.02f;
+template <typename T> constexpr float kOff = elem_traits<T>::kIsBf16 ? 1.5e-3f : 5e-4f;
 // alpha = 1.5: steps from the sums of u^2 and u and the members' number.  With the same members the sum of u^2 is a parabola in the threshold; the
 // members that change are few, near u = 0, and their density there follows from the three sums (members_density: exact for u distributed evenly
 // and exponentially; for a normal distribution above a threshold 0.4 spreads over its mean and more within 2.5 %, at the mean 7 % too high, half a spread below it 18 %, a
@@ -70,8 +77,8 @@ __device__ __forceinline__ float normal_threshold(float ns2) {
 }
 constexpr int kSample = 256;  // keys of the sample that a row's first threshold comes from
 
-template <typename T, int D, int AM, bool kTaus>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd16_kernel(AttnParams p) {
+// A row block.  Returns whether it has to be gone through again, from the output walk on (kOff; `turn`: how many times it has been).
+template <typename T, int D, int AM, bool kTaus> __device__ __forceinline__ bool row_block(const AttnParams& p, int turn) {
   constexpr int kTR = D == 64 ? 128 : 64;  // two stages of K and V in 64 KB either way: two workgroups a CU
   using TL = Tile<T, D, kTR>;
   constexpr int kRow = TL::kRow, kRows = kMaskRows, kBlk = kTR / 32, G = TL::kG;
@@ -80,20 +87,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr bool kSet = AM == ATT_15;  // steps with the members' number (set_step)
   __shared__ __align__(1024) unsigned char smem[4 * TL::kBytes];  // two stages of a K and a V tile
   __shared__ uint32_t more_flag[4];
+  __shared__ float slope_lds[kSet ? 256 : 1], t_lds[kSet ? 256 : 1];  // a lane's sum of u behind its last step, about, and its threshold, for another turn
   extern __shared__ uint32_t mask_lds[];  // the tile mask of the row block, where one is asked for
   const LeftOver left(p.block_flags, p.queue);
-  if (left.none()) return;
-  const int tid = threadIdx.x;
+  if (left.none()) return false;
+  int tid = threadIdx.x;
+  if constexpr (kSet) asm volatile("" : "+v"(tid));  // (nothing is kept in registers from turn to turn: D = 128's walks would spill, 10 % of the time)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
   const int N = p.N, group = p.Hq / p.Hkv, n_blk = (N + kRows - 1) / kRows;
   int bkv, mi, hg;
-  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_blk, group, p.causal != 0, 2ll * N * kRow, bkv, mi, hg)) return;
+  if (!xcd_block_map(p.varlen != nullptr, p.B * p.Hkv, n_blk, group, p.causal != 0, 2ll * N * kRow, bkv, mi, hg)) return false;
   const BatchItem item = batch_item(p.varlen, p.varlen_bits, p.B, N, bkv / p.Hkv, p.Hkv, n_blk * group, p.causal == 0, 2);
   const int b = item.b, L = item.L, kvh = bkv % p.Hkv, h = kvh * group + hg, bh = b * p.Hq + h;
   bkv = b * p.Hkv + kvh;
   const int mblk = n_blk - 1 - mi, m0 = mblk * kRows;
-  if (!left.takes((size_t)bh * p.n_mblk + mblk)) return;
+  if (!left.takes((size_t)bh * p.n_mblk + mblk)) return false;
   const size_t q_row0 = (size_t)bh * N;
   unsigned char* const out = reinterpret_cast<unsigned char*>(p.out) + q_row0 * kRow;
   int32_t* const bmask = p.bmask ? p.bmask + ((size_t)bh * p.n_mblk + mblk) * p.mask_words : nullptr;
@@ -101,7 +110,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     zero_rows(out + (size_t)m0 * kRow, (N - m0 < kRows ? N - m0 : kRows) * kRow, tid);
     if (bmask)
       for (int i = tid; i < p.mask_words; i += 256) bmask[i] = 0;
-    return;
+    return false;
   }
   const int wave_row0 = m0 + 32 * wave, qi = wave_row0 + lq;
   const bool live = qi < L;
@@ -128,9 +137,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // ---- a first threshold from a sample of the keys, or the threshold itself where the sample is all of them ----
   const int n_key_blk = (key_hi + 31) / 32;
   const bool all_sampled = n_key_blk * 32 <= kSample;
-  float t;  // in z units
+  float t = 0.f;  // in z units
   bool flat = false;  // hundreds of members, alpha = 1.5
-  {
+  if (turn == 0) {
     // block x of the sample (alpha = 1.5: in the middle of its eighth of the keys, for scores that rise or fall along the sequence)
     auto block_of = [&](int x) { return all_sampled ? x : (int)((kSet ? (2ll * x + 1) * whole / 2 : (long long)x * whole) / (kSample / 32)); };
 #pragma unroll
@@ -351,8 +360,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __syncthreads();
     return (more_flag[0] | more_flag[1] | more_flag[2] | more_flag[3]) != 0u;
   };
-  if (!all_sampled) {
-    bool done = false;
+  bool done = false;
+  bool far = turn != 0;  // the last step was beyond kSure, or the sums were moved (alpha = 1.5)
+  if (kSet && turn != 0) {
+    t = t_lds[tid];
+  } else if (!all_sampled) {
     if constexpr (kSet) {
       // A step on every fourth tile (the first part), one on the others, and one on all of them: the first part's sums at the threshold
       // that the second part gave, and the second's, which are known for the one before, moved there.  From 1792 keys on (at 1700 the quarter is too
@@ -384,8 +396,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const float step = step_of(1.f, true);
             ok = fabsf(step) <= near_of();
             if (live) t += step;
+            slope_lds[tid] = s1 - members * step;
           }
           done = !any_wave(live && !ok);
+          far = true;
         }
       }
     } else {
@@ -414,6 +428,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (in_range()) {
           step = fmaxf(step, step_of(1.f, it < 6));
           near = near_of();
+          far = kSet && fabsf(step) > kSure<T> * s0 * fast_rcp(s1);
+          if constexpr (kSet) slope_lds[tid] = s1 - members * step;
         }
         if (live) t += step;
         low -= step;
@@ -424,22 +440,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     idle = false;
   }
 
-  // ---- output ----
-  if (!live) t = INFINITY;  // rows behind the sequence's end are copies of its last, with thresholds that no walk has moved: no weights and no marks of theirs
-  if (bmask)
-    for (int i = tid; i < p.mask_words; i += 256) mask_lds[i] = 0u;
   f32x16 o[TL::kDB];
-#pragma unroll
-  for (int db = 0; db < TL::kDB; ++db)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) o[db][i] = 0.f;
-  f32x4_t zacc = {0.f, 0.f, 0.f, 0.f};  // the sum of the rounded weights, those that the product takes
+  f32x4_t zacc;  // the sum of the rounded weights, those that the product takes
   f32x16 zero;
 #pragma unroll
   for (int i = 0; i < 16; ++i) zero[i] = 0.f;
-  // The sums at t, in fp32, for the threshold that is kept.  (From the rounded weights' sum it would be off by up to 2e-3 of the mean of u in bf16: roundings cancel
-  // neither over a few members nor over equal ones.)
-  float q0 = 0.f, q1 = 0.f;
+  // The sums at t, in fp32, for the threshold that is kept, and alpha = 1.5 for whether t was right (kOff).  (From the rounded weights' sum it would be off by up to 2e-3 of the
+  // mean of u in bf16: roundings cancel neither over a few members nor over equal ones.)
+  float q0, q1;
   auto prob = [&](float x) -> float {
     // (within 1 but for the last step's remainder)
     const float u = __builtin_amdgcn_fmed3f(fmaf(x, qs, -t), 0.f, 1.f);
@@ -454,10 +462,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       e1 = fast_exp2(fast_log2(u) * (c0 - 1.f));  // (0 at 0)
       pr = e1 * u;
     }
-    if constexpr (kTaus) {
+    if constexpr (kTaus || kSet) {
       q0 += pr;
-      q1 += e1;
-      asm volatile("" : "+v"(q0), "+v"(q1));  // (else the compiler gathers the terms of a block, in 36 registers)
+      if constexpr (kTaus) {
+        q1 += e1;
+        asm volatile("" : "+v"(q0), "+v"(q1));  // (else the compiler gathers the terms of a block, in 36 registers)
+      } else {
+        asm volatile("" : "+v"(q0));
+      }
     }
     return pr;
   };
@@ -475,6 +487,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   auto mark = [&](uint32_t weights, int k0) {
     if (bmask && __builtin_amdgcn_ballot_w64(weights != 0u) != 0ull && lane == 0) atomicOr(&mask_lds[k0 >> 11], 1u << ((k0 >> 6) & 31));
   };
+  // ---- output ----
+  if (!live) t = INFINITY;  // rows behind the sequence's end are copies of its last, with thresholds that no walk has moved: no weights and no marks of theirs
+  if (bmask)
+    for (int i = tid; i < p.mask_words; i += 256) mask_lds[i] = 0u;
+#pragma unroll
+  for (int db = 0; db < TL::kDB; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[db][i] = 0.f;
+  zacc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  q0 = q1 = 0.f;
   walk(
       every, nt, true,
       [&](int blk, int k0) {
@@ -519,6 +541,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             });
         mark(any, k0);
       });
+  if constexpr (kSet) {
+    const float off = total(q0) - 1.f;
+    const bool wrong = live && far && fabsf(off) > kOff<T>;
+    if (turn < 2 && any_wave(wrong)) {
+      t_lds[tid] = wrong ? fmaf(0.5f * off, fast_rcp(slope_lds[tid]), t) : t;
+      return true;
+    }
+  }
   const float zsum = total(zacc[0]);
   if constexpr (kTaus) {
     q0 = total(q0);
@@ -531,6 +561,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   BwdTiles<T, D>::store_rows(o, inv, smem + wave * 32 * kRow, out, wave_row0, N, lane);
   if (bmask)
     for (int i = tid; i < p.mask_words; i += 256) bmask[i] = (int32_t)mask_lds[i];
+  return false;
+}
+
+template <typename T, int D, int AM, bool kTaus>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd16_kernel(AttnParams p) {
+  for (int turn = 0; row_block<T, D, AM, kTaus>(p, turn); ++turn) {
+  }
 }
 
 }  // namespace fwd16

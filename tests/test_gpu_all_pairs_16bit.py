@@ -191,6 +191,28 @@ def test_thresholds_of_scores_that_are_not_normal(no_supports, scores, N, D, dty
     assert err.max() < 3 * UNIT[dtype], err.max()
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("N", [1100, 2048, 4096])
+@pytest.mark.parametrize("values", [4, 7, 9, 15, 23, 39])
+def test_thresholds_of_scores_of_few_values(no_supports, values, N, D):
+    """Normal scores on a grid of 1 / values times three spreads: members come and go by hundreds, which the steps' densities do not expect.  Every row has a spread
+    of its own.  Bound, row by row: the weight's and the result's rounding, 2^-11 each at most -- equal weights round alike --, on average half of that, and as a root of squares
+    what is left of the threshold, sums off by 5e-4 and as much of the weights.  (f16: bf16's roundings alone reach 4.5e-3 here, as much as a wrong threshold.)"""
+    dtype = torch.float16
+    g = torch.Generator().manual_seed(values)
+    x = (values * torch.randn(N, generator=g) / 3).round() / values
+    q, k, v, dout, varlen = problem(1, 8, 8, N, D, dtype, 1.0, [N])
+    q.zero_()
+    k.zero_()
+    spread = torch.logspace(-1.7, 0.3, 8 * N)  # of the scores times 1/2
+    q[..., 0] = (spread * 2 * D ** 0.5 / x.std()).reshape(1, 8, N).to(dtype)
+    k[..., 0] = x.to(dtype)
+    got = run(q, k, v, dout, varlen, 1.5, False, train=False)[0].double().cpu()[:, :, ::37]
+    want = exact.dense_entmax_attention(q[:, :, ::37], k, v, 1.5, False, None).double()
+    err = (got - want).norm(dim=-1) / want.norm(dim=-1)
+    assert err.max() < 2 * UNIT[dtype], err.max()
+
+
 @pytest.mark.parametrize("scores", ["even", "rising"])
 def test_scores_with_an_upper_end_take_no_longer_than_normal_ones(no_supports, scores):
     """Normal scores of spread 1/4 (about 70 members of 4096 keys) take about three walks over the keys in front of the output's, even ones of that spread (400 members)
