@@ -576,9 +576,17 @@ inline bool rows_fit_grid(long long rows, long long nvec) {
 
 // The places that rows of `nvec` chunks ask for: where they do not start on a line, up to seven more, in front of the first chunk.  Rows of a few
 // hundred bytes do without where they have none to spare (32768 rows, bf16, 249 columns: 13.7 us with, 9.8 without; fp32, 125: 8.6, 7.7; beyond the line bf16,
-// 1019: 26.0, 30.1; fp32, 505: 23.6, 27.4).
+// 1019: 26.0, 30.1; fp32, 505: 23.6, 27.4).  So do longer ones where the seven would take them to an instance of as many threads and twice the chunks a thread, half of
+// them empty, or forward to the one of 1024 threads.  us, 96 MiB in bf16 and as many chunks in fp32, seven
+// places always -> so: bf16, 250 chunks 38.5 -> 35.0, and one column more 40.9 -> 36.0; 1018 37.4 -> 34.7; 8186 41.9 -> 36.6; backward fp32, 2042 and one column more 40.4 -> 37.7, bf16
+// 42.2 -> 39.0.  At the other lines the next instance has more threads: fp32, 125 chunks 43.3 with none, 34.3 with seven; 509 36.4, 34.4; 4093 40.1, 37.3; backward bf16, 8189 39.9, 37.3.
 constexpr long long kRowsShort = 64;
-inline long long rows_places(long long rows, long long nvec, int shape) { return shape == 1 && nvec > kRowsShort && rows_fit_grid(rows, nvec + 7) ? nvec + 7 : nvec; }
+inline long long rows_places(long long rows, long long nvec, int shape, bool backward) {
+  if (shape != 1 || nvec <= kRowsShort || !rows_fit_grid(rows, nvec + 7)) return nvec;
+  auto over = [nvec](long long line) { return nvec <= line && nvec + 7 > line; };
+  if (over(256) || over(1024) || over(2048) || (!backward && over(8192))) return nvec;
+  return nvec + 7;
+}
 
 // 0: the rows' chunks are aligned and fill them, and the rows start on 128-byte lines or are short; 1: they have edges, or start inside a line; 2: neither (bases that differ in their offset from a 16-byte
 // boundary, elements off their own alignment, very short ragged rows, more chunks than the registers hold, more rows than a
@@ -606,7 +614,7 @@ template <typename T, int AM> static void launch_fwd(const RowsParams& p, hipStr
     if (shape == 0) hipLaunchKernelGGL((entmax_rows_reg_kernel<T, AM, NC, TPR, false>), grid, block, 0, s, p);              \
     else hipLaunchKernelGGL((entmax_rows_reg_kernel<T, AM, NC, TPR, true>), grid, block, 0, s, p);                          \
   } while (0)
-  ADSP_ROWS_DISPATCH(rows_places(p.rows, p.cols / elem_traits<T>::kVec, shape), ADSP_ROWS_FWD);
+  ADSP_ROWS_DISPATCH(rows_places(p.rows, p.cols / elem_traits<T>::kVec, shape, false), ADSP_ROWS_FWD);
 }
 
 template <typename T, int AM>
@@ -624,7 +632,7 @@ static void launch_bwd(const void* y, const void* dy, void* dx, long long rows, 
     if (shape == 0) hipLaunchKernelGGL((entmax_rows_bwd_reg_kernel<T, AM, NC, TPR, false>), grid, block, 0, s, y, dy, dx, rows, cols, cf); \
     else hipLaunchKernelGGL((entmax_rows_bwd_reg_kernel<T, AM, NC, TPR, true>), grid, block, 0, s, y, dy, dx, rows, cols, cf);      \
   } while (0)
-  ADSP_ROWS_DISPATCH(rows_places(rows, cols / elem_traits<T>::kVec, shape), ADSP_ROWS_BWD);
+  ADSP_ROWS_DISPATCH(rows_places(rows, cols / elem_traits<T>::kVec, shape, true), ADSP_ROWS_BWD);
 }
 
 }  // namespace adsp

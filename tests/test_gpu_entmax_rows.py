@@ -274,6 +274,25 @@ def test_rows_that_start_inside_a_line(chunks, extra, alpha, dtype):
         assert (b[:per] == 7.0).all() and (b[per + rows * cols:] == 7.0).all()
 
 
+@pytest.mark.parametrize("few,many", [(246, 250), (8180, 8186)])
+def test_rows_that_nearly_fill_an_instance_take_as_long_as_shorter_ones(few, many):
+    """Rows with seven places to spare in their instance, and rows that would need the next one for them, whose threads are half empty there: as many bytes,
+    1.15 times as long.  Bound: 1.05, for the clock's wandering."""
+    took = {few: [], many: []}
+    x = {chunks: torch.empty((192 << 20) // (16 * chunks), chunks * 8 + 1, device=DEV).normal_().mul_(2).bfloat16() for chunks in took}
+    for _ in range(12):
+        for chunks in took:
+            A.triton_entmax(x[chunks])
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(4):
+                A.triton_entmax(x[chunks])
+            end.record()
+            end.synchronize()
+            took[chunks].append(start.elapsed_time(end))
+    assert min(took[many]) < 1.05 * min(took[few]), {k: min(v) for k, v in took.items()}
+
+
 def test_more_short_ragged_rows_than_a_grid_of_row_blocks_holds():
     """2^28 rows of 7: sixteen threads a row would be a launch of 2^32 threads, which HIP refuses; forward and backward."""
     rows, cols = 1 << 28, 7
