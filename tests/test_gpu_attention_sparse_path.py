@@ -332,6 +332,28 @@ def test_two_waves_keep_what_one_wave_keeps(H, N, D):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,N,D,alpha,causal,scale", [
+    (4, 640, 128, 1.5, False, 0.7),   # some row blocks of a head are served
+    (4, 2048, 64, 1.5, True, 1.0),
+    (4, 16384, 64, 1.5, False, 1.0),  # lists that are nearly full
+    (4, 16384, 128, 1.333, True, 2.0),
+    (3, 8192, 64, 2.0, False, 0.5),
+])
+def test_two_waves_serve_what_one_wave_serves(dtype, H, N, D, alpha, causal, scale):
+    """The same heads by themselves, with two waves to 32 rows, and as the first item of a batch of more than 512 row blocks, with one: no row block that one
+    wave serves is given up with two, by the flags in the kept supports."""
+    q, k, v = (t.to(DEV) for t in qkv(1, H, H, N, D, dtype, seed=N + D, scale=scale))
+    blocks = (N + 127) // 128
+    served = []
+    for copies in (1, 512 // (H * blocks) + 1):
+        varlen = torch.full((copies,), N, dtype=torch.int32, device=DEV)
+        sup = _attention.launch_forward(*[t.repeat(copies, 1, 1, 1) for t in (q, k, v)], version=2 if causal and alpha == 1.5 else 1, alpha=alpha,
+                                        is_causal=causal, niter=10, varlen=varlen, keep_supports="always")[3]
+        served.append(sup.view(torch.uint8)[:4 * H * blocks].view(torch.int32).view(H, blocks) != 0)
+    assert served[1].any() and not (served[1] & ~served[0]).any(), [int(x.sum()) for x in served]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,H,N,D,causal,lens", [
     (4, 32, 700, 64, True, [700, 256, 255, 1]),  # two workgroups a head, eleven pieces; sequences the probe does not look at
     (2, 20, 1990, 128, False, [1990, 1025]),     # eight of eight pieces
