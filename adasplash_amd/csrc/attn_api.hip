@@ -669,10 +669,10 @@ static int attn_common(const void* q, const void* k, const void* v, void* out, f
   }
   // All pairs, 16-bit types: where more than one solver step is asked for, or a step without the histogram, the kernel that starts
   // from a sample of the keys converges in one or two walks.  4 x 16 heads, N = 4096, D = 64, flat scores, not causal (ten steps allowed):
-  // 2240 -> 583 us; D = 128: 3530 -> 973; 8 heads, N = 8192, alpha = 1.333: 2860 -> 1020.  A single step behind the histogram, the causal
+  // 2240 -> 644 us; D = 128: 3530 -> 1067; 8 heads, N = 8192, alpha = 1.333: 2860 -> 1020.  A single step behind the histogram, the causal
   // entry point's default, stays with the kernel below: it is less exact (relative error 6.1e-3 against 2.3e-3, more for longer rows), but its results are those of
-  // one step, and of the times either kernel has the better ones: causal, 345 against 312 us, D = 128 580 against 531, but with q of spread 1/2 335 against 430 and
-  // 2 x 8 heads, N = 16384, D = 128 2110 against 2540.
+  // one step, and of the times either kernel has the better ones: causal, 391 against 391 us, D = 128 599 against 597, 2 x 8 heads, N = 16384, D = 128 2174 against 1980, but
+  // with q of spread 1/2 338 against 486.
   if (dtype != ADSP_F32 && (D == 64 || D == 128) && !tile_counts && alpha >= 1.125 && alpha <= 2.0 && (niter >= 2 || (niter == 1 && !use_hist))) {
     const int rc = ADSP_CALL_16(launch_attn_fwd16, D, dtype, p, am, s);
     return rc == 0 && hipGetLastError() == hipSuccess ? ADSP_OK : ADSP_ERR_LAUNCH;

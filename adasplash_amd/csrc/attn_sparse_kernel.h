@@ -1113,9 +1113,9 @@ template <typename T, int D, int AM, int KP> static int launch_attn_sparse_one(c
 
 // Two waves share 32 rows (KP = 2) in launches of up to 512 row blocks: two workgroups of eight waves a CU are then all of them at
 // once, where one wave for 32 rows leaves a CU eight waves and the launch lasts as long as the chain of stages of its longest item,
-// of which KP = 2 halves each.  us, KP = 1 -> 2, whole forwards, causal unless noted: 32/8 heads, N = 2048, D = 128, q of spread 1 and 3: 120 -> 100,
-// 92 -> 79; 16/8, N = 4096, D = 128: 184 -> 137; 8, N = 8192, D = 64: 575 -> 499 with the gradients; 2 x 16 of up to 2000, D = 64: 113 -> 87; 16, N = 4096, D = 64,
-// alpha = 2, full: 119 -> 102.  Beyond the line KP = 1 has its waves side by side anyway: 2 x 32/8, N = 2048, D = 128: 171 -> 214, 3 x 16, N = 2048, D = 64:
+// of which KP = 2 halves each.  us, KP = 1 -> 2 with all else the same, whole forwards, causal unless noted: 32/8 heads, N = 2048, D = 128, q of spread 1 and 3: 125 -> 104,
+// 88 -> 79; 16/8, N = 4096, D = 128: 178 -> 133; 8, N = 8192, D = 64: 430 -> 352 with the gradients; 2 x 16 of up to 2000, D = 64: 108 -> 83; 16, N = 4096, D = 64,
+// alpha = 2, full: 119 -> 105.  Beyond the line KP = 1 has its waves side by side anyway: 2 x 32/8, N = 2048, D = 128: 171 -> 214, 3 x 16, N = 2048, D = 64:
 // 122 -> 133, 16, N = 8192, D = 64: 597 -> 616 (f16).
 template <typename T, int D> static int launch_attn_sparse(const AttnParams& p, int am, int max_slots, hipStream_t s) {
   if ((long long)p.B * p.Hq * p.n_mblk <= 512) {
