@@ -349,7 +349,7 @@ template <typename T, int D, int AM, bool kTaus> __device__ __forceinline__ bool
     if constexpr (kSet) return set ? set_step(s0 * ratio, s1 * ratio, members * ratio, c0) : f32path::norm_step<AM>(s0 * ratio, s1 * ratio, c0);
     else return f32path::norm_step<AM>(s0 * ratio, s1 * ratio, c0);
   };
-  auto near_of = [&]() -> float {  // (few members have no density to go by)
+  auto near_of = [&]() -> float {  // (few members have no density to go by, and may have a bulk of keys just below their threshold: limits as wide as Newton's left errors of 1e-2 there)
     if constexpr (kSet) return kNear<T, AM> * s1 * fast_rcp(members) * __builtin_amdgcn_sqrtf(fminf(members * (1.f / 256.f), 1.f));
     else return kNear<T, AM> * s0 * fast_rcp(s1);
   };
